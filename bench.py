@@ -235,17 +235,15 @@ def compare(d, d_ref, diag):
 
 def packet_roofline(n, w, K, kernel_ms, kernel, traffic):
     """Roofline of a packet-traversal launch, priced on the bytes it must fetch: per wavefront,
-    each interior node record (32 K bytes: K child boxes, references and counts), each triangle
-    record it copies for evaluation (128 B), each culling-record load of the screen (4
-    triangles, 128 B) and each leaf-slab load (4 B), fetched once for the wavefront's 64
-    queries, plus per query its point (12 B) and its result (4 B). The counts come from the
+    each interior node record (the walk's 160-byte node), each triangle record it copies for evaluation (128 B) and each culling-record load of
+    the screen (4 triangles, 128 B), fetched once for the wavefront's 64 queries, plus per query its point (12 B) and its result (4 B). The counts come from the
     counting variant of the same launch (work[4], work[5], pair counters [2], [3]). The per-query figure beside it
     (every query's own node and triangle reads, 16 + 28 K per node + 36 per triangle) is what 64
     separate traversals would read; a packet shares those reads, so that figure is not an HBM
     rate and is reported for reference only. With w[8], w[9] (the pair counters) the evaluation
     work is reported too: (query, triangle) pairs per query, 64-lane evaluation batches per
     wavefront, and the share of batch lanes used."""
-    byts = 16 * n + w[4] * 32 * K + w[5] * 128 + (w[10] * 128 + w[11] * 4 if len(w) >= 12 else 0)
+    byts = 16 * n + w[4] * 160 + w[5] * 128 + (w[10] * 128 if len(w) >= 12 else 0)
     gbs = byts / (kernel_ms * 1e-3) / 1e9
     lane = 16 * n + w[0] * 28 * K + w[1] * 36
     return {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -471,7 +469,7 @@ def batched_bench(a):
                       "launch": "persistent" if plan.persistent else "one wavefront per packet",
                       "tune_ms": info["tune_ms"]},
            "graph_replay_ms": round(replay_ms, 3),
-           "roofline": packet_roofline(nq, c, K, kms, f"batch32_kernel<{K},{info['stack_capacity'] // 64},false,"
+           "roofline": packet_roofline(nq, c, K, kms, f"batch32_kernel<{info['stack_capacity'] // 64},false,"
                                        f"{str(plan.persistent).lower()}>",
                                        profiled_traffic("batch32", "batch32_many_meshes_256_counters.txt")),
            "correctness": {"sample": f"{checked} queries (200 strided of every 16th mesh) against the oracle",
@@ -521,7 +519,7 @@ def main():
     plain = lambda: mesh.query(qt, out=out)  # noqa: E731
     learned = lambda: mesh.query(qt, out=out_l, learned_bound=True)  # noqa: E731
     K = info["branching"]
-    kname = f"sdf32_kernel<{K},{info['stack_capacity'] // 64},false,{{mode}}>"
+    kname = f"sdf32_kernel<{info['stack_capacity'] // 64},false,{{mode}},false>"
 
     def work(**kw):
         w = torch.zeros(12, dtype=torch.int64, device=dev)  # work[0..7], then the pair counters

@@ -61,11 +61,9 @@ static double heavy_factor(uint64_t n) { return n >= (1u << 22) ? 6.0 : 3.0; }
 
 // Subtree roots for split packets: breadth-first from the root, each interior entry replaced by
 // its children until there are at least `target` roots (leaves stay as they are).
-template <int K>
-static std::vector<ebgpu::SplitRoot> split_frontier(const ebgpu::PackedMesh& pm, std::size_t target)
+static std::vector<ebgpu::SplitRoot> split_frontier(const ebgpu::WalkTree& wt, std::size_t target)
 {
-  const auto*                   nodes = reinterpret_cast<const ebgpu::Node<K>*>(pm.nodes.data());
-  std::vector<ebgpu::SplitRoot> cur{{0u, 0u, {pm.lo[0], pm.lo[1], pm.lo[2]}, {pm.hi[0], pm.hi[1], pm.hi[2]}}};
+  std::vector<ebgpu::SplitRoot> cur{{0u, 0u, {0u, 0u}}};
   while (cur.size() < target) {
     std::vector<ebgpu::SplitRoot> next;
     bool                          grew = false;
@@ -75,10 +73,10 @@ static std::vector<ebgpu::SplitRoot> split_frontier(const ebgpu::PackedMesh& pm,
         next.push_back(r);
         continue;
       }
-      const ebgpu::Node<K>& nd = nodes[r.ref];
-      for (int k = 0; k < K; k++) {
+      const ebgpu::WalkNode& nd = wt.nodes[r.ref];
+      for (int k = 0; k < 4; k++) {
         if (nd.cnt[k] == ebgpu::kInvalid) continue;
-        next.push_back({nd.ref[k], nd.cnt[k], {nd.lox[k], nd.loy[k], nd.loz[k]}, {nd.hix[k], nd.hiy[k], nd.hiz[k]}});
+        next.push_back({nd.ref[k], nd.cnt[k] & (ebgpu::kBoxChild - 1u), {0u, 0u}});
       }
       grew = true;
     }
@@ -159,15 +157,70 @@ static ebg_status adopt_gpu_mesh(ebg_mesh* m, ebgpu::GpuBuiltMesh& g)
   return finalize_mesh(m, g.meta);
 }
 
-// Split frontier, counts, stack banks, bounds and the device view of an uploaded mesh.
+// The FP32 walk's tree and records, from the packed tree and the device's vertex positions (the
+// same for every builder): topology and boxes on the host, cylinders and discs on the device.
+static ebg_status build_walk(ebg_mesh* m, const ebgpu::PackedMesh& pm)
+{
+  ebgpu::MeshDev& d = m->dev;
+  // squares and products of squares of lengths must stay within FP32's range: meshes whose size is
+  // far from 1 are scaled by a power of two (exact)
+  d.scale = 1.0f;
+  if (pm.diag > 0.0 && (pm.diag < 0x1p-8 || pm.diag > 0x1p24))
+    d.scale = float(std::ldexp(1.0, std::clamp(-std::ilogb(pm.diag), -126, 126)));
+  d.inv_scale = 1.0f / d.scale;
+
+  ebgpu::WalkTree wt;
+  ebgpu::build_walk_tree(pm, d.scale, wt);
+  m->wbanks = (wt.stack_need + 63) / 64;
+  if (m->wbanks > 4)
+    return fail(EBG_STACK_OVERFLOW, "tree needs a traversal stack of " + std::to_string(wt.stack_need) +
+                                      " entries (max 256); use a smaller branching factor");
+  if (m->wbanks == 3) m->wbanks = 4;
+  const std::vector<ebgpu::SplitRoot> roots = split_frontier(wt, kSplitRoots);
+  EBG_HIP(upload(m->split_roots, roots));
+  m->num_split_roots = uint32_t(roots.size());
+
+  std::vector<uint32_t> small, large;
+  std::vector<float>    none(8 * 4 * wt.nodes.size(), -1.0f);
+  for (uint32_t i = 0; i < 4 * wt.nodes.size(); i++) {
+    const uint32_t c = wt.range[2 * i + 1] - wt.range[2 * i];
+    if (c) (c > ebgpu::kWalkLarge ? large : small).push_back(i);
+  }
+  DevBuf range, ls, ll, discs, off;
+  EBG_HIP(upload(m->wnodes, wt.nodes));
+  EBG_HIP(upload(range, wt.range));
+  EBG_HIP(upload(ls, small));
+  EBG_HIP(upload(ll, large));
+  EBG_HIP(upload(discs, none));
+  EBG_HIP(upload(off, std::vector<uint32_t>(16, 0u)));
+  EBG_HIP(m->frames.reserve(sizeof(ebgpu::FrameRec) * std::max<uint64_t>(m->nt, 1)));
+  EBG_HIP(m->tdisc.reserve(sizeof(ebgpu::TriDisc) * (m->nt + ebgpu::kSphPad)));
+  EBG_HIP(ebgpu::launch_frames(d.tripos, m->nt, d.scale, m->frames.as<ebgpu::FrameRec>(), m->tdisc.as<ebgpu::TriDisc>(),
+                               off.as<uint32_t>(), nullptr));
+  EBG_HIP(ebgpu::launch_walk_nodes(d.tripos, range.as<uint32_t>(), ls.as<uint32_t>(), uint32_t(small.size()),
+                                   ll.as<uint32_t>(), uint32_t(large.size()), d.scale, discs.as<float>(),
+                                   m->wnodes.as<ebgpu::WalkNode>(), uint32_t(wt.nodes.size()), nullptr));
+  uint32_t bits = 0;
+  EBG_HIP(hipStreamSynchronize(nullptr));
+  EBG_HIP(hipMemcpy(&bits, off.p, 4, hipMemcpyDeviceToHost));
+  float offs;
+  std::memcpy(&offs, &bits, 4);
+  // see cull_radius2
+  d.cull_abs = std::nextafter(float(double(offs) + 0x1p-18 * double(pm.hmax) * d.scale), INFINITY);
+  d.wnodes   = m->wnodes.as<ebgpu::WalkNode>();
+  d.tdisc    = m->tdisc.as<ebgpu::TriDisc>();
+  d.frames   = m->frames.as<ebgpu::FrameRec>();
+  std::vector<uint32_t> first;
+  ebgpu::child_first_triangles(pm, first);
+  EBG_HIP(upload(m->nfirst, first));
+  d.nfirst = m->nfirst.as<uint32_t>();
+  d.K      = uint32_t(pm.K);
+  return EBG_OK;
+}
+
+// Counts, stack banks, bounds and the device view of an uploaded mesh.
 static ebg_status finalize_mesh(ebg_mesh* m, const ebgpu::PackedMesh& pm)
 {
-  {
-    const std::vector<ebgpu::SplitRoot> roots =
-      pm.K == 4 ? split_frontier<4>(pm, kSplitRoots) : split_frontier<8>(pm, kSplitRoots);
-    EBG_HIP(upload(m->split_roots, roots));
-    m->num_split_roots = uint32_t(roots.size());
-  }
   m->K          = pm.K;
   m->leaf       = pm.leaf_size;
   m->num_nodes  = pm.num_nodes;
@@ -203,17 +256,11 @@ static ebg_status finalize_mesh(ebg_mesh* m, const ebgpu::PackedMesh& pm)
   d.hmax          = pm.hmax;
   EBG_HIP(upload(m->status, std::vector<uint32_t>(16, 0u)));
   d.status = m->status.as<uint32_t>();
-  // leaf slabs, from the device arrays (the same for every builder)
-  EBG_HIP(m->lthick.reserve(4 * std::max<uint64_t>(m->nt, 1)));
-  EBG_HIP(ebgpu::launch_leaf_slabs(m->nodes.p, pm.num_nodes, pm.K, d.tsph, d.tripos, m->lthick.as<float>(), nullptr));
-  EBG_HIP(hipStreamSynchronize(nullptr));
-  d.lthick        = m->lthick.as<float>();
-  EBG_HIP(m->frames.reserve(sizeof(ebgpu::FrameRec) * std::max<uint64_t>(m->nt, 1)));
-  EBG_HIP(ebgpu::launch_frames(d.tripos, m->nt, m->frames.as<ebgpu::FrameRec>(), nullptr));
-  EBG_HIP(hipStreamSynchronize(nullptr));
-  d.frames        = m->frames.as<ebgpu::FrameRec>();
+  const ebg_status ws = build_walk(m, pm);
+  if (ws != EBG_OK) return ws;
   m->device_bytes = m->nodes.bytes + m->tris.bytes + m->tripos.bytes + m->tsph.bytes + m->feat.bytes + m->vn32.bytes +
-                    m->en32.bytes + m->vn64.bytes + m->en64.bytes + m->fn64.bytes + m->lthick.bytes + m->frames.bytes;
+                    m->en32.bytes + m->vn64.bytes + m->en64.bytes + m->fn64.bytes + m->wnodes.bytes + m->tdisc.bytes +
+                    m->frames.bytes + m->nfirst.bytes;
   return EBG_OK;
 }
 
@@ -455,7 +502,7 @@ ebg_status ensure_cost_grid(ebg_mesh* m, hipStream_t s)
   q.n           = 64 * ng;
   q.out_d       = dd.as<float>();
   q.packet_cost = m->cost_grid.as<uint32_t>();
-  EBG_HIP(ebgpu::launch_sdf32(m->dev, m->K, m->banks, q, true, s));
+  EBG_HIP(ebgpu::launch_sdf32(m->dev, m->wbanks, q, true, s));
   std::vector<uint32_t> cost(ng);
   EBG_HIP(hipMemcpyAsync(cost.data(), m->cost_grid.p, 4 * ng, hipMemcpyDeviceToHost, s));
   EBG_HIP(hipStreamSynchronize(s));
@@ -592,7 +639,7 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   // events bracket the FP32 traversal (one launch for the bulk and the split items, then the
   // split packets' resolve)
   if (timed) EBG_HIP(hipEventRecord(m->ev0, s));
-  EBG_HIP(launch_sdf32(m->dev, m->K, m->banks, a, count, s));
+  EBG_HIP(launch_sdf32(m->dev, m->wbanks, a, count, s));
   if (heavy_first) EBG_HIP(launch_sdf32_resolve(m->dev, a, s));
   if (timed) {
     EBG_HIP(hipEventRecord(m->ev1, s));

@@ -68,7 +68,7 @@ __global__ __launch_bounds__(256) void batch_keys_kernel(const BatchItemDev* __r
 }
 
 // One packet: the wavefront's 64 queries of one item against its mesh.
-template <int K, int NB, bool COUNT>
+template <int NB, bool COUNT>
 __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, PairLds* pl)
 {
   const SWords<4>    pk = sload<4>(a.packets + 4 * (size_t)p);
@@ -78,25 +78,32 @@ __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, Pai
 
   const uint32_t lane   = __lane_id();
   const uint32_t j      = first + lane;
-  const bool     active = j < it.n;
+  bool           active = j < it.n;
   uint32_t       qi     = 0;
-  float          px = 0.0f, py = 0.0f, pz = 0.0f, bound = -1.0f;
+  float          px = 0.0f, py = 0.0f, pz = 0.0f;
   if (active) {
-    qi    = a.sorted ? (uint32_t)(a.sorted[it.base + j] - it.base) : j;
-    px    = it.pts[3 * (size_t)qi];
-    py    = it.pts[3 * (size_t)qi + 1];
-    pz    = it.pts[3 * (size_t)qi + 2];
-    bound = INFINITY;
+    qi = a.sorted ? (uint32_t)(a.sorted[it.base + j] - it.base) : j;
+    px = it.pts[3 * (size_t)qi] * m.scale;
+    py = it.pts[3 * (size_t)qi + 1] * m.scale;
+    pz = it.pts[3 * (size_t)qi + 2] * m.scale;
+    if (!(px == px && py == py && pz == pz)) { // NaN: no closest triangle, the lane takes no part
+      px = py = pz = 0.0f;
+      active       = false;
+    }
   }
   float    best = INFINITY;
-  uint32_t btri = kInvalid, bfeat = 0, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
+  uint32_t btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
   PairCounts pc{0u, 0u, 0u, 0u};
-  traverse<K, NB, float, COUNT, false, false, true>(m, px, py, pz, bound, best, btri, bfeat, n_inner, n_tris, w_inner,
-                                                    w_tris, nullptr, pl, &pc);
+  mesh_walk<NB, COUNT, false>(m, 0u, 0u, px, py, pz, active ? INFINITY : -1.0f, best, btri, n_inner, n_tris, w_inner,
+                              w_tris, nullptr, pl, &pc);
+  px *= m.inv_scale;
+  py *= m.inv_scale;
+  pz *= m.inv_scale;
+  best *= m.inv_scale * m.inv_scale;
   const bool found = active && btri != kInvalid;
   float      d     = 0.0f;
   if (found) {
-    d            = resolve32(m, btri, bfeat, best, px, py, pz);
+    d            = resolve32(m, btri, closest_feature(m, btri, px, py, pz), best, px, py, pz);
     it.out[qi]   = d;
     if (it.tri) it.tri[qi] = m.tris[btri].face;
   }
@@ -125,8 +132,8 @@ __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, Pai
 // PERSIST = false: one wavefront per packet (the early list first, then the table without the
 // early packets). PERSIST = true: a grid that fits the device at once; each wavefront takes queue
 // entries in the same order until the queue is exhausted (no wavefront waits on another).
-template <int K, int NB, bool COUNT, bool PERSIST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 4 ? 8 : 1))) void batch32_kernel(const BatchArgs a)
+template <int NB, bool COUNT, bool PERSIST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8 : (NB == 2 ? 6 : 4)))) void batch32_kernel(const BatchArgs a)
 {
   extern __shared__ PairLds pair_lds[]; // one per wavefront of the workgroup
   PairLds* const pl = &pair_lds[uni(threadIdx.x >> 6)];
@@ -147,7 +154,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 4 ? 8 
         p = w - skip;
         if (p >= a.num_packets || (a.early_blocks && a.flag[p])) continue;
       }
-      batch_packet<K, NB, COUNT>(a, p, pl);
+      batch_packet<NB, COUNT>(a, p, pl);
     }
   }
   else {
@@ -173,7 +180,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 4 ? 8 
     }
     else p = w;
     if (p >= a.num_packets) return; // whole wavefront (p is wave-uniform)
-    batch_packet<K, NB, COUNT>(a, p, pl);
+    batch_packet<NB, COUNT>(a, p, pl);
   }
 }
 
@@ -267,31 +274,31 @@ __global__ __launch_bounds__(256) void batch_mark_kernel(const BatchArgs a)
   }
 }
 
-template <int K, int NB>
+template <int NB>
 hipError_t launch32(const BatchArgs& a, int wg, bool count, hipStream_t s)
 {
   const size_t lds = (size_t)(wg / 64) * sizeof(PairLds);
   if (a.persist_blocks) {
     if (!a.queue) return hipErrorInvalidValue;
-    if (count) hipLaunchKernelGGL((batch32_kernel<K, NB, true, true>), dim3(a.persist_blocks), dim3(wg), lds, s, a);
-    else hipLaunchKernelGGL((batch32_kernel<K, NB, false, true>), dim3(a.persist_blocks), dim3(wg), lds, s, a);
+    if (count) hipLaunchKernelGGL((batch32_kernel<NB, true, true>), dim3(a.persist_blocks), dim3(wg), lds, s, a);
+    else hipLaunchKernelGGL((batch32_kernel<NB, false, true>), dim3(a.persist_blocks), dim3(wg), lds, s, a);
     return hipGetLastError();
   }
   const uint32_t wpb    = (uint32_t)wg / 64u;
   const uint32_t blocks = (a.num_packets + wpb - 1) / wpb + a.early_blocks;
   if (blocks == 0) return hipSuccess;
-  if (count) hipLaunchKernelGGL((batch32_kernel<K, NB, true, false>), dim3(blocks), dim3(wg), lds, s, a);
-  else hipLaunchKernelGGL((batch32_kernel<K, NB, false, false>), dim3(blocks), dim3(wg), lds, s, a);
+  if (count) hipLaunchKernelGGL((batch32_kernel<NB, true, false>), dim3(blocks), dim3(wg), lds, s, a);
+  else hipLaunchKernelGGL((batch32_kernel<NB, false, false>), dim3(blocks), dim3(wg), lds, s, a);
   return hipGetLastError();
 }
 
-template <int K, int NB>
+template <int NB>
 hipError_t persist_blocks(int wg, bool count, uint32_t* blocks)
 {
   int        nb = 0, dev = 0, cus = 0;
   const size_t lds = (size_t)(wg / 64) * sizeof(PairLds);
-  hipError_t   e   = count ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch32_kernel<K, NB, true, true>, wg, lds)
-                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch32_kernel<K, NB, false, true>, wg, lds);
+  hipError_t   e   = count ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch32_kernel<NB, true, true>, wg, lds)
+                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch32_kernel<NB, false, true>, wg, lds);
   if (e != hipSuccess) return e;
   if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
   if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
@@ -333,31 +340,21 @@ hipError_t launch_batch_mark(const BatchArgs& a, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t launch_batch32(const BatchArgs& a, int K, int banks, int wg, bool count, hipStream_t s)
+hipError_t launch_batch32(const BatchArgs& a, int banks, int wg, bool count, hipStream_t s)
 {
   if (wg != 64 && wg != 128 && wg != 256) return hipErrorInvalidValue;
   if (a.early_blocks && (!a.flag || !a.early_list || !a.early_count)) return hipErrorInvalidValue;
-  if (K == 4) {
-    if (banks <= 1) return launch32<4, 1>(a, wg, count, s);
-    if (banks == 2) return launch32<4, 2>(a, wg, count, s);
-    return launch32<4, 4>(a, wg, count, s);
-  }
-  if (banks <= 1) return launch32<8, 1>(a, wg, count, s);
-  if (banks == 2) return launch32<8, 2>(a, wg, count, s);
-  return launch32<8, 4>(a, wg, count, s);
+  if (banks <= 1) return launch32<1>(a, wg, count, s);
+  if (banks == 2) return launch32<2>(a, wg, count, s);
+  return launch32<4>(a, wg, count, s);
 }
 
-hipError_t batch32_persistent_blocks(int K, int banks, int wg, bool count, uint32_t* blocks)
+hipError_t batch32_persistent_blocks(int banks, int wg, bool count, uint32_t* blocks)
 {
   if (wg != 64 && wg != 128 && wg != 256) return hipErrorInvalidValue;
-  if (K == 4) {
-    if (banks <= 1) return persist_blocks<4, 1>(wg, count, blocks);
-    if (banks == 2) return persist_blocks<4, 2>(wg, count, blocks);
-    return persist_blocks<4, 4>(wg, count, blocks);
-  }
-  if (banks <= 1) return persist_blocks<8, 1>(wg, count, blocks);
-  if (banks == 2) return persist_blocks<8, 2>(wg, count, blocks);
-  return persist_blocks<8, 4>(wg, count, blocks);
+  if (banks <= 1) return persist_blocks<1>(wg, count, blocks);
+  if (banks == 2) return persist_blocks<2>(wg, count, blocks);
+  return persist_blocks<4>(wg, count, blocks);
 }
 
 hipError_t launch_batch64(const BatchArgs& a, int K, int banks, hipStream_t s)

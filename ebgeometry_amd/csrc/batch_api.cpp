@@ -21,7 +21,7 @@ struct ebg_batch
 {
   std::vector<ebg_mesh*> meshes; // owned
   DevBuf                 meshdev;
-  int                    K = 4, leaf = 8, banks = 1;
+  int                    K = 4, leaf = 8, banks = 1, wbanks = 1;
   bool                   tuned = false;
   double                 tune_ms[4]{-1, -1, -1, -1};
   double                 build_seconds = 0;
@@ -221,7 +221,7 @@ ebg_status enqueue(ebg_batch_plan* p, hipStream_t s, bool events)
     a.persist_blocks = p->persist_blocks;
   }
   if (events) EBG_HIP(hipEventRecord(p->ev0, s));
-  EBG_HIP(ebgpu::launch_batch32(a, b->K, b->banks, p->wg, p->work != nullptr, s));
+  EBG_HIP(ebgpu::launch_batch32(a, b->wbanks, p->wg, p->work != nullptr, s));
   if (events) EBG_HIP(hipEventRecord(p->ev1, s));
   if (p->fp64) {
     // the list follows the packet table (presort order), so FP64 wavefronts hold neighbouring
@@ -342,7 +342,8 @@ ebg_status ebg_batch_create(const float* const* xyz, const uint64_t* nv, const u
   std::vector<ebgpu::MeshDev> md(num_meshes);
   for (uint64_t i = 0; i < num_meshes; i++) {
     md[i]    = b->meshes[i]->dev;
-    b->banks = std::max(b->banks, b->meshes[i]->banks);
+    b->banks  = std::max(b->banks, b->meshes[i]->banks);
+    b->wbanks = std::max(b->wbanks, b->meshes[i]->wbanks);
     b->num_triangles += b->meshes[i]->nt;
   }
   const hipError_t e = upload(b->meshdev, md);
@@ -521,7 +522,7 @@ ebg_status ebg_batch_plan_create(ebg_batch* b, const ebg_batch_item* items, uint
   auto set_shape = [&](int wg, bool persistent) -> hipError_t {
     p->wg         = wg;
     p->persistent = persistent;
-    return persistent ? ebgpu::batch32_persistent_blocks(b->K, b->banks, wg, p->work != nullptr, &p->persist_blocks)
+    return persistent ? ebgpu::batch32_persistent_blocks(b->wbanks, wg, p->work != nullptr, &p->persist_blocks)
                       : hipSuccess;
   };
   if ((e = set_shape(p->wg, p->persistent)) != hipSuccess) return bail(e, "occupancy");

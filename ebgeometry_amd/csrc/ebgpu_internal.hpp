@@ -48,14 +48,39 @@ struct alignas(64) Node
 static_assert(sizeof(Node<4>) == 128, "Node<4> layout");
 static_assert(sizeof(Node<8>) == 256, "Node<8> layout");
 
-// A subtree root (node reference and box, as on the traversal stack): the roots of a frontier
-// that covers the whole tree let several wavefronts share one expensive packet.
+// Node of the FP32 mesh walk: 4 children, each bounded by 8 floats v[k]. A node is of one of two
+// kinds, flagged in every cnt word:
+//   disc node  child k lies in the cylinder about c = v[0..2] with unit axis n = v[3..5], radius R
+//              and half-height t = v[7] along n; v[6] = 4 R^2.
+//   box node   (kBoxChild set) child k lies in the box lo = v[0..2], hi = v[3..5].
+// A patch of a surface is flat at the scale of the lower levels: its cylinder is a thin disc in the
+// patch's own plane, far closer to the patch than its axis-aligned box. Coordinates are the mesh's
+// times MeshDev::scale.
+constexpr uint32_t kBoxChild = 0x80u;
+struct alignas(32) WalkNode
+{
+  float    v[4][8];
+  uint32_t ref[4]; // as in Node
+  uint32_t cnt[4]; // 0: interior child; 1..16: leaf triangle count; | kBoxChild; kInvalid: empty slot
+};
+static_assert(sizeof(WalkNode) == 160, "WalkNode layout");
+
+// Culling record of one triangle: the disc (centre c, unit normal n, radius R) of its plane that
+// holds it, with 4 R^2 and -R^2 (inflated for the FP32 test).
+struct alignas(32) TriDisc
+{
+  float c[3], n[3], r2x4, nr2;
+};
+static_assert(sizeof(TriDisc) == 32, "TriDisc layout");
+
+// A subtree root of the FP32 walk's tree: the roots of a frontier that covers the whole tree let
+// several wavefronts share one expensive packet.
 struct SplitRoot
 {
   uint32_t ref, cnt; // cnt == 0: interior node ref; 1..16: leaf of cnt triangles from ref
-  float    lo[3], hi[3];
+  uint32_t pad[2];
 };
-static_assert(sizeof(SplitRoot) == 32, "SplitRoot layout");
+static_assert(sizeof(SplitRoot) == 16, "SplitRoot layout");
 
 struct alignas(64) TriRec
 {
@@ -111,10 +136,15 @@ struct MeshDev
   uint32_t        num_tris;
   uint32_t*       status; // device word: bit 0 set when a traversal found its stack too small
   float           hmax;   // longest triangle edge (rounded up): scale of the FP32 distance error
-  uint32_t        pad0;
-  const float*    lthick; // per leaf, at its first triangle: slab half-thickness about that
-                          // triangle's plane holding the whole leaf (rounded up); may be null
-  const FrameRec*  frames; // per triangle (leaf order); may be null
+  float           cull_abs; // FP32 walk: absolute widening of the cull radius (scaled units)
+  // The FP32 walk's tree and records, all in coordinates times `scale` (a power of two, 1 unless
+  // the mesh is very small or very large), so that its squared quantities stay in FP32's range.
+  const WalkNode* wnodes;
+  const TriDisc*  tdisc;  // per triangle (leaf order), padded by kSphPad
+  const FrameRec* frames; // per triangle (leaf order)
+  float           scale, inv_scale;
+  const uint32_t* nfirst; // K per node of `nodes`: each child's first triangle (kInvalid: empty slot)
+  uint32_t        K, pad0;
 };
 static_assert(sizeof(MeshDev) % 16 == 0, "MeshDev is read with 16-byte scalar loads");
 constexpr uint32_t kStatusStackOverflow = 1u;

@@ -218,8 +218,10 @@ struct ebg_mesh
   double                 build_seconds = 0;
   ebgpu::DevBuf          nodes, tris, tripos, tsph, feat, vn32, en32, vn64, en64, fn64;
   ebgpu::DevBuf          area_cdf; // normalised cumulative triangle area, leaf order (training samples)
-  ebgpu::DevBuf          lthick;   // MeshDev::lthick (one float per triangle, set at leaf starts)
-  ebgpu::DevBuf          frames;   // MeshDev::frames (one FrameRec per triangle)
+  // the FP32 walk's tree and records (MeshDev::wnodes, tdisc, frames) and its stack banks
+  ebgpu::DevBuf          wnodes, tdisc, frames;
+  ebgpu::DevBuf          nfirst; // MeshDev::nfirst
+  int                    wbanks = 1;
   // cost grid of the split schedule (built at the first large presorted query): per cell, the
   // work of a packet of 64 queries spread over the cell
   ebgpu::DevBuf          cost_grid;

@@ -26,7 +26,7 @@ struct QueryArgs
   uint32_t*           fallback_list;  // queries whose seeded radius held no triangle
   uint32_t*           fallback_count;
   unsigned long long* work;      // [inner nodes, triangles] accumulated (null = not counted)
-  unsigned long long* pair_work; // counting launches: [pairs, pair batches, culling loads, slab loads]
+  unsigned long long* pair_work; // counting launches: [pairs, pair batches, culling loads, leaves screened]
   float               slack_abs; // FP64 recheck: bound = (|d| + slack_abs + slack_rel*|d|)^2
   float               slack_rel;
   uint32_t*           packet_cost; // counting launches: per packet, the nodes + triangles its wavefront fetched
@@ -87,8 +87,8 @@ hipError_t launch_recheck_compact(const uint64_t* mask, uint64_t n, const uint32
 // the plain pass (outputs, recheck list).
 hipError_t launch_sdf32_resolve(const MeshDev& m, const QueryArgs& a, hipStream_t s);
 
-// FP32 packet traversal. K = 4 or 8; banks = stack capacity / 64 (1..4).
-hipError_t launch_sdf32(const MeshDev& m, int K, int banks, const QueryArgs& a, bool count, hipStream_t s);
+// FP32 packet traversal over the walk tree; banks = its stack capacity / 64 (1..4).
+hipError_t launch_sdf32(const MeshDev& m, int banks, const QueryArgs& a, bool count, hipStream_t s);
 // FP64 traversal that recomputes distance, closest face and sign exactly as the reference's
 // double-precision lane kernel; seeded from the FP32 result (bound |d| + slack).
 hipError_t launch_sdf64(const MeshDev& m, int K, int banks, const QueryArgs& a, hipStream_t s);
@@ -136,7 +136,7 @@ struct BatchArgs
   uint32_t*           recheck_list; // packet << 6 | lane, in packet order (launch_recheck_compact)
   uint32_t*           recheck_count;
   unsigned long long* work;        // [0] inner, [1] triangles, [4]/[5] per wavefront (null = off)
-  unsigned long long* pair_work;   // counting launches: [pairs, pair batches, culling loads, slab loads]
+  unsigned long long* pair_work;   // counting launches: [pairs, pair batches, culling loads, leaves screened]
   // Early packets (early_blocks = 0: none): batch_mark lists the packets whose most expensive
   // query (the cost-grid value of its cell in its mesh's grid) reaches the mesh's threshold;
   // the first early_blocks workgroups of batch32 take them, the rest skip flagged packets.
@@ -158,9 +158,9 @@ hipError_t launch_batch_mark(const BatchArgs& a, hipStream_t s);
 hipError_t launch_batch_keys(const BatchItemDev* items, uint32_t num_items, uint64_t total, void* keys, bool narrow,
                              hipStream_t s);
 // wg = 64, 128 or 256 lanes per workgroup (1, 2 or 4 packets).
-hipError_t launch_batch32(const BatchArgs& a, int K, int banks, int wg, bool count, hipStream_t s);
+hipError_t launch_batch32(const BatchArgs& a, int banks, int wg, bool count, hipStream_t s);
 // Workgroups of wg lanes of the persistent batch32 that fit the device at once (occupancy x CUs).
-hipError_t batch32_persistent_blocks(int K, int banks, int wg, bool count, uint32_t* blocks);
+hipError_t batch32_persistent_blocks(int banks, int wg, bool count, uint32_t* blocks);
 // FP64 pass over the compacted recheck list (a.recheck_list == null skips); a fixed grid
 // strides over groups of 64 entries.
 hipError_t launch_batch64(const BatchArgs& a, int K, int banks, hipStream_t s);
@@ -190,11 +190,19 @@ hipError_t launch_knn(const CloudDev& c, int K, int banks, const KnnArgs& a, hip
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s);
 // v[i] <- map[v[i]] where v[i] < nmap (polygon meshes: triangle index -> face index)
 hipError_t launch_map_u32(uint32_t* v, uint64_t n, const uint32_t* map, uint32_t nmap, hipStream_t s);
-// Per leaf, at its first triangle: the slab half-thickness about that triangle's plane
-hipError_t launch_leaf_slabs(const void* nodes, uint32_t num_nodes, int K, const float* tsph, const float* tripos,
-                             float* lthick, hipStream_t s);
-// Per triangle (leaf order): its record in a frame of its own plane, from the FP32 vertices
-hipError_t launch_frames(const float* tripos, uint64_t nt, FrameRec* out, hipStream_t s);
+// Per triangle (leaf order), from the FP32 vertices times scale: its record in a frame of its own
+// plane and its culling disc; *off (zero on entry) gets the bits of the mesh's largest distance of
+// a corner from its triangle's disc
+hipError_t launch_frames(const float* tripos, uint64_t nt, float scale, FrameRec* out, TriDisc* disc, uint32_t* off,
+                         hipStream_t s);
+// The walk tree's cylinders: range holds 2 words per child slot (4 slots per node); the listed
+// slots (small: walked by a wavefront each, large: by a 1024-lane workgroup) get 8 floats of discs,
+// the others must hold a negative seventh; then each node takes its children's cylinders or keeps
+// their boxes
+constexpr uint32_t kWalkLarge = 1024; // triangles of a large slot
+hipError_t launch_walk_nodes(const float* tripos, const uint32_t* range, const uint32_t* small, uint32_t num_small,
+                             const uint32_t* large, uint32_t num_large, float scale, float* discs, WalkNode* nodes,
+                             uint32_t num_nodes, hipStream_t s);
 // n doubles -> floats (round to nearest even) and n floats -> doubles
 hipError_t launch_f64_to_f32(const double* in, float* out, uint64_t n, hipStream_t s);
 

@@ -660,6 +660,121 @@ int compute_stack_need(const PackedMesh& m)
   return 1 + std::max(0, stack_need_rec<8>(reinterpret_cast<const Node<8>*>(m.nodes.data()), 0));
 }
 
+namespace {
+
+template <int K>
+struct WalkEmitter
+{
+  const Node<K>* in;
+  float          scale;
+  WalkTree&      out;
+
+  struct Range
+  {
+    uint32_t first = kInvalid, last = 0, count = 0; // count: triangles in the subtree
+  };
+
+  std::vector<int> children(uint32_t i) const
+  {
+    std::vector<int> c;
+    for (int k = 0; k < K; k++)
+      if (in[i].cnt[k] != kInvalid) c.push_back(k);
+    return c;
+  }
+
+  // A walk node over the children kids of in[i]; returns its index, the triangles below it and
+  // the stack its walk needs beyond its own entry.
+  uint32_t emit(uint32_t i, const std::vector<int>& kids, Range& all, int& need)
+  {
+    const uint32_t me = uint32_t(out.nodes.size());
+    out.nodes.emplace_back();
+    out.range.resize(8 * out.nodes.size(), 0u);
+    WalkNode nd{};
+    for (int k = 0; k < 4; k++) nd.cnt[k] = kInvalid;
+    const int m = int(kids.size()), slots = std::min(m, 4);
+    int       deepest = 0;
+    for (int k = 0; k < slots; k++) {
+      // slots share the children evenly, in order
+      const std::vector<int> part(kids.begin() + k * m / slots, kids.begin() + (k + 1) * m / slots);
+      const Node<K>&         n = in[i];
+      float                  lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+      for (int c : part) {
+        const float a[3] = {n.lox[c], n.loy[c], n.loz[c]}, b[3] = {n.hix[c], n.hiy[c], n.hiz[c]};
+        for (int x = 0; x < 3; x++) {
+          lo[x] = std::min(lo[x], a[x]);
+          hi[x] = std::max(hi[x], b[x]);
+        }
+      }
+      for (int x = 0; x < 3; x++) {
+        nd.v[k][x]     = lo[x] * scale;
+        nd.v[k][3 + x] = hi[x] * scale;
+      }
+      Range r;
+      int   deep = 0;
+      if (part.size() == 1 && n.cnt[part[0]] != 0u) {
+        nd.ref[k] = n.ref[part[0]];
+        nd.cnt[k] = n.cnt[part[0]] | kBoxChild;
+        r         = {nd.ref[k], nd.ref[k] + n.cnt[part[0]], n.cnt[part[0]]};
+      }
+      else {
+        nd.cnt[k] = kBoxChild;
+        nd.ref[k] = part.size() == 1 ? emit(n.ref[part[0]], children(n.ref[part[0]]), r, deep) : emit(i, part, r, deep);
+      }
+      deepest = std::max(deepest, deep);
+      if (r.count == r.last - r.first) {
+        out.range[8 * me + 2 * k]     = r.first;
+        out.range[8 * me + 2 * k + 1] = r.last;
+      }
+      all.first = std::min(all.first, r.first);
+      all.last  = std::max(all.last, r.last);
+      all.count += r.count;
+    }
+    out.nodes[me] = nd;
+    need          = slots - 1 + deepest;
+    return me;
+  }
+};
+
+} // namespace
+
+void build_walk_tree(const PackedMesh& pm, float scale, WalkTree& out)
+{
+  out.nodes.clear();
+  out.range.clear();
+  int  need = 0;
+  auto run  = [&](auto tag) {
+    constexpr int         KK = decltype(tag)::value;
+    WalkEmitter<KK>       e{reinterpret_cast<const Node<KK>*>(pm.nodes.data()), scale, out};
+    typename WalkEmitter<KK>::Range all;
+    e.emit(0, e.children(0), all, need);
+  };
+  if (pm.K == 4) run(std::integral_constant<int, 4>{});
+  else run(std::integral_constant<int, 8>{});
+  out.stack_need = 1 + std::max(0, need);
+}
+
+namespace {
+template <int K>
+uint32_t child_first_rec(const Node<K>* nodes, uint32_t i, std::vector<uint32_t>& out)
+{
+  uint32_t least = kInvalid;
+  for (int k = 0; k < K; k++) {
+    if (nodes[i].cnt[k] == kInvalid) continue;
+    const uint32_t f = nodes[i].cnt[k] ? nodes[i].ref[k] : child_first_rec<K>(nodes, nodes[i].ref[k], out);
+    out[size_t(K) * i + k] = f;
+    least                  = std::min(least, f);
+  }
+  return least;
+}
+} // namespace
+
+void child_first_triangles(const PackedMesh& pm, std::vector<uint32_t>& out)
+{
+  out.assign(size_t(pm.K) * pm.num_nodes, kInvalid);
+  if (pm.K == 4) child_first_rec<4>(reinterpret_cast<const Node<4>*>(pm.nodes.data()), 0, out);
+  else child_first_rec<8>(reinterpret_cast<const Node<8>*>(pm.nodes.data()), 0, out);
+}
+
 bool build_sah_mesh(const float* xyz, std::size_t nv, const uint32_t* tri, std::size_t nt, int K, int leaf_size,
                     const PseudoNormals& pn, PackedMesh& out, std::string& err)
 {

@@ -103,6 +103,22 @@ static_assert(sizeof(BinNode) == 40, "BinNode layout (also written by the GPU bu
 // diagonal and stack need of out (not its order).
 void collapse_binary(const std::vector<BinNode>& bn, int32_t root, int K, WideBvh& out);
 
+// The tree of the FP32 mesh walk: WalkNodes over the same leaves as a packed tree of Node<K>
+// records (K = 8: a node's more than 4 children are grouped in neighbours under 4), DFS pre-order,
+// root at 0, every child with its box (times scale) and flagged kBoxChild; and per child slot
+// (4 per node) the leaf-order range [first, last) of its triangles (equal: not contiguous).
+struct WalkTree
+{
+  std::vector<WalkNode> nodes;
+  std::vector<uint32_t> range;
+  int                   stack_need = 0;
+};
+void build_walk_tree(const PackedMesh& pm, float scale, WalkTree& out);
+
+// Per node of a packed tree, the first triangle (leaf order) of each of its K children (kInvalid
+// for an empty slot); within a node they ascend with the slot.
+void child_first_triangles(const PackedMesh& pm, std::vector<uint32_t>& out);
+
 // 64-bit FNV-1a over the bytes of the vertex and triangle arrays (identifies the mesh a trained
 // network belongs to).
 inline uint64_t mesh_hash(const float* xyz, uint64_t nv, const uint32_t* tri, uint64_t nt)

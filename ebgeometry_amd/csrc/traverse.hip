@@ -6,12 +6,17 @@
 //     no LDS and no scratch;
 //   * a node or triangle record is fetched once per wavefront with scalar loads into SGPRs
 //     and every lane tests its own query against it;
-//   * a child is pushed when any lane's box distance is within that lane's bound (ballot);
-//     children are ordered by the box distance seen by the packet's middle lane (nearest
-//     popped first), which is the reference's descending-d^2 push order
+//   * a child is pushed when its bound (a cylinder along the patch of surface it holds, or a box:
+//     WalkNode) is within any lane's cull radius (ballot); children are ordered by the distance
+//     seen by the packet's middle lane (to the box, or to the cylinder's centre; nearest popped
+//     first), which is the reference's descending-d^2 push order
 //     (Source/EBGeometry_BVHImplem.hpp:1178-1194) applied to the packet;
-//   * on pop, each lane re-tests the entry box against its current bound (the reference's
-//     `entry.dist2 > curBest2` check, :1145-1149); the entry is skipped when no lane needs it.
+//   * on pop, each lane re-tests the entry's bound against its current cull radius (the
+//     reference's `entry.dist2 > curBest2` check, :1145-1149); the entry is skipped when no lane
+//     needs it.
+// The cylinders took the 16M-query launch on the 327,680-face displaced sphere (K = 4, leaves of 16)
+// from 11.0 to 4.86 ms a pass, 1M queries on the 20,480-face unit sphere from 4.98 to 1.01 ms and 1M
+// closest faces on an 81,920-face sphere from 10.8 to 2.8 ms.
 // Queries arrive presorted along a Hilbert curve, so the 64 queries of a wave are spatial
 // neighbours and visit nearly the same nodes.
 //
@@ -47,15 +52,51 @@ enum Mode : int
   kSeeded = 1
 };
 
+// Whether a depth-first walk of the packed tree that takes a node's children in the order of their
+// box distances from (rx, ry, rz) -- nearest first, on equal distances the later slot first -- meets
+// triangle a before triangle b.
+template <int K>
+__device__ __forceinline__ bool met_before_k(const MeshDev& m, uint32_t a, uint32_t b, float rx, float ry, float rz)
+{
+  const Node<K>* nodes = static_cast<const Node<K>*>(m.nodes);
+  uint32_t       i     = 0;
+  for (;;) {
+    const uint32_t* f  = m.nfirst + (size_t)K * i;
+    int             ka = 0, kb = 0; // the children holding a and b (the slots' first triangles ascend)
+    for (int k = 1; k < K; k++) {
+      if (f[k] == kInvalid) continue;
+      if (f[k] <= a) ka = k;
+      if (f[k] <= b) kb = k;
+    }
+    const Node<K>& nd = nodes[i];
+    if (ka != kb) {
+      const float da = box_d2<float>(rx, ry, rz, nd.lox[ka], nd.loy[ka], nd.loz[ka], nd.hix[ka], nd.hiy[ka], nd.hiz[ka]);
+      const float db = box_d2<float>(rx, ry, rz, nd.lox[kb], nd.loy[kb], nd.loz[kb], nd.hix[kb], nd.hiy[kb], nd.hiz[kb]);
+      return da < db || (da == db && ka > kb);
+    }
+    if (nd.cnt[ka] != 0u) return a < b; // one leaf: in its order
+    i = nd.ref[ka];
+  }
+}
+__device__ __forceinline__ bool met_before(const MeshDev& m, uint32_t a, uint32_t b, float rx, float ry, float rz)
+{
+  return m.K == 4u ? met_before_k<4>(m, a, b, rx, ry, rz) : met_before_k<8>(m, a, b, rx, ry, rz);
+}
+
 // Closest face of a lane whose FP32 walk kept more than one triangle inside the band of its
 // minimum (FaceCands): the kept triangles are evaluated with the FP64 lane formulas and the
-// first strict FP64 minimum (in FP32 order) wins, as TriMeshSDF::getClosestTriangle keeps the
-// first strict minimum (Source/EBGeometry_MeshDistanceFunctionsImplem.hpp:511-549). Returns the
+// FP64 minimum wins; among exact FP64 ties (faces meeting at the closest edge or vertex) the one of
+// the smallest FP32 distance, and among those the one that a walk of the packed tree by box
+// distances from the packet's representative point r meets first, as
+// TriMeshSDF::getClosestTriangle keeps the first strict minimum of its walk
+// (Source/EBGeometry_MeshDistanceFunctionsImplem.hpp:511-549). That order is a rule on the tree and
+// the packet, so the choice does not depend on the order in which this walk met them. Returns the
 // FP64 signed distance of that face.
 __device__ __forceinline__ float decide_face64(const MeshDev& m, const FaceCands& fc, float lim, float px, float py,
-                                               float pz, uint32_t& btri)
+                                               float pz, float rx, float ry, float rz, uint32_t& btri)
 {
   double   bd = INFINITY;
+  float    bd32 = INFINITY;
   uint32_t bt = fc.t[0], bf = 0;
 #pragma unroll
   for (int i = 0; i < kFaceCands; i++) {
@@ -64,10 +105,12 @@ __device__ __forceinline__ float decide_face64(const MeshDev& m, const FaceCands
       double         d2;
       uint32_t       f;
       tri_eval64(m.tripos + 12 * (size_t)t, m.fn64 + 4 * (size_t)t, px, py, pz, d2, f);
-      if (d2 < bd) {
-        bd = d2;
-        bt = t;
-        bf = f;
+      // the list ascends in d32, so a tie with a smaller d32 is already held
+      if (d2 < bd || (d2 == bd && fc.d[i] == bd32 && met_before(m, t, bt, rx, ry, rz))) {
+        bd   = d2;
+        bd32 = fc.d[i];
+        bt   = t;
+        bf   = f;
       }
     }
   }
@@ -79,34 +122,40 @@ __device__ __forceinline__ float decide_face64(const MeshDev& m, const FaceCands
 // FACE (closest faces requested): each lane decides its face exactly (decide_face64); a lane
 // whose band held more triangles than its list goes to the FP64 pass with the near-surface ones.
 // Distance-only variants (!FACE) evaluate leaves pair-compacted in the wavefront's PairLds.
-template <int K, int NB, bool COUNT, int MODE, bool FACE>
+template <int NB, bool COUNT, int MODE, bool FACE>
 __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& a, uint64_t n, uint64_t pk, PairLds* pl)
 {
   const uint64_t tid    = pk * 64u + (uint64_t)__lane_id();
-  const bool     active = tid < n;
-  uint32_t   qi     = 0;
-  float      px = 0.0f, py = 0.0f, pz = 0.0f, bound = -1.0f;
+  bool           active = tid < n;
+  uint32_t       qi     = 0;
+  float          px = 0.0f, py = 0.0f, pz = 0.0f, bound = -1.0f;
+  const float    sc = m.scale, ds = FACE ? 1.0f : sc * sc; // distance^2 units of the walk (mesh_walk)
   if (active) {
     qi = a.idx ? a.idx[tid] : (uint32_t)tid;
-    px = a.pts[3 * (size_t)qi];
-    py = a.pts[3 * (size_t)qi + 1];
-    pz = a.pts[3 * (size_t)qi + 2];
+    px = a.pts[3 * (size_t)qi] * sc;
+    py = a.pts[3 * (size_t)qi + 1] * sc;
+    pz = a.pts[3 * (size_t)qi + 2] * sc;
     if (MODE == kSeeded) {
       const float r = a.seed_r[qi];
-      bound         = r * r;
+      bound         = r * r * ds;
     }
     else {
       bound = INFINITY;
     }
+    // a NaN coordinate has no closest triangle: its lane takes no part (and writes nothing)
+    if (!(px == px && py == py && pz == pz)) {
+      px = py = pz = 0.0f;
+      bound        = -1.0f;
+      active       = false;
+    }
   }
   float    best = INFINITY;
-  uint32_t btri = kInvalid, bfeat = 0, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
+  uint32_t btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
   const float seed2 = bound;
   FaceCands   fc;
   if constexpr (FACE) fc.init(m.hmax);
   PairCounts pc{0u, 0u, 0u, 0u};
-  traverse<K, NB, float, COUNT, false, FACE, !FACE>(m, px, py, pz, bound, best, btri, bfeat, n_inner, n_tris, w_inner,
-                                                    w_tris, &fc, pl, &pc);
+  mesh_walk<NB, COUNT, FACE>(m, 0u, 0u, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, &fc, pl, &pc);
 
   // Exact only if some triangle lies within the seeded radius: otherwise nodes between the
   // seeded radius and the true distance were pruned, and the query must be redone unseeded.
@@ -119,15 +168,14 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
     const uint64_t rmask = ballot(redo);
     if (rmask) {
       float     best2 = INFINITY;
-      uint32_t  btri2 = kInvalid, bfeat2 = 0, f_inner = 0, f_tris = 0;
+      uint32_t  btri2 = kInvalid, f_inner = 0, f_tris = 0;
       FaceCands fc2;
       if constexpr (FACE) fc2.init(m.hmax);
-      traverse<K, NB, float, COUNT, false, FACE, !FACE>(m, px, py, pz, redo ? INFINITY : -1.0f, best2, btri2, bfeat2,
-                                                        f_inner, f_tris, w_inner, w_tris, &fc2, pl, &pc);
+      mesh_walk<NB, COUNT, FACE>(m, 0u, 0u, px, py, pz, redo ? INFINITY : -1.0f, best2, btri2, f_inner, f_tris, w_inner,
+                                 w_tris, &fc2, pl, &pc);
       if (redo) {
-        best  = best2;
-        btri  = btri2;
-        bfeat = bfeat2;
+        best = best2;
+        btri = btri2;
         if constexpr (FACE) fc = fc2;
       }
       found = active && btri != kInvalid;
@@ -142,17 +190,26 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
       }
     }
   }
+  // back to the mesh's own units (a power of two: exact)
+  px *= m.inv_scale;
+  py *= m.inv_scale;
+  pz *= m.inv_scale;
+  if constexpr (!FACE) best *= m.inv_scale * m.inv_scale;
+  // the packet's representative point: its middle lane's, or its first query's
+  const int rep = rep_lane(active ? 0.0f : -1.0f);
+  [[maybe_unused]] const float rx = rdlanef(px, rep), ry = rdlanef(py, rep), rz = rdlanef(pz, rep);
   float d   = 0.0f;
   bool  ovf = false; // FACE: the band held more triangles than the list
   if (found) {
-    d = resolve32(m, btri, bfeat, best, px, py, pz);
+    d = resolve32(m, btri, closest_feature(m, btri, px, py, pz), best, px, py, pz);
     if constexpr (FACE) {
       // a second triangle inside the band: decide in FP64 among the kept ones, unless the
       // query is a near-surface one (the FP64 pass decides those from scratch) or the band
       // overflowed the list (then the FP64 pass decides it too)
       const float lim = fc.band(best);
       ovf             = fc.evict <= lim;
-      if (!ovf && fc.d[1] <= lim && !(fabsf(d) < a.recheck_abs)) d = decide_face64(m, fc, lim, px, py, pz, btri);
+      if (!ovf && fc.d[1] <= lim && !(fabsf(d) < a.recheck_abs))
+        d = decide_face64(m, fc, lim, px, py, pz, rx, ry, rz, btri);
     }
     a.out_d[qi] = d;
     if (a.out_tri) a.out_tri[qi] = m.tris[btri].face;
@@ -185,26 +242,29 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
 // One split item: subtree root r for the 64 queries of listed packet j, unseeded; each lane's
 // (d^2, triangle) is folded into the packet's keys. d^2 >= 0, so its bits order like the value;
 // on equal d^2 the lower triangle index wins.
-template <int K, int NB, bool COUNT>
+template <int NB, bool COUNT>
 __device__ __forceinline__ void split_item(const MeshDev& m, const QueryArgs& a, uint32_t j, uint32_t r, PairLds* pl)
 {
   const uint64_t pk     = a.split_list[j];
   const uint32_t lane   = __lane_id();
   const uint64_t tid    = pk * 64u + lane;
-  const bool     active = tid < a.n;
+  bool           active = tid < a.n;
   float          px = 0.0f, py = 0.0f, pz = 0.0f;
   if (active) {
     const uint32_t qi = a.idx ? a.idx[tid] : (uint32_t)tid;
-    px                = a.pts[3 * (size_t)qi];
-    py                = a.pts[3 * (size_t)qi + 1];
-    pz                = a.pts[3 * (size_t)qi + 2];
+    px                = a.pts[3 * (size_t)qi] * m.scale;
+    py                = a.pts[3 * (size_t)qi + 1] * m.scale;
+    pz                = a.pts[3 * (size_t)qi + 2] * m.scale;
+    if (!(px == px && py == py && pz == pz)) { // as in sdf32_packet
+      px = py = pz = 0.0f;
+      active       = false;
+    }
   }
   const SplitRoot rt = sload_record(a.split_roots + r);
-  const Entry     start{rt.ref, rt.cnt, rt.lo[0], rt.lo[1], rt.lo[2], rt.hi[0], rt.hi[1], rt.hi[2]};
   float           best = INFINITY;
-  uint32_t        btri = kInvalid, bfeat = 0, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
-  traverse_from<K, NB, float, COUNT, false, false, true>(m, start, px, py, pz, active ? INFINITY : -1.0f, best, btri,
-                                                        bfeat, n_inner, n_tris, w_inner, w_tris, nullptr, pl);
+  uint32_t        btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
+  mesh_walk<NB, COUNT, false>(m, rt.ref, rt.cnt, px, py, pz, active ? INFINITY : -1.0f, best, btri, n_inner, n_tris,
+                              w_inner, w_tris, nullptr, pl, nullptr);
   if (active && btri != kInvalid)
     atomicMin(a.split_keys + 64 * (size_t)j + lane, ((unsigned long long)__float_as_uint(best) << 32) | btri);
   if (COUNT && a.work) {
@@ -223,8 +283,8 @@ __device__ __forceinline__ void split_item(const MeshDev& m, const QueryArgs& a,
 // mapped XCD-aware so that each XCD works through one contiguous (Morton) range of queries.
 // The leading split_blocks workgroups (dispatched first) work through the split items instead,
 // beside the packets of the bulk; packets flagged in heavy_flag are skipped.
-template <int K, int NB, bool COUNT, int MODE, bool FACE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 4 && !FACE ? 8 : 1))) void sdf32_kernel(const MeshDev m, const QueryArgs a)
+template <int NB, bool COUNT, int MODE, bool FACE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FACE ? 1 : (NB == 1 ? 8 : (NB == 2 ? 6 : 4))))) void sdf32_kernel(const MeshDev m, const QueryArgs a)
 {
   const uint32_t wave = uni(threadIdx.x >> 6); // known uniform: list entries load as scalars
   extern __shared__ PairLds pair_lds[];        // one per wavefront (distance-only variants)
@@ -235,7 +295,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 4 && !
       const uint32_t items = min(*a.split_count, a.split_cap) * a.split_nroots;
       for (uint32_t w = b * 4u + wave; w < items; w += a.split_blocks * 4u) {
         const uint32_t j = w / a.split_nroots;
-        split_item<K, NB, COUNT>(m, a, j, w - j * a.split_nroots, pl);
+        split_item<NB, COUNT>(m, a, j, w - j * a.split_nroots, pl);
       }
       return;
     }
@@ -245,7 +305,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 4 && !
   if (a.early_blocks) {
     if (b < a.early_blocks) {
       const uint32_t j = b * 4u + wave;
-      if (j < min(*a.early_count, a.early_cap)) sdf32_packet<K, NB, COUNT, MODE, FACE>(m, a, a.n, a.early_list[j], pl);
+      if (j < min(*a.early_count, a.early_cap)) sdf32_packet<NB, COUNT, MODE, FACE>(m, a, a.n, a.early_list[j], pl);
       return;
     }
     b -= a.early_blocks;
@@ -256,7 +316,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K == 4 && !
   const uint64_t pk  = (uint64_t)blk * 4u + wave;
   if (pk * 64u >= n) return;                    // whole wavefront past the end
   if (a.heavy_flag && a.heavy_flag[pk]) return; // whole wavefront: a split or early packet
-  sdf32_packet<K, NB, COUNT, MODE, FACE>(m, a, n, pk, pl);
+  sdf32_packet<NB, COUNT, MODE, FACE>(m, a, n, pk, pl);
 }
 
 // One wavefront per listed packet: the winning triangle of each query, as the plain pass ends.
@@ -279,7 +339,8 @@ __global__ __launch_bounds__(256) void sdf32_resolve_kernel(const MeshDev m, con
       float       d2;
       uint32_t    feat;
       tri_eval32<true>(m.tris[t], px, py, pz, d2, feat);
-      d           = resolve32(m, t, feat, __uint_as_float((uint32_t)(key >> 32)), px, py, pz);
+      d2          = __uint_as_float((uint32_t)(key >> 32)) * (m.inv_scale * m.inv_scale); // the walk's, unscaled
+      d           = resolve32(m, t, feat, d2, px, py, pz);
       a.out_d[qi] = d;
       if (a.out_tri) a.out_tri[qi] = m.tris[t].face;
       found = true;
@@ -366,23 +427,23 @@ __global__ __launch_bounds__(256) void sdf64_kernel(const MeshDev m, const Query
     sdf64_block<K, NB>(m, a, n, lane < kSdf64Lanes ? w * kSdf64Lanes + lane : n);
 }
 
-template <int K, int NB, int MODE, bool FACE>
+template <int NB, int MODE, bool FACE>
 void launch32f(const MeshDev& m, const QueryArgs& a, bool count, uint32_t blocks, hipStream_t s)
 {
   const size_t lds = FACE ? 0 : 4 * sizeof(PairLds);
-  if (count) hipLaunchKernelGGL((sdf32_kernel<K, NB, true, MODE, FACE>), dim3(blocks), dim3(256), lds, s, m, a);
-  else hipLaunchKernelGGL((sdf32_kernel<K, NB, false, MODE, FACE>), dim3(blocks), dim3(256), lds, s, m, a);
+  if (count) hipLaunchKernelGGL((sdf32_kernel<NB, true, MODE, FACE>), dim3(blocks), dim3(256), lds, s, m, a);
+  else hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, FACE>), dim3(blocks), dim3(256), lds, s, m, a);
 }
 
 // closest faces requested: the exact-face variant (its split packets are off: see launch32)
-template <int K, int NB, int MODE>
+template <int NB, int MODE>
 void launch32m(const MeshDev& m, const QueryArgs& a, bool count, uint32_t blocks, hipStream_t s)
 {
-  if (a.out_tri) launch32f<K, NB, MODE, true>(m, a, count, blocks, s);
-  else launch32f<K, NB, MODE, false>(m, a, count, blocks, s);
+  if (a.out_tri) launch32f<NB, MODE, true>(m, a, count, blocks, s);
+  else launch32f<NB, MODE, false>(m, a, count, blocks, s);
 }
 
-template <int K, int NB>
+template <int NB>
 hipError_t launch32(const MeshDev& m, const QueryArgs& a, bool count, hipStream_t s)
 {
   const uint32_t blocks = (uint32_t)((a.n + 255) / 256) + a.split_blocks + a.early_blocks;
@@ -395,10 +456,10 @@ hipError_t launch32(const MeshDev& m, const QueryArgs& a, bool count, hipStream_
   if (a.early_blocks && (!a.early_list || !a.early_count || !a.heavy_flag)) return hipErrorInvalidValue;
   if (a.seed_r) {
     if (!a.fallback_count) return hipErrorInvalidValue;
-    launch32m<K, NB, kSeeded>(m, a, count, blocks, s);
+    launch32m<NB, kSeeded>(m, a, count, blocks, s);
   }
   else {
-    launch32m<K, NB, kPlain>(m, a, count, blocks, s);
+    launch32m<NB, kPlain>(m, a, count, blocks, s);
   }
   return hipGetLastError();
 }
@@ -414,16 +475,11 @@ hipError_t launch64(const MeshDev& m, const QueryArgs& a, hipStream_t s)
 
 } // namespace
 
-hipError_t launch_sdf32(const MeshDev& m, int K, int banks, const QueryArgs& a, bool count, hipStream_t s)
+hipError_t launch_sdf32(const MeshDev& m, int banks, const QueryArgs& a, bool count, hipStream_t s)
 {
-  if (K == 4) {
-    if (banks <= 1) return launch32<4, 1>(m, a, count, s);
-    if (banks == 2) return launch32<4, 2>(m, a, count, s);
-    return launch32<4, 4>(m, a, count, s);
-  }
-  if (banks <= 1) return launch32<8, 1>(m, a, count, s);
-  if (banks == 2) return launch32<8, 2>(m, a, count, s);
-  return launch32<8, 4>(m, a, count, s);
+  if (banks <= 1) return launch32<1>(m, a, count, s);
+  if (banks == 2) return launch32<2>(m, a, count, s);
+  return launch32<4>(m, a, count, s);
 }
 
 namespace {

@@ -615,6 +615,114 @@ __device__ __forceinline__ int rep_lane(R bound)
   return ((act >> 32) & 1ull) ? 32 : (act ? __builtin_ctzll(act) : 0);
 }
 
+// ---------------------------------------------------------------------------------------
+// the FP32 mesh walk: cylinder bounds, pair-compacted leaves
+// ---------------------------------------------------------------------------------------
+
+// The walk's stack, in VGPR lanes like LaneStack: an entry is a child of a WalkNode (its
+// reference, its count word with the stamp above it, its 8 bound floats).
+struct WalkEntry
+{
+  uint32_t ref, cnt;
+  float    v[8];
+};
+
+template <int NB>
+struct WalkStack
+{
+  uint32_t ref[NB], cnt[NB];
+  float    v[8][NB];
+
+  __device__ __forceinline__ void init()
+  {
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      ref[i] = cnt[i] = 0u;
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j][i] = 0.0f;
+    }
+  }
+  __device__ __forceinline__ void put(int pos, uint32_t r, uint32_t c, const float* b)
+  {
+    const int l = pos & 63;
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      if ((pos >> 6) == i) {
+        ref[i] = wrlane(r, l, ref[i]);
+        cnt[i] = wrlane(c, l, cnt[i]);
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j][i] = wrlanef(b[j], l, v[j][i]);
+      }
+    }
+  }
+  __device__ __forceinline__ uint32_t ref_at(int pos) const
+  {
+    uint32_t x = 0u;
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+      if ((pos >> 6) == i) x = rdlane(ref[i], pos & 63);
+    return x;
+  }
+  __device__ __forceinline__ uint32_t cnt_at(int pos) const
+  {
+    uint32_t x = 0u;
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+      if ((pos >> 6) == i) x = rdlane(cnt[i], pos & 63);
+    return x;
+  }
+  __device__ __forceinline__ void bound_at(int pos, float* b) const
+  {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      b[j] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NB; i++)
+        if ((pos >> 6) == i) b[j] = rdlanef(v[j][i], pos & 63);
+    }
+  }
+};
+
+// The squared cull radius of a lane whose bound on d^2 is `bound` (all scaled): (d (1 + 2^-17) +
+// cull_abs)^2. It covers, for every triangle whose evaluated distance^2 is at most `bound`: the
+// FP32 error of that evaluation (cull_abs holds 2^-18 of the longest edge), the distance of the
+// triangles' corners from their rounded discs (the largest is in cull_abs) and the part of the
+// tests' own rounding that scales with the distance; the part that scales with a record's size is
+// in its inflated radius and height. So no cull changes the walk's minimum. A lane without a
+// query (bound < 0) gets -1, which every test rejects.
+__device__ __forceinline__ float cull_radius2(const MeshDev& m, float bound)
+{
+  const float r = fmaf(__builtin_amdgcn_sqrtf(bound), 1.0f + 0x1p-17f, m.cull_abs);
+  return bound < 0.0f ? -1.0f : r * r;
+}
+
+// Lanes within their cull radius of a cylinder (see WalkNode): with s = p - c, h the distance
+// beyond the end planes and rho the distance from the axis, the cylinder is within b of p when
+// h <= b and rho - R <= sqrt(b^2 - h^2) =: sqrt(w), that is
+//   B := s.s - (n.s)^2 - R^2 - w <= 2 R sqrt(w), tested without the root as B |B| <= 4 R^2 w.
+// 18 VALU instructions (a box takes 13: one SGPR operand per instruction, so med3(p, lo, hi) costs
+// a move), for a bound that follows a surface patch: against the boxes and the bounding-sphere and plane
+// tests it visits 34 instead of 74 nodes, 16 instead of 63 leaves and 27 instead of 108 pairs per
+// query (16M queries, 327,680-face displaced sphere). Both conditions are tested as "not beyond",
+// so an overflow or a NaN keeps the lane.
+__device__ __forceinline__ uint64_t disc_lanes(const float* v, float px, float py, float pz, float b2, float& s2)
+{
+  const float sx = px - v[0], sy = py - v[1], sz = pz - v[2];
+  s2             = sx * sx + sy * sy + sz * sz;
+  const float pd = v[3] * sx + v[4] * sy + v[5] * sz;
+  const float q  = fmaf(-pd, pd, fmaf(v[6], -0.25f, s2));
+  const float h  = fmaxf(fabsf(pd) - v[7], 0.0f);
+  const float w  = fmaf(-h, h, b2);
+  const float B  = q - w;
+  return ballot(!(B * fabsf(B) > v[6] * w)) & ballot(!(w < 0.0f));
+}
+
+__device__ __forceinline__ uint64_t walk_box_lanes(const float* v, float px, float py, float pz, float b2, float& d2)
+{
+  d2 = box_d2<float>(px, py, pz, v[0], v[1], v[2], v[3], v[4], v[5]);
+  return ballot(d2 <= b2);
+}
+
 // Per-wavefront LDS of the pair-compacted leaf evaluation (leaf_pairs): the leaf's triangle
 // records, every (lane, triangle) pair the screen passed, and each lane's best key.
 struct alignas(64) PairLds
@@ -627,79 +735,54 @@ static_assert(kMaxLeaf <= 16, "leaf slots are 4 bits");
 static_assert(sizeof(PairLds) == 4608, "PairLds layout");
 
 // Counting walks (wave-uniform): the pairs the pair-compacted leaves evaluated, their 64-lane
-// batches, the culling-record loads of the screen (4 triangles, 128 B each) and the leaves whose
-// slab was tested (one 4-B load each).
+// batches, the culling-record loads of the screen (4 triangles, 128 B each) and the leaves screened.
 struct PairCounts
 {
   uint32_t pairs, batches, groups, leaves;
 };
 
-// FP32 distance-only leaf, compacted: the screen (bounding sphere and plane against each lane's
-// bound, as in the wavefront-wide leaf) is run for every triangle of the leaf, and each passing
+// FP32 distance-only leaf, compacted: the screen (each triangle's disc against each lane's cull
+// radius, disc_lanes without a height) is run for every triangle of the leaf, and each passing
 // (lane, triangle) pair is appended to a list in LDS; then each lane evaluates one pair at a time
 // -- its triangle's record read from LDS, its query point from the pair's lane (ds_bpermute) --
 // and folds (d^2, triangle) into the pair lane's best key with an LDS atomic minimum. A
 // wavefront-wide evaluation costs a full evaluation's instructions whenever one lane needs the
 // triangle; here 64 needed pairs share those instructions, whichever lanes and triangles they
-// come from. A pair is evaluated on the triangle's in-plane frame (frame_eval32, a third fewer
-// instructions than tri_eval32), over the pairs the wavefront-wide leaf would evaluate (the
-// screen is the same conservative test, against bounds tightened once per leaf instead of per
-// triangle). The walk's d^2 is this function's minimum (among equal d^2 the lower triangle
-// index wins), whichever packets and subtree walks the query was part of; it agrees with the
-// wavefront-wide leaf's tri_eval32 minimum to FP32 rounding, and where two triangles' distances
-// agree to rounding the two may pick different ones.
-// Before the screen, the leaf's slab (MeshDev::lthick, about its first triangle's plane) skips
-// leaves that no lane comes within. The leaf's records are fetched (one 32-byte piece per lane)
-// only when some pair needs them: loading every visited leaf ahead of the screen, to hide the
-// load's latency behind it, fetched three leaves for each one used (1.4x the DRAM traffic) and
-// was 1% slower.
+// come from. The walk's d^2 is frame_eval32's minimum (among equal d^2 the lower triangle index
+// wins), whichever packets and subtree walks the query was part of.
 template <bool COUNT>
 __device__ __forceinline__ void leaf_pairs(const MeshDev& m, uint32_t first, uint32_t cnt, float px, float py,
-                                           float pz, float& bound, float& best, uint32_t& btri, uint32_t& n_tris,
-                                           uint32_t& w_tris, PairLds& L, PairCounts* pc)
+                                           float pz, float b2, float& bound, float& best, uint32_t& btri,
+                                           uint32_t& n_tris, uint32_t& w_tris, PairLds& L, PairCounts* pc)
 {
   const uint32_t lane = __lane_id();
   const uint32_t q0   = 2u * lane; // this lane's 16-byte pieces q0, q0 + 1 of the leaf's records
   const bool     mine = q0 < 8u * cnt;
   const float4* __restrict__ src = reinterpret_cast<const float4*>(m.frames + first);
 
-  const float rb = __builtin_amdgcn_sqrtf(bound) * 1.000001f; // 1-ulp hardware root, rounded up
-  SWords<32>  sp = sload<32>(m.tsph + 8 * (size_t)first); // culling records of the first 4 triangles
-  if (m.lthick) {
-    // the leaf's slab (its first triangle's plane, widened to hold the whole leaf) is a lower
-    // bound on every lane's distance to it: the screen is skipped when no lane reaches it. The
-    // plane comes with the first culling records (the same round trip).
-    typedef const __attribute__((address_space(4))) float ConstF;
-    const float t  = *(ConstF*)(m.lthick + first);
-    const float pd = fmaf(__uint_as_float(sp.w[4]), px,
-                          fmaf(__uint_as_float(sp.w[5]), py, fmaf(__uint_as_float(sp.w[6]), pz, __uint_as_float(sp.w[7]))));
-    if (COUNT && pc) {
-      pc->leaves++;
-      pc->groups++;
-    }
-    if (ballot(fabsf(pd) <= rb + t) == 0) return;
-    if (COUNT && pc) pc->groups += (cnt + 3u) / 4u - 1u;
+  if (COUNT && pc) {
+    pc->leaves++;
+    pc->groups += (cnt + 3u) / 4u;
   }
-  else if (COUNT && pc) pc->groups += (cnt + 3u) / 4u;
   uint32_t total = 0; // pairs listed (wave-uniform)
   for (uint32_t c0 = 0; c0 < cnt; c0 += 4) {
-    if (c0) sp = sload<32>(m.tsph + 8 * (size_t)(first + c0));
+    const SWords<32> sp = sload<32>(m.tdisc + first + c0); // culling records of 4 triangles
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       if (c0 + i < cnt) {
         const float sx = px - __uint_as_float(sp.w[8 * i]), sy = py - __uint_as_float(sp.w[8 * i + 1]),
                     sz = pz - __uint_as_float(sp.w[8 * i + 2]);
-        const float lim  = rb + __uint_as_float(sp.w[8 * i + 3]);
-        const bool  in_s = sx * sx + sy * sy + sz * sz <= lim * lim;
-        const float pd   = fmaf(__uint_as_float(sp.w[8 * i + 4]), px,
-                                fmaf(__uint_as_float(sp.w[8 * i + 5]), py,
-                                     fmaf(__uint_as_float(sp.w[8 * i + 6]), pz, __uint_as_float(sp.w[8 * i + 7]))));
-        const bool  in_p = fabsf(pd) <= rb;
-        if (COUNT) n_tris += (in_s && in_p) ? 1u : 0u;
-        const uint64_t pm = ballot(in_s) & ballot(in_p);
+        const float pd = __uint_as_float(sp.w[8 * i + 3]) * sx + __uint_as_float(sp.w[8 * i + 4]) * sy +
+                         __uint_as_float(sp.w[8 * i + 5]) * sz;
+        // disc_lanes with t = 0: (n.s)^2 + w = b2
+        const float w = fmaf(-pd, pd, b2);
+        const float B = fmaf(sz, sz, fmaf(sy, sy, fmaf(sx, sx, __uint_as_float(sp.w[8 * i + 7])))) - b2;
+        const bool  in_r = !(B * fabsf(B) > __uint_as_float(sp.w[8 * i + 6]) * w), in_p = !(w < 0.0f);
+        if (COUNT) n_tris += (in_r && in_p) ? 1u : 0u;
+        const uint64_t pm = ballot(in_r) & ballot(in_p);
         if (pm) {
-          // this lane's bit of pm is in_s && in_p: the write is predicated on the compares
-          if (in_s && in_p) L.pair[mbcnt(pm, total)] = (uint16_t)((lane << 4) | (c0 + (uint32_t)i));
+          // this lane's bit of pm is in_r && in_p: the write is predicated on the compares
+          if (in_r && in_p) L.pair[mbcnt(pm, total)] = (uint16_t)((lane << 4) | (c0 + (uint32_t)i));
           total += (uint32_t)__popcll(pm);
         }
       }
@@ -743,20 +826,178 @@ __device__ __forceinline__ void leaf_pairs(const MeshDev& m, uint32_t first, uin
   bound             = best < bound ? best : bound; // bound stays min(bound, best)
 }
 
+// Closest-face leaf: a triangle is evaluated by the whole wavefront when some lane's cull radius
+// reaches its disc; the cull bound is the band of the minimum (FaceCands::band), the distances are
+// in the mesh's own units, and every triangle inside the band is kept in fc.
+template <bool COUNT>
+__device__ __forceinline__ void leaf_face(const MeshDev& m, uint32_t first, uint32_t cnt, float px, float py, float pz,
+                                          float& b2, float& bound, float& best, uint32_t& btri, uint32_t& n_tris,
+                                          uint32_t& w_tris, FaceCands& fc)
+{
+  const float ux = px * m.inv_scale, uy = py * m.inv_scale, uz = pz * m.inv_scale, ss = m.scale * m.scale;
+  for (uint32_t c0 = 0; c0 < cnt; c0 += 4) {
+    const SWords<32> sp   = sload<32>(m.tdisc + first + c0);
+    uint32_t         need = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      if (c0 + i < cnt) {
+        const float sx = px - __uint_as_float(sp.w[8 * i]), sy = py - __uint_as_float(sp.w[8 * i + 1]),
+                    sz = pz - __uint_as_float(sp.w[8 * i + 2]);
+        const float pd = __uint_as_float(sp.w[8 * i + 3]) * sx + __uint_as_float(sp.w[8 * i + 4]) * sy +
+                         __uint_as_float(sp.w[8 * i + 5]) * sz;
+        const float w = fmaf(-pd, pd, b2);
+        const float B = fmaf(sz, sz, fmaf(sy, sy, fmaf(sx, sx, __uint_as_float(sp.w[8 * i + 7])))) - b2;
+        const bool  in_r = !(B * fabsf(B) > __uint_as_float(sp.w[8 * i + 6]) * w), in_p = !(w < 0.0f);
+        if (COUNT) n_tris += (in_r && in_p) ? 1u : 0u;
+        need |= (ballot(in_r) & ballot(in_p)) ? (1u << i) : 0u;
+      }
+    }
+    while (need) {
+      const uint32_t t = first + c0 + (uint32_t)__builtin_ctz(need);
+      need &= need - 1u;
+      const TriRec rec = sload_record(m.tris + t);
+      // the distance to the triangle's plane is a lower bound on the distance to it
+      const float fd = rec.n[0] * (ux - rec.v0[0]) + rec.n[1] * (uy - rec.v0[1]) + rec.n[2] * (uz - rec.v0[2]);
+      if (ballot(fd * fd <= bound) == 0) continue;
+      if (COUNT) w_tris++;
+      float    d2;
+      uint32_t f = 0;
+      tri_eval32<false>(rec, ux, uy, uz, d2, f);
+      if (d2 <= fc.lim) {
+        fc.insert(d2, t);
+        if (d2 < best) {
+          best   = d2;
+          btri   = t;
+          fc.lim = fc.band(d2);
+          bound  = fc.lim < bound ? fc.lim : bound;
+          b2     = cull_radius2(m, bound * ss);
+        }
+      }
+    }
+  }
+}
+
+// The walk from a node (interior: cnt0 = 0, or a leaf) over the mesh's WalkNodes. px, py, pz are
+// scaled. Distance-only (FACE = false): bound, best scaled, leaves by leaf_pairs. FACE: bound,
+// best in the mesh's own units, leaves by leaf_face. bound < 0: a lane without a query.
+template <int NB, bool COUNT, bool FACE>
+__device__ __forceinline__ void mesh_walk(const MeshDev& m, uint32_t ref0, uint32_t cnt0, float px, float py, float pz,
+                                          float bound, float& best, uint32_t& btri, uint32_t& n_inner, uint32_t& n_tris,
+                                          uint32_t& w_inner, uint32_t& w_tris, FaceCands* fc, PairLds* pl,
+                                          PairCounts* pc)
+{
+  WalkStack<NB> st;
+  st.init();
+  const int   lane = __lane_id();
+  const int   rep  = rep_lane(bound);
+  const float ss   = FACE ? m.scale * m.scale : 1.0f;
+  float       b2   = cull_radius2(m, FACE ? bound * ss : bound);
+  // Stamp of the bounds: it advances after every leaf that tightened some lane's bound, and each
+  // pushed entry carries it above the count's bits. An entry whose stamp is current was pushed
+  // because some lane reached it, and no bound has changed since, so the test at the pop would
+  // pass again: it is skipped (the bound floats are not even read). A skipped test can only
+  // cost work, never change a result; the counting walk always tests (its start entry carries a
+  // box that every lane with a query reaches).
+  uint32_t    stamp = 1u;
+  int         top   = 0;
+  const float everywhere[8] = {-INFINITY, -INFINITY, -INFINITY, INFINITY, INFINITY, INFINITY, 0.0f, 0.0f};
+  st.put(top++, ref0, cnt0 | kBoxChild | (stamp << kStampShift), everywhere);
+
+  while (top > 0) {
+    --top;
+    const uint32_t ecnt = st.cnt_at(top);
+    bool           need = true;
+    if (COUNT || (ecnt >> kStampShift) != stamp) {
+      float v[8], key;
+      st.bound_at(top, v);
+      const uint64_t mask = (ecnt & kBoxChild) ? walk_box_lanes(v, px, py, pz, b2, key)
+                                               : disc_lanes(v, px, py, pz, b2, key);
+      if (mask == 0) continue;
+      if (COUNT) need = ((mask >> lane) & 1ull) != 0;
+    }
+    const uint32_t eref = uni(st.ref_at(top)), cnt = ecnt & (kBoxChild - 1u);
+
+    if (cnt == 0u) {
+      if (COUNT) { n_inner += need ? 1u : 0u; w_inner++; }
+      const WalkNode nd  = sload_record(m.wnodes + eref);
+      const uint32_t tag = stamp << kStampShift;
+      uint64_t       msk[4];
+      uint32_t       key[4];
+      if (nd.cnt[0] & kBoxChild) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          msk[k] = 0;
+          key[k] = 0xFFFFFFFFu;
+          if (nd.cnt[k] != kInvalid) {
+            float d2;
+            msk[k] = walk_box_lanes(nd.v[k], px, py, pz, b2, d2);
+            key[k] = rdlane(__float_as_uint(d2), rep);
+          }
+        }
+      }
+      else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          msk[k] = 0;
+          key[k] = 0xFFFFFFFFu;
+          if (nd.cnt[k] != kInvalid) {
+            float s2; // order by the distance to the cylinder's centre
+            msk[k] = disc_lanes(nd.v[k], px, py, pz, b2, s2);
+            key[k] = rdlane(__float_as_uint(s2), rep);
+          }
+        }
+      }
+      int pushed = 0;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        if (!msk[k]) continue;
+        int rank = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          if (j == k || !msk[j]) continue;
+          rank += (key[j] > key[k] || (key[j] == key[k] && j < k)) ? 1 : 0;
+        }
+        st.put(top + rank, nd.ref[k], nd.cnt[k] | tag, nd.v[k]);
+        pushed++;
+      }
+      top += pushed;
+      // The capacity is the tree's exact worst case, computed at build time; should a walk ever
+      // exceed it, the pushes beyond it were dropped: record that in the mesh's status word
+      // (the host reports it) and go on with the entries that are held.
+      if (top > 64 * NB) {
+        if (lane == 0 && m.status) atomicOr(m.status, kStatusStackOverflow);
+        top = 64 * NB;
+      }
+    }
+    else {
+      const float bound0 = bound;
+      if constexpr (FACE) leaf_face<COUNT>(m, eref, cnt, px, py, pz, b2, bound, best, btri, n_tris, w_tris, *fc);
+      else leaf_pairs<COUNT>(m, eref, cnt, px, py, pz, b2, bound, best, btri, n_tris, w_tris, *pl, pc);
+      if (ballot(bound < bound0)) {
+        stamp++;
+        if constexpr (!FACE) b2 = cull_radius2(m, bound);
+      }
+    }
+  }
+}
+
+// The closest feature of the winning triangle (per-lane record load), at the point in the mesh's
+// own units.
+__device__ __forceinline__ uint32_t closest_feature(const MeshDev& m, uint32_t t, float px, float py, float pz)
+{
+  float    d2;
+  uint32_t f;
+  tri_eval32<true>(m.tris[t], px, py, pz, d2, f);
+  return f;
+}
+
 // R = float: FP32 pass on TriRec records. R = double: FP64 recheck on raw positions.
 // The walk starts at `start` (the root, or a subtree root of a split packet).
-// FACE (FP32 only): the cull bound is the band of the minimum (FaceCands::band) rather than the
-// minimum itself, the plane culls are off (their FP32 error is one of the coordinates, not of
-// the distance), and every triangle inside the band is kept in fc.
-// PAIRS (FP32 distance-only walks): leaves are evaluated by leaf_pairs in the wavefront's PairLds.
-template <int K, int NB, class R, bool COUNT, bool WMIN = (sizeof(R) == 8), bool FACE = false, bool PAIRS = false>
+template <int K, int NB, class R, bool COUNT, bool WMIN = (sizeof(R) == 8)>
 __device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& start, R px, R py, R pz, R bound, R& best,
                                               uint32_t& btri, uint32_t& bfeat, uint32_t& n_inner, uint32_t& n_tris,
-                                              uint32_t& w_inner, uint32_t& w_tris, FaceCands* fc = nullptr,
-                                              PairLds* pl = nullptr, PairCounts* pc = nullptr)
+                                              uint32_t& w_inner, uint32_t& w_tris)
 {
-  static_assert(!FACE || sizeof(R) == 4, "closest-face candidates: FP32 walk only");
-  static_assert(!PAIRS || (sizeof(R) == 4 && !FACE), "pair-compacted leaves: FP32 distance-only walks");
   const Node<K>* __restrict__ nodes = static_cast<const Node<K>*>(m.nodes);
   LaneStack<NB>               st;
   st.init();
@@ -795,11 +1036,6 @@ __device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& sta
         top = 64 * NB;
       }
     }
-    else if constexpr (PAIRS) {
-      const R bound0 = bound;
-      leaf_pairs<COUNT>(m, uni(eref), cnt, px, py, pz, bound, best, btri, n_tris, w_tris, *pl, pc);
-      if (ballot(bound < bound0)) stamp++;
-    }
     else {
       // leaf: a triangle is evaluated by the whole wavefront (keeping the minimum is exact for
       // every lane) unless, for every lane, its bounding sphere or its plane lies beyond the
@@ -815,7 +1051,7 @@ __device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& sta
       [[maybe_unused]] float cull = 0.0f; // FP32 distance-only walks: the lower-bound cull's limit
       if constexpr (sizeof(R) == 4) {
         rb = __builtin_amdgcn_sqrtf(bound) * 1.000001f; // 1-ulp hardware root, rounded up
-        if constexpr (!FACE) cull = cull_band(bound, m.hmax);
+        cull = cull_band(bound, m.hmax);
       }
       else rb = sqrt(bound);
       for (uint32_t c0 = 0; c0 < cnt; c0 += 4) {
@@ -829,7 +1065,7 @@ __device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& sta
             const R    lim = rb + R(__uint_as_float(sp.w[8 * i + 3]));
             const bool in_s = sx * sx + sy * sy + sz * sz <= lim * lim;
             bool       in_p = true;
-            if constexpr (sizeof(R) == 4 && !FACE) {
+            if constexpr (sizeof(R) == 4) {
               // the FP32 plane (rounded normal and offset) may misjudge by a few ulps of the
               // coordinates; the FP64 pass, whose seed only just contains the minimum, skips it
               const float pd = fmaf(__uint_as_float(sp.w[8 * i + 4]), px,
@@ -850,27 +1086,8 @@ __device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& sta
           uint32_t f = 0;
           if constexpr (sizeof(R) == 4) {
             const TriRec rec = sload_record(m.tris + t);
-            if constexpr (!FACE) {
-              if (!tri_eval32_culled(rec, px, py, pz, cull, d2)) continue;
-              if (COUNT) w_tris++;
-            }
-            else {
-              // the distance to the triangle's plane is a lower bound on the distance to it
-              const float fd = rec.n[0] * (px - rec.v0[0]) + rec.n[1] * (py - rec.v0[1]) + rec.n[2] * (pz - rec.v0[2]);
-              if (ballot(fd * fd <= bound) == 0) continue;
-              if (COUNT) w_tris++;
-              tri_eval32<false>(rec, px, py, pz, d2, f);
-              if (d2 <= fc->lim) {
-                fc->insert(d2, t);
-                if (d2 < best) {
-                  best    = d2;
-                  btri    = t;
-                  fc->lim = fc->band(d2);
-                  bound   = fc->lim < bound ? fc->lim : bound;
-                }
-              }
-              continue;
-            }
+            if (!tri_eval32_culled(rec, px, py, pz, cull, d2)) continue;
+            if (COUNT) w_tris++;
           }
           else {
             if (COUNT) w_tris++;
@@ -887,7 +1104,7 @@ __device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& sta
             btri  = t;
             bfeat = f;
             bound = d2 < bound ? d2 : bound; // bound stays min(bound, best)
-            if constexpr (sizeof(R) == 4 && !FACE) cull = cull_band(bound, m.hmax);
+            if constexpr (sizeof(R) == 4) cull = cull_band(bound, m.hmax);
           }
         }
       }
@@ -903,14 +1120,12 @@ __device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& sta
   }
 }
 
-template <int K, int NB, class R, bool COUNT, bool WMIN = (sizeof(R) == 8), bool FACE = false, bool PAIRS = false>
+template <int K, int NB, class R, bool COUNT, bool WMIN = (sizeof(R) == 8)>
 __device__ __forceinline__ void traverse(const MeshDev& m, R px, R py, R pz, R bound, R& best, uint32_t& btri,
-                                         uint32_t& bfeat, uint32_t& n_inner, uint32_t& n_tris, uint32_t& w_inner, uint32_t& w_tris,
-                                         FaceCands* fc = nullptr, PairLds* pl = nullptr, PairCounts* pc = nullptr)
+                                         uint32_t& bfeat, uint32_t& n_inner, uint32_t& n_tris, uint32_t& w_inner, uint32_t& w_tris)
 {
   const Entry root{0u, 0u, m.root_lo[0], m.root_lo[1], m.root_lo[2], m.root_hi[0], m.root_hi[1], m.root_hi[2]};
-  traverse_from<K, NB, R, COUNT, WMIN, FACE, PAIRS>(m, root, px, py, pz, bound, best, btri, bfeat, n_inner, n_tris,
-                                                    w_inner, w_tris, fc, pl, pc);
+  traverse_from<K, NB, R, COUNT, WMIN>(m, root, px, py, pz, bound, best, btri, bfeat, n_inner, n_tris, w_inner, w_tris);
 }
 
 } // namespace dev

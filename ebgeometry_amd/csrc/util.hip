@@ -61,53 +61,199 @@ __global__ void grid_points_kernel(GridSpec g, float* __restrict__ out)
   out[3 * p + 2]   = __double2float_rn(__dadd_rn(g.origin[2], __dmul_rn((double)k, g.spacing[2])));
 }
 
-// Slab of each leaf about its first triangle's plane (n, d of that triangle's culling record):
-// every vertex x of the leaf has |n.x + d| <= t, computed in FP64 from the exact vertex
-// positions, then widened so that the FP32 test |n.p + d| <= rb + t of the traversal never
-// rejects a leaf within rb of p: by 2^-20 (|d| + max |x|_1) for the FP32 evaluation of n.p + d
-// and the rounding of rb + t, then rounded up to FP32. (The part of the FP32 error that scales
-// with |p - x|, and |n| != 1, are covered by the 1e-6 the traversal adds to rb.)
-template <int K>
-__global__ __launch_bounds__(256) void leaf_slab_kernel(const Node<K>* __restrict__ nodes, uint32_t num_nodes,
-                                                        const float* __restrict__ tsph,
-                                                        const float* __restrict__ tripos, float* __restrict__ lthick)
+// Reductions over a workgroup of B threads, every thread getting the result.
+template <int B, class Op>
+__device__ __forceinline__ double block_reduce(double v, Op op)
 {
-  const uint64_t g = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (g >= (uint64_t)num_nodes * K) return;
-  const Node<K>& nd  = nodes[g / K];
-  const uint32_t k   = (uint32_t)(g % K);
-  const uint32_t cnt = nd.cnt[k];
-  if (cnt == 0u || cnt == kInvalid) return;
-  const uint32_t first = nd.ref[k];
-  const double   nx = tsph[8 * (size_t)first + 4], ny = tsph[8 * (size_t)first + 5];
-  const double   nz = tsph[8 * (size_t)first + 6], d = tsph[8 * (size_t)first + 7];
-  double         t = 0.0, r1 = 0.0;
-  for (uint32_t j = first; j < first + cnt; j++) {
-    const float* x = tripos + 12 * (size_t)j;
+  for (int o = 32; o > 0; o >>= 1) v = op(v, __shfl_xor(v, o, 64));
+  if constexpr (B > 64) {
+    __shared__ double sh[B / 64];
+    __syncthreads();
+    if ((threadIdx.x & 63u) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = sh[0];
+    for (int i = 1; i < B / 64; i++) v = op(v, sh[i]);
+  }
+  return v;
+}
+template <int B>
+__device__ __forceinline__ double block_sum(double v)
+{
+  return block_reduce<B>(v, [](double a, double b) { return a + b; });
+}
+template <int B>
+__device__ __forceinline__ double block_max(double v)
+{
+  return block_reduce<B>(v, [](double a, double b) { return fmax(a, b); });
+}
+
+// The cylinder of a range of triangles (one workgroup per listed child slot): axis along the
+// area-weighted normal, centre by extents along the axis and two directions across it, then moved
+// towards the farthest corner a few times (keeping the best), radius and half-height measured
+// from the centre and axis as rounded to FP32. The FP32 test (disc_lanes) rounds its own
+// quantities by up to 2^-21 of the record's size and of the cull radius, squared; the record's
+// part is covered here: R^2 + 2^-18 (R + t)^2, t + 2^-19 (R + t), rounded up. Everything depends
+// on the set of triangles only, up to the FP64 rounding of the normal's sum. A range whose normal
+// cancels has no axis: v[6] = -1, its node keeps the boxes.
+template <int B>
+__global__ __launch_bounds__(B) void walk_disc_kernel(const float* __restrict__ tripos, const uint32_t* __restrict__ range,
+                                                      const uint32_t* __restrict__ list, double scale,
+                                                      float* __restrict__ discs)
+{
+  const uint32_t slot = list[blockIdx.x], f = range[2 * (size_t)slot], l = range[2 * (size_t)slot + 1];
+  float*         out  = discs + 8 * (size_t)slot;
+  double         N[3] = {0.0, 0.0, 0.0}, A = 0.0;
+  for (uint32_t t = f + threadIdx.x; t < l; t += B) {
+    const float* x = tripos + 12 * (size_t)t;
+    double       a[3], b[3];
+    for (int c = 0; c < 3; c++) {
+      a[c] = ((double)x[3 + c] - x[c]) * scale;
+      b[c] = ((double)x[6 + c] - x[c]) * scale;
+    }
+    const double cx = a[1] * b[2] - a[2] * b[1], cy = a[2] * b[0] - a[0] * b[2], cz = a[0] * b[1] - a[1] * b[0];
+    N[0] += cx;
+    N[1] += cy;
+    N[2] += cz;
+    A += sqrt(cx * cx + cy * cy + cz * cz);
+  }
+  for (int c = 0; c < 3; c++) N[c] = block_sum<B>(N[c]);
+  A               = block_sum<B>(A);
+  const double nl = sqrt(N[0] * N[0] + N[1] * N[1] + N[2] * N[2]);
+  if (!(nl > 0.3 * A)) { // whole workgroup
+    if (threadIdx.x == 0) out[6] = -1.0f;
+    return;
+  }
+  float  nr[3];
+  double n[3], u[3], w[3];
+  for (int c = 0; c < 3; c++) n[c] = nr[c] = (float)(N[c] / nl);
+  {
+    const int m = fabs(n[0]) < 0.7 ? 0 : 1; // a coordinate axis away from n
+    double    q = 0.0;
+    for (int c = 0; c < 3; c++) u[c] = (c == m ? 1.0 : 0.0) - n[m] * n[c] / (n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+    for (int c = 0; c < 3; c++) q += u[c] * u[c];
+    for (int c = 0; c < 3; c++) u[c] /= sqrt(q);
+    const double nn = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+    w[0] = (n[1] * u[2] - n[2] * u[1]) / nn;
+    w[1] = (n[2] * u[0] - n[0] * u[2]) / nn;
+    w[2] = (n[0] * u[1] - n[1] * u[0]) / nn;
+  }
+  // extents along u, w and the axis (as -min, max)
+  double e[6];
+  for (int i = 0; i < 6; i++) e[i] = -INFINITY;
+  for (uint32_t t = f + threadIdx.x; t < l; t += B) {
+    const float* x = tripos + 12 * (size_t)t;
     for (int v = 0; v < 3; v++) {
-      const double px = x[3 * v], py = x[3 * v + 1], pz = x[3 * v + 2];
-      t  = fmax(t, fabs(nx * px + ny * py + nz * pz + d));
-      r1 = fmax(r1, fabs(px) + fabs(py) + fabs(pz));
+      const double px = x[3 * v] * scale, py = x[3 * v + 1] * scale, pz = x[3 * v + 2] * scale;
+      const double pu = u[0] * px + u[1] * py + u[2] * pz, pw = w[0] * px + w[1] * py + w[2] * pz,
+                   ph = n[0] * px + n[1] * py + n[2] * pz;
+      e[0] = fmax(e[0], -pu), e[1] = fmax(e[1], pu);
+      e[2] = fmax(e[2], -pw), e[3] = fmax(e[3], pw);
+      e[4] = fmax(e[4], -ph), e[5] = fmax(e[5], ph);
     }
   }
-  const double w = t * (1.0 + 0x1p-20) + 0x1p-20 * (fabs(d) + r1);
-  lthick[first]  = __double2float_ru(w);
+  for (int i = 0; i < 6; i++) e[i] = block_max<B>(e[i]);
+  double       cu = 0.5 * (e[1] - e[0]), cw = 0.5 * (e[3] - e[2]), bu = cu, bw = cw, best = INFINITY;
+  const double ch = 0.5 * (e[5] - e[4]) / (n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+  for (int it = 0; it < 8; it++) {
+    double far = -1.0, fu = 0.0, fw = 0.0; // the farthest corner in the plane (ties: largest pu, then pw)
+    for (uint32_t t = f + threadIdx.x; t < l; t += B) {
+      const float* x = tripos + 12 * (size_t)t;
+      for (int v = 0; v < 3; v++) {
+        const double px = x[3 * v] * scale, py = x[3 * v + 1] * scale, pz = x[3 * v + 2] * scale;
+        const double pu = u[0] * px + u[1] * py + u[2] * pz, pw = w[0] * px + w[1] * py + w[2] * pz;
+        const double d  = (pu - cu) * (pu - cu) + (pw - cw) * (pw - cw);
+        if (d > far || (d == far && (pu > fu || (pu == fu && pw > fw)))) {
+          far = d;
+          fu  = pu;
+          fw  = pw;
+        }
+      }
+    }
+    const double m  = block_max<B>(far);
+    const double mu = block_max<B>(far == m ? fu : -INFINITY);
+    const double mw = block_max<B>(far == m && fu == mu ? fw : -INFINITY);
+    if (m < best) {
+      best = m;
+      bu   = cu;
+      bw   = cw;
+    }
+    cu += (mu - cu) * (0.5 / (it + 2));
+    cw += (mw - cw) * (0.5 / (it + 2));
+  }
+  float cr[3];
+  for (int c = 0; c < 3; c++) cr[c] = (float)(bu * u[c] + bw * w[c] + ch * n[c]);
+  double t2 = 0.0, r2 = 0.0;
+  for (uint32_t t = f + threadIdx.x; t < l; t += B) {
+    const float* x = tripos + 12 * (size_t)t;
+    for (int v = 0; v < 3; v++) {
+      const double sx = x[3 * v] * scale - cr[0], sy = x[3 * v + 1] * scale - cr[1], sz = x[3 * v + 2] * scale - cr[2];
+      const double pd = n[0] * sx + n[1] * sy + n[2] * sz;
+      t2              = fmax(t2, fabs(pd));
+      r2              = fmax(r2, sx * sx + sy * sy + sz * sz - pd * pd);
+    }
+  }
+  t2 = block_max<B>(t2);
+  r2 = block_max<B>(r2);
+  if (threadIdx.x == 0) {
+    const double s = sqrt(r2) + t2;
+    for (int c = 0; c < 3; c++) {
+      out[c]     = cr[c];
+      out[3 + c] = nr[c];
+    }
+    out[6] = __double2float_ru(4.0 * (r2 + 0x1p-18 * s * s) * (1.0 + 1e-12));
+    out[7] = __double2float_ru((t2 + 0x1p-19 * s) * (1.0 + 1e-12));
+  }
+}
+
+// Per node: its children's cylinders in place of their boxes where every child has one that is
+// flat (t < 0.4 R: a patch bent further than that is left to its box, whose distance also orders
+// the children better: 40 against 60 nodes per packet on the 327,680-face displaced sphere) and
+// the cylinders, grown by a quarter of their radius, hold less volume than the boxes grown alike
+// (axis-aligned flat patches keep their boxes).
+__global__ __launch_bounds__(256) void walk_node_kernel(WalkNode* __restrict__ nodes, uint32_t num_nodes,
+                                                        const float* __restrict__ discs)
+{
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= num_nodes) return;
+  WalkNode& nd = nodes[i];
+  double    vd = 0.0, vb = 0.0;
+  for (int k = 0; k < 4; k++) {
+    if (nd.cnt[k] == kInvalid) continue;
+    const float* d = discs + 8 * ((size_t)4 * i + k);
+    if (!(d[6] >= 0.0f)) return;
+    const double R = 0.5 * sqrt((double)d[6]), t = d[7], g = 0.25 * R;
+    if (!(t < 0.4 * R)) return;
+    vd += 2.0 * (t + g) * M_PI * (R + g) * (R + g);
+    vb += ((double)nd.v[k][3] - nd.v[k][0] + 2 * g) * ((double)nd.v[k][4] - nd.v[k][1] + 2 * g) *
+          ((double)nd.v[k][5] - nd.v[k][2] + 2 * g);
+  }
+  if (!(vd < vb)) return;
+  for (int k = 0; k < 4; k++) {
+    if (nd.cnt[k] == kInvalid) continue;
+    for (int j = 0; j < 8; j++) nd.v[k][j] = discs[8 * ((size_t)4 * i + k) + j];
+    nd.cnt[k] &= ~kBoxChild;
+  }
 }
 
 // The in-plane frame record of each triangle (FrameRec), in FP64 from the FP32 vertices: the
 // longest edge becomes A -> B (a zero-length longest edge, a point triangle, takes the x axis),
 // ey is the unit part of C - A normal to ex (when C lies on the line AB, any unit vector normal
 // to ex: then c = 0 and no point is inside the face), ez = ex x ey. The edge parameters of a
-// zero-length edge are 0, so that edge's closest point is its start.
-__global__ __launch_bounds__(256) void frame_kernel(const float* __restrict__ tripos, uint64_t nt,
-                                                    FrameRec* __restrict__ out)
+// zero-length edge are 0, so that edge's closest point is its start. Beside it the triangle's
+// culling disc: the smallest circle of its plane that holds it (on the longest edge when the angle
+// at C is not acute, else through the corners), radius and the corners' distance from the disc's
+// plane measured from the centre and normal as rounded to FP32; the largest such distance of the
+// mesh goes to *off (float bits, zero on entry). All times `scale`.
+__global__ __launch_bounds__(256) void frame_kernel(const float* __restrict__ tripos, uint64_t nt, double scale,
+                                                    FrameRec* __restrict__ out, TriDisc* __restrict__ disc,
+                                                    uint32_t* __restrict__ off)
 {
   const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= nt) return;
   const float* x = tripos + 12 * i;
   double       P[3][3];
   for (int v = 0; v < 3; v++)
-    for (int c = 0; c < 3; c++) P[v][c] = x[3 * v + c];
+    for (int c = 0; c < 3; c++) P[v][c] = x[3 * v + c] * scale;
   double L[3];
   for (int j = 0; j < 3; j++) {
     const int k = j == 2 ? 0 : j + 1;
@@ -170,14 +316,52 @@ __global__ __launch_bounds__(256) void frame_kernel(const float* __restrict__ tr
   r.k2u = L2 > 0.0 ? (float)(b / L2) : 0.0f;
   r.k2v = L2 > 0.0 ? (float)(cc / L2) : 0.0f;
   out[i] = r;
+
+  double ou = 0.5 * a, ov = 0.0; // circle centre in the frame
+  if ((b - ou) * (b - ou) + cc * cc > ou * ou) ov = 0.5 * (b * b - a * b + cc * cc) / cc;
+  TriDisc d;
+  for (int c = 0; c < 3; c++) {
+    d.c[c] = (float)(A[c] + ou * ex[c] + ov * ey[c]);
+    d.n[c] = (float)ez[c];
+  }
+  double t2 = 0.0, r2 = 0.0;
+  for (int v = 0; v < 3; v++) {
+    const double sx = P[v][0] - d.c[0], sy = P[v][1] - d.c[1], sz = P[v][2] - d.c[2];
+    const double pd = (double)d.n[0] * sx + (double)d.n[1] * sy + (double)d.n[2] * sz;
+    t2              = fmax(t2, fabs(pd));
+    r2              = fmax(r2, sx * sx + sy * sy + sz * sz - pd * pd);
+  }
+  const double g = (r2 + 0x1p-18 * (sqrt(r2) + t2) * (sqrt(r2) + t2)) * (1.0 + 1e-12);
+  d.r2x4  = __double2float_ru(4.0 * g);
+  d.nr2   = -__double2float_ru(g);
+  disc[i] = d;
+  // the distance from the disc's plane, and the part of the test's own rounding that scales with
+  // the record's size (as in walk_disc_kernel)
+  atomicMax(off, __float_as_uint(__double2float_ru((t2 + 0x1p-19 * (sqrt(r2) + t2)) * (1.0 + 1e-12))));
 }
 
 } // namespace
 
-hipError_t launch_frames(const float* tripos, uint64_t nt, FrameRec* out, hipStream_t s)
+hipError_t launch_frames(const float* tripos, uint64_t nt, float scale, FrameRec* out, TriDisc* disc, uint32_t* off,
+                         hipStream_t s)
 {
   if (nt == 0) return hipSuccess;
-  hipLaunchKernelGGL(frame_kernel, dim3((uint32_t)((nt + 255) / 256)), dim3(256), 0, s, tripos, nt, out);
+  hipLaunchKernelGGL(frame_kernel, dim3((uint32_t)((nt + 255) / 256)), dim3(256), 0, s, tripos, nt, (double)scale, out,
+                     disc, off);
+  return hipGetLastError();
+}
+
+hipError_t launch_walk_nodes(const float* tripos, const uint32_t* range, const uint32_t* small, uint32_t num_small,
+                             const uint32_t* large, uint32_t num_large, float scale, float* discs, WalkNode* nodes,
+                             uint32_t num_nodes, hipStream_t s)
+{
+  if (num_small)
+    hipLaunchKernelGGL(walk_disc_kernel<64>, dim3(num_small), dim3(64), 0, s, tripos, range, small, (double)scale, discs);
+  if (num_large)
+    hipLaunchKernelGGL(walk_disc_kernel<1024>, dim3(num_large), dim3(1024), 0, s, tripos, range, large, (double)scale,
+                       discs);
+  if (num_nodes)
+    hipLaunchKernelGGL(walk_node_kernel, dim3((num_nodes + 255) / 256), dim3(256), 0, s, nodes, num_nodes, discs);
   return hipGetLastError();
 }
 
@@ -207,22 +391,6 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, uint32_t v, hipStream_t s)
 {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(fill_u32_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
-  return hipGetLastError();
-}
-
-hipError_t launch_leaf_slabs(const void* nodes, uint32_t num_nodes, int K, const float* tsph, const float* tripos,
-                             float* lthick, hipStream_t s)
-{
-  const uint64_t n = (uint64_t)num_nodes * (uint64_t)K;
-  if (n == 0) return hipSuccess;
-  const dim3 grid((uint32_t)((n + 255) / 256));
-  if (K == 4)
-    hipLaunchKernelGGL(leaf_slab_kernel<4>, grid, dim3(256), 0, s, static_cast<const Node<4>*>(nodes), num_nodes,
-                       tsph, tripos, lthick);
-  else if (K == 8)
-    hipLaunchKernelGGL(leaf_slab_kernel<8>, grid, dim3(256), 0, s, static_cast<const Node<8>*>(nodes), num_nodes,
-                       tsph, tripos, lthick);
-  else return hipErrorInvalidValue;
   return hipGetLastError();
 }
 

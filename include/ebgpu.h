@@ -166,7 +166,7 @@ typedef struct ebg_query_opts
                               (query, triangle) pairs evaluated by the pair-compacted leaves,
                               [1] their 64-lane evaluation batches, [2] the screen's loads of
                               culling records (4 triangles, 128 B each, per wavefront), [3] the
-                              leaves whose slab was tested (one 4-B load each, per wavefront).
+                              leaves whose triangles were screened (per wavefront).
                               NULL = not counted.                                            */
 } ebg_query_opts;
 
