@@ -43,20 +43,31 @@ void set_last_error(const std::string& s) { g_last_error = s; }
 // so the last of them to finish sets the end of the launch. A 32^3 grid over the mesh box (grown
 // by 10% per side) holds, per cell, the work of one packet of 64 queries spread over the cell
 // (4x4x4 lattice), measured once by a counting traversal; from then on every presorted query of
-// at least 2^14 points lists the packets whose most expensive cell reaches kHeavyFactor times the
+// at least kHandMaxQ points lists the packets whose most expensive cell reaches kHeavyFactor times the
 // grid mean; the leading workgroups of the traversal launch share each listed packet among
 // wavefronts that each walk one subtree of a frontier covering the tree, beside the bulk; the
 // packets between kEarlyFactor and that threshold start next, before the bulk in curve order.
 // Measured on the 327,680-face displaced sphere (K=4, leaf 16): kHeavyFactor 6 above 2^22
 // queries (the launch is full, and splitting costs extra work), 3 below (spare capacity); more
 // than 16 subtree roots only adds work.
-constexpr uint64_t kHeavyMinQ   = 1u << 14;
+constexpr uint64_t kHeavyMinQ   = 1u << 14; // ebg_mesh_last_split_packets counts from here on
 constexpr uint32_t kSplitBlocks = 2048; // workgroups that stride over the split items
 constexpr std::size_t kSplitRoots = 16;
 // Packets at >= 1.5x the grid mean that are not split are listed too and start right after the
 // split items, before the bulk (Hilbert-ordered 16M queries on the 327,680-face displaced sphere: 20.4 -> 17.4 ms).
 constexpr double kEarlyFactor = 1.5;
 static double heavy_factor(uint64_t n) { return n >= (1u << 22) ? 6.0 : 3.0; }
+// Below kHandMaxQ queries a wavefront that has visited kHandBudget[0] nodes and leaves hands the
+// rest of its walk on (HandOn) instead: nothing to measure beforehand, and any packet that turns
+// out long is shared, which is what a call needs whose launch is over before its longest packet is.
+// 1M uniform queries on the 20,480-face unit sphere: 1.07 ms split by the cost grid, 0.86 ms handed
+// on; 100 queries on it 3.65 -> 0.35 ms. The line lies where the launch itself is long enough to
+// hide the known long packets started first: 2M seeded queries on 81,920 faces take 1.34 ms split,
+// 1.49 ms handed on, 5.2M 2.14 against 2.45 ms, 16M on 327,680 faces 5.03 against 5.63 ms.
+// Budgets and spreads: (200, 100, 32, 16) 0.93 ms, (150, 60, 48, 32) 0.87, (100, 60, 32, 32) 0.86 on
+// the 1M queries.
+constexpr uint32_t kHandBudget[2] = {150, 60};
+constexpr int32_t  kHandSpread[2] = {48, 32};
 
 
 // Subtree roots for split packets: breadth-first from the root, each interior entry replaced by
@@ -532,15 +543,16 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   // counting launches run unsplit: the counters describe the plain traversal's own work; so do
   // closest-face queries (each lane decides its face from the band of its own whole walk)
   const bool face        = d_tri != nullptr;
-  const bool heavy_first = o.presort && n >= kHeavyMinQ && !o.work && !face && (may_alloc || m->grid_ready);
-  m->last_split           = heavy_first;
-  m->last_split_cap       = heavy_first ? Workspace::heavy_cap(n) : 0;
+  const bool hand_on     = !o.work && !face && n < kHandMaxQ;
+  const bool heavy_first = o.presort && n >= kHandMaxQ && !o.work && !face && (may_alloc || m->grid_ready);
+  m->last_split_cap      = heavy_first ? Workspace::heavy_cap(n)
+                                       : (hand_on && o.presort && n >= kHeavyMinQ ? ws.hand.slot_cap : 0);
   if (heavy_first) {
     const ebg_status gs = ensure_cost_grid(m, s);
     if (gs != EBG_OK) return gs;
   }
-  uint32_t* cnt = ws.counters; // [0] recheck, [1] fallback, [2] split packets, [3] early packets
-  EBG_HIP(launch_fill_u32(cnt, 4, 0u, s));
+  uint32_t* cnt = ws.counters; // [0] recheck, [1] fallback; [2] split, [3] early packets or [2..4] HandOn::counts
+  EBG_HIP(launch_fill_u32(cnt, 8, 0u, s));
 
   // The bound network needs no presort (it writes the radius by query index), so it runs on a
   // second stream of the handle, in query order, while the presort runs on the caller's stream.
@@ -636,11 +648,20 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
     }
   }
 
+  if (hand_on) {
+    a.hand = ws.hand;
+    for (int i = 0; i < 2; i++) {
+      a.hand.budget[i] = kHandBudget[i];
+      a.hand.spread[i] = kHandSpread[i];
+    }
+  }
+
   // events bracket the FP32 traversal (one launch for the bulk and the split items, then the
-  // split packets' resolve)
+  // split packets' resolve; or the packets, the handed-on items and their packets' end)
   if (timed) EBG_HIP(hipEventRecord(m->ev0, s));
   EBG_HIP(launch_sdf32(m->dev, m->wbanks, a, count, s));
   if (heavy_first) EBG_HIP(launch_sdf32_resolve(m->dev, a, s));
+  if (hand_on) EBG_HIP(launch_sdf32_handed(m->dev, m->wbanks, a, s));
   if (timed) {
     EBG_HIP(hipEventRecord(m->ev1, s));
     m->timed = true;
@@ -797,7 +818,7 @@ int64_t ebg_mesh_last_split_packets(const ebg_mesh* cm)
   ebg_mesh* m = const_cast<ebg_mesh*>(cm);
   if (!m) return -1;
   std::lock_guard<std::recursive_mutex> lock(m->mu);
-  if (!m->ws.cap || !m->last_split) return 0;
+  if (!m->ws.cap || !m->last_split_cap) return 0;
   uint32_t c = 0;
   if (hipDeviceSynchronize() != hipSuccess) return -1;
   if (hipMemcpy(&c, m->ws.counters() + 2, 4, hipMemcpyDeviceToHost) != hipSuccess) return -1;

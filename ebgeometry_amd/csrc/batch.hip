@@ -94,8 +94,11 @@ __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, Pai
   float    best = INFINITY;
   uint32_t btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
   PairCounts pc{0u, 0u, 0u, 0u};
-  mesh_walk<NB, COUNT, false>(m, 0u, 0u, px, py, pz, active ? INFINITY : -1.0f, best, btri, n_inner, n_tris, w_inner,
-                              w_tris, nullptr, pl, &pc);
+  float      bound = active ? INFINITY : -1.0f;
+  Walk<NB>   wk;
+  wk.start(0u, 0u);
+  mesh_walk<NB, COUNT, false, false>(m, wk, ~0u, 0, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris,
+                                     nullptr, pl, &pc);
   px *= m.inv_scale;
   py *= m.inv_scale;
   pz *= m.inv_scale;

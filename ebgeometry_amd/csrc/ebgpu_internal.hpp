@@ -149,6 +149,29 @@ struct MeshDev
 static_assert(sizeof(MeshDev) % 16 == 0, "MeshDev is read with 16-byte scalar loads");
 constexpr uint32_t kStatusStackOverflow = 1u;
 
+// Handing on the rest of a long walk (slot_cap = 0: never). A wavefront whose walk of its packet
+// has visited budget[0] nodes and leaves takes a slot, stores each lane's (d^2, triangle) so far in
+// keys[64 slot + lane] and the packet in list[slot], appends its stack to items[0], and ends. The
+// items are walked by a wavefront each in two more launches (one item: the subtree at `ref` for
+// the 64 queries of the slot's packet, from the bounds of its keys, folding into the keys with an
+// atomic minimum): the first hands on again after budget[1] visits, to items[1], the second walks
+// to the end. A last launch finishes the listed packets from their keys. A wavefront that finds
+// no room walks on instead.
+struct HandItem
+{
+  uint32_t slot, ref, cnt, pad; // slot kInvalid: no item
+};
+struct HandOn
+{
+  uint32_t            budget[2];
+  int32_t             spread[2]; // entries the stack is spread to before it is appended (at most 60)
+  uint32_t            slot_cap, item_cap;
+  uint32_t*           list;
+  unsigned long long* keys;
+  HandItem*           items[2];
+  uint32_t*           counts; // slots, items[0], items[1] (zero at the first launch)
+};
+
 // ---------------------------------------------------------------------------------------------
 // CSG union scenes: primitives in BVH leaf order
 // ---------------------------------------------------------------------------------------------

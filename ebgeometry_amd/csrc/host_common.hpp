@@ -75,8 +75,8 @@ hipError_t upload(DevBuf& b, const std::vector<T>& v)
 
 // Device memory of one query call, carved from a workspace: the presort keys and permutation,
 // the radix sort's scratch, the bounding-box partials, the FP64 recheck list, the counters, the
-// seeded radii, the recheck lane masks and the split/early packet schedule, for up to `cap`
-// queries.
+// seeded radii, the recheck lane masks and the split/early packet schedule or the handed-on
+// packets, for up to `cap` queries.
 struct WsView
 {
   uint64_t            cap = 0;
@@ -86,19 +86,24 @@ struct WsView
   void*               sort_scratch = nullptr; // radix_sort_scratch_bytes(cap)
   void*               box = nullptr;          // 6 doubles x (kBboxParts + 1)
   uint32_t*           recheck_list = nullptr; // cap
-  uint32_t*           counters = nullptr;     // 4: recheck, fallback, split packets, early packets
+  uint32_t*           counters = nullptr;     // 8: recheck, fallback, HandOn::counts (3), unused
   float*              seeds = nullptr;        // cap
   uint64_t*           rmask = nullptr;        // packets(cap)
   uint8_t*            heavy_flag = nullptr;   // packets(cap)
   uint32_t*           heavy_list = nullptr;   // heavy_cap(cap)
   unsigned long long* heavy_keys = nullptr;   // 64 x heavy_cap(cap)
   uint32_t*           early_list = nullptr;   // early_cap(cap)
+  HandOn              hand{};                 // lists of hand_slots(cap), hand_items(cap); no budgets
 };
+
+// Calls of fewer queries hand long walks on (HandOn); larger presorted ones split the packets that
+// their cost grid finds expensive.
+constexpr uint64_t kHandMaxQ = 1u << 20;
 
 // Query workspace, grown on demand.
 struct Workspace
 {
-  DevBuf   codes, codes_sorted, perm, sort_scratch, box, lists, seeds, sched, rmask;
+  DevBuf   codes, codes_sorted, perm, sort_scratch, box, lists, seeds, sched, handed, rmask;
   uint64_t cap = 0;
 
   hipError_t ensure(uint64_t n)
@@ -117,6 +122,7 @@ struct Workspace
     if ((e = rmask.reserve(8 * packets(m))) != hipSuccess) return e; // recheck lane mask per packet
     // split packets: one flag byte per packet, the list of split packets, 64 result keys each
     if ((e = sched.reserve(sched_early_offset(m) + 4 * (size_t)early_cap(m))) != hipSuccess) return e;
+    if ((e = handed.reserve(hand_bytes(m))) != hipSuccess) return e;
     cap = m;
     return hipSuccess;
   }
@@ -133,9 +139,33 @@ struct Workspace
   {
     return reinterpret_cast<unsigned long long*>(sched.as<uint8_t>() + sched_keys_offset(cap));
   }
+  // Room for handed-on packets: 1 in 16 (64-query packets), and at least 1,024, with 32 items each.
+  static uint32_t    hand_slots(uint64_t n) { return (uint32_t)(packets(std::min(n, kHandMaxQ)) / 16 + 1024); }
+  static uint32_t    hand_items(uint64_t n) { return 32 * hand_slots(n); }
+  static std::size_t hand_bytes(uint64_t n)
+  {
+    return part(4 * (std::size_t)hand_slots(n)) + part(512 * (std::size_t)hand_slots(n)) +
+           2 * part(sizeof(HandItem) * (std::size_t)hand_items(n));
+  }
+  static HandOn hand_view(uint8_t* base, uint64_t n, uint32_t* counts)
+  {
+    HandOn h{};
+    h.slot_cap = hand_slots(n);
+    h.item_cap = hand_items(n);
+    h.list     = reinterpret_cast<uint32_t*>(base);
+    base += part(4 * (std::size_t)h.slot_cap);
+    h.keys = reinterpret_cast<unsigned long long*>(base);
+    base += part(512 * (std::size_t)h.slot_cap);
+    for (int i = 0; i < 2; i++) {
+      h.items[i] = reinterpret_cast<HandItem*>(base);
+      base += part(sizeof(HandItem) * (std::size_t)h.item_cap);
+    }
+    h.counts = counts;
+    return h;
+  }
   uint32_t* recheck_list() const { return lists.as<uint32_t>(); }
   uint32_t* fallback_list() const { return lists.as<uint32_t>() + cap; }
-  uint32_t* counters() const { return lists.as<uint32_t>() + 2 * cap; } // [0] recheck [1] fallback [2] split [3] early
+  uint32_t* counters() const { return lists.as<uint32_t>() + 2 * cap; } // as WsView::counters
 
   WsView view() const
   {
@@ -154,6 +184,7 @@ struct Workspace
     v.heavy_list   = heavy_list();
     v.heavy_keys   = heavy_keys();
     v.early_list   = early_list();
+    v.hand         = hand_view(handed.as<uint8_t>(), cap, v.counters + 2);
     return v;
   }
 
@@ -163,8 +194,8 @@ struct Workspace
   {
     const uint64_t np = packets(cap);
     return 3 * part(4 * cap) + part(radix_sort_scratch_bytes(cap)) + part(sizeof(double) * 6 * (kBboxParts + 1)) +
-           part(4 * cap) + part(16) + part(4 * cap) + part(8 * np) + part(np) + part(4 * (size_t)heavy_cap(cap)) +
-           part(512 * (size_t)heavy_cap(cap)) + part(4 * (size_t)early_cap(cap));
+           part(4 * cap) + part(32) + part(4 * cap) + part(8 * np) + part(np) + part(4 * (size_t)heavy_cap(cap)) +
+           part(512 * (size_t)heavy_cap(cap)) + part(4 * (size_t)early_cap(cap)) + hand_bytes(cap);
   }
   static WsView carve(uint8_t* base, uint64_t cap)
   {
@@ -182,13 +213,14 @@ struct Workspace
     v.sort_scratch = take(radix_sort_scratch_bytes(cap));
     v.box          = take(sizeof(double) * 6 * (kBboxParts + 1));
     v.recheck_list = reinterpret_cast<uint32_t*>(take(4 * cap));
-    v.counters     = reinterpret_cast<uint32_t*>(take(16));
+    v.counters     = reinterpret_cast<uint32_t*>(take(32));
     v.seeds        = reinterpret_cast<float*>(take(4 * cap));
     v.rmask        = reinterpret_cast<uint64_t*>(take(8 * np));
     v.heavy_flag   = take(np);
     v.heavy_list   = reinterpret_cast<uint32_t*>(take(4 * (size_t)heavy_cap(cap)));
     v.heavy_keys   = reinterpret_cast<unsigned long long*>(take(512 * (size_t)heavy_cap(cap)));
     v.early_list   = reinterpret_cast<uint32_t*>(take(4 * (size_t)early_cap(cap)));
+    v.hand         = hand_view(take(hand_bytes(cap)), cap, v.counters + 2);
     return v;
   }
 };
@@ -233,8 +265,7 @@ struct ebg_mesh
   bool                   grid_ready = false;
   float                  grid_lo[3]{}, grid_scale[3]{};
   double                 grid_mean = 0; // mean packet cost over the grid cells
-  bool                   last_split     = false; // the last query listed split packets ...
-  int64_t                last_split_cap = 0;     // ... up to this many
+  int64_t                last_split_cap = 0; // the last query could split or hand on this many packets
   std::vector<float>     host_xyz; // vertex positions (scene instance bounds)
   std::vector<uint32_t>  order;    // original face index of each leaf-order triangle
   // polygon meshes: the polygon each triangle was clipped from (host and device copies); the
@@ -271,10 +302,9 @@ constexpr uint32_t kCostGrid = 32; // cells per axis of a mesh's packet cost gri
 ebg_status ensure_cost_grid(ebg_mesh* m, hipStream_t s);
 // Validate a lattice (origin, spacing, dims; at most 2^32-1 points) into g; n = its point count.
 ebg_status grid_spec(const double* origin, const double* spacing, const uint64_t* dims, GridSpec& g, uint64_t& n);
-// The mesh query pipeline (presort, [bound network], FP32 traversal with split packets, FP64
+// The mesh query pipeline (presort, [bound network], FP32 traversal with handed-on packets, FP64
 // recheck) over a caller-chosen workspace of at least n queries. With may_alloc false nothing is
-// allocated or created: split packets only if the cost grid already exists, the bound network
-// on the caller's stream, no traversal timing. The caller holds m->mu.
+// allocated or created: the bound network runs on the caller's stream, no traversal timing. The caller holds m->mu.
 ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_dist, uint32_t* d_tri,
                           const ebg_query_opts& o, const WsView& ws, bool may_alloc);
 inline void mesh_retain(ebg_mesh* m) { m->refs.fetch_add(1); }

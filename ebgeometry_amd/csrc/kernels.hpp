@@ -46,6 +46,7 @@ struct QueryArgs
   const uint32_t*     early_list;
   const uint32_t*     early_count;
   uint32_t            early_cap, early_blocks;
+  HandOn              hand; // (not together with split packets)
 };
 
 // Cost flags of the split schedule, set while the presort keys are made: a query whose
@@ -86,6 +87,10 @@ hipError_t launch_recheck_compact(const uint64_t* mask, uint64_t n, const uint32
 // After the FP32 launch: the split packets' winning triangles classified, signed and written like
 // the plain pass (outputs, recheck list).
 hipError_t launch_sdf32_resolve(const MeshDev& m, const QueryArgs& a, hipStream_t s);
+
+// After the FP32 launch: the handed-on items, then the listed packets' winning triangles
+// classified, signed and written like the plain pass (outputs, recheck list).
+hipError_t launch_sdf32_handed(const MeshDev& m, int banks, const QueryArgs& a, hipStream_t s);
 
 // FP32 packet traversal over the walk tree; banks = its stack capacity / 64 (1..4).
 hipError_t launch_sdf32(const MeshDev& m, int banks, const QueryArgs& a, bool count, hipStream_t s);

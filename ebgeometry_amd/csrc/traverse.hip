@@ -122,7 +122,7 @@ __device__ __forceinline__ float decide_face64(const MeshDev& m, const FaceCands
 // FACE (closest faces requested): each lane decides its face exactly (decide_face64); a lane
 // whose band held more triangles than its list goes to the FP64 pass with the near-surface ones.
 // Distance-only variants (!FACE) evaluate leaves pair-compacted in the wavefront's PairLds.
-template <int NB, bool COUNT, int MODE, bool FACE>
+template <int NB, bool COUNT, int MODE, bool FACE, bool HAND>
 __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& a, uint64_t n, uint64_t pk, PairLds* pl)
 {
   const uint64_t tid    = pk * 64u + (uint64_t)__lane_id();
@@ -155,38 +155,62 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
   FaceCands   fc;
   if constexpr (FACE) fc.init(m.hmax);
   PairCounts pc{0u, 0u, 0u, 0u};
-  mesh_walk<NB, COUNT, FACE>(m, 0u, 0u, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, &fc, pl, &pc);
-
-  // Exact only if some triangle lies within the seeded radius: otherwise nodes between the
-  // seeded radius and the true distance were pruned, and the query must be redone unseeded.
-  // The redo runs here, in the same wavefront (the other lanes sit it out with bound -1), so a
-  // rare expensive query is hidden among the other wavefronts of the launch instead of being
-  // serialised in a launch of its own.
-  bool found = active && btri != kInvalid && best <= seed2;
-  if (MODE == kSeeded) {
-    const bool     redo  = active && !found;
-    const uint64_t rmask = ballot(redo);
-    if (rmask) {
-      float     best2 = INFINITY;
-      uint32_t  btri2 = kInvalid, f_inner = 0, f_tris = 0;
-      FaceCands fc2;
-      if constexpr (FACE) fc2.init(m.hmax);
-      mesh_walk<NB, COUNT, FACE>(m, 0u, 0u, px, py, pz, redo ? INFINITY : -1.0f, best2, btri2, f_inner, f_tris, w_inner,
-                                 w_tris, &fc2, pl, &pc);
-      if (redo) {
-        best = best2;
-        btri = btri2;
-        if constexpr (FACE) fc = fc2;
+  Walk<NB>   wk;
+  wk.start(0u, 0u);
+  // A seeded walk is exact only for the lanes that found a triangle within their seed: for the
+  // others, nodes between the seed and the true distance were pruned. Those lanes walk again
+  // unseeded (from the distances they have), in the same wavefront, while the others sit it out
+  // with bound -1; a rare expensive query is so hidden among the other wavefronts of the launch.
+  bool     seeded = MODE == kSeeded, redo = false;
+  uint32_t budget = HAND ? a.hand.budget[0] : ~0u;
+  [[maybe_unused]] uint32_t s_inner = 0, s_tris = 0; // the seeded walk's counts
+  for (;;) {
+    mesh_walk<NB, COUNT, FACE, HAND>(m, wk, budget, HAND ? a.hand.spread[0] : 0, px, py, pz, bound, best, btri, n_inner,
+                                     n_tris, w_inner, w_tris, &fc, pl, &pc);
+    const bool missed = MODE == kSeeded && seeded && active && !(btri != kInvalid && best <= seed2);
+    if (HAND && wk.top > 0) {
+      const uint64_t mmask = ballot(missed);
+      if (mmask) {
+        // the pruned part is not on the stack: start over without the seeds
+        seeded = false;
+        wk.start(0u, 0u);
+        if (__lane_id() == 0) atomicAdd(a.fallback_count, (uint32_t)__popcll(mmask));
       }
-      found = active && btri != kInvalid;
-      if (__lane_id() == 0) atomicAdd(a.fallback_count, (uint32_t)__popcll(rmask));
-      if (COUNT && a.work) {
-        const uint64_t fi = wave_sum_u64(redo ? (uint64_t)f_inner : 0ull);
-        const uint64_t ft = wave_sum_u64(redo ? (uint64_t)f_tris : 0ull);
-        if (__lane_id() == 0) {
-          atomicAdd(a.work + 6, (unsigned long long)fi);
-          atomicAdd(a.work + 7, (unsigned long long)ft);
-        }
+      if (hand_on(a.hand, wk, (uint32_t)pk, best, btri)) return; // whole wavefront
+      if (MODE == kSeeded && !redo && active) bound = best;
+      budget = ~0u;
+      continue;
+    }
+    if (MODE != kSeeded) break;
+    const uint64_t rmask = ballot(missed);
+    if (!rmask) break;
+    seeded = false;
+    redo   = missed;
+    if (__lane_id() == 0) atomicAdd(a.fallback_count, (uint32_t)__popcll(rmask));
+    if constexpr (FACE) {
+      if (redo) {
+        fc.init(m.hmax);
+        best = INFINITY;
+        btri = kInvalid;
+      }
+    }
+    s_inner = n_inner;
+    s_tris  = n_tris;
+    bound   = redo ? best : -1.0f;
+    wk.start(0u, 0u);
+  }
+  const bool found = active && btri != kInvalid;
+  if constexpr (MODE == kSeeded && COUNT) {
+    if (ballot(redo) && a.work) { // the redone lanes' counts of their second walk
+      const uint64_t fi = wave_sum_u64(redo ? (uint64_t)(n_inner - s_inner) : 0ull);
+      const uint64_t ft = wave_sum_u64(redo ? (uint64_t)(n_tris - s_tris) : 0ull);
+      if (__lane_id() == 0) {
+        atomicAdd(a.work + 6, (unsigned long long)fi);
+        atomicAdd(a.work + 7, (unsigned long long)ft);
+      }
+      if (redo) {
+        n_inner = s_inner;
+        n_tris  = s_tris;
       }
     }
   }
@@ -263,8 +287,11 @@ __device__ __forceinline__ void split_item(const MeshDev& m, const QueryArgs& a,
   const SplitRoot rt = sload_record(a.split_roots + r);
   float           best = INFINITY;
   uint32_t        btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
-  mesh_walk<NB, COUNT, false>(m, rt.ref, rt.cnt, px, py, pz, active ? INFINITY : -1.0f, best, btri, n_inner, n_tris,
-                              w_inner, w_tris, nullptr, pl, nullptr);
+  float           bound = active ? INFINITY : -1.0f;
+  Walk<NB>        wk;
+  wk.start(rt.ref, rt.cnt);
+  mesh_walk<NB, COUNT, false, false>(m, wk, ~0u, 0, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, nullptr, pl,
+                              nullptr);
   if (active && btri != kInvalid)
     atomicMin(a.split_keys + 64 * (size_t)j + lane, ((unsigned long long)__float_as_uint(best) << 32) | btri);
   if (COUNT && a.work) {
@@ -283,7 +310,7 @@ __device__ __forceinline__ void split_item(const MeshDev& m, const QueryArgs& a,
 // mapped XCD-aware so that each XCD works through one contiguous (Morton) range of queries.
 // The leading split_blocks workgroups (dispatched first) work through the split items instead,
 // beside the packets of the bulk; packets flagged in heavy_flag are skipped.
-template <int NB, bool COUNT, int MODE, bool FACE>
+template <int NB, bool COUNT, int MODE, bool FACE, bool HAND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FACE ? 1 : (NB == 1 ? 8 : (NB == 2 ? 6 : 4))))) void sdf32_kernel(const MeshDev m, const QueryArgs a)
 {
   const uint32_t wave = uni(threadIdx.x >> 6); // known uniform: list entries load as scalars
@@ -305,7 +332,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FACE ? 1 : 
   if (a.early_blocks) {
     if (b < a.early_blocks) {
       const uint32_t j = b * 4u + wave;
-      if (j < min(*a.early_count, a.early_cap)) sdf32_packet<NB, COUNT, MODE, FACE>(m, a, a.n, a.early_list[j], pl);
+      if (j < min(*a.early_count, a.early_cap)) sdf32_packet<NB, COUNT, MODE, FACE, HAND>(m, a, a.n, a.early_list[j], pl);
       return;
     }
     b -= a.early_blocks;
@@ -316,41 +343,87 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FACE ? 1 : 
   const uint64_t pk  = (uint64_t)blk * 4u + wave;
   if (pk * 64u >= n) return;                    // whole wavefront past the end
   if (a.heavy_flag && a.heavy_flag[pk]) return; // whole wavefront: a split or early packet
-  sdf32_packet<NB, COUNT, MODE, FACE>(m, a, n, pk, pl);
+  sdf32_packet<NB, COUNT, MODE, FACE, HAND>(m, a, n, pk, pl);
 }
 
-// One wavefront per listed packet: the winning triangle of each query, as the plain pass ends.
-__global__ __launch_bounds__(256) void sdf32_resolve_kernel(const MeshDev m, const QueryArgs a)
+// The items handed on (HandOn): wavefronts stride over items[STAGE]. Each walks its subtree for the
+// 64 queries of the slot's packet from the distances found so far and folds what it finds into
+// the keys. d^2 >= 0, so its bits order like the value; on equal d^2 the lower triangle index
+// wins, as within a walk. Stage 0 hands on again after budget[1] visits, stage 1 walks to the end.
+template <int NB, int STAGE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8 : (NB == 2 ? 6 : 4)))) void sdf32_items_kernel(const MeshDev m, const QueryArgs a)
 {
-  const uint32_t j = uni(blockIdx.x * 4u + (threadIdx.x >> 6));
-  if (j >= min(*a.split_count, a.split_cap)) return; // whole wavefront
-  const uint64_t pk     = a.split_list[j];
-  const uint64_t tid    = pk * 64u + __lane_id();
-  const bool     active = tid < a.n;
-  bool           found  = false;
-  uint32_t       qi     = 0;
-  float          d      = 0.0f;
-  if (active) {
-    qi                           = a.idx ? a.idx[tid] : (uint32_t)tid;
-    const unsigned long long key = a.split_keys[64 * (size_t)j + __lane_id()];
-    const uint32_t           t   = (uint32_t)key;
-    if (t != kInvalid) {
-      const float px = a.pts[3 * (size_t)qi], py = a.pts[3 * (size_t)qi + 1], pz = a.pts[3 * (size_t)qi + 2];
-      float       d2;
-      uint32_t    feat;
-      tri_eval32<true>(m.tris[t], px, py, pz, d2, feat);
-      d2          = __uint_as_float((uint32_t)(key >> 32)) * (m.inv_scale * m.inv_scale); // the walk's, unscaled
-      d           = resolve32(m, t, feat, d2, px, py, pz);
-      a.out_d[qi] = d;
-      if (a.out_tri) a.out_tri[qi] = m.tris[t].face;
-      found = true;
+  const uint32_t wave = uni(threadIdx.x >> 6), lane = __lane_id();
+  extern __shared__ PairLds pair_lds[];
+  PairLds* const pl = &pair_lds[wave];
+  const uint32_t n  = min(a.hand.counts[1 + STAGE], a.hand.item_cap);
+  for (uint32_t w = uni(blockIdx.x * 4u + wave); w < n; w += gridDim.x * 4u) {
+    const SWords<4> it = sload<4>(a.hand.items[STAGE] + w);
+    if (it.w[0] == kInvalid) continue;
+    const uint32_t      slot = it.w[0];
+    const uint64_t      tid  = (uint64_t)uni(a.hand.list[slot]) * 64u + lane;
+    unsigned long long* keys = a.hand.keys + 64 * (size_t)slot + lane;
+    const uint64_t      key  = *keys;
+    float               px = 0.0f, py = 0.0f, pz = 0.0f, bound = -1.0f;
+    if (tid < a.n) {
+      const uint32_t qi = a.idx ? a.idx[tid] : (uint32_t)tid;
+      px                = a.pts[3 * (size_t)qi] * m.scale;
+      py                = a.pts[3 * (size_t)qi + 1] * m.scale;
+      pz                = a.pts[3 * (size_t)qi + 2] * m.scale;
+      bound             = __uint_as_float((uint32_t)(key >> 32));
+      if (!(px == px && py == py && pz == pz)) { // as in sdf32_packet
+        px = py = pz = 0.0f;
+        bound        = -1.0f;
+      }
     }
+    float    best = __uint_as_float((uint32_t)(key >> 32));
+    uint32_t btri = (uint32_t)key, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
+    Walk<NB> wk;
+    wk.start(it.w[1], it.w[2]);
+    uint32_t budget = STAGE == 0 ? a.hand.budget[1] : ~0u;
+    for (;;) {
+      mesh_walk<NB, false, false, true>(m, wk, budget, a.hand.spread[1], px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, nullptr,
+                                  pl, nullptr);
+      if (wk.top == 0 || append_items(wk, slot, a.hand.items[1], a.hand.counts + 2, a.hand.item_cap)) break;
+      budget = ~0u; // no room: walk on
+    }
+    const uint64_t now = ((uint64_t)__float_as_uint(best) << 32) | btri;
+    if (now < key) atomicMin(keys, (unsigned long long)now);
   }
-  if (a.recheck_mask) {
-    const uint64_t rm = ballot(found && fabsf(d) < a.recheck_abs);
-    if (__lane_id() == 0) a.recheck_mask[pk] = rm;
+}
+
+// Wavefronts stride over the listed packets (split or handed on): the winning triangle of each
+// query from the packet's keys, as the plain pass ends.
+__global__ __launch_bounds__(256) void sdf32_resolve_kernel(const MeshDev m, const QueryArgs a, const uint32_t* list,
+                                                            const unsigned long long* result_keys, const uint32_t* count,
+                                                            uint32_t cap)
+{
+  const uint32_t n = min(*count, cap);
+  for (uint32_t j = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); j < n; j += gridDim.x * 4u) {
+    const uint32_t pk = uni(list[j]);
+    if (pk == kInvalid) continue;
+    const uint64_t tid   = (uint64_t)pk * 64u + __lane_id();
+    bool           found = false;
+    uint32_t       qi    = 0;
+    float          d     = 0.0f;
+    if (tid < a.n) {
+      qi                           = a.idx ? a.idx[tid] : (uint32_t)tid;
+      const unsigned long long key = result_keys[64 * (size_t)j + __lane_id()];
+      const uint32_t           t   = (uint32_t)key;
+      if (t != kInvalid) {
+        const float px = a.pts[3 * (size_t)qi], py = a.pts[3 * (size_t)qi + 1], pz = a.pts[3 * (size_t)qi + 2];
+        const float d2 = __uint_as_float((uint32_t)(key >> 32)) * (m.inv_scale * m.inv_scale); // the walk's, unscaled
+        d              = resolve32(m, t, closest_feature(m, t, px, py, pz), d2, px, py, pz);
+        a.out_d[qi]    = d;
+        found          = true;
+      }
+    }
+    if (a.recheck_mask) {
+      const uint64_t rm = ballot(found && fabsf(d) < a.recheck_abs);
+      if (__lane_id() == 0) a.recheck_mask[pk] = rm;
+    }
+    else if (a.recheck_list) wave_append(found && fabsf(d) < a.recheck_abs, qi, a.recheck_list, a.recheck_count);
   }
-  else if (a.recheck_list) wave_append(found && fabsf(d) < a.recheck_abs, qi, a.recheck_list, a.recheck_count);
 }
 
 // one wavefront per 64 consecutive packets
@@ -431,8 +504,10 @@ template <int NB, int MODE, bool FACE>
 void launch32f(const MeshDev& m, const QueryArgs& a, bool count, uint32_t blocks, hipStream_t s)
 {
   const size_t lds = FACE ? 0 : 4 * sizeof(PairLds);
-  if (count) hipLaunchKernelGGL((sdf32_kernel<NB, true, MODE, FACE>), dim3(blocks), dim3(256), lds, s, m, a);
-  else hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, FACE>), dim3(blocks), dim3(256), lds, s, m, a);
+  if (count) hipLaunchKernelGGL((sdf32_kernel<NB, true, MODE, FACE, false>), dim3(blocks), dim3(256), lds, s, m, a);
+  else if (a.hand.slot_cap && !FACE)
+    hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, FACE, !FACE>), dim3(blocks), dim3(256), lds, s, m, a);
+  else hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, FACE, false>), dim3(blocks), dim3(256), lds, s, m, a);
 }
 
 // closest faces requested: the exact-face variant (its split packets are off: see launch32)
@@ -450,6 +525,9 @@ hipError_t launch32(const MeshDev& m, const QueryArgs& a, bool count, hipStream_
   if (blocks == 0) return hipSuccess;
   if (a.count_ptr) return hipErrorInvalidValue;
   if (a.split_blocks && (!a.split_nroots || !a.split_count || !a.heavy_flag)) return hipErrorInvalidValue;
+  if (a.hand.slot_cap && (a.split_blocks || a.out_tri || !a.hand.list || !a.hand.keys || !a.hand.items[0] ||
+                          !a.hand.items[1] || !a.hand.counts))
+    return hipErrorInvalidValue;
   // exact closest faces need each lane's whole candidate band in one walk: no split packets, and
   // the FP64 pass must follow (lanes whose band overflowed are listed for it)
   if (a.out_tri && (a.split_blocks || (!a.recheck_mask && !a.recheck_list))) return hipErrorInvalidValue;
@@ -553,10 +631,35 @@ hipError_t launch_recheck_compact(const uint64_t* mask, uint64_t n, const uint32
 
 hipError_t launch_sdf32_resolve(const MeshDev& m, const QueryArgs& a, hipStream_t s)
 {
-  const uint32_t blocks = (a.split_cap + 3) / 4;
-  if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(sdf32_resolve_kernel, dim3(blocks), dim3(256), 0, s, m, a);
+  if (a.split_cap == 0) return hipSuccess;
+  hipLaunchKernelGGL(sdf32_resolve_kernel, dim3(std::min((a.split_cap + 3u) / 4u, kListGrid)), dim3(256), 0, s, m, a,
+                     a.split_list, a.split_keys, a.split_count, a.split_cap);
   return hipGetLastError();
+}
+
+namespace {
+
+// The lists' lengths are only known on the device: fixed grids stride over them.
+template <int NB>
+hipError_t launch_handed(const MeshDev& m, const QueryArgs& a, hipStream_t s)
+{
+  const size_t   lds    = 4 * sizeof(PairLds);
+  const uint32_t blocks = (uint32_t)std::clamp<uint64_t>((a.n + 255) / 256 * 8u, 512u, kListGrid);
+  hipLaunchKernelGGL((sdf32_items_kernel<NB, 0>), dim3(blocks), dim3(256), lds, s, m, a);
+  hipLaunchKernelGGL((sdf32_items_kernel<NB, 1>), dim3(blocks), dim3(256), lds, s, m, a);
+  hipLaunchKernelGGL(sdf32_resolve_kernel, dim3(std::min(blocks, (a.hand.slot_cap + 3u) / 4u)), dim3(256), 0, s, m, a,
+                     a.hand.list, a.hand.keys, a.hand.counts, a.hand.slot_cap);
+  return hipGetLastError();
+}
+
+} // namespace
+
+hipError_t launch_sdf32_handed(const MeshDev& m, int banks, const QueryArgs& a, hipStream_t s)
+{
+  if (a.n == 0 || !a.hand.slot_cap) return hipSuccess;
+  if (banks <= 1) return launch_handed<1>(m, a, s);
+  if (banks == 2) return launch_handed<2>(m, a, s);
+  return launch_handed<4>(m, a, s);
 }
 
 hipError_t launch_sdf64(const MeshDev& m, int K, int banks, const QueryArgs& a, hipStream_t s)

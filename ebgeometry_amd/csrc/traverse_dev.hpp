@@ -877,17 +877,134 @@ __device__ __forceinline__ void leaf_face(const MeshDev& m, uint32_t first, uint
   }
 }
 
-// The walk from a node (interior: cnt0 = 0, or a leaf) over the mesh's WalkNodes. px, py, pz are
-// scaled. Distance-only (FACE = false): bound, best scaled, leaves by leaf_pairs. FACE: bound,
-// best in the mesh's own units, leaves by leaf_face. bound < 0: a lane without a query.
-template <int NB, bool COUNT, bool FACE>
-__device__ __forceinline__ void mesh_walk(const MeshDev& m, uint32_t ref0, uint32_t cnt0, float px, float py, float pz,
-                                          float bound, float& best, uint32_t& btri, uint32_t& n_inner, uint32_t& n_tris,
+// A walk's state between calls of mesh_walk (wave-uniform but for the stack's lanes).
+template <int NB>
+struct Walk
+{
+  WalkStack<NB> st;
+  int           top;
+  uint32_t      stamp;
+
+  // Start at a node (interior: cnt = 0, or a leaf).
+  __device__ __forceinline__ void start(uint32_t ref, uint32_t cnt)
+  {
+    const float everywhere[8] = {-INFINITY, -INFINITY, -INFINITY, INFINITY, INFINITY, INFINITY, 0.0f, 0.0f};
+    st.init();
+    top   = 0;
+    stamp = 1u;
+    st.put(top++, ref, cnt | kBoxChild | (stamp << kStampShift), everywhere);
+  }
+};
+
+// Append the walk's stack to a list of items of `slot`. The stack's entries lie in its lanes, so
+// each lane stores its own. Without room nothing is listed (slots of the list taken by the attempt
+// hold kInvalid) and false is returned.
+template <int NB>
+__device__ __forceinline__ bool append_items(const Walk<NB>& wk, uint32_t slot, HandItem* items, uint32_t* count,
+                                             uint32_t cap)
+{
+  const uint32_t lane = __lane_id();
+  uint32_t       base = 0;
+  if (lane == 0) base = atomicAdd(count, (uint32_t)wk.top);
+  base            = rdlane(base, 0);
+  const bool fits = base <= cap && (uint32_t)wk.top <= cap - base;
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    const uint32_t pos = 64u * i + lane;
+    if (pos < (uint32_t)wk.top && base <= cap && pos < cap - base)
+      items[base + pos] = HandItem{fits ? slot : kInvalid, wk.st.ref[i], wk.st.cnt[i] & (kBoxChild - 1u), 0u};
+  }
+  return fits;
+}
+
+// Hand the rest of the walk of `packet` on (see HandOn); false: no room, walk on.
+template <int NB>
+__device__ __forceinline__ bool hand_on(const HandOn& h, const Walk<NB>& wk, uint32_t packet, float best, uint32_t btri)
+{
+  const uint32_t lane = __lane_id();
+  uint32_t       j    = 0;
+  if (lane == 0) j = atomicAdd(h.counts, 1u);
+  j = rdlane(j, 0);
+  if (j >= h.slot_cap) return false;
+  const bool ok                = append_items(wk, j, h.items[0], h.counts + 1, h.item_cap);
+  h.keys[64 * (size_t)j + lane] = ((unsigned long long)__float_as_uint(best) << 32) | btri;
+  if (lane == 0) h.list[j] = ok ? packet : kInvalid;
+  return ok;
+}
+
+// Visit a node: test its children and push the ones some lane reaches, ranked so that the farthest
+// from the representative lane's point lies deepest and the nearest is popped next (a box by its
+// distance, a cylinder by the distance to its centre).
+template <int NB>
+__device__ __forceinline__ void push_walk_children(const MeshDev& m, Walk<NB>& wk, uint32_t node, float px, float py,
+                                                   float pz, float b2, int rep)
+{
+  const WalkNode nd  = sload_record(m.wnodes + node);
+  const uint32_t tag = wk.stamp << kStampShift;
+  uint64_t       msk[4];
+  uint32_t       key[4];
+  if (nd.cnt[0] & kBoxChild) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      msk[k] = 0;
+      key[k] = 0xFFFFFFFFu;
+      if (nd.cnt[k] != kInvalid) {
+        float d2;
+        msk[k] = walk_box_lanes(nd.v[k], px, py, pz, b2, d2);
+        key[k] = rdlane(__float_as_uint(d2), rep);
+      }
+    }
+  }
+  else {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      msk[k] = 0;
+      key[k] = 0xFFFFFFFFu;
+      if (nd.cnt[k] != kInvalid) {
+        float s2;
+        msk[k] = disc_lanes(nd.v[k], px, py, pz, b2, s2);
+        key[k] = rdlane(__float_as_uint(s2), rep);
+      }
+    }
+  }
+  int pushed = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    if (!msk[k]) continue;
+    int rank = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      if (j == k || !msk[j]) continue;
+      rank += (key[j] > key[k] || (key[j] == key[k] && j < k)) ? 1 : 0;
+    }
+    wk.st.put(wk.top + rank, nd.ref[k], nd.cnt[k] | tag, nd.v[k]);
+    pushed++;
+  }
+  wk.top += pushed;
+  // The capacity is the tree's exact worst case, computed at build time; should a walk ever exceed
+  // it, the pushes beyond it were dropped: record that in the mesh's status word (the host reports
+  // it) and go on with the entries that are held.
+  if (wk.top > 64 * NB) {
+    if (__lane_id() == 0 && m.status) atomicOr(m.status, kStatusStackOverflow);
+    wk.top = 64 * NB;
+  }
+}
+
+// The walk over the mesh's WalkNodes from wk's stack until it is empty or (HAND) `budget` nodes and
+// leaves have been visited. Then the stack is spread for handing on: its lowest entries, the largest
+// subtrees, are replaced by their children until there are `spread` entries (a depth-first stack
+// alone holds a few subtrees of a quarter of the rest, a sixteenth, ...). px, py, pz are scaled. Distance-only (FACE = false): bound, best scaled,
+// leaves by leaf_pairs. FACE: bound, best in the mesh's own units, leaves by leaf_face. bound < 0:
+// a lane without a query.
+template <int NB, bool COUNT, bool FACE, bool HAND>
+__device__ __forceinline__ void mesh_walk(const MeshDev& m, Walk<NB>& wk, uint32_t budget, int spread, float px, float py, float pz,
+                                          float& bound, float& best, uint32_t& btri, uint32_t& n_inner, uint32_t& n_tris,
                                           uint32_t& w_inner, uint32_t& w_tris, FaceCands* fc, PairLds* pl,
                                           PairCounts* pc)
 {
-  WalkStack<NB> st;
-  st.init();
+  WalkStack<NB>& st    = wk.st;
+  int&           top   = wk.top;
+  uint32_t&      stamp = wk.stamp;
   const int   lane = __lane_id();
   const int   rep  = rep_lane(bound);
   const float ss   = FACE ? m.scale * m.scale : 1.0f;
@@ -898,12 +1015,7 @@ __device__ __forceinline__ void mesh_walk(const MeshDev& m, uint32_t ref0, uint3
   // pass again: it is skipped (the bound floats are not even read). A skipped test can only
   // cost work, never change a result; the counting walk always tests (its start entry carries a
   // box that every lane with a query reaches).
-  uint32_t    stamp = 1u;
-  int         top   = 0;
-  const float everywhere[8] = {-INFINITY, -INFINITY, -INFINITY, INFINITY, INFINITY, INFINITY, 0.0f, 0.0f};
-  st.put(top++, ref0, cnt0 | kBoxChild | (stamp << kStampShift), everywhere);
-
-  while (top > 0) {
+  while (top > 0 && (!HAND || budget > 0u)) {
     --top;
     const uint32_t ecnt = st.cnt_at(top);
     bool           need = true;
@@ -916,58 +1028,11 @@ __device__ __forceinline__ void mesh_walk(const MeshDev& m, uint32_t ref0, uint3
       if (COUNT) need = ((mask >> lane) & 1ull) != 0;
     }
     const uint32_t eref = uni(st.ref_at(top)), cnt = ecnt & (kBoxChild - 1u);
+    if constexpr (HAND) budget--;
 
     if (cnt == 0u) {
       if (COUNT) { n_inner += need ? 1u : 0u; w_inner++; }
-      const WalkNode nd  = sload_record(m.wnodes + eref);
-      const uint32_t tag = stamp << kStampShift;
-      uint64_t       msk[4];
-      uint32_t       key[4];
-      if (nd.cnt[0] & kBoxChild) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          msk[k] = 0;
-          key[k] = 0xFFFFFFFFu;
-          if (nd.cnt[k] != kInvalid) {
-            float d2;
-            msk[k] = walk_box_lanes(nd.v[k], px, py, pz, b2, d2);
-            key[k] = rdlane(__float_as_uint(d2), rep);
-          }
-        }
-      }
-      else {
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-          msk[k] = 0;
-          key[k] = 0xFFFFFFFFu;
-          if (nd.cnt[k] != kInvalid) {
-            float s2; // order by the distance to the cylinder's centre
-            msk[k] = disc_lanes(nd.v[k], px, py, pz, b2, s2);
-            key[k] = rdlane(__float_as_uint(s2), rep);
-          }
-        }
-      }
-      int pushed = 0;
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        if (!msk[k]) continue;
-        int rank = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          if (j == k || !msk[j]) continue;
-          rank += (key[j] > key[k] || (key[j] == key[k] && j < k)) ? 1 : 0;
-        }
-        st.put(top + rank, nd.ref[k], nd.cnt[k] | tag, nd.v[k]);
-        pushed++;
-      }
-      top += pushed;
-      // The capacity is the tree's exact worst case, computed at build time; should a walk ever
-      // exceed it, the pushes beyond it were dropped: record that in the mesh's status word
-      // (the host reports it) and go on with the entries that are held.
-      if (top > 64 * NB) {
-        if (lane == 0 && m.status) atomicOr(m.status, kStatusStackOverflow);
-        top = 64 * NB;
-      }
+      push_walk_children(m, wk, eref, px, py, pz, b2, rep);
     }
     else {
       const float bound0 = bound;
@@ -977,6 +1042,19 @@ __device__ __forceinline__ void mesh_walk(const MeshDev& m, uint32_t ref0, uint3
         stamp++;
         if constexpr (!FACE) b2 = cull_radius2(m, bound);
       }
+    }
+  }
+  if constexpr (HAND) {
+    // out of budget: spread the stack (rare)
+    for (int bot = 0; bot < top && top < spread; bot++) {
+      const uint32_t ecnt = st.cnt_at(bot);
+      if ((ecnt & (kBoxChild - 1u)) != 0u) continue; // a leaf stays as it is
+      const uint32_t eref = uni(st.ref_at(bot));
+      float          v[8];
+      top--; // the top entry takes its place
+      st.bound_at(top, v);
+      st.put(bot, st.ref_at(top), st.cnt_at(top), v);
+      push_walk_children(m, wk, eref, px, py, pz, b2, rep);
     }
   }
 }

@@ -175,10 +175,11 @@ void ebg_query_opts_default(ebg_query_opts* opts);
 
 /* d_pts: n float32 xyz triples; d_dist: n float32; d_tri (nullable): n uint32 face indices
  * (closest face, up to exact ties). Device pointers, asynchronous on opts->stream.
- * Split packets: with presort on and n >= 2^14, packets of 64 queries whose estimated cost (a
- * 32^3 grid of measured packet costs over the mesh box, built at the first such call) is a few
- * times the grid mean are each shared among 16 wavefronts walking disjoint subtrees, unseeded,
- * inside the same traversal launch; results are those of the plain traversal. */
+ * Long packets are shared: with presort on and n >= 2^20, packets of 64 queries whose estimated cost
+ * (a 32^3 grid of measured packet costs over the mesh box, built at the first such call) is a few
+ * times the grid mean are each split among 16 wavefronts walking disjoint subtrees, unseeded,
+ * inside the same traversal launch; in smaller calls a wavefront that finds its packet long hands
+ * the rest of its walk on to others. Results are those of the plain traversal. */
 ebg_status ebg_query_sdf(const ebg_mesh* mesh, const float* d_pts, uint64_t n, float* d_dist,
                          uint32_t* d_tri, const ebg_query_opts* opts);
 /* Allocation-free form of ebg_query_sdf. No counterpart in the reference: for callers that
@@ -188,9 +189,7 @@ ebg_status ebg_query_sdf(const ebg_mesh* mesh, const float* d_pts, uint64_t n, f
  * array of 40 MiB per GPU, held from the library's first use on that GPU until the process ends,
  * which limits a call to n <= EBG_NOALLOC_MAX_QUERIES (larger n: EBG_INVALID_ARG). Every call on
  * one GPU shares that array: calls that overlap on one GPU (other streams, other threads) race
- * and must be serialised by the caller. Differences from ebg_query_sdf: split packets are used
- * only once an ebg_query_sdf call of >= 2^14 presorted queries has built the mesh's cost grid;
- * the learned bound's network runs on opts->stream before the traversal (no second stream); the
+ * and must be serialised by the caller. Differences from ebg_query_sdf: the learned bound's network runs on opts->stream before the traversal (no second stream); the
  * traversal is not timed (ebg_mesh_last_traversal_ms keeps the previous value). */
 #define EBG_NOALLOC_MAX_QUERIES 1048576u
 ebg_status ebg_query_sdf_noalloc(const ebg_mesh* mesh, const float* d_pts, uint64_t n, float* d_dist,
@@ -235,8 +234,8 @@ double ebg_mesh_last_traversal_ms(const ebg_mesh* mesh);
  * expected outcome. No counterpart in the reference (its stack is a fixed 256 entries,
  * Source/EBGeometry_BVHImplem.hpp:1138). */
 ebg_status ebg_mesh_check(const ebg_mesh* mesh);
-/* Number of split packets of the last query on `mesh` (0 if none were split, <0 on error).
- * Diagnostic with no counterpart in the reference; waits for the device. */
+/* Number of packets of the last presorted query of at least 2^14 points on `mesh` that were split
+ * or handed on (0 if none were, or for smaller calls; <0 on error). Diagnostic with no counterpart in the reference; waits for the device. */
 int64_t ebg_mesh_last_split_packets(const ebg_mesh* mesh);
 
 /* ---------------------------------------------------------------------------------------- */
