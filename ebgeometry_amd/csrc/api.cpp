@@ -540,12 +540,11 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
     EBG_HIP(hipEventCreate(&m->ev1));
   }
   const bool timed = m->ev0 && may_alloc;
-  // counting launches run unsplit: the counters describe the plain traversal's own work; so do
-  // closest-face queries (each lane decides its face from the band of its own whole walk)
+  // counting launches run unsplit: the counters describe the plain traversal's own work
   const bool face        = d_tri != nullptr;
-  const bool hand_on     = !o.work && !face && n < kHandMaxQ;
-  const bool heavy_first = o.presort && n >= kHandMaxQ && !o.work && !face && (may_alloc || m->grid_ready);
-  m->last_split_cap      = heavy_first ? Workspace::heavy_cap(n)
+  const bool hand_on     = !o.work && n < kHandMaxQ;
+  const bool heavy_first = o.presort && n >= kHandMaxQ && !o.work && (may_alloc || m->grid_ready);
+  m->last_split_cap      = face ? 0 : heavy_first ? Workspace::heavy_cap(n)
                                        : (hand_on && o.presort && n >= kHeavyMinQ ? ws.hand.slot_cap : 0);
   if (heavy_first) {
     const ebg_status gs = ensure_cost_grid(m, s);
@@ -611,8 +610,9 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   }
   if (fork) EBG_HIP(hipStreamWaitEvent(s, m->ev_join, 0));
 
-  // the FP64 pass also decides the closest face of the lanes whose FP32 band overflowed
-  const bool recheck = o.fp64_recheck || o.fp64_all || face;
+  // the FP64 decision: of every query when faces are asked for, else of the near-surface ones
+  const bool all64   = o.fp64_all || face;
+  const bool recheck = o.fp64_recheck && !all64;
   QueryArgs a{};
   a.pts            = d_pts;
   a.idx            = idx;
@@ -620,7 +620,7 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   a.seed_r         = seeds;
   a.out_d          = d_dist;
   a.out_tri        = d_tri;
-  a.recheck_abs    = o.fp64_all ? INFINITY : (o.fp64_recheck ? float(o.recheck_eps * m->diag) : 0.0f);
+  a.recheck_abs    = recheck ? float(o.recheck_eps * m->diag) : 0.0f;
   a.recheck_list   = recheck ? ws.recheck_list : nullptr;
   a.recheck_count  = cnt;
   a.recheck_mask   = recheck ? ws.rmask : nullptr;
@@ -667,27 +667,20 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
     m->timed = true;
   }
 
-  if (recheck) {
-    // the list follows the presort order, so FP64 packets hold neighbouring queries
+  if (recheck) // the list follows the presort order, so FP64 packets hold neighbouring queries
     EBG_HIP(launch_recheck_compact(a.recheck_mask, n, idx, ws.recheck_list, cnt, s));
+  if (recheck || all64) {
     QueryArgs r = a;
-    r.idx       = ws.recheck_list;
-    r.count_ptr        = cnt;
-    r.seed_r           = nullptr;
-    r.recheck_list     = nullptr;
-    r.recheck_mask     = nullptr;
-    r.fallback_list    = nullptr;
-    r.work             = nullptr;
-    r.pair_work        = nullptr;
-    // bound (|d32| (1 + rel) + abs)^2 always contains the FP64 minimum: FP32 distances are
-    // accurate to a few ulp of the coordinates
-    r.slack_abs = float(1e-5 * m->diag);
-    r.slack_rel = 1e-4f;
-    EBG_HIP(launch_sdf64(m->dev, m->K, m->banks, r, s));
+    if (recheck) {
+      r.idx       = ws.recheck_list;
+      r.count_ptr = cnt;
+    }
+    EBG_HIP(launch_sdf64(m->dev, m->wbanks, r, s));
+    if (all64 && count) EBG_HIP(launch_fill_u32(cnt, 1, uint32_t(n), s));
   }
   // polygon meshes report the face each closest triangle was clipped from
   if (d_tri && m->tri_face.p) EBG_HIP(launch_map_u32(d_tri, n, m->tri_face.as<uint32_t>(), uint32_t(m->nt), s));
-  if (count) EBG_HIP(launch_add_counts(a.work, recheck ? cnt : nullptr, seeds ? cnt + 1 : nullptr, s));
+  if (count) EBG_HIP(launch_add_counts(a.work, recheck || all64 ? cnt : nullptr, seeds ? cnt + 1 : nullptr, s));
   return EBG_OK;
 }
 

@@ -97,8 +97,7 @@ __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, Pai
   float      bound = active ? INFINITY : -1.0f;
   Walk<NB>   wk;
   wk.start(0u, 0u);
-  mesh_walk<NB, COUNT, false, false>(m, wk, ~0u, 0, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris,
-                                     nullptr, pl, &pc);
+  mesh_walk<NB, COUNT, false>(m, wk, ~0u, 0, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, pl, &pc);
   px *= m.inv_scale;
   py *= m.inv_scale;
   pz *= m.inv_scale;
@@ -189,11 +188,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8
 
 // One wavefront per 64 consecutive entries of the recheck list (packet << 6 | lane, in packet
 // order: neighbouring queries, mostly of one item). The wavefront takes the distinct items of its
-// entries in turn; each listed query is redone in FP64, seeded with (|d32| (1 + 1e-4) +
-// slack_abs)^2, which contains the FP64 minimum.
+// entries in turn; each listed query is decided in FP64 from its FP32 distance (band_walk).
 constexpr uint32_t kBatch64Lanes = 64; // list entries per wavefront (32 measured the same on 256 meshes, 60M queries)
-template <int K, int NB>
-__device__ __forceinline__ void batch64_group(const BatchArgs& a, uint32_t count, uint32_t g)
+template <int NB>
+__device__ __forceinline__ void batch64_group(const BatchArgs& a, uint32_t count, uint32_t g, BandLds& L)
 {
   const uint32_t lane   = __lane_id();
   const uint32_t e      = g * kBatch64Lanes + lane;
@@ -213,34 +211,35 @@ __device__ __forceinline__ void batch64_group(const BatchArgs& a, uint32_t count
     const BatchItemDev it = sload_record(a.items + cur);
     const MeshDev      m  = sload_record(a.meshes + it.mesh);
     uint32_t           qi = 0;
-    double             px = 0.0, py = 0.0, pz = 0.0, bound = -1.0;
+    float              px = 0.0f, py = 0.0f, pz = 0.0f, d32 = 0.0f;
     if (mine) {
-      qi             = a.sorted ? (uint32_t)(a.sorted[it.base + j] - it.base) : j;
-      px             = it.pts[3 * (size_t)qi];
-      py             = it.pts[3 * (size_t)qi + 1];
-      pz             = it.pts[3 * (size_t)qi + 2];
-      const double r = fabs((double)it.out[qi]) * (1.0 + 1e-4) + (double)it.slack_abs;
-      bound          = r * r;
+      qi  = a.sorted ? (uint32_t)(a.sorted[it.base + j] - it.base) : j;
+      px  = it.pts[3 * (size_t)qi];
+      py  = it.pts[3 * (size_t)qi + 1];
+      pz  = it.pts[3 * (size_t)qi + 2];
+      d32 = it.out[qi];
     }
-    double   best = INFINITY;
-    uint32_t btri = kInvalid, bfeat = 0, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
-    const double seed2 = bound;
-    traverse<K, NB, double, false>(m, px, py, pz, bound, best, btri, bfeat, n_inner, n_tris, w_inner, w_tris);
-    if (mine && btri != kInvalid && best <= seed2) {
-      it.out[qi] = (float)resolve64(m, btri, bfeat, best, px, py, pz);
-      if (it.tri) it.tri[qi] = m.feat[8 * (size_t)btri + 6];
+    const int rep = rep_lane(mine ? 0.0f : -1.0f);
+    double    d2;
+    uint32_t  tri;
+    band_walk<NB>(m, px, py, pz, d32, mine, rdlanef(px, rep), rdlanef(py, rep), rdlanef(pz, rep), L, d2, tri);
+    if (mine && tri != kInvalid) {
+      it.out[qi] = signed_distance64(m, tri, px, py, pz);
+      if (it.tri) it.tri[qi] = m.feat[8 * (size_t)tri + 6];
     }
   }
 }
 
 // A fixed grid of wavefronts strides over the groups (their number is only known on the device).
-template <int K, int NB>
+template <int NB>
 __global__ __launch_bounds__(256) void batch64_kernel(const BatchArgs a)
 {
+  __shared__ BandLds lds[4];
   const uint32_t count  = *a.recheck_count;
   const uint32_t groups = (count + kBatch64Lanes - 1u) / kBatch64Lanes;
   const uint32_t waves  = gridDim.x * 4u;
-  for (uint32_t g = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); g < groups; g += waves) batch64_group<K, NB>(a, count, g);
+  for (uint32_t g = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); g < groups; g += waves) 
+    batch64_group<NB>(a, count, g, lds[uni(threadIdx.x >> 6)]);
 }
 
 // One wavefront per packet: the largest cost-grid value over its queries' cells in its mesh's
@@ -309,11 +308,11 @@ hipError_t persist_blocks(int wg, bool count, uint32_t* blocks)
   return hipSuccess;
 }
 
-template <int K, int NB>
+template <int NB>
 hipError_t launch64(const BatchArgs& a, hipStream_t s)
 {
   if (a.num_packets == 0 || !a.recheck_list) return hipSuccess;
-  hipLaunchKernelGGL((batch64_kernel<K, NB>), dim3(std::min<uint32_t>((a.num_packets + 3) / 4, 2048u)), dim3(256), 0, s,
+  hipLaunchKernelGGL((batch64_kernel<NB>), dim3(std::min<uint32_t>((a.num_packets + 3) / 4, 2048u)), dim3(256), 0, s,
                      a);
   return hipGetLastError();
 }
@@ -360,16 +359,11 @@ hipError_t batch32_persistent_blocks(int banks, int wg, bool count, uint32_t* bl
   return persist_blocks<4>(wg, count, blocks);
 }
 
-hipError_t launch_batch64(const BatchArgs& a, int K, int banks, hipStream_t s)
+hipError_t launch_batch64(const BatchArgs& a, int banks, hipStream_t s)
 {
-  if (K == 4) {
-    if (banks <= 1) return launch64<4, 1>(a, s);
-    if (banks == 2) return launch64<4, 2>(a, s);
-    return launch64<4, 4>(a, s);
-  }
-  if (banks <= 1) return launch64<8, 1>(a, s);
-  if (banks == 2) return launch64<8, 2>(a, s);
-  return launch64<8, 4>(a, s);
+  if (banks <= 1) return launch64<1>(a, s);
+  if (banks == 2) return launch64<2>(a, s);
+  return launch64<4>(a, s);
 }
 
 } // namespace ebgpu

@@ -228,7 +228,7 @@ ebg_status enqueue(ebg_batch_plan* p, hipStream_t s, bool events)
     // queries
     EBG_HIP(ebgpu::launch_recheck_compact(a.recheck_mask, uint64_t(p->num_packets) * 64, nullptr, a.recheck_list,
                                           a.recheck_count, s));
-    EBG_HIP(ebgpu::launch_batch64(a, b->K, b->banks, s));
+    EBG_HIP(ebgpu::launch_batch64(a, b->wbanks, s));
   }
   return EBG_OK;
 }

@@ -94,9 +94,10 @@ hipError_t launch_sdf32_handed(const MeshDev& m, int banks, const QueryArgs& a, 
 
 // FP32 packet traversal over the walk tree; banks = its stack capacity / 64 (1..4).
 hipError_t launch_sdf32(const MeshDev& m, int banks, const QueryArgs& a, bool count, hipStream_t s);
-// FP64 traversal that recomputes distance, closest face and sign exactly as the reference's
-// double-precision lane kernel; seeded from the FP32 result (bound |d| + slack).
-hipError_t launch_sdf64(const MeshDev& m, int K, int banks, const QueryArgs& a, hipStream_t s);
+// FP64 decision of distance, closest face and sign with the reference's double-precision lane
+// formulas, from the FP32 distances in out_d: over a.idx / *a.count_ptr when count_ptr is set, else
+// over all a.n queries in the order a.idx.
+hipError_t launch_sdf64(const MeshDev& m, int banks, const QueryArgs& a, hipStream_t s);
 
 // CSG union scenes (scene.hip). KM = branching of the instanced meshes (all equal); banks =
 // stack capacity / 64 for both the scene tree and the mesh trees. Work counters: [0] interior
@@ -168,7 +169,7 @@ hipError_t launch_batch32(const BatchArgs& a, int banks, int wg, bool count, hip
 hipError_t batch32_persistent_blocks(int banks, int wg, bool count, uint32_t* blocks);
 // FP64 pass over the compacted recheck list (a.recheck_list == null skips); a fixed grid
 // strides over groups of 64 entries.
-hipError_t launch_batch64(const BatchArgs& a, int K, int banks, hipStream_t s);
+hipError_t launch_batch64(const BatchArgs& a, int banks, hipStream_t s);
 
 // csg.hip: CSG programs. FP32 pass over a.n queries (a.idx: presort order), appending
 // |v| < a.recheck_abs to the recheck list; FP64 pass over that list (a.idx, *a.count_ptr).

@@ -52,84 +52,15 @@ enum Mode : int
   kSeeded = 1
 };
 
-// Whether a depth-first walk of the packed tree that takes a node's children in the order of their
-// box distances from (rx, ry, rz) -- nearest first, on equal distances the later slot first -- meets
-// triangle a before triangle b.
-template <int K>
-__device__ __forceinline__ bool met_before_k(const MeshDev& m, uint32_t a, uint32_t b, float rx, float ry, float rz)
-{
-  const Node<K>* nodes = static_cast<const Node<K>*>(m.nodes);
-  uint32_t       i     = 0;
-  for (;;) {
-    const uint32_t* f  = m.nfirst + (size_t)K * i;
-    int             ka = 0, kb = 0; // the children holding a and b (the slots' first triangles ascend)
-    for (int k = 1; k < K; k++) {
-      if (f[k] == kInvalid) continue;
-      if (f[k] <= a) ka = k;
-      if (f[k] <= b) kb = k;
-    }
-    const Node<K>& nd = nodes[i];
-    if (ka != kb) {
-      const float da = box_d2<float>(rx, ry, rz, nd.lox[ka], nd.loy[ka], nd.loz[ka], nd.hix[ka], nd.hiy[ka], nd.hiz[ka]);
-      const float db = box_d2<float>(rx, ry, rz, nd.lox[kb], nd.loy[kb], nd.loz[kb], nd.hix[kb], nd.hiy[kb], nd.hiz[kb]);
-      return da < db || (da == db && ka > kb);
-    }
-    if (nd.cnt[ka] != 0u) return a < b; // one leaf: in its order
-    i = nd.ref[ka];
-  }
-}
-__device__ __forceinline__ bool met_before(const MeshDev& m, uint32_t a, uint32_t b, float rx, float ry, float rz)
-{
-  return m.K == 4u ? met_before_k<4>(m, a, b, rx, ry, rz) : met_before_k<8>(m, a, b, rx, ry, rz);
-}
-
-// Closest face of a lane whose FP32 walk kept more than one triangle inside the band of its
-// minimum (FaceCands): the kept triangles are evaluated with the FP64 lane formulas and the
-// FP64 minimum wins; among exact FP64 ties (faces meeting at the closest edge or vertex) the one of
-// the smallest FP32 distance, and among those the one that a walk of the packed tree by box
-// distances from the packet's representative point r meets first, as
-// TriMeshSDF::getClosestTriangle keeps the first strict minimum of its walk
-// (Source/EBGeometry_MeshDistanceFunctionsImplem.hpp:511-549). That order is a rule on the tree and
-// the packet, so the choice does not depend on the order in which this walk met them. Returns the
-// FP64 signed distance of that face.
-__device__ __forceinline__ float decide_face64(const MeshDev& m, const FaceCands& fc, float lim, float px, float py,
-                                               float pz, float rx, float ry, float rz, uint32_t& btri)
-{
-  double   bd = INFINITY;
-  float    bd32 = INFINITY;
-  uint32_t bt = fc.t[0], bf = 0;
-#pragma unroll
-  for (int i = 0; i < kFaceCands; i++) {
-    if (fc.d[i] <= lim && fc.t[i] != kInvalid) {
-      const uint32_t t = fc.t[i];
-      double         d2;
-      uint32_t       f;
-      tri_eval64(m.tripos + 12 * (size_t)t, m.fn64 + 4 * (size_t)t, px, py, pz, d2, f);
-      // the list ascends in d32, so a tie with a smaller d32 is already held
-      if (d2 < bd || (d2 == bd && fc.d[i] == bd32 && met_before(m, t, bt, rx, ry, rz))) {
-        bd   = d2;
-        bd32 = fc.d[i];
-        bt   = t;
-        bf   = f;
-      }
-    }
-  }
-  btri = bt;
-  return (float)resolve64(m, bt, bf, bd, px, py, pz);
-}
-
 // One packet: the 64 queries pk*64 .. pk*64+63 of the (presorted) query order, one per lane.
-// FACE (closest faces requested): each lane decides its face exactly (decide_face64); a lane
-// whose band held more triangles than its list goes to the FP64 pass with the near-surface ones.
-// Distance-only variants (!FACE) evaluate leaves pair-compacted in the wavefront's PairLds.
-template <int NB, bool COUNT, int MODE, bool FACE, bool HAND>
+template <int NB, bool COUNT, int MODE, bool HAND>
 __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& a, uint64_t n, uint64_t pk, PairLds* pl)
 {
   const uint64_t tid    = pk * 64u + (uint64_t)__lane_id();
   bool           active = tid < n;
   uint32_t       qi     = 0;
   float          px = 0.0f, py = 0.0f, pz = 0.0f, bound = -1.0f;
-  const float    sc = m.scale, ds = FACE ? 1.0f : sc * sc; // distance^2 units of the walk (mesh_walk)
+  const float    sc = m.scale;
   if (active) {
     qi = a.idx ? a.idx[tid] : (uint32_t)tid;
     px = a.pts[3 * (size_t)qi] * sc;
@@ -137,7 +68,7 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
     pz = a.pts[3 * (size_t)qi + 2] * sc;
     if (MODE == kSeeded) {
       const float r = a.seed_r[qi];
-      bound         = r * r * ds;
+      bound         = r * r * (sc * sc);
     }
     else {
       bound = INFINITY;
@@ -152,8 +83,6 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
   float    best = INFINITY;
   uint32_t btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
   const float seed2 = bound;
-  FaceCands   fc;
-  if constexpr (FACE) fc.init(m.hmax);
   PairCounts pc{0u, 0u, 0u, 0u};
   Walk<NB>   wk;
   wk.start(0u, 0u);
@@ -165,8 +94,8 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
   uint32_t budget = HAND ? a.hand.budget[0] : ~0u;
   [[maybe_unused]] uint32_t s_inner = 0, s_tris = 0; // the seeded walk's counts
   for (;;) {
-    mesh_walk<NB, COUNT, FACE, HAND>(m, wk, budget, HAND ? a.hand.spread[0] : 0, px, py, pz, bound, best, btri, n_inner,
-                                     n_tris, w_inner, w_tris, &fc, pl, &pc);
+    mesh_walk<NB, COUNT, HAND>(m, wk, budget, HAND ? a.hand.spread[0] : 0, px, py, pz, bound, best, btri, n_inner, n_tris,
+                               w_inner, w_tris, pl, &pc);
     const bool missed = MODE == kSeeded && seeded && active && !(btri != kInvalid && best <= seed2);
     if (HAND && wk.top > 0) {
       const uint64_t mmask = ballot(missed);
@@ -187,13 +116,6 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
     seeded = false;
     redo   = missed;
     if (__lane_id() == 0) atomicAdd(a.fallback_count, (uint32_t)__popcll(rmask));
-    if constexpr (FACE) {
-      if (redo) {
-        fc.init(m.hmax);
-        best = INFINITY;
-        btri = kInvalid;
-      }
-    }
     s_inner = n_inner;
     s_tris  = n_tris;
     bound   = redo ? best : -1.0f;
@@ -218,27 +140,14 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
   px *= m.inv_scale;
   py *= m.inv_scale;
   pz *= m.inv_scale;
-  if constexpr (!FACE) best *= m.inv_scale * m.inv_scale;
-  // the packet's representative point: its middle lane's, or its first query's
-  const int rep = rep_lane(active ? 0.0f : -1.0f);
-  [[maybe_unused]] const float rx = rdlanef(px, rep), ry = rdlanef(py, rep), rz = rdlanef(pz, rep);
-  float d   = 0.0f;
-  bool  ovf = false; // FACE: the band held more triangles than the list
+  best *= m.inv_scale * m.inv_scale;
+  float d = 0.0f;
   if (found) {
     d = resolve32(m, btri, closest_feature(m, btri, px, py, pz), best, px, py, pz);
-    if constexpr (FACE) {
-      // a second triangle inside the band: decide in FP64 among the kept ones, unless the
-      // query is a near-surface one (the FP64 pass decides those from scratch) or the band
-      // overflowed the list (then the FP64 pass decides it too)
-      const float lim = fc.band(best);
-      ovf             = fc.evict <= lim;
-      if (!ovf && fc.d[1] <= lim && !(fabsf(d) < a.recheck_abs))
-        d = decide_face64(m, fc, lim, px, py, pz, rx, ry, rz, btri);
-    }
     a.out_d[qi] = d;
     if (a.out_tri) a.out_tri[qi] = m.tris[btri].face;
   }
-  const bool rchk = found && (fabsf(d) < a.recheck_abs || ovf);
+  const bool rchk = found && fabsf(d) < a.recheck_abs;
   if (a.recheck_mask) {
     const uint64_t rm = ballot(rchk);
     if (__lane_id() == 0) a.recheck_mask[pk] = rm;
@@ -290,8 +199,7 @@ __device__ __forceinline__ void split_item(const MeshDev& m, const QueryArgs& a,
   float           bound = active ? INFINITY : -1.0f;
   Walk<NB>        wk;
   wk.start(rt.ref, rt.cnt);
-  mesh_walk<NB, COUNT, false, false>(m, wk, ~0u, 0, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, nullptr, pl,
-                              nullptr);
+  mesh_walk<NB, COUNT, false>(m, wk, ~0u, 0, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, pl, nullptr);
   if (active && btri != kInvalid)
     atomicMin(a.split_keys + 64 * (size_t)j + lane, ((unsigned long long)__float_as_uint(best) << 32) | btri);
   if (COUNT && a.work) {
@@ -310,12 +218,12 @@ __device__ __forceinline__ void split_item(const MeshDev& m, const QueryArgs& a,
 // mapped XCD-aware so that each XCD works through one contiguous (Morton) range of queries.
 // The leading split_blocks workgroups (dispatched first) work through the split items instead,
 // beside the packets of the bulk; packets flagged in heavy_flag are skipped.
-template <int NB, bool COUNT, int MODE, bool FACE, bool HAND>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FACE ? 1 : (NB == 1 ? 8 : (NB == 2 ? 6 : 4))))) void sdf32_kernel(const MeshDev m, const QueryArgs a)
+template <int NB, bool COUNT, int MODE, bool HAND>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8 : (NB == 2 ? 6 : 4)))) void sdf32_kernel(const MeshDev m, const QueryArgs a)
 {
   const uint32_t wave = uni(threadIdx.x >> 6); // known uniform: list entries load as scalars
-  extern __shared__ PairLds pair_lds[];        // one per wavefront (distance-only variants)
-  PairLds* const pl = FACE ? nullptr : &pair_lds[wave];
+  extern __shared__ PairLds pair_lds[];        // one per wavefront
+  PairLds* const pl = &pair_lds[wave];
   uint32_t       b = blockIdx.x, nb = gridDim.x;
   if (a.split_blocks) {
     if (b < a.split_blocks) {
@@ -332,7 +240,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FACE ? 1 : 
   if (a.early_blocks) {
     if (b < a.early_blocks) {
       const uint32_t j = b * 4u + wave;
-      if (j < min(*a.early_count, a.early_cap)) sdf32_packet<NB, COUNT, MODE, FACE, HAND>(m, a, a.n, a.early_list[j], pl);
+      if (j < min(*a.early_count, a.early_cap)) sdf32_packet<NB, COUNT, MODE, HAND>(m, a, a.n, a.early_list[j], pl);
       return;
     }
     b -= a.early_blocks;
@@ -343,7 +251,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FACE ? 1 : 
   const uint64_t pk  = (uint64_t)blk * 4u + wave;
   if (pk * 64u >= n) return;                    // whole wavefront past the end
   if (a.heavy_flag && a.heavy_flag[pk]) return; // whole wavefront: a split or early packet
-  sdf32_packet<NB, COUNT, MODE, FACE, HAND>(m, a, n, pk, pl);
+  sdf32_packet<NB, COUNT, MODE, HAND>(m, a, n, pk, pl);
 }
 
 // The items handed on (HandOn): wavefronts stride over items[STAGE]. Each walks its subtree for the
@@ -382,8 +290,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8
     wk.start(it.w[1], it.w[2]);
     uint32_t budget = STAGE == 0 ? a.hand.budget[1] : ~0u;
     for (;;) {
-      mesh_walk<NB, false, false, true>(m, wk, budget, a.hand.spread[1], px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, nullptr,
-                                  pl, nullptr);
+      mesh_walk<NB, false, true>(m, wk, budget, a.hand.spread[1], px, py, pz, bound, best, btri, n_inner, n_tris, w_inner,
+                                 w_tris, pl, nullptr);
       if (wk.top == 0 || append_items(wk, slot, a.hand.items[1], a.hand.counts + 2, a.hand.item_cap)) break;
       budget = ~0u; // no room: walk on
     }
@@ -415,7 +323,8 @@ __global__ __launch_bounds__(256) void sdf32_resolve_kernel(const MeshDev m, con
         const float d2 = __uint_as_float((uint32_t)(key >> 32)) * (m.inv_scale * m.inv_scale); // the walk's, unscaled
         d              = resolve32(m, t, closest_feature(m, t, px, py, pz), d2, px, py, pz);
         a.out_d[qi]    = d;
-        found          = true;
+        if (a.out_tri) a.out_tri[qi] = m.tris[t].face;
+        found = true;
       }
     }
     if (a.recheck_mask) {
@@ -454,68 +363,71 @@ __global__ __launch_bounds__(256) void recheck_compact_kernel(const uint64_t* __
   }
 }
 
-template <int K, int NB>
-__device__ __forceinline__ void sdf64_block(const MeshDev& m, const QueryArgs& a, uint64_t n, uint64_t tid)
+// The FP64 decision of the closest triangle (band_walk) of one lane's query tid, at most one per
+// lane; (rx, ry, rz) is the wavefront's representative point.
+template <int NB>
+__device__ __forceinline__ void band_block(const MeshDev& m, const QueryArgs& a, bool active, uint64_t tid, BandLds& L)
 {
-  const bool active = tid < n;
-  uint32_t   qi     = 0;
-  double     px = 0.0, py = 0.0, pz = 0.0, bound = -1.0;
+  uint32_t qi = 0;
+  float    px = 0.0f, py = 0.0f, pz = 0.0f, d32 = 0.0f;
   if (active) {
-    qi = a.idx ? a.idx[tid] : (uint32_t)tid;
-    px = a.pts[3 * (size_t)qi];
-    py = a.pts[3 * (size_t)qi + 1];
-    pz = a.pts[3 * (size_t)qi + 2];
-    if (a.slack_abs > 0.0f) {
-      const double r = fabs((double)a.out_d[qi]) * (1.0 + (double)a.slack_rel) + (double)a.slack_abs;
-      bound          = r * r;
+    qi  = a.idx ? a.idx[tid] : (uint32_t)tid;
+    px  = a.pts[3 * (size_t)qi];
+    py  = a.pts[3 * (size_t)qi + 1];
+    pz  = a.pts[3 * (size_t)qi + 2];
+    if (!(px == px && py == py && pz == pz)) { // NaN: no closest triangle (sdf32_packet wrote nothing)
+      px = py = pz = 0.0f;
+      active       = false;
     }
-    else {
-      bound = INFINITY;
-    }
+    else d32 = a.out_d[qi];
   }
-  double   best = INFINITY;
-  uint32_t btri = kInvalid, bfeat = 0, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
-  const double seed2 = bound;
-  traverse<K, NB, double, false>(m, px, py, pz, bound, best, btri, bfeat, n_inner, n_tris, w_inner, w_tris);
-  const bool found = active && btri != kInvalid && best <= seed2;
-  if (found) {
-    a.out_d[qi] = (float)resolve64(m, btri, bfeat, best, px, py, pz);
-    if (a.out_tri) a.out_tri[qi] = m.feat[8 * (size_t)btri + 6];
+  const int rep = rep_lane(active ? 0.0f : -1.0f);
+  double    d2;
+  uint32_t  tri;
+  band_walk<NB>(m, px, py, pz, d32, active, rdlanef(px, rep), rdlanef(py, rep), rdlanef(pz, rep), L, d2, tri);
+  if (active && tri != kInvalid) {
+    a.out_d[qi] = signed_distance64(m, tri, px, py, pz);
+    if (a.out_tri) a.out_tri[qi] = m.feat[8 * (size_t)tri + 6];
   }
-  if (a.fallback_list) wave_append(active && !found, qi, a.fallback_list, a.fallback_count);
 }
 
-// FP64 pass over a device-side list (a.idx, count *a.count_ptr) or over all a.n queries; a fixed
-// grid of wavefronts strides over the entries, kSdf64Lanes per wavefront (the other lanes sit
-// out). Near-surface queries are sparse even in presort order, so a wavefront walks several
-// paths; with 32 entries its slowest wavefronts end earlier (16M queries, 327,680-face displaced sphere: 0.31 -> 0.23 ms).
-constexpr uint32_t kSdf64Lanes = 32;
-template <int K, int NB>
-__global__ __launch_bounds__(256) void sdf64_kernel(const MeshDev m, const QueryArgs a)
+// Every query: one wavefront per packet, as the FP32 pass.
+template <int NB>
+__global__ __launch_bounds__(256) void band_all_kernel(const MeshDev m, const QueryArgs a)
 {
-  const uint64_t n     = a.count_ptr ? (uint64_t)*a.count_ptr : a.n;
-  const uint32_t lane  = __lane_id();
+  const uint32_t wave = uni(threadIdx.x >> 6);
+  __shared__ BandLds lds[4];
+  const uint64_t pk  = (uint64_t)xcd_remap(blockIdx.x, gridDim.x) * 4u + wave;
+  const uint64_t tid = pk * 64u + __lane_id();
+  if (pk * 64u >= a.n) return; // whole wavefront past the end
+  band_block<NB>(m, a, tid < a.n, tid, lds[wave]);
+}
+
+// A device-side list (a.idx, its length *a.count_ptr): a fixed grid of wavefronts strides over the
+// entries, kBandLanes per wavefront (the other lanes sit out). Near-surface queries are sparse
+// even in presort order, so a wavefront walks several paths, and the last to end is the one with
+// the most.
+constexpr uint32_t kBandLanes = 32;
+template <int NB>
+__global__ __launch_bounds__(256) void band_list_kernel(const MeshDev m, const QueryArgs a)
+{
+  const uint32_t wave = uni(threadIdx.x >> 6), lane = __lane_id();
+  __shared__ BandLds lds[4];
+  const uint64_t n     = *a.count_ptr;
   const uint64_t waves = (uint64_t)gridDim.x * 4u;
-  for (uint64_t w = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); w * kSdf64Lanes < n; w += waves)
-    sdf64_block<K, NB>(m, a, n, lane < kSdf64Lanes ? w * kSdf64Lanes + lane : n);
+  for (uint64_t w = uni(blockIdx.x * 4u + wave); w * kBandLanes < n; w += waves) {
+    const uint64_t tid = w * kBandLanes + lane;
+    band_block<NB>(m, a, lane < kBandLanes && tid < n, tid, lds[wave]);
+  }
 }
 
-template <int NB, int MODE, bool FACE>
-void launch32f(const MeshDev& m, const QueryArgs& a, bool count, uint32_t blocks, hipStream_t s)
-{
-  const size_t lds = FACE ? 0 : 4 * sizeof(PairLds);
-  if (count) hipLaunchKernelGGL((sdf32_kernel<NB, true, MODE, FACE, false>), dim3(blocks), dim3(256), lds, s, m, a);
-  else if (a.hand.slot_cap && !FACE)
-    hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, FACE, !FACE>), dim3(blocks), dim3(256), lds, s, m, a);
-  else hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, FACE, false>), dim3(blocks), dim3(256), lds, s, m, a);
-}
-
-// closest faces requested: the exact-face variant (its split packets are off: see launch32)
 template <int NB, int MODE>
 void launch32m(const MeshDev& m, const QueryArgs& a, bool count, uint32_t blocks, hipStream_t s)
 {
-  if (a.out_tri) launch32f<NB, MODE, true>(m, a, count, blocks, s);
-  else launch32f<NB, MODE, false>(m, a, count, blocks, s);
+  const size_t lds = 4 * sizeof(PairLds);
+  if (count) hipLaunchKernelGGL((sdf32_kernel<NB, true, MODE, false>), dim3(blocks), dim3(256), lds, s, m, a);
+  else if (a.hand.slot_cap) hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, true>), dim3(blocks), dim3(256), lds, s, m, a);
+  else hipLaunchKernelGGL((sdf32_kernel<NB, false, MODE, false>), dim3(blocks), dim3(256), lds, s, m, a);
 }
 
 template <int NB>
@@ -525,12 +437,9 @@ hipError_t launch32(const MeshDev& m, const QueryArgs& a, bool count, hipStream_
   if (blocks == 0) return hipSuccess;
   if (a.count_ptr) return hipErrorInvalidValue;
   if (a.split_blocks && (!a.split_nroots || !a.split_count || !a.heavy_flag)) return hipErrorInvalidValue;
-  if (a.hand.slot_cap && (a.split_blocks || a.out_tri || !a.hand.list || !a.hand.keys || !a.hand.items[0] ||
+  if (a.hand.slot_cap && (a.split_blocks || !a.hand.list || !a.hand.keys || !a.hand.items[0] ||
                           !a.hand.items[1] || !a.hand.counts))
     return hipErrorInvalidValue;
-  // exact closest faces need each lane's whole candidate band in one walk: no split packets, and
-  // the FP64 pass must follow (lanes whose band overflowed are listed for it)
-  if (a.out_tri && (a.split_blocks || (!a.recheck_mask && !a.recheck_list))) return hipErrorInvalidValue;
   if (a.early_blocks && (!a.early_list || !a.early_count || !a.heavy_flag)) return hipErrorInvalidValue;
   if (a.seed_r) {
     if (!a.fallback_count) return hipErrorInvalidValue;
@@ -542,12 +451,14 @@ hipError_t launch32(const MeshDev& m, const QueryArgs& a, bool count, hipStream_
   return hipGetLastError();
 }
 
-template <int K, int NB>
+template <int NB>
 hipError_t launch64(const MeshDev& m, const QueryArgs& a, hipStream_t s)
 {
-  const uint32_t blocks = std::min<uint32_t>((uint32_t)((a.n + 255) / 256), kListGrid);
+  const uint32_t blocks = (uint32_t)((a.n + 255) / 256);
   if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL((sdf64_kernel<K, NB>), dim3(blocks), dim3(256), 0, s, m, a);
+  if (a.count_ptr)
+    hipLaunchKernelGGL(band_list_kernel<NB>, dim3(std::min<uint32_t>(2u * blocks, kListGrid)), dim3(256), 0, s, m, a);
+  else hipLaunchKernelGGL(band_all_kernel<NB>, dim3(blocks), dim3(256), 0, s, m, a);
   return hipGetLastError();
 }
 
@@ -662,16 +573,11 @@ hipError_t launch_sdf32_handed(const MeshDev& m, int banks, const QueryArgs& a, 
   return launch_handed<4>(m, a, s);
 }
 
-hipError_t launch_sdf64(const MeshDev& m, int K, int banks, const QueryArgs& a, hipStream_t s)
+hipError_t launch_sdf64(const MeshDev& m, int banks, const QueryArgs& a, hipStream_t s)
 {
-  if (K == 4) {
-    if (banks <= 1) return launch64<4, 1>(m, a, s);
-    if (banks == 2) return launch64<4, 2>(m, a, s);
-    return launch64<4, 4>(m, a, s);
-  }
-  if (banks <= 1) return launch64<8, 1>(m, a, s);
-  if (banks == 2) return launch64<8, 2>(m, a, s);
-  return launch64<8, 4>(m, a, s);
+  if (banks <= 1) return launch64<1>(m, a, s);
+  if (banks == 2) return launch64<2>(m, a, s);
+  return launch64<4>(m, a, s);
 }
 
 } // namespace ebgpu

@@ -501,62 +501,6 @@ __device__ __forceinline__ void wave_append(bool pred, uint32_t idx, uint32_t* l
 }
 
 // ---------------------------------------------------------------------------------------
-// closest-face candidates (exact closest face from an FP32 walk)
-// ---------------------------------------------------------------------------------------
-
-// The FP32 distance of a point to a triangle differs from the FP64 lane formula's by at most
-// E(d) = 2^-21 (d + 2 hmax) (d the distance, hmax the mesh's longest edge: every rounding acts on
-// a vector no longer than d + 2 hmax; measured maximum 3 * 2^-24 (d + 2 hmax)). So the face that
-// is closest in FP64 has an FP32 distance within 2 E of the FP32 minimum, and a lane that keeps
-// every triangle inside that band can decide its face exactly, in FP64, among them.
-constexpr int kFaceCands = 8;
-
-struct FaceCands
-{
-  float    d[kFaceCands]; // FP32 d^2 of the kept triangles, ascending (+inf: empty slot)
-  uint32_t t[kFaceCands];
-  float    lim;           // band of the current minimum: triangles with d^2 <= lim are kept
-  float    evict;         // smallest d^2 pushed out of a full list
-  float    habs;          // 2^-19 hmax: the band's absolute part
-
-  __device__ __forceinline__ void init(float hmax)
-  {
-#pragma unroll
-    for (int i = 0; i < kFaceCands; i++) {
-      d[i] = INFINITY;
-      t[i] = kInvalid;
-    }
-    lim   = INFINITY;
-    evict = INFINITY;
-    habs  = hmax * 0x1p-19f;
-  }
-
-  // band(d^2) = (d (1 + 2^-20) + 2^-19 hmax)^2, rounded up
-  __device__ __forceinline__ float band(float d2) const
-  {
-    const float r = fmaf(__builtin_amdgcn_sqrtf(d2), 1.0f + 0x1p-20f, habs);
-    return r * r * (1.0f + 0x1p-21f);
-  }
-
-  // Sorted insert (fixed positions only: the list stays in VGPRs); a value pushed out of the
-  // full list is remembered in `evict`.
-  __device__ __forceinline__ void insert(float x, uint32_t xt)
-  {
-#pragma unroll
-    for (int i = 0; i < kFaceCands; i++) {
-      const bool     sw = x < d[i];
-      const float    od = d[i];
-      const uint32_t ot = t[i];
-      d[i]              = sw ? x : od;
-      t[i]              = sw ? xt : ot;
-      x                 = sw ? od : x;
-      xt                = sw ? ot : xt;
-    }
-    evict = fminf(evict, x);
-  }
-};
-
-// ---------------------------------------------------------------------------------------
 // the packet traversal
 // ---------------------------------------------------------------------------------------
 
@@ -741,6 +685,45 @@ struct PairCounts
   uint32_t pairs, batches, groups, leaves;
 };
 
+// A value of another lane (byte address 4 * lane); all 64 lanes take part (an inactive source lane
+// would not be read).
+__device__ __forceinline__ float bperm(int addr, float x)
+{
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(x)));
+}
+
+// The screen of one triangle: its disc (record i of sp) against each lane's cull radius, disc_lanes
+// with t = 0, where (n.s)^2 + w = b2. The lanes it may reach write `entry` to the pair list
+// from place `total` on (mine: this lane is one); returns their number.
+__device__ __forceinline__ uint32_t list_pairs(const SWords<32>& sp, int i, float px, float py, float pz, float b2,
+                                               uint32_t entry, uint32_t total, uint16_t* list, bool& mine)
+{
+  const float sx = px - __uint_as_float(sp.w[8 * i]), sy = py - __uint_as_float(sp.w[8 * i + 1]),
+              sz = pz - __uint_as_float(sp.w[8 * i + 2]);
+  const float pd = __uint_as_float(sp.w[8 * i + 3]) * sx + __uint_as_float(sp.w[8 * i + 4]) * sy +
+                   __uint_as_float(sp.w[8 * i + 5]) * sz;
+  const float w = fmaf(-pd, pd, b2);
+  const float B = fmaf(sz, sz, fmaf(sy, sy, fmaf(sx, sx, __uint_as_float(sp.w[8 * i + 7])))) - b2;
+  const bool  in_r = !(B * fabsf(B) > __uint_as_float(sp.w[8 * i + 6]) * w), in_p = !(w < 0.0f);
+  const uint64_t pm = ballot(in_r) & ballot(in_p);
+  mine              = in_r && in_p;
+  if (pm == 0) return 0u;
+  // this lane's bit of pm is in_r && in_p: the write is predicated on the compares
+  if (mine) list[mbcnt(pm, total)] = (uint16_t)entry;
+  return (uint32_t)__popcll(pm);
+}
+
+// Copy a leaf's frame records to LDS, two 16-byte pieces per lane.
+__device__ __forceinline__ void copy_records(const MeshDev& m, uint32_t first, uint32_t cnt, float4* rec)
+{
+  const uint32_t q0 = 2u * __lane_id();
+  const float4* __restrict__ src = reinterpret_cast<const float4*>(m.frames + first);
+  if (q0 < 8u * cnt) {
+    rec[q0]     = src[q0];
+    rec[q0 + 1] = src[q0 + 1];
+  }
+}
+
 // FP32 distance-only leaf, compacted: the screen (each triangle's disc against each lane's cull
 // radius, disc_lanes without a height) is run for every triangle of the leaf, and each passing
 // (lane, triangle) pair is appended to a list in LDS; then each lane evaluates one pair at a time
@@ -756,10 +739,6 @@ __device__ __forceinline__ void leaf_pairs(const MeshDev& m, uint32_t first, uin
                                            uint32_t& n_tris, uint32_t& w_tris, PairLds& L, PairCounts* pc)
 {
   const uint32_t lane = __lane_id();
-  const uint32_t q0   = 2u * lane; // this lane's 16-byte pieces q0, q0 + 1 of the leaf's records
-  const bool     mine = q0 < 8u * cnt;
-  const float4* __restrict__ src = reinterpret_cast<const float4*>(m.frames + first);
-
   if (COUNT && pc) {
     pc->leaves++;
     pc->groups += (cnt + 3u) / 4u;
@@ -770,21 +749,9 @@ __device__ __forceinline__ void leaf_pairs(const MeshDev& m, uint32_t first, uin
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       if (c0 + i < cnt) {
-        const float sx = px - __uint_as_float(sp.w[8 * i]), sy = py - __uint_as_float(sp.w[8 * i + 1]),
-                    sz = pz - __uint_as_float(sp.w[8 * i + 2]);
-        const float pd = __uint_as_float(sp.w[8 * i + 3]) * sx + __uint_as_float(sp.w[8 * i + 4]) * sy +
-                         __uint_as_float(sp.w[8 * i + 5]) * sz;
-        // disc_lanes with t = 0: (n.s)^2 + w = b2
-        const float w = fmaf(-pd, pd, b2);
-        const float B = fmaf(sz, sz, fmaf(sy, sy, fmaf(sx, sx, __uint_as_float(sp.w[8 * i + 7])))) - b2;
-        const bool  in_r = !(B * fabsf(B) > __uint_as_float(sp.w[8 * i + 6]) * w), in_p = !(w < 0.0f);
-        if (COUNT) n_tris += (in_r && in_p) ? 1u : 0u;
-        const uint64_t pm = ballot(in_r) & ballot(in_p);
-        if (pm) {
-          // this lane's bit of pm is in_r && in_p: the write is predicated on the compares
-          if (in_r && in_p) L.pair[mbcnt(pm, total)] = (uint16_t)((lane << 4) | (c0 + (uint32_t)i));
-          total += (uint32_t)__popcll(pm);
-        }
+        bool mine;
+        total += list_pairs(sp, i, px, py, pz, b2, (lane << 4) | (c0 + (uint32_t)i), total, L.pair, mine);
+        if (COUNT) n_tris += mine ? 1u : 0u;
       }
     }
   }
@@ -796,10 +763,7 @@ __device__ __forceinline__ void leaf_pairs(const MeshDev& m, uint32_t first, uin
       pc->batches += (total + 63u) / 64u;
     }
   }
-  if (mine) {
-    L.rec[q0]     = src[q0];
-    L.rec[q0 + 1] = src[q0 + 1];
-  }
+  copy_records(m, first, cnt, L.rec);
   L.best[lane] = ((uint64_t)__float_as_uint(best) << 32) | btri;
   wave_lds_handoff();
   for (uint32_t b0 = 0; b0 < total; b0 += 64) {
@@ -807,11 +771,8 @@ __device__ __forceinline__ void leaf_pairs(const MeshDev& m, uint32_t first, uin
     const bool     ok = k < total;
     uint32_t       e  = lane << 4; // idle lanes: their own point
     if (ok) e = L.pair[k];
-    // all 64 lanes take part in the permutes (an inactive source lane would not be read)
     const int   sa = (int)((e >> 4) << 2);
-    const float qx = __int_as_float(__builtin_amdgcn_ds_bpermute(sa, __float_as_int(px)));
-    const float qy = __int_as_float(__builtin_amdgcn_ds_bpermute(sa, __float_as_int(py)));
-    const float qz = __int_as_float(__builtin_amdgcn_ds_bpermute(sa, __float_as_int(pz)));
+    const float qx = bperm(sa, px), qy = bperm(sa, py), qz = bperm(sa, pz);
     if (ok) {
       const uint32_t slot = e & 15u;
       const float    d2   = frame_eval32(*reinterpret_cast<const FrameRec*>(&L.rec[8 * slot]), qx, qy, qz);
@@ -826,53 +787,117 @@ __device__ __forceinline__ void leaf_pairs(const MeshDev& m, uint32_t first, uin
   bound             = best < bound ? best : bound; // bound stays min(bound, best)
 }
 
-// Closest-face leaf: a triangle is evaluated by the whole wavefront when some lane's cull radius
-// reaches its disc; the cull bound is the band of the minimum (FaceCands::band), the distances are
-// in the mesh's own units, and every triangle inside the band is kept in fc.
-template <bool COUNT>
-__device__ __forceinline__ void leaf_face(const MeshDev& m, uint32_t first, uint32_t cnt, float px, float py, float pz,
-                                          float& b2, float& bound, float& best, uint32_t& btri, uint32_t& n_tris,
-                                          uint32_t& w_tris, FaceCands& fc)
+// Whether a depth-first walk of the packed tree that takes a node's children in the order of their
+// box distances from (rx, ry, rz) -- nearest first, on equal distances the later slot first -- meets
+// triangle a before triangle b.
+template <int K>
+__device__ __forceinline__ bool met_before_k(const MeshDev& m, uint32_t a, uint32_t b, float rx, float ry, float rz)
 {
-  const float ux = px * m.inv_scale, uy = py * m.inv_scale, uz = pz * m.inv_scale, ss = m.scale * m.scale;
-  for (uint32_t c0 = 0; c0 < cnt; c0 += 4) {
-    const SWords<32> sp   = sload<32>(m.tdisc + first + c0);
-    uint32_t         need = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      if (c0 + i < cnt) {
-        const float sx = px - __uint_as_float(sp.w[8 * i]), sy = py - __uint_as_float(sp.w[8 * i + 1]),
-                    sz = pz - __uint_as_float(sp.w[8 * i + 2]);
-        const float pd = __uint_as_float(sp.w[8 * i + 3]) * sx + __uint_as_float(sp.w[8 * i + 4]) * sy +
-                         __uint_as_float(sp.w[8 * i + 5]) * sz;
-        const float w = fmaf(-pd, pd, b2);
-        const float B = fmaf(sz, sz, fmaf(sy, sy, fmaf(sx, sx, __uint_as_float(sp.w[8 * i + 7])))) - b2;
-        const bool  in_r = !(B * fabsf(B) > __uint_as_float(sp.w[8 * i + 6]) * w), in_p = !(w < 0.0f);
-        if (COUNT) n_tris += (in_r && in_p) ? 1u : 0u;
-        need |= (ballot(in_r) & ballot(in_p)) ? (1u << i) : 0u;
-      }
+  const Node<K>* nodes = static_cast<const Node<K>*>(m.nodes);
+  uint32_t       i     = 0;
+  for (;;) {
+    const uint32_t* f  = m.nfirst + (size_t)K * i;
+    int             ka = 0, kb = 0; // the children holding a and b (the slots' first triangles ascend)
+    for (int k = 1; k < K; k++) {
+      if (f[k] == kInvalid) continue;
+      if (f[k] <= a) ka = k;
+      if (f[k] <= b) kb = k;
     }
-    while (need) {
-      const uint32_t t = first + c0 + (uint32_t)__builtin_ctz(need);
-      need &= need - 1u;
-      const TriRec rec = sload_record(m.tris + t);
-      // the distance to the triangle's plane is a lower bound on the distance to it
-      const float fd = rec.n[0] * (ux - rec.v0[0]) + rec.n[1] * (uy - rec.v0[1]) + rec.n[2] * (uz - rec.v0[2]);
-      if (ballot(fd * fd <= bound) == 0) continue;
-      if (COUNT) w_tris++;
-      float    d2;
-      uint32_t f = 0;
-      tri_eval32<false>(rec, ux, uy, uz, d2, f);
-      if (d2 <= fc.lim) {
-        fc.insert(d2, t);
-        if (d2 < best) {
-          best   = d2;
-          btri   = t;
-          fc.lim = fc.band(d2);
-          bound  = fc.lim < bound ? fc.lim : bound;
-          b2     = cull_radius2(m, bound * ss);
+    const Node<K>& nd = nodes[i];
+    if (ka != kb) {
+      const float da = box_d2<float>(rx, ry, rz, nd.lox[ka], nd.loy[ka], nd.loz[ka], nd.hix[ka], nd.hiy[ka], nd.hiz[ka]);
+      const float db = box_d2<float>(rx, ry, rz, nd.lox[kb], nd.loy[kb], nd.loz[kb], nd.hix[kb], nd.hiy[kb], nd.hiz[kb]);
+      return da < db || (da == db && ka > kb);
+    }
+    if (nd.cnt[ka] != 0u) return a < b; // one leaf: in its order
+    i = nd.ref[ka];
+  }
+}
+__device__ __forceinline__ bool met_before(const MeshDev& m, uint32_t a, uint32_t b, float rx, float ry, float rz)
+{
+  return m.K == 4u ? met_before_k<4>(m, a, b, rx, ry, rz) : met_before_k<8>(m, a, b, rx, ry, rz);
+}
+
+// Per-wavefront LDS of the FP64 decision (leaf_band): a leaf's records and pairs as in PairLds, and
+// each lane's FP64 minimum so far, its triangle, and the lane that may update them.
+struct alignas(64) BandLds
+{
+  float4   rec[kMaxLeaf * 8];
+  uint64_t best[64]; // bits of the smallest FP64 distance^2
+  uint32_t tri[64];
+  uint16_t pair[kMaxLeaf * 64];
+  uint16_t claim[64];
+};
+static_assert(sizeof(BandLds) == 5120 - 128, "BandLds layout");
+
+// Leaf of the FP64 decision: the pairs within the lanes' cull radii are evaluated in FP32 as by
+// leaf_pairs, those within the lane's band (d^2 <= lim) again with the FP64 lane formulas, and
+// folded into the lane's FP64 minimum. Among exact FP64 ties (faces meeting at the closest edge or
+// vertex) the triangle of the smallest tri_eval32 distance is kept, and among those the one that a
+// walk of the packed tree by box distances from the packet's representative point r meets first,
+// as TriMeshSDF::getClosestTriangle keeps the first strict minimum of its walk
+// (Source/EBGeometry_MeshDistanceFunctionsImplem.hpp:511-549): a rule on the tree and the packet,
+// whatever order this walk meets them in.
+__device__ __forceinline__ void leaf_band(const MeshDev& m, uint32_t first, uint32_t cnt, float px, float py, float pz,
+                                          float b2, float lim, float rx, float ry, float rz, BandLds& L)
+{
+  const uint32_t lane = __lane_id();
+  uint32_t       total = 0;
+  bool           mine;
+  for (uint32_t c0 = 0; c0 < cnt; c0 += 4) {
+    const SWords<32> sp = sload<32>(m.tdisc + first + c0);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (c0 + i < cnt) total += list_pairs(sp, i, px, py, pz, b2, (lane << 4) | (c0 + (uint32_t)i), total, L.pair, mine);
+  }
+  if (total == 0) return;
+  copy_records(m, first, cnt, L.rec);
+  wave_lds_handoff();
+  // FP32: the pairs inside the band, compacted to the front of the list
+  uint32_t kept = 0;
+  for (uint32_t b0 = 0; b0 < total; b0 += 64) {
+    const bool     ok = b0 + lane < total;
+    const uint32_t e  = ok ? L.pair[b0 + lane] : lane << 4;
+    const int      sa = (int)((e >> 4) << 2);
+    const float    qx = bperm(sa, px), qy = bperm(sa, py), qz = bperm(sa, pz), ql = bperm(sa, lim);
+    const bool     in = ok && frame_eval32(*reinterpret_cast<const FrameRec*>(&L.rec[8 * (e & 15u)]), qx, qy, qz) <= ql;
+    const uint64_t im = ballot(in);
+    wave_lds_handoff(); // the batch has been read before its places are written
+    if (in) L.pair[mbcnt(im, kept)] = (uint16_t)e;
+    kept += (uint32_t)__popcll(im);
+  }
+  wave_lds_handoff();
+  for (uint32_t b0 = 0; b0 < kept; b0 += 64) {
+    bool           pending = b0 + lane < kept;
+    const uint32_t e       = pending ? L.pair[b0 + lane] : lane << 4;
+    const uint32_t own = e >> 4, t = first + (e & 15u);
+    const int      sa = (int)(own << 2);
+    const float    ux = bperm(sa, px) * m.inv_scale, uy = bperm(sa, py) * m.inv_scale, uz = bperm(sa, pz) * m.inv_scale;
+    double         d2 = 0.0;
+    uint32_t       f;
+    if (pending) tri_eval64(m.tripos + 12 * (size_t)t, m.fn64 + 4 * (size_t)t, ux, uy, uz, d2, f);
+    // pairs of one lane fold one after the other: each round every lane with pairs left is claimed
+    // by one of them
+    while (ballot(pending)) {
+      if (pending) L.claim[own] = (uint16_t)lane;
+      wave_lds_handoff();
+      if (pending && L.claim[own] == lane) {
+        const double   held = __longlong_as_double((long long)L.best[own]);
+        const uint32_t h    = L.tri[own];
+        bool           take = d2 < held;
+        if (d2 == held && h != kInvalid) {
+          float da, db;
+          tri_eval32<false>(m.tris[t], ux, uy, uz, da, f);
+          tri_eval32<false>(m.tris[h], ux, uy, uz, db, f);
+          take = da < db || (da == db && met_before(m, t, h, rx, ry, rz));
         }
+        if (take) {
+          L.best[own] = (uint64_t)__double_as_longlong(d2);
+          L.tri[own]  = t;
+        }
+        pending = false;
       }
+      wave_lds_handoff();
     }
   }
 }
@@ -993,22 +1018,19 @@ __device__ __forceinline__ void push_walk_children(const MeshDev& m, Walk<NB>& w
 // The walk over the mesh's WalkNodes from wk's stack until it is empty or (HAND) `budget` nodes and
 // leaves have been visited. Then the stack is spread for handing on: its lowest entries, the largest
 // subtrees, are replaced by their children until there are `spread` entries (a depth-first stack
-// alone holds a few subtrees of a quarter of the rest, a sixteenth, ...). px, py, pz are scaled. Distance-only (FACE = false): bound, best scaled,
-// leaves by leaf_pairs. FACE: bound, best in the mesh's own units, leaves by leaf_face. bound < 0:
-// a lane without a query.
-template <int NB, bool COUNT, bool FACE, bool HAND>
+// alone holds a few subtrees of a quarter of the rest, a sixteenth, ...). px, py, pz, bound, best are
+// scaled; bound < 0: a lane without a query.
+template <int NB, bool COUNT, bool HAND>
 __device__ __forceinline__ void mesh_walk(const MeshDev& m, Walk<NB>& wk, uint32_t budget, int spread, float px, float py, float pz,
                                           float& bound, float& best, uint32_t& btri, uint32_t& n_inner, uint32_t& n_tris,
-                                          uint32_t& w_inner, uint32_t& w_tris, FaceCands* fc, PairLds* pl,
-                                          PairCounts* pc)
+                                          uint32_t& w_inner, uint32_t& w_tris, PairLds* pl, PairCounts* pc)
 {
   WalkStack<NB>& st    = wk.st;
   int&           top   = wk.top;
   uint32_t&      stamp = wk.stamp;
   const int   lane = __lane_id();
   const int   rep  = rep_lane(bound);
-  const float ss   = FACE ? m.scale * m.scale : 1.0f;
-  float       b2   = cull_radius2(m, FACE ? bound * ss : bound);
+  float       b2   = cull_radius2(m, bound);
   // Stamp of the bounds: it advances after every leaf that tightened some lane's bound, and each
   // pushed entry carries it above the count's bits. An entry whose stamp is current was pushed
   // because some lane reached it, and no bound has changed since, so the test at the pop would
@@ -1036,11 +1058,10 @@ __device__ __forceinline__ void mesh_walk(const MeshDev& m, Walk<NB>& wk, uint32
     }
     else {
       const float bound0 = bound;
-      if constexpr (FACE) leaf_face<COUNT>(m, eref, cnt, px, py, pz, b2, bound, best, btri, n_tris, w_tris, *fc);
-      else leaf_pairs<COUNT>(m, eref, cnt, px, py, pz, b2, bound, best, btri, n_tris, w_tris, *pl, pc);
+      leaf_pairs<COUNT>(m, eref, cnt, px, py, pz, b2, bound, best, btri, n_tris, w_tris, *pl, pc);
       if (ballot(bound < bound0)) {
         stamp++;
-        if constexpr (!FACE) b2 = cull_radius2(m, bound);
+        b2 = cull_radius2(m, bound);
       }
     }
   }
@@ -1057,6 +1078,49 @@ __device__ __forceinline__ void mesh_walk(const MeshDev& m, Walk<NB>& wk, uint32
       push_walk_children(m, wk, eref, px, py, pz, b2, rep);
     }
   }
+}
+
+// The closest triangle in FP64, given a distance d32 that an FP32 walk found (|d32| for lanes with
+// a query; tri kInvalid where the lane has none). The FP32 distance of a point to a triangle, by
+// either evaluation, is within E(d) = 2^-21 (d + 2 hmax) of the FP64 lane formula's (every rounding
+// acts on a vector no longer than d + 2 hmax; the largest measured is 3 * 2^-24 (d + 2 hmax)), so
+// the FP64-closest triangle has an FP32 distance within 2 E of the minimum: one walk with that
+// band as its fixed radius meets it, and the FP64 formulas decide among the few triangles inside
+// the band (leaf_band). Nothing tightens, so no entry is tested again. px, py, pz: the mesh's own
+// units; (rx, ry, rz): the packet's representative point, for ties.
+template <int NB>
+__device__ __forceinline__ void band_walk(const MeshDev& m, float px, float py, float pz, float d32, bool active,
+                                          float rx, float ry, float rz, BandLds& L, double& d2, uint32_t& tri)
+{
+  const uint32_t lane = __lane_id();
+  const float    r    = fmaf(fabsf(d32), 1.0f + 0x1p-19f, m.hmax * 0x1p-18f) * m.scale;
+  const float    lim  = r * r * (1.0f + 0x1p-20f);
+  const float    b2   = cull_radius2(m, active ? lim : -1.0f);
+  const float    sx = px * m.scale, sy = py * m.scale, sz = pz * m.scale;
+  const int      rep = rep_lane(b2);
+  L.best[lane]       = (uint64_t)__double_as_longlong((double)INFINITY);
+  L.tri[lane]        = kInvalid;
+  wave_lds_handoff();
+  Walk<NB> wk;
+  wk.start(0u, 0u);
+  while (wk.top > 0) {
+    --wk.top;
+    const uint32_t cnt = wk.st.cnt_at(wk.top) & (kBoxChild - 1u), ref = uni(wk.st.ref_at(wk.top));
+    if (cnt == 0u) push_walk_children(m, wk, ref, sx, sy, sz, b2, rep);
+    else leaf_band(m, ref, cnt, sx, sy, sz, b2, lim, rx, ry, rz, L);
+  }
+  wave_lds_handoff();
+  d2  = __longlong_as_double((long long)L.best[lane]);
+  tri = L.tri[lane];
+}
+
+// The FP64 signed distance of triangle t at a point (per-lane).
+__device__ __forceinline__ float signed_distance64(const MeshDev& m, uint32_t t, float px, float py, float pz)
+{
+  double   d2;
+  uint32_t f;
+  tri_eval64(m.tripos + 12 * (size_t)t, m.fn64 + 4 * (size_t)t, px, py, pz, d2, f);
+  return (float)resolve64(m, t, f, d2, px, py, pz);
 }
 
 // The closest feature of the winning triangle (per-lane record load), at the point in the mesh's
