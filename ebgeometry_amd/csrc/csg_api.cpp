@@ -308,8 +308,12 @@ ebg_status ebg_csg_query(const ebg_csg* cg, const float* d_pts, uint64_t n, floa
   EBG_HIP(ws.ensure(n));
   uint32_t* cnt = ws.counters();
   EBG_HIP(ebgpu::launch_fill_u32(cnt, 2, 0u, s));
-  const uint32_t* idx = nullptr;
-  if (o.presort && n > 1) {
+  // only tree walks (BVH unions, meshes) gain from neighbouring queries in a wavefront; a program of
+  // analytic leaves runs the same instructions for any points, and in query order its reads and
+  // writes are coalesced (2M queries, 12 blended parts: 368 -> 216 us)
+  const bool      walks = !g->nodes.empty() || !g->meshes.empty();
+  const uint32_t* idx   = nullptr;
+  if (o.presort && n > 1 && walks) {
     EBG_HIP(ebgpu::presort(ws.view(), d_pts, n, s));
     idx = ws.perm.as<uint32_t>();
   }
