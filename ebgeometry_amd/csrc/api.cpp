@@ -589,8 +589,10 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
     cf.heavy = uint32_t(std::max(1.0, heavy_factor(n) * m->grid_mean));
     cf.early = uint32_t(std::max(1.0, kEarlyFactor * m->grid_mean));
   }
-  const uint32_t* idx = nullptr;
-  if (o.presort && n > 1) {
+  const uint32_t  narrow = heavy_first ? 0u : packet_narrow(n);
+  const uint32_t* idx    = nullptr;
+  // one query per wavefront needs no order (closest faces: ties are settled per presorted packet)
+  if (o.presort && n > 1 && (narrow < 6 || face)) {
     EBG_HIP(presort(ws, d_pts, n, s, heavy_first ? &cf : nullptr));
     idx = ws.perm;
   }
@@ -617,6 +619,7 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   a.pts            = d_pts;
   a.idx            = idx;
   a.n              = n;
+  a.narrow         = narrow;
   a.seed_r         = seeds;
   a.out_d          = d_dist;
   a.out_tri        = d_tri;
@@ -668,7 +671,7 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   }
 
   if (recheck) // the list follows the presort order, so FP64 packets hold neighbouring queries
-    EBG_HIP(launch_recheck_compact(a.recheck_mask, n, idx, ws.recheck_list, cnt, s));
+    EBG_HIP(launch_recheck_compact(a.recheck_mask, n, idx, ws.recheck_list, cnt, s, narrow));
   if (recheck || all64) {
     QueryArgs r = a;
     if (recheck) {

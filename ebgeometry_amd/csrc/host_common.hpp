@@ -88,7 +88,7 @@ struct WsView
   uint32_t*           recheck_list = nullptr; // cap
   uint32_t*           counters = nullptr;     // 8: recheck, fallback, HandOn::counts (3), unused
   float*              seeds = nullptr;        // cap
-  uint64_t*           rmask = nullptr;        // packets(cap)
+  uint64_t*           rmask = nullptr;        // mask_packets(cap)
   uint8_t*            heavy_flag = nullptr;   // packets(cap)
   uint32_t*           heavy_list = nullptr;   // heavy_cap(cap)
   unsigned long long* heavy_keys = nullptr;   // 64 x heavy_cap(cap)
@@ -119,7 +119,7 @@ struct Workspace
     // recheck list, fallback list, 2 counters (+pad)
     if ((e = lists.reserve(8 * m + 256)) != hipSuccess) return e;
     if ((e = seeds.reserve(4 * m)) != hipSuccess) return e;
-    if ((e = rmask.reserve(8 * packets(m))) != hipSuccess) return e; // recheck lane mask per packet
+    if ((e = rmask.reserve(8 * mask_packets(m))) != hipSuccess) return e; // recheck lane mask per packet
     // split packets: one flag byte per packet, the list of split packets, 64 result keys each
     if ((e = sched.reserve(sched_early_offset(m) + 4 * (size_t)early_cap(m))) != hipSuccess) return e;
     if ((e = handed.reserve(hand_bytes(m))) != hipSuccess) return e;
@@ -127,6 +127,8 @@ struct Workspace
     return hipSuccess;
   }
   static uint64_t packets(uint64_t n) { return (n + 63) / 64; }
+  // packets of any call of at most n queries, narrowed ones included
+  static uint64_t mask_packets(uint64_t n) { return std::max(packets(n), kNarrowPackets); }
   static uint32_t heavy_cap(uint64_t n) { return (uint32_t)(packets(n) / 64 + 64); }
   static size_t   sched_list_offset(uint64_t n) { return (packets(n) + 255) & ~size_t(255); }
   static size_t   sched_keys_offset(uint64_t n) { return sched_list_offset(n) + ((4 * (size_t)heavy_cap(n) + 255) & ~size_t(255)); }
@@ -194,7 +196,7 @@ struct Workspace
   {
     const uint64_t np = packets(cap);
     return 3 * part(4 * cap) + part(radix_sort_scratch_bytes(cap)) + part(sizeof(double) * 6 * (kBboxParts + 1)) +
-           part(4 * cap) + part(32) + part(4 * cap) + part(8 * np) + part(np) + part(4 * (size_t)heavy_cap(cap)) +
+           part(4 * cap) + part(32) + part(4 * cap) + part(8 * mask_packets(cap)) + part(np) + part(4 * (size_t)heavy_cap(cap)) +
            part(512 * (size_t)heavy_cap(cap)) + part(4 * (size_t)early_cap(cap)) + hand_bytes(cap);
   }
   static WsView carve(uint8_t* base, uint64_t cap)
@@ -215,7 +217,7 @@ struct Workspace
     v.recheck_list = reinterpret_cast<uint32_t*>(take(4 * cap));
     v.counters     = reinterpret_cast<uint32_t*>(take(32));
     v.seeds        = reinterpret_cast<float*>(take(4 * cap));
-    v.rmask        = reinterpret_cast<uint64_t*>(take(8 * np));
+    v.rmask        = reinterpret_cast<uint64_t*>(take(8 * mask_packets(cap)));
     v.heavy_flag   = take(np);
     v.heavy_list   = reinterpret_cast<uint32_t*>(take(4 * (size_t)heavy_cap(cap)));
     v.heavy_keys   = reinterpret_cast<unsigned long long*>(take(512 * (size_t)heavy_cap(cap)));

@@ -29,6 +29,8 @@ struct QueryArgs
   unsigned long long* pair_work; // counting launches: [pairs, pair batches, culling loads, leaves screened]
   float               slack_abs; // FP64 recheck: bound = (|d| + slack_abs + slack_rel*|d|)^2
   float               slack_rel;
+  // queries per packet (wavefront): 64 >> narrow
+  uint32_t            narrow;
   uint32_t*           packet_cost; // counting launches: per packet, the nodes + triangles its wavefront fetched
   // Split packets (split_blocks = 0: none). The first split_blocks workgroups of the FP32 launch
   // stride over the items (j, r), j < min(*split_count, split_cap), r < split_nroots: walk subtree
@@ -78,11 +80,11 @@ struct HeavyMarkArgs
 };
 hipError_t launch_heavy_mark(const HeavyMarkArgs& h, hipStream_t s);
 
-// Recheck list from the per-packet masks of n threads: one wavefront per 64 consecutive packets
-// appends their flagged queries (idx[thread], or the thread) with one atomic on *count, in packet
-// order, so each run of the list covers a compact stretch of the presort curve.
+// Recheck list from the per-packet masks of n threads (64 >> narrow per packet): one wavefront per
+// 64 consecutive packets appends their flagged queries (idx[thread], or the thread) with one atomic
+// on *count, in packet order, so each run of the list covers a compact stretch of the presort curve.
 hipError_t launch_recheck_compact(const uint64_t* mask, uint64_t n, const uint32_t* idx, uint32_t* list,
-                                  uint32_t* count, hipStream_t s);
+                                  uint32_t* count, hipStream_t s, uint32_t narrow = 0);
 
 // After the FP32 launch: the split packets' winning triangles classified, signed and written like
 // the plain pass (outputs, recheck list).
@@ -91,6 +93,18 @@ hipError_t launch_sdf32_resolve(const MeshDev& m, const QueryArgs& a, hipStream_
 // After the FP32 launch: the handed-on items, then the listed packets' winning triangles
 // classified, signed and written like the plain pass (outputs, recheck list).
 hipError_t launch_sdf32_handed(const MeshDev& m, int banks, const QueryArgs& a, hipStream_t s);
+
+// Packets of a call of n queries are narrowed until they are enough wavefronts to spread over the
+// device (kNarrowPackets): the 64 lanes of a packet walk the union of their paths one node after the
+// other, which a call of few queries cannot hide behind other packets.
+constexpr uint64_t kNarrowPackets = 4096;
+inline uint64_t num_packets(uint64_t n, uint32_t narrow) { return (n + (64u >> narrow) - 1) / (64u >> narrow); }
+inline uint32_t packet_narrow(uint64_t n)
+{
+  uint32_t k = 0;
+  while (k < 6 && num_packets(n, k + 1) <= kNarrowPackets) k++;
+  return k;
+}
 
 // FP32 packet traversal over the walk tree; banks = its stack capacity / 64 (1..4).
 hipError_t launch_sdf32(const MeshDev& m, int banks, const QueryArgs& a, bool count, hipStream_t s);

@@ -56,8 +56,9 @@ enum Mode : int
 template <int NB, bool COUNT, int MODE, bool HAND>
 __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& a, uint64_t n, uint64_t pk, PairLds* pl)
 {
-  const uint64_t tid    = pk * 64u + (uint64_t)__lane_id();
-  bool           active = tid < n;
+  const uint32_t width  = 64u >> a.narrow;
+  const uint64_t tid    = pk * width + (uint64_t)__lane_id();
+  bool           active = __lane_id() < (int)width && tid < n;
   uint32_t       qi     = 0;
   float          px = 0.0f, py = 0.0f, pz = 0.0f, bound = -1.0f;
   const float    sc = m.scale;
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8
   const uint32_t blk = xcd_remap(b, nb);
   const uint64_t n   = a.n;
   const uint64_t pk  = (uint64_t)blk * 4u + wave;
-  if (pk * 64u >= n) return;                    // whole wavefront past the end
+  if (pk * (64u >> a.narrow) >= n) return;      // whole wavefront past the end
   if (a.heavy_flag && a.heavy_flag[pk]) return; // whole wavefront: a split or early packet
   sdf32_packet<NB, COUNT, MODE, HAND>(m, a, n, pk, pl);
 }
@@ -269,11 +270,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8
     const SWords<4> it = sload<4>(a.hand.items[STAGE] + w);
     if (it.w[0] == kInvalid) continue;
     const uint32_t      slot = it.w[0];
-    const uint64_t      tid  = (uint64_t)uni(a.hand.list[slot]) * 64u + lane;
+    const uint32_t      width = 64u >> a.narrow;
+    const uint64_t      tid   = (uint64_t)uni(a.hand.list[slot]) * width + lane;
     unsigned long long* keys = a.hand.keys + 64 * (size_t)slot + lane;
     const uint64_t      key  = *keys;
     float               px = 0.0f, py = 0.0f, pz = 0.0f, bound = -1.0f;
-    if (tid < a.n) {
+    if (lane < width && tid < a.n) {
       const uint32_t qi = a.idx ? a.idx[tid] : (uint32_t)tid;
       px                = a.pts[3 * (size_t)qi] * m.scale;
       py                = a.pts[3 * (size_t)qi + 1] * m.scale;
@@ -310,11 +312,12 @@ __global__ __launch_bounds__(256) void sdf32_resolve_kernel(const MeshDev m, con
   for (uint32_t j = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); j < n; j += gridDim.x * 4u) {
     const uint32_t pk = uni(list[j]);
     if (pk == kInvalid) continue;
-    const uint64_t tid   = (uint64_t)pk * 64u + __lane_id();
+    const uint32_t width = 64u >> a.narrow;
+    const uint64_t tid   = (uint64_t)pk * width + __lane_id();
     bool           found = false;
     uint32_t       qi    = 0;
     float          d     = 0.0f;
-    if (tid < a.n) {
+    if (__lane_id() < (int)width && tid < a.n) {
       qi                           = a.idx ? a.idx[tid] : (uint32_t)tid;
       const unsigned long long key = result_keys[64 * (size_t)j + __lane_id()];
       const uint32_t           t   = (uint32_t)key;
@@ -338,7 +341,7 @@ __global__ __launch_bounds__(256) void sdf32_resolve_kernel(const MeshDev m, con
 // one wavefront per 64 consecutive packets
 __global__ __launch_bounds__(256) void recheck_compact_kernel(const uint64_t* __restrict__ mask, uint64_t npk,
                                                               const uint32_t* __restrict__ idx, uint32_t* __restrict__ list,
-                                                              uint32_t* __restrict__ count)
+                                                              uint32_t* __restrict__ count, uint32_t width)
 {
   const uint64_t chunk = (uint64_t)uni(blockIdx.x * 4u + (threadIdx.x >> 6));
   const int      lane  = __lane_id();
@@ -357,19 +360,23 @@ __global__ __launch_bounds__(256) void recheck_compact_kernel(const uint64_t* __
   if (lane == 0) base = atomicAdd(count, total);
   uint32_t pos = rdlane(base, 0) + inc - c;
   while (mk) {
-    const uint64_t tid = pk * 64u + (uint64_t)(__ffsll((unsigned long long)mk) - 1);
+    const uint64_t tid = pk * width + (uint64_t)(__ffsll((unsigned long long)mk) - 1);
     mk &= mk - 1ull;
     list[pos++] = idx ? idx[tid] : (uint32_t)tid;
   }
 }
 
 // The FP64 decision of the closest triangle (band_walk) of one lane's query tid, at most one per
-// lane; (rx, ry, rz) is the wavefront's representative point.
+// lane. For ties: the representative point of the 64-query packet (of the presort order, whatever
+// the width of the wavefront's) that holds the wavefront's first query: its middle query, or its
+// first.
 template <int NB>
-__device__ __forceinline__ void band_block(const MeshDev& m, const QueryArgs& a, bool active, uint64_t tid, BandLds& L)
+__device__ __forceinline__ void band_block(const MeshDev& m, const QueryArgs& a, bool active, uint64_t tid0, uint64_t n,
+                                           BandLds& L)
 {
-  uint32_t qi = 0;
-  float    px = 0.0f, py = 0.0f, pz = 0.0f, d32 = 0.0f;
+  const uint64_t tid = tid0 + __lane_id();
+  uint32_t       qi  = 0;
+  float          px = 0.0f, py = 0.0f, pz = 0.0f, d32 = 0.0f;
   if (active) {
     qi  = a.idx ? a.idx[tid] : (uint32_t)tid;
     px  = a.pts[3 * (size_t)qi];
@@ -381,10 +388,12 @@ __device__ __forceinline__ void band_block(const MeshDev& m, const QueryArgs& a,
     }
     else d32 = a.out_d[qi];
   }
-  const int rep = rep_lane(active ? 0.0f : -1.0f);
-  double    d2;
-  uint32_t  tri;
-  band_walk<NB>(m, px, py, pz, d32, active, rdlanef(px, rep), rdlanef(py, rep), rdlanef(pz, rep), L, d2, tri);
+  const uint64_t g0 = tid0 & ~63ull, rt = g0 + 32u < n ? g0 + 32u : g0;
+  const uint32_t rq = a.idx ? a.idx[rt] : (uint32_t)rt;
+  double         d2;
+  uint32_t       tri;
+  band_walk<NB>(m, px, py, pz, d32, active, a.pts[3 * (size_t)rq], a.pts[3 * (size_t)rq + 1], a.pts[3 * (size_t)rq + 2], L,
+                d2, tri);
   if (active && tri != kInvalid) {
     a.out_d[qi] = signed_distance64(m, tri, px, py, pz);
     if (a.out_tri) a.out_tri[qi] = m.feat[8 * (size_t)tri + 6];
@@ -395,19 +404,17 @@ __device__ __forceinline__ void band_block(const MeshDev& m, const QueryArgs& a,
 template <int NB>
 __global__ __launch_bounds__(256) void band_all_kernel(const MeshDev m, const QueryArgs a)
 {
-  const uint32_t wave = uni(threadIdx.x >> 6);
+  const uint32_t wave = uni(threadIdx.x >> 6), width = 64u >> a.narrow;
   __shared__ BandLds lds[4];
-  const uint64_t pk  = (uint64_t)xcd_remap(blockIdx.x, gridDim.x) * 4u + wave;
-  const uint64_t tid = pk * 64u + __lane_id();
-  if (pk * 64u >= a.n) return; // whole wavefront past the end
-  band_block<NB>(m, a, tid < a.n, tid, lds[wave]);
+  const uint64_t tid0 = ((uint64_t)xcd_remap(blockIdx.x, gridDim.x) * 4u + wave) * width;
+  if (tid0 >= a.n) return; // whole wavefront past the end
+  band_block<NB>(m, a, __lane_id() < (int)width && tid0 + __lane_id() < a.n, tid0, a.n, lds[wave]);
 }
 
 // A device-side list (a.idx, its length *a.count_ptr): a fixed grid of wavefronts strides over the
-// entries, kBandLanes per wavefront (the other lanes sit out). Near-surface queries are sparse
-// even in presort order, so a wavefront walks several paths, and the last to end is the one with
-// the most.
-constexpr uint32_t kBandLanes = 32;
+// entries, at most 32 per wavefront (the other lanes sit out), fewer when the list is short.
+// Near-surface queries are sparse even in presort order, so a wavefront walks several paths, and
+// the last to end is the one with the most.
 template <int NB>
 __global__ __launch_bounds__(256) void band_list_kernel(const MeshDev m, const QueryArgs a)
 {
@@ -415,10 +422,10 @@ __global__ __launch_bounds__(256) void band_list_kernel(const MeshDev m, const Q
   __shared__ BandLds lds[4];
   const uint64_t n     = *a.count_ptr;
   const uint64_t waves = (uint64_t)gridDim.x * 4u;
-  for (uint64_t w = uni(blockIdx.x * 4u + wave); w * kBandLanes < n; w += waves) {
-    const uint64_t tid = w * kBandLanes + lane;
-    band_block<NB>(m, a, lane < kBandLanes && tid < n, tid, lds[wave]);
-  }
+  uint32_t       width = 32u;
+  while (width > 1u && n <= (uint64_t)(width / 2u) * min(waves, (uint64_t)kNarrowPackets)) width /= 2u;
+  for (uint64_t w = uni(blockIdx.x * 4u + wave); w * width < n; w += waves)
+    band_block<NB>(m, a, lane < width && w * width + lane < n, w * width, n, lds[wave]);
 }
 
 template <int NB, int MODE>
@@ -433,9 +440,9 @@ void launch32m(const MeshDev& m, const QueryArgs& a, bool count, uint32_t blocks
 template <int NB>
 hipError_t launch32(const MeshDev& m, const QueryArgs& a, bool count, hipStream_t s)
 {
-  const uint32_t blocks = (uint32_t)((a.n + 255) / 256) + a.split_blocks + a.early_blocks;
+  const uint32_t blocks = (uint32_t)((num_packets(a.n, a.narrow) + 3) / 4) + a.split_blocks + a.early_blocks;
   if (blocks == 0) return hipSuccess;
-  if (a.count_ptr) return hipErrorInvalidValue;
+  if (a.count_ptr || a.narrow > 6 || (a.narrow && (a.split_blocks || a.early_blocks))) return hipErrorInvalidValue;
   if (a.split_blocks && (!a.split_nroots || !a.split_count || !a.heavy_flag)) return hipErrorInvalidValue;
   if (a.hand.slot_cap && (a.split_blocks || !a.hand.list || !a.hand.keys || !a.hand.items[0] ||
                           !a.hand.items[1] || !a.hand.counts))
@@ -454,11 +461,13 @@ hipError_t launch32(const MeshDev& m, const QueryArgs& a, bool count, hipStream_
 template <int NB>
 hipError_t launch64(const MeshDev& m, const QueryArgs& a, hipStream_t s)
 {
-  const uint32_t blocks = (uint32_t)((a.n + 255) / 256);
-  if (blocks == 0) return hipSuccess;
-  if (a.count_ptr)
-    hipLaunchKernelGGL(band_list_kernel<NB>, dim3(std::min<uint32_t>(2u * blocks, kListGrid)), dim3(256), 0, s, m, a);
-  else hipLaunchKernelGGL(band_all_kernel<NB>, dim3(blocks), dim3(256), 0, s, m, a);
+  if (a.n == 0) return hipSuccess;
+  if (a.count_ptr) {
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((a.n + 3) / 4, kListGrid);
+    hipLaunchKernelGGL(band_list_kernel<NB>, dim3(blocks), dim3(256), 0, s, m, a);
+  }
+  else
+    hipLaunchKernelGGL(band_all_kernel<NB>, dim3((uint32_t)((num_packets(a.n, a.narrow) + 3) / 4)), dim3(256), 0, s, m, a);
   return hipGetLastError();
 }
 
@@ -530,13 +539,13 @@ hipError_t launch_heavy_mark(const HeavyMarkArgs& h, hipStream_t s)
 }
 
 hipError_t launch_recheck_compact(const uint64_t* mask, uint64_t n, const uint32_t* idx, uint32_t* list,
-                                  uint32_t* count, hipStream_t s)
+                                  uint32_t* count, hipStream_t s, uint32_t narrow)
 {
-  const uint64_t npk    = (n + 63) / 64;
+  const uint64_t npk    = num_packets(n, narrow);
   const uint64_t chunks = (npk + 63) / 64;
   if (chunks == 0) return hipSuccess;
   hipLaunchKernelGGL(recheck_compact_kernel, dim3((uint32_t)((chunks + 3) / 4)), dim3(256), 0, s, mask, npk, idx, list,
-                     count);
+                     count, 64u >> narrow);
   return hipGetLastError();
 }
 
