@@ -158,7 +158,7 @@ ebg_status ebg_csg_create(const ebg_csg_op* ops, uint64_t num_ops, uint64_t main
     if (!meshes[j]) return fail(EBG_INVALID_ARG, "null mesh handle");
     if (KM && meshes[j]->K != KM) return fail(EBG_INVALID_ARG, "all program meshes must have the same branching");
     KM         = meshes[j]->K;
-    mesh_banks = std::max(mesh_banks, meshes[j]->banks);
+    mesh_banks = std::max({mesh_banks, meshes[j]->banks, meshes[j]->wbanks});
   }
   if (!KM) KM = 4;
 

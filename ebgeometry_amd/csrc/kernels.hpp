@@ -116,7 +116,7 @@ hipError_t launch_sdf64(const MeshDev& m, int banks, const QueryArgs& a, hipStre
 // CSG union scenes (scene.hip). KM = branching of the instanced meshes (all equal); banks =
 // stack capacity / 64 for both the scene tree and the mesh trees. Work counters: [0] interior
 // nodes, [1] triangles, [4]/[5] their wave-level fetches, [6] primitives, [7] wave-level.
-hipError_t launch_scene32(const SceneDev& sc, int KM, int banks, const QueryArgs& a, bool count, hipStream_t s);
+hipError_t launch_scene32(const SceneDev& sc, int banks, const QueryArgs& a, bool count, hipStream_t s);
 // FP64 pass over a.idx / a.count_ptr, seeded with |v32| (1 + slack_rel) + slack_abs.
 hipError_t launch_scene64(const SceneDev& sc, int KM, int banks, const QueryArgs& a, hipStream_t s);
 

@@ -89,7 +89,7 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
     if (!meshes[j]) return fail(EBG_INVALID_ARG, "null mesh handle");
     if (KM && meshes[j]->K != KM) return fail(EBG_INVALID_ARG, "all scene meshes must have the same branching");
     KM         = meshes[j]->K;
-    mesh_banks = std::max(mesh_banks, meshes[j]->banks);
+    mesh_banks = std::max({mesh_banks, meshes[j]->banks, meshes[j]->wbanks});
   }
   if (!KM) KM = 4;
 
@@ -314,7 +314,7 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
   const bool count = o.work != nullptr;
 
   EBG_HIP(hipEventRecord(sc->ev0, s));
-  EBG_HIP(ebgpu::launch_scene32(sc->dev, sc->KM, sc->banks, a, count, s));
+  EBG_HIP(ebgpu::launch_scene32(sc->dev, sc->banks, a, count, s));
   EBG_HIP(hipEventRecord(sc->ev1, s));
   sc->timed = true;
   if (recheck) {

@@ -693,10 +693,10 @@ __device__ __forceinline__ float bperm(int addr, float x)
 }
 
 // The screen of one triangle: its disc (record i of sp) against each lane's cull radius, disc_lanes
-// with t = 0, where (n.s)^2 + w = b2. The lanes it may reach write `entry` to the pair list
-// from place `total` on (mine: this lane is one); returns their number.
-__device__ __forceinline__ uint32_t list_pairs(const SWords<32>& sp, int i, float px, float py, float pz, float b2,
-                                               uint32_t entry, uint32_t total, uint16_t* list, bool& mine)
+// with t = 0, where (n.s)^2 + w = b2. Returns the mask of the lanes it may reach (mine: this lane's
+// bit, from the compares).
+__device__ __forceinline__ uint64_t disc_reaches(const SWords<32>& sp, int i, float px, float py, float pz, float b2,
+                                                 bool& mine)
 {
   const float sx = px - __uint_as_float(sp.w[8 * i]), sy = py - __uint_as_float(sp.w[8 * i + 1]),
               sz = pz - __uint_as_float(sp.w[8 * i + 2]);
@@ -705,11 +705,18 @@ __device__ __forceinline__ uint32_t list_pairs(const SWords<32>& sp, int i, floa
   const float w = fmaf(-pd, pd, b2);
   const float B = fmaf(sz, sz, fmaf(sy, sy, fmaf(sx, sx, __uint_as_float(sp.w[8 * i + 7])))) - b2;
   const bool  in_r = !(B * fabsf(B) > __uint_as_float(sp.w[8 * i + 6]) * w), in_p = !(w < 0.0f);
-  const uint64_t pm = ballot(in_r) & ballot(in_p);
-  mine              = in_r && in_p;
+  mine             = in_r && in_p;
+  return ballot(in_r) & ballot(in_p);
+}
+
+// The lanes that a triangle may reach write `entry` to the pair list from place `total` on; returns
+// their number.
+__device__ __forceinline__ uint32_t list_pairs(const SWords<32>& sp, int i, float px, float py, float pz, float b2,
+                                               uint32_t entry, uint32_t total, uint16_t* list, bool& mine)
+{
+  const uint64_t pm = disc_reaches(sp, i, px, py, pz, b2, mine);
   if (pm == 0) return 0u;
-  // this lane's bit of pm is in_r && in_p: the write is predicated on the compares
-  if (mine) list[mbcnt(pm, total)] = (uint16_t)entry;
+  if (mine) list[mbcnt(pm, total)] = (uint16_t)entry; // predicated on the compares
   return (uint32_t)__popcll(pm);
 }
 
@@ -1076,6 +1083,73 @@ __device__ __forceinline__ void mesh_walk(const MeshDev& m, Walk<NB>& wk, uint32
       st.bound_at(top, v);
       st.put(bot, st.ref_at(top), st.cnt_at(top), v);
       push_walk_children(m, wk, eref, px, py, pz, b2, rep);
+    }
+  }
+}
+
+// The walk for kernels without the pair-compacted leaves' LDS (mesh instances of scenes, mesh
+// leaves of programs): a triangle is evaluated by the whole wavefront when some lane's cull radius
+// reaches its disc, behind the lower-bound cull of tri_eval32_culled. px, py, pz, bound and best are
+// in the mesh's own units; bound < 0: a lane without a query. Lanes meet triangles that only others
+// asked for too, so with a finite bound `best` is the lane's minimum only if it is within it.
+template <int NB, bool COUNT>
+__device__ __forceinline__ void wide_walk(const MeshDev& m, float px, float py, float pz, float bound, float& best,
+                                          uint32_t& btri, uint32_t& n_inner, uint32_t& n_tris, uint32_t& w_inner,
+                                          uint32_t& w_tris)
+{
+  const int   lane = __lane_id(), rep = rep_lane(bound);
+  const float ss = m.scale * m.scale, sx = px * m.scale, sy = py * m.scale, sz = pz * m.scale;
+  float       b2   = cull_radius2(m, bound * ss);
+  Walk<NB>    wk;
+  wk.start(0u, 0u);
+  while (wk.top > 0) {
+    --wk.top;
+    const uint32_t ecnt = wk.st.cnt_at(wk.top);
+    bool           need = true;
+    if (COUNT || (ecnt >> kStampShift) != wk.stamp) {
+      float v[8], key;
+      wk.st.bound_at(wk.top, v);
+      const uint64_t mask = (ecnt & kBoxChild) ? walk_box_lanes(v, sx, sy, sz, b2, key)
+                                               : disc_lanes(v, sx, sy, sz, b2, key);
+      if (mask == 0) continue;
+      if (COUNT) need = ((mask >> lane) & 1ull) != 0;
+    }
+    const uint32_t eref = uni(wk.st.ref_at(wk.top)), cnt = ecnt & (kBoxChild - 1u);
+    if (cnt == 0u) {
+      if (COUNT) { n_inner += need ? 1u : 0u; w_inner++; }
+      push_walk_children(m, wk, eref, sx, sy, sz, b2, rep);
+      continue;
+    }
+    const float bound0 = bound;
+    float       cull   = cull_band(bound, m.hmax);
+    for (uint32_t c0 = 0; c0 < cnt; c0 += 4) {
+      const SWords<32> sp     = sload<32>(m.tdisc + eref + c0);
+      uint32_t         needed = 0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (c0 + i < cnt) {
+          bool mine;
+          if (disc_reaches(sp, i, sx, sy, sz, b2, mine)) needed |= 1u << i;
+          if (COUNT) n_tris += mine ? 1u : 0u;
+        }
+      }
+      while (needed) {
+        const uint32_t t = eref + c0 + (uint32_t)__builtin_ctz(needed);
+        needed &= needed - 1u;
+        float d2;
+        if (!tri_eval32_culled(sload_record(m.tris + t), px, py, pz, cull, d2)) continue;
+        if (COUNT) w_tris++;
+        if (d2 < best) {
+          best  = d2;
+          btri  = t;
+          bound = d2 < bound ? d2 : bound; // bound stays min(bound, best)
+          cull  = cull_band(bound, m.hmax);
+        }
+      }
+    }
+    if (ballot(bound < bound0)) {
+      wk.stamp++;
+      b2 = cull_radius2(m, bound * ss);
     }
   }
 }
