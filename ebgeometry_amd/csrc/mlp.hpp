@@ -69,6 +69,7 @@ struct Mlp
   float*    adam_m  = nullptr;
   float*    adam_v  = nullptr;
   uint16_t* wtrain  = nullptr;   // kBfTotal BF16, row-major [in][out]
+  uint16_t* wtrain_t = nullptr;  // the same, [out][in] per layer
   uint16_t* winfer  = nullptr;   // kBfInfer BF16, inference fragment layout
   int       step    = 0;
   ~Mlp();
@@ -88,20 +89,18 @@ hipError_t mlp_sync_bf16(Mlp& m, hipStream_t s);
 hipError_t mlp_forward(const Mlp& m, const float* pts, const uint32_t* idx, uint64_t n, bool seed_mode, float scale,
                        float offset, float* out, hipStream_t s);
 
-// Training state for one batch size.
+// Training state: partial gradients of a step's workgroups (grown on demand) and the loss sum.
 struct MlpTrainBuffers
 {
-  int       batch = 0;
-  uint16_t* x0    = nullptr; // B x 64
-  uint16_t* h[4]  = {};      // B x 128 each
-  uint16_t* dl[4] = {};      // B x 128 each (deltas)
-  float*    g     = nullptr; // B
-  float*    loss  = nullptr; // 1
+  int    parts = 0;
+  float* part  = nullptr; // parts x kMaster
+  float* loss  = nullptr; // 1
   ~MlpTrainBuffers();
-  hipError_t ensure(int b);
+  hipError_t ensure(int batch);
 };
+int mlp_train_blocks(int n); // workgroups, hence partial gradients, of a step of n rows
 
-// Loss and full parameter gradient (into m.grad, master layout) for n <= buffers.batch points
+// Loss and full parameter gradient (into m.grad, master layout) for n points
 // with targets |d| (physical units). The summed loss is added to tb.loss[0].
 // On failure *why (nullable) names the check that failed.
 hipError_t mlp_loss_grad(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, int n,
@@ -109,8 +108,9 @@ hipError_t mlp_loss_grad(Mlp& m, MlpTrainBuffers& tb, const float* pts, const fl
 // Host-only: run the shape and extent checks of every launch of the training steps that
 // ebg_mlp_train enqueues for these sizes (full batches and the last, partial one). No GPU.
 bool mlp_check_train_schedule(uint64_t num_samples, int batch, std::string* why);
-// One Adam step on m (uses m.grad), then refresh the BF16 copies.
-hipError_t mlp_adam(Mlp& m, float lr, hipStream_t s);
+// One training step: loss, gradient, Adam and the BF16 training copies (not the inference copy).
+hipError_t mlp_step(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, int n, float lr, hipStream_t s,
+                    std::string* why);
 // Copy the gradient out in the public parameter order (device pointer, kMlpParams floats).
 hipError_t mlp_grad_public(const Mlp& m, float* out, hipStream_t s);
 
