@@ -66,8 +66,7 @@ static double heavy_factor(uint64_t n) { return n >= (1u << 22) ? 6.0 : 3.0; }
 // 1.49 ms handed on, 5.2M 2.14 against 2.45 ms, 16M on 327,680 faces 5.03 against 5.63 ms.
 // Budgets and spreads: (200, 100, 32, 16) 0.93 ms, (150, 60, 48, 32) 0.87, (100, 60, 32, 32) 0.86 on
 // the 1M queries.
-constexpr uint32_t kHandBudget[2] = {150, 60};
-constexpr int32_t  kHandSpread[2] = {48, 32};
+
 
 
 // Subtree roots for split packets: breadth-first from the root, each interior entry replaced by
@@ -654,8 +653,8 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   if (hand_on) {
     a.hand = ws.hand;
     for (int i = 0; i < 2; i++) {
-      a.hand.budget[i] = kHandBudget[i];
-      a.hand.spread[i] = kHandSpread[i];
+      a.hand.budget[i] = ebgpu::kHandBudget[i];
+      a.hand.spread[i] = ebgpu::kHandSpread[i];
     }
   }
 

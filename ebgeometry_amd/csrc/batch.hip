@@ -67,37 +67,30 @@ __global__ __launch_bounds__(256) void batch_keys_kernel(const BatchItemDev* __r
   keys[g] = KeyT(((uint64_t)lo << 24) | hilbert_index<8>(x[0], x[1], x[2]));
 }
 
-// One packet: the wavefront's 64 queries of one item against its mesh.
-template <int NB, bool COUNT>
-__device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, PairLds* pl)
+// A lane's query of packet p (item it, first query `first`): its index in the item and its point in
+// the walk's units. False: no query, or a NaN coordinate (no closest triangle; nothing is written).
+__device__ __forceinline__ bool batch_query(const BatchArgs& a, const BatchItemDev& it, const MeshDev& m, uint32_t first,
+                                            uint32_t& qi, float& px, float& py, float& pz)
 {
-  const SWords<4>    pk = sload<4>(a.packets + 4 * (size_t)p);
-  const uint32_t     item = pk.w[0], first = pk.w[1];
-  const BatchItemDev it   = sload_record(a.items + item);
-  const MeshDev      m    = sload_record(a.meshes + it.mesh);
+  const uint32_t j = first + __lane_id();
+  qi               = 0;
+  px = py = pz = 0.0f;
+  if (j >= it.n) return false;
+  qi = a.sorted ? (uint32_t)(a.sorted[it.base + j] - it.base) : j;
+  px = it.pts[3 * (size_t)qi] * m.scale;
+  py = it.pts[3 * (size_t)qi + 1] * m.scale;
+  pz = it.pts[3 * (size_t)qi + 2] * m.scale;
+  if (px == px && py == py && pz == pz) return true;
+  px = py = pz = 0.0f;
+  return false;
+}
 
-  const uint32_t lane   = __lane_id();
-  const uint32_t j      = first + lane;
-  bool           active = j < it.n;
-  uint32_t       qi     = 0;
-  float          px = 0.0f, py = 0.0f, pz = 0.0f;
-  if (active) {
-    qi = a.sorted ? (uint32_t)(a.sorted[it.base + j] - it.base) : j;
-    px = it.pts[3 * (size_t)qi] * m.scale;
-    py = it.pts[3 * (size_t)qi + 1] * m.scale;
-    pz = it.pts[3 * (size_t)qi + 2] * m.scale;
-    if (!(px == px && py == py && pz == pz)) { // NaN: no closest triangle, the lane takes no part
-      px = py = pz = 0.0f;
-      active       = false;
-    }
-  }
-  float    best = INFINITY;
-  uint32_t btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
-  PairCounts pc{0u, 0u, 0u, 0u};
-  float      bound = active ? INFINITY : -1.0f;
-  Walk<NB>   wk;
-  wk.start(0u, 0u);
-  mesh_walk<NB, COUNT, false>(m, wk, ~0u, 0, px, py, pz, bound, best, btri, n_inner, n_tris, w_inner, w_tris, pl, &pc);
+// The end of a packet: classify, sign and write each lane's closest triangle, and the packet's
+// recheck mask. Point and distance^2 in the walk's units.
+__device__ __forceinline__ void batch_finish(const BatchArgs& a, const BatchItemDev& it, const MeshDev& m, uint32_t p,
+                                             bool active, uint32_t qi, float px, float py, float pz, float best,
+                                             uint32_t btri)
+{
   px *= m.inv_scale;
   py *= m.inv_scale;
   pz *= m.inv_scale;
@@ -111,12 +104,39 @@ __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, Pai
   }
   if (a.recheck_mask) {
     const uint64_t mask = ballot(found && fabsf(d) < it.recheck_abs);
-    if (lane == 0) a.recheck_mask[p] = mask;
+    if (__lane_id() == 0) a.recheck_mask[p] = mask;
   }
+}
+
+// One packet: the wavefront's 64 queries of one item against its mesh. HAND: a long walk is handed
+// on (HandOn).
+template <int NB, bool COUNT, bool HAND>
+__device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, PairLds* pl)
+{
+  const SWords<4>    pk = sload<4>(a.packets + 4 * (size_t)p);
+  const BatchItemDev it = sload_record(a.items + pk.w[0]);
+  const MeshDev      m  = sload_record(a.meshes + it.mesh);
+  uint32_t           qi;
+  float              px, py, pz;
+  const bool         active = batch_query(a, it, m, pk.w[1], qi, px, py, pz);
+  float              best = INFINITY, bound = active ? INFINITY : -1.0f;
+  uint32_t           btri = kInvalid, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
+  PairCounts         pc{0u, 0u, 0u, 0u};
+  Walk<NB>           wk;
+  wk.start(0u, 0u);
+  uint32_t budget = HAND ? a.hand.budget[0] : ~0u;
+  for (;;) {
+    mesh_walk<NB, COUNT, HAND>(m, wk, budget, HAND ? a.hand.spread[0] : 0, px, py, pz, bound, best, btri, n_inner, n_tris,
+                               w_inner, w_tris, pl, &pc);
+    if (!HAND || wk.top == 0) break;
+    if (hand_on(a.hand, wk, p, best, btri)) return; // whole wavefront
+    budget = ~0u;
+  }
+  batch_finish(a, it, m, p, active, qi, px, py, pz, best, btri);
   if (COUNT && a.work) {
     const uint64_t si = wave_sum_u64(active ? (uint64_t)n_inner : 0ull);
     const uint64_t st = wave_sum_u64(active ? (uint64_t)n_tris : 0ull);
-    if (lane == 0) {
+    if (__lane_id() == 0) {
       atomicAdd(a.work, (unsigned long long)si);
       atomicAdd(a.work + 1, (unsigned long long)st);
       atomicAdd(a.work + 4, (unsigned long long)w_inner);
@@ -131,10 +151,64 @@ __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, Pai
   }
 }
 
+// The items handed on, as sdf32_items_kernel: stage 0 hands on again, stage 1 walks to the end.
+template <int NB, int STAGE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8 : (NB == 2 ? 6 : 4)))) void batch_items_kernel(const BatchArgs a)
+{
+  const uint32_t wave = uni(threadIdx.x >> 6);
+  extern __shared__ PairLds pair_lds[];
+  PairLds* const pl = &pair_lds[wave];
+  const uint32_t n  = min(a.hand.counts[1 + STAGE], a.hand.item_cap);
+  for (uint32_t w = uni(blockIdx.x * 4u + wave); w < n; w += gridDim.x * 4u) {
+    const SWords<4> hi = sload<4>(a.hand.items[STAGE] + w);
+    if (hi.w[0] == kInvalid) continue;
+    const uint32_t      slot = hi.w[0];
+    const SWords<4>     pk   = sload<4>(a.packets + 4 * (size_t)uni(a.hand.list[slot]));
+    const BatchItemDev  it   = sload_record(a.items + pk.w[0]);
+    const MeshDev       m    = sload_record(a.meshes + it.mesh);
+    unsigned long long* keys = a.hand.keys + 64 * (size_t)slot + __lane_id();
+    const uint64_t      key  = *keys;
+    uint32_t            qi;
+    float               px, py, pz;
+    const bool          active = batch_query(a, it, m, pk.w[1], qi, px, py, pz);
+    float               best = __uint_as_float((uint32_t)(key >> 32)), bound = active ? best : -1.0f;
+    uint32_t            btri = (uint32_t)key, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
+    Walk<NB>            wk;
+    wk.start(hi.w[1], hi.w[2]);
+    uint32_t budget = STAGE == 0 ? a.hand.budget[1] : ~0u;
+    for (;;) {
+      mesh_walk<NB, false, true>(m, wk, budget, a.hand.spread[1], px, py, pz, bound, best, btri, n_inner, n_tris, w_inner,
+                                 w_tris, pl, nullptr);
+      if (wk.top == 0 || append_items(wk, slot, a.hand.items[1], a.hand.counts + 2, a.hand.item_cap)) break;
+      budget = ~0u; // no room: walk on
+    }
+    const uint64_t now = ((uint64_t)__float_as_uint(best) << 32) | btri;
+    if (now < key) atomicMin(keys, (unsigned long long)now);
+  }
+}
+
+// The handed-on packets' end, from their keys.
+__global__ __launch_bounds__(256) void batch_resolve_kernel(const BatchArgs a)
+{
+  const uint32_t n = min(a.hand.counts[0], a.hand.slot_cap);
+  for (uint32_t s = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); s < n; s += gridDim.x * 4u) {
+    const uint32_t p = uni(a.hand.list[s]);
+    if (p == kInvalid) continue;
+    const SWords<4>    pk = sload<4>(a.packets + 4 * (size_t)p);
+    const BatchItemDev it = sload_record(a.items + pk.w[0]);
+    const MeshDev      m  = sload_record(a.meshes + it.mesh);
+    uint32_t           qi;
+    float              px, py, pz;
+    const bool         active = batch_query(a, it, m, pk.w[1], qi, px, py, pz);
+    const uint64_t     key    = a.hand.keys[64 * (size_t)s + __lane_id()];
+    batch_finish(a, it, m, p, active, qi, px, py, pz, __uint_as_float((uint32_t)(key >> 32)), (uint32_t)key);
+  }
+}
+
 // PERSIST = false: one wavefront per packet (the early list first, then the table without the
 // early packets). PERSIST = true: a grid that fits the device at once; each wavefront takes queue
 // entries in the same order until the queue is exhausted (no wavefront waits on another).
-template <int NB, bool COUNT, bool PERSIST>
+template <int NB, bool COUNT, bool PERSIST, bool HAND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8 : (NB == 2 ? 6 : 4)))) void batch32_kernel(const BatchArgs a)
 {
   extern __shared__ PairLds pair_lds[]; // one per wavefront of the workgroup
@@ -156,7 +230,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8
         p = w - skip;
         if (p >= a.num_packets || (a.early_blocks && a.flag[p])) continue;
       }
-      batch_packet<NB, COUNT>(a, p, pl);
+      batch_packet<NB, COUNT, HAND>(a, p, pl);
     }
   }
   else {
@@ -182,7 +256,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8
     }
     else p = w;
     if (p >= a.num_packets) return; // whole wavefront (p is wave-uniform)
-    batch_packet<NB, COUNT>(a, p, pl);
+    batch_packet<NB, COUNT, HAND>(a, p, pl);
   }
 }
 
@@ -276,31 +350,47 @@ __global__ __launch_bounds__(256) void batch_mark_kernel(const BatchArgs a)
   }
 }
 
+// launch shape: PERSIST and HAND are the plan's, counting launches hand nothing on
+template <int NB, bool PERSIST>
+auto batch32_of(bool count, bool hand)
+{
+  return count ? batch32_kernel<NB, true, PERSIST, false>
+               : (hand ? batch32_kernel<NB, false, PERSIST, true> : batch32_kernel<NB, false, PERSIST, false>);
+}
+
 template <int NB>
 hipError_t launch32(const BatchArgs& a, int wg, bool count, hipStream_t s)
 {
-  const size_t lds = (size_t)(wg / 64) * sizeof(PairLds);
+  const size_t   lds  = (size_t)(wg / 64) * sizeof(PairLds);
+  const uint32_t wpb  = (uint32_t)wg / 64u;
+  const bool     hand = a.hand.slot_cap != 0 && !count;
+  if (hand && (!a.hand.list || !a.hand.keys || !a.hand.items[0] || !a.hand.items[1] || !a.hand.counts))
+    return hipErrorInvalidValue;
   if (a.persist_blocks) {
     if (!a.queue) return hipErrorInvalidValue;
-    if (count) hipLaunchKernelGGL((batch32_kernel<NB, true, true>), dim3(a.persist_blocks), dim3(wg), lds, s, a);
-    else hipLaunchKernelGGL((batch32_kernel<NB, false, true>), dim3(a.persist_blocks), dim3(wg), lds, s, a);
-    return hipGetLastError();
+    hipLaunchKernelGGL((batch32_of<NB, true>(count, hand)), dim3(a.persist_blocks), dim3(wg), lds, s, a);
   }
-  const uint32_t wpb    = (uint32_t)wg / 64u;
-  const uint32_t blocks = (a.num_packets + wpb - 1) / wpb + a.early_blocks;
-  if (blocks == 0) return hipSuccess;
-  if (count) hipLaunchKernelGGL((batch32_kernel<NB, true, false>), dim3(blocks), dim3(wg), lds, s, a);
-  else hipLaunchKernelGGL((batch32_kernel<NB, false, false>), dim3(blocks), dim3(wg), lds, s, a);
+  else {
+    const uint32_t blocks = (a.num_packets + wpb - 1) / wpb + a.early_blocks;
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL((batch32_of<NB, false>(count, hand)), dim3(blocks), dim3(wg), lds, s, a);
+  }
+  if (hand) {
+    const size_t   l4 = 4 * sizeof(PairLds);
+    const uint32_t g  = std::clamp<uint32_t>(2u * a.num_packets, 512u, 2048u);
+    hipLaunchKernelGGL((batch_items_kernel<NB, 0>), dim3(g), dim3(256), l4, s, a);
+    hipLaunchKernelGGL((batch_items_kernel<NB, 1>), dim3(g), dim3(256), l4, s, a);
+    hipLaunchKernelGGL(batch_resolve_kernel, dim3(std::min(g, (a.hand.slot_cap + 3u) / 4u)), dim3(256), 0, s, a);
+  }
   return hipGetLastError();
 }
 
 template <int NB>
-hipError_t persist_blocks(int wg, bool count, uint32_t* blocks)
+hipError_t persist_blocks(int wg, bool count, bool hand, uint32_t* blocks)
 {
-  int        nb = 0, dev = 0, cus = 0;
+  int          nb = 0, dev = 0, cus = 0;
   const size_t lds = (size_t)(wg / 64) * sizeof(PairLds);
-  hipError_t   e   = count ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch32_kernel<NB, true, true>, wg, lds)
-                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch32_kernel<NB, false, true>, wg, lds);
+  hipError_t   e   = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch32_of<NB, true>(count, hand), wg, lds);
   if (e != hipSuccess) return e;
   if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
   if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
@@ -351,12 +441,12 @@ hipError_t launch_batch32(const BatchArgs& a, int banks, int wg, bool count, hip
   return launch32<4>(a, wg, count, s);
 }
 
-hipError_t batch32_persistent_blocks(int banks, int wg, bool count, uint32_t* blocks)
+hipError_t batch32_persistent_blocks(int banks, int wg, bool count, bool hand, uint32_t* blocks)
 {
   if (wg != 64 && wg != 128 && wg != 256) return hipErrorInvalidValue;
-  if (banks <= 1) return persist_blocks<1>(wg, count, blocks);
-  if (banks == 2) return persist_blocks<2>(wg, count, blocks);
-  return persist_blocks<4>(wg, count, blocks);
+  if (banks <= 1) return persist_blocks<1>(wg, count, hand, blocks);
+  if (banks == 2) return persist_blocks<2>(wg, count, hand, blocks);
+  return persist_blocks<4>(wg, count, hand, blocks);
 }
 
 hipError_t launch_batch64(const BatchArgs& a, int banks, hipStream_t s)

@@ -41,6 +41,8 @@ struct ebg_batch_plan
   DevBuf          items, packets, keys, keys_sorted, sorted, scratch, rmask, recheck, counter;
   DevBuf          grids, flags, early; // early packets: per-mesh grid records, packet flags, list
   uint32_t        early_cap = 0;       // 0: no early packets
+  DevBuf          handed;              // HandOn's lists
+  bool            hand = false;        // long walks are handed on
   int             wg = 256;
   bool            persistent = false;  // one grid that fits the device, wavefronts take packets from a queue
   uint32_t        persist_blocks = 0;
@@ -190,9 +192,16 @@ ebg_status enqueue(ebg_batch_plan* p, hipStream_t s, bool events)
   a.recheck_count = p->counter.as<uint32_t>();
   a.work          = p->work;
   a.pair_work     = p->work ? p->pair_work : nullptr;
-  // counters: [0] recheck list, [1] early list, [2] persistent queue (a fill kernel, so that a
-  // captured plan clears them on every replay)
-  if (p->fp64 || p->early_cap || p->persistent) EBG_HIP(ebgpu::launch_fill_u32(a.recheck_count, 3, 0u, s));
+  // counters: [0] recheck list, [1] early list, [2] persistent queue, [4..6] HandOn::counts (a fill
+  // kernel, so that a captured plan clears them on every replay)
+  EBG_HIP(ebgpu::launch_fill_u32(a.recheck_count, 8, 0u, s));
+  if (p->hand) {
+    a.hand = ebgpu::Workspace::hand_view(p->handed.as<uint8_t>(), p->total, p->counter.as<uint32_t>() + 4);
+    for (int i = 0; i < 2; i++) {
+      a.hand.budget[i] = ebgpu::kHandBudget[i];
+      a.hand.spread[i] = ebgpu::kHandSpread[i];
+    }
+  }
   if (p->presort && p->total > 1) {
     int item_bits = 1;
     while ((1ull << item_bits) < p->num_items) item_bits++;
@@ -238,6 +247,9 @@ ebg_status enqueue(ebg_batch_plan* p, hipStream_t s, bool events)
 // Early packets of a plan: meshes from 16,384 faces get a cost grid; packets at >= 2x their
 // mesh's grid mean start first (256-mesh workload: 66.8 -> 55.4 ms; 1.5x: 56.3, 3x: 55.4).
 constexpr uint64_t kEarlyMinFaces = 16384;
+// Plans of fewer queries hand long walks on (HandOn) besides: such a launch is over before its
+// longest packets are, early or not (32 meshes of 1,280 to 81,920 faces, 5M queries: 4.1 -> 1.6 ms).
+constexpr uint64_t kHandMaxTotal = 1u << 23;
 constexpr double   kEarlyFactor   = 2.0;
 
 double elapsed_ms(hipEvent_t a, hipEvent_t b)
@@ -476,6 +488,8 @@ ebg_status ebg_batch_plan_create(ebg_batch* b, const ebg_batch_item* items, uint
   if ((e = p->rmask.reserve(8 * std::max<uint64_t>(p->num_packets, 1))) != hipSuccess) return bail(e, "recheck");
   if ((e = p->recheck.reserve(4 * (p->fp64 ? cap : 1))) != hipSuccess) return bail(e, "recheck");
   if ((e = p->counter.reserve(256)) != hipSuccess) return bail(e, "counter");
+  p->hand = total < kHandMaxTotal && !p->work;
+  if (p->hand && (e = p->handed.reserve(ebgpu::Workspace::hand_bytes(total))) != hipSuccess) return bail(e, "hand-on lists");
   if ((e = hipEventCreate(&p->ev0)) != hipSuccess || (e = hipEventCreate(&p->ev1)) != hipSuccess)
     return bail(e, "events");
 
@@ -522,7 +536,7 @@ ebg_status ebg_batch_plan_create(ebg_batch* b, const ebg_batch_item* items, uint
   auto set_shape = [&](int wg, bool persistent) -> hipError_t {
     p->wg         = wg;
     p->persistent = persistent;
-    return persistent ? ebgpu::batch32_persistent_blocks(b->wbanks, wg, p->work != nullptr, &p->persist_blocks)
+    return persistent ? ebgpu::batch32_persistent_blocks(b->wbanks, wg, p->work != nullptr, p->hand, &p->persist_blocks)
                       : hipSuccess;
   };
   if ((e = set_shape(p->wg, p->persistent)) != hipSuccess) return bail(e, "occupancy");

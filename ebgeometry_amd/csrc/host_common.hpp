@@ -98,7 +98,9 @@ struct WsView
 
 // Calls of fewer queries hand long walks on (HandOn); larger presorted ones split the packets that
 // their cost grid finds expensive.
-constexpr uint64_t kHandMaxQ = 1u << 20;
+constexpr uint64_t kHandMaxQ      = 1u << 20;
+constexpr uint32_t kHandBudget[2] = {150, 60}; // HandOn::budget (measured: api.cpp)
+constexpr int32_t  kHandSpread[2] = {48, 32};
 
 // Query workspace, grown on demand.
 struct Workspace
@@ -122,7 +124,7 @@ struct Workspace
     if ((e = rmask.reserve(8 * mask_packets(m))) != hipSuccess) return e; // recheck lane mask per packet
     // split packets: one flag byte per packet, the list of split packets, 64 result keys each
     if ((e = sched.reserve(sched_early_offset(m) + 4 * (size_t)early_cap(m))) != hipSuccess) return e;
-    if ((e = handed.reserve(hand_bytes(m))) != hipSuccess) return e;
+    if ((e = handed.reserve(hand_bytes(std::min(m, kHandMaxQ)))) != hipSuccess) return e;
     cap = m;
     return hipSuccess;
   }
@@ -142,7 +144,7 @@ struct Workspace
     return reinterpret_cast<unsigned long long*>(sched.as<uint8_t>() + sched_keys_offset(cap));
   }
   // Room for handed-on packets: 1 in 16 (64-query packets), and at least 1,024, with 32 items each.
-  static uint32_t    hand_slots(uint64_t n) { return (uint32_t)(packets(std::min(n, kHandMaxQ)) / 16 + 1024); }
+  static uint32_t    hand_slots(uint64_t n) { return (uint32_t)(packets(n) / 16 + 1024); }
   static uint32_t    hand_items(uint64_t n) { return 32 * hand_slots(n); }
   static std::size_t hand_bytes(uint64_t n)
   {
@@ -186,7 +188,7 @@ struct Workspace
     v.heavy_list   = heavy_list();
     v.heavy_keys   = heavy_keys();
     v.early_list   = early_list();
-    v.hand         = hand_view(handed.as<uint8_t>(), cap, v.counters + 2);
+    v.hand         = hand_view(handed.as<uint8_t>(), std::min(cap, kHandMaxQ), v.counters + 2);
     return v;
   }
 
@@ -197,7 +199,7 @@ struct Workspace
     const uint64_t np = packets(cap);
     return 3 * part(4 * cap) + part(radix_sort_scratch_bytes(cap)) + part(sizeof(double) * 6 * (kBboxParts + 1)) +
            part(4 * cap) + part(32) + part(4 * cap) + part(8 * mask_packets(cap)) + part(np) + part(4 * (size_t)heavy_cap(cap)) +
-           part(512 * (size_t)heavy_cap(cap)) + part(4 * (size_t)early_cap(cap)) + hand_bytes(cap);
+           part(512 * (size_t)heavy_cap(cap)) + part(4 * (size_t)early_cap(cap)) + hand_bytes(std::min(cap, kHandMaxQ));
   }
   static WsView carve(uint8_t* base, uint64_t cap)
   {
@@ -222,7 +224,7 @@ struct Workspace
     v.heavy_list   = reinterpret_cast<uint32_t*>(take(4 * (size_t)heavy_cap(cap)));
     v.heavy_keys   = reinterpret_cast<unsigned long long*>(take(512 * (size_t)heavy_cap(cap)));
     v.early_list   = reinterpret_cast<uint32_t*>(take(4 * (size_t)early_cap(cap)));
-    v.hand         = hand_view(take(hand_bytes(cap)), cap, v.counters + 2);
+    v.hand         = hand_view(take(hand_bytes(std::min(cap, kHandMaxQ))), std::min(cap, kHandMaxQ), v.counters + 2);
     return v;
   }
 };

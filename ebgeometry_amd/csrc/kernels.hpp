@@ -170,6 +170,7 @@ struct BatchArgs
   // then the packet table -- from *queue (zero at launch) until all queue_total are taken.
   uint32_t*           queue;
   uint32_t            queue_total, persist_blocks;
+  HandOn              hand;        // slots hold packets of the table
 };
 
 hipError_t launch_batch_mark(const BatchArgs& a, hipStream_t s);
@@ -177,10 +178,11 @@ hipError_t launch_batch_mark(const BatchArgs& a, hipStream_t s);
 // keys: uint32 when narrow (at most 256 items: 8 item bits + 24 curve bits), else uint64
 hipError_t launch_batch_keys(const BatchItemDev* items, uint32_t num_items, uint64_t total, void* keys, bool narrow,
                              hipStream_t s);
-// wg = 64, 128 or 256 lanes per workgroup (1, 2 or 4 packets).
+// wg = 64, 128 or 256 lanes per workgroup (1, 2 or 4 packets); the handed-on items and their packets'
+// end follow in launches of their own.
 hipError_t launch_batch32(const BatchArgs& a, int banks, int wg, bool count, hipStream_t s);
 // Workgroups of wg lanes of the persistent batch32 that fit the device at once (occupancy x CUs).
-hipError_t batch32_persistent_blocks(int banks, int wg, bool count, uint32_t* blocks);
+hipError_t batch32_persistent_blocks(int banks, int wg, bool count, bool hand, uint32_t* blocks);
 // FP64 pass over the compacted recheck list (a.recheck_list == null skips); a fixed grid
 // strides over groups of 64 entries.
 hipError_t launch_batch64(const BatchArgs& a, int banks, hipStream_t s);
