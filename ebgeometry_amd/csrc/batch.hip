@@ -260,16 +260,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 8
   }
 }
 
-// One wavefront per 64 consecutive entries of the recheck list (packet << 6 | lane, in packet
+// One wavefront per `width` consecutive entries of the recheck list (packet << 6 | lane, in packet
 // order: neighbouring queries, mostly of one item). The wavefront takes the distinct items of its
 // entries in turn; each listed query is decided in FP64 from its FP32 distance (band_walk).
-constexpr uint32_t kBatch64Lanes = 64; // list entries per wavefront (32 measured the same on 256 meshes, 60M queries)
 template <int NB>
-__device__ __forceinline__ void batch64_group(const BatchArgs& a, uint32_t count, uint32_t g, BandLds& L)
+__device__ __forceinline__ void batch64_group(const BatchArgs& a, uint32_t count, uint32_t g, uint32_t width, BandLds& L)
 {
   const uint32_t lane   = __lane_id();
-  const uint32_t e      = g * kBatch64Lanes + lane;
-  const bool     listed = lane < kBatch64Lanes && e < count;
+  const uint32_t e      = g * width + lane;
+  const bool     listed = lane < width && e < count;
   uint32_t       item = kInvalid, j = 0;
   if (listed) {
     const uint32_t en  = a.recheck_list[e];
@@ -310,10 +309,12 @@ __global__ __launch_bounds__(256) void batch64_kernel(const BatchArgs a)
 {
   __shared__ BandLds lds[4];
   const uint32_t count  = *a.recheck_count;
-  const uint32_t groups = (count + kBatch64Lanes - 1u) / kBatch64Lanes;
   const uint32_t waves  = gridDim.x * 4u;
+  uint32_t       width  = 64u; // entries per wavefront: fewer when the list is short
+  while (width > 1u && count <= width / 2u * min(waves, (uint32_t)kNarrowPackets)) width /= 2u;
+  const uint32_t groups = (count + width - 1u) / width;
   for (uint32_t g = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); g < groups; g += waves) 
-    batch64_group<NB>(a, count, g, lds[uni(threadIdx.x >> 6)]);
+    batch64_group<NB>(a, count, g, width, lds[uni(threadIdx.x >> 6)]);
 }
 
 // One wavefront per packet: the largest cost-grid value over its queries' cells in its mesh's
@@ -402,7 +403,7 @@ template <int NB>
 hipError_t launch64(const BatchArgs& a, hipStream_t s)
 {
   if (a.num_packets == 0 || !a.recheck_list) return hipSuccess;
-  hipLaunchKernelGGL((batch64_kernel<NB>), dim3(std::min<uint32_t>((a.num_packets + 3) / 4, 2048u)), dim3(256), 0, s,
+  hipLaunchKernelGGL((batch64_kernel<NB>), dim3(std::min<uint32_t>(16u * a.num_packets, 2048u)), dim3(256), 0, s,
                      a);
   return hipGetLastError();
 }
