@@ -263,6 +263,8 @@ struct ebg_mesh
   ebgpu::DevBuf          cost_grid;
   ebgpu::DevBuf          split_roots; // SplitRoot frontier covering the tree
   ebgpu::DevBuf          status;      // one device word, MeshDev::status
+  std::mutex             host_mu;       // guards host_io
+  ebgpu::DevBuf          host_io;       // host-array queries: points, distances, faces
   ebgpu::DevBuf          pts32, dist32; // FP64-point queries: the points rounded to FP32, FP32 results
   uint64_t               hash = 0;      // FNV-1a of the vertex and triangle arrays given at creation
   uint32_t               num_split_roots = 0;

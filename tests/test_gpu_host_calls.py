@@ -1,0 +1,35 @@
+"""Host-array calls share one buffer of the handle: sizes up and down, and several threads at once,
+give the values of the device-array call."""
+import threading
+
+import numpy as np
+import pytest
+
+from ebgeometry_amd import TriMeshSDF
+from ebgeometry_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+
+def test_sizes_and_threads(cuda):
+    import torch
+    v, f = wl.displaced_icosphere(3, 33)
+    m = TriMeshSDF(v, f)
+    sets = [wl.mixed_queries(n, v, f, 34 + n) for n in (1, 5000, 64, 70_001, 3)]
+    ref = [m.query(torch.from_numpy(q).to(cuda)).cpu().numpy() for q in sets]
+    for q, r in zip(sets, ref):
+        assert np.array_equal(m.signed_distance(q), r)
+    bad = []
+
+    def work(k):
+        for rep in range(5):
+            j = (k + rep) % len(sets)
+            if not np.array_equal(m.signed_distance(sets[j]), ref[j]):
+                bad.append((k, j))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
