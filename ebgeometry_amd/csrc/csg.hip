@@ -32,13 +32,12 @@ namespace {
 
 using namespace dev;
 
-// Per-workgroup LDS of W lanes: FP32 40 KB at W = 256, FP64 40 KB at W = 128.
-template <class R, uint32_t W>
-struct CsgLds
-{
-  R v[kCsgMaxValues][W];    // value stack
-  R p[kCsgMaxPoints][3][W]; // saved points
-};
+// Per-workgroup LDS of W lanes: the program's value stack (CsgDev::vrows rows of W) and its saved
+// points (3 rows each). Sized by what the program reaches, so that small programs fill the SIMDs:
+// with room for the deepest program in every workgroup (40 KB, 4 wavefronts per SIMD) and the walks'
+// registers in every kernel, 2M points of 12 blended parts and 3 holes took 162 us in FP32 and 24 in
+// FP64, now 98 and 17: 8 wavefronts per SIMD, bound by the issue of the leaves' arithmetic.
+extern __shared__ __attribute__((aligned(16))) unsigned char csg_lds[];
 
 // One lane's interpreter state; its stack entries are vcol[i * W], pcol[(3 d + c) * W].
 template <class R>
@@ -50,6 +49,13 @@ struct CsgLane
   R*       pcol;
   uint32_t w;          // lanes per workgroup (the column stride)
 };
+
+template <class R>
+__device__ __forceinline__ CsgLane<R> csg_lane(const CsgDev& g, uint32_t w)
+{
+  R* v = reinterpret_cast<R*>(csg_lds) + threadIdx.x;
+  return CsgLane<R>{R(0), R(0), R(0), 0, 0, v, v + g.vrows * w, w};
+}
 
 template <class R>
 struct CsgParams
@@ -194,7 +200,7 @@ __device__ __forceinline__ R& pat(CsgLane<R>& L, int d, int c)
 
 // One instruction other than a BVH union. `need`: this lane wants the value (mesh walks leave
 // the other lanes out).
-template <class R, int KM, int NB>
+template <class R, int KM, int NB, bool WALKS>
 __device__ __forceinline__ void csg_step(const CsgDev& g, const CsgParams<R>& q, CsgLane<R>& L, bool need)
 {
   const uint32_t op = q.op;
@@ -202,7 +208,7 @@ __device__ __forceinline__ void csg_step(const CsgDev& g, const CsgParams<R>& q,
     vat(L, L.vtop++) = leaf_value<R>(q, L.x, L.y, L.z);
     return;
   }
-  if (op == kCsgMesh) {
+  if (WALKS && op == kCsgMesh) {
     const MeshDev md   = sload_record(g.meshes + q.n);
     R             best = R(INFINITY);
     uint32_t      btri = kInvalid, bfeat = 0, c0 = 0, c1 = 0, c2 = 0, c3 = 0;
@@ -343,7 +349,7 @@ __device__ __forceinline__ void csg_bvh(const CsgDev& g, const CsgParams<R>& q, 
       if (ballot(pn) == 0) continue;
       const int base = L.vtop;
       for (uint32_t k = uni(pr.start); k < uni(pr.start) + uni(pr.count); k++)
-        csg_step<R, KM, NB>(g, fetch<R>(g, k), L, pn);
+        csg_step<R, KM, NB, true>(g, fetch<R>(g, k), L, pn);
       const R v = vat(L, base);
       L.vtop    = base;
       if (pn) {
@@ -362,105 +368,111 @@ __device__ __forceinline__ void csg_bvh(const CsgDev& g, const CsgParams<R>& q, 
   vat(L, L.vtop++) = smooth ? smooth_min<R>(a, b, q.p[0], q.n) : a;
 }
 
-template <class R, int KM, int NB>
+template <class R, int KM, int NB, bool WALKS>
 __device__ __forceinline__ R csg_run(const CsgDev& g, CsgLane<R>& L, bool active)
 {
   for (uint32_t i = 0; i < g.main_count; i++) {
     const CsgParams<R> q = fetch<R>(g, i);
-    if (q.op == kCsgBvhUnion || q.op == kCsgBvhSmoothUnion) csg_bvh<R, KM, NB>(g, q, L, active);
-    else csg_step<R, KM, NB>(g, q, L, active);
+    if (WALKS && (q.op == kCsgBvhUnion || q.op == kCsgBvhSmoothUnion)) csg_bvh<R, KM, NB>(g, q, L, active);
+    else csg_step<R, KM, NB, WALKS>(g, q, L, active);
   }
   return vat(L, 0);
 }
 
-template <int KM, int NB>
+// WALKS = false: programs without BVH unions and meshes.
+template <int NB, bool WALKS>
 __global__ __launch_bounds__(256) void csg32_kernel(const CsgDev g, const QueryArgs a)
 {
-  __shared__ CsgLds<float, 256> lds;
   const uint32_t blk = xcd_remap(blockIdx.x, gridDim.x);
   const uint64_t n   = a.n;
   if ((uint64_t)blk * 256u >= n) return; // whole workgroup
   const uint64_t tid    = (uint64_t)blk * 256u + threadIdx.x;
   const bool     active = tid < n;
   uint32_t       qi     = 0;
-  CsgLane<float> L{0.0f, 0.0f, 0.0f, 0, 0, &lds.v[0][threadIdx.x], &lds.p[0][0][threadIdx.x], 256u};
+  CsgLane<float> L      = csg_lane<float>(g, 256u);
   if (active) {
     qi  = a.idx ? a.idx[tid] : (uint32_t)tid;
     L.x = a.pts[3 * (size_t)qi];
     L.y = a.pts[3 * (size_t)qi + 1];
     L.z = a.pts[3 * (size_t)qi + 2];
   }
-  const float v = csg_run<float, KM, NB>(g, L, active);
+  const float v = csg_run<float, 4, NB, WALKS>(g, L, active);
   if (active) a.out_d[qi] = v;
   if (a.recheck_list) wave_append(active && fabsf(v) < a.recheck_abs, qi, a.recheck_list, a.recheck_count);
 }
 
 // FP64 pass over the device-side recheck list (length *a.count_ptr): a fixed grid strides over it.
-template <int KM, int NB>
+template <int KM, int NB, bool WALKS>
 __global__ __launch_bounds__(128) void csg64_kernel(const CsgDev g, const QueryArgs a)
 {
-  __shared__ CsgLds<double, 128> lds;
   const uint64_t n     = *a.count_ptr;
   const uint64_t waves = (uint64_t)gridDim.x * 2u;
   for (uint64_t w = uni(blockIdx.x * 2u + (threadIdx.x >> 6)); w * 64u < n; w += waves) {
     const uint64_t  tid    = w * 64u + __lane_id();
     const bool      active = tid < n;
     uint32_t        qi     = 0;
-    CsgLane<double> L{0.0, 0.0, 0.0, 0, 0, &lds.v[0][threadIdx.x], &lds.p[0][0][threadIdx.x], 128u};
+    CsgLane<double> L      = csg_lane<double>(g, 128u);
     if (active) {
       qi  = a.idx[tid];
       L.x = a.pts[3 * (size_t)qi];
       L.y = a.pts[3 * (size_t)qi + 1];
       L.z = a.pts[3 * (size_t)qi + 2];
     }
-    const double v = csg_run<double, KM, NB>(g, L, active);
+    const double v = csg_run<double, KM, NB, WALKS>(g, L, active);
     if (active) a.out_d[qi] = (float)v;
   }
 }
 
-template <int KM, int NB>
+std::size_t csg_lds_bytes(const CsgDev& g, std::size_t elem, std::size_t w) { return (g.vrows + 3u * g.prows) * w * elem; }
+
+template <int NB, bool WALKS>
 hipError_t launch32(const CsgDev& g, const QueryArgs& a, hipStream_t s)
 {
   const uint32_t blocks = (uint32_t)((a.n + 255) / 256);
   if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL((csg32_kernel<KM, NB>), dim3(blocks), dim3(256), 0, s, g, a);
+  hipLaunchKernelGGL((csg32_kernel<NB, WALKS>), dim3(blocks), dim3(256), csg_lds_bytes(g, sizeof(float), 256), s, g, a);
   return hipGetLastError();
 }
 
-template <int KM, int NB>
+template <int KM, int NB, bool WALKS>
 hipError_t launch64(const CsgDev& g, const QueryArgs& a, hipStream_t s)
 {
   if (!a.count_ptr || !a.idx) return hipErrorInvalidValue;
   const uint32_t blocks = std::min<uint32_t>((uint32_t)((a.n + 127) / 128), 2048u);
   if (blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL((csg64_kernel<KM, NB>), dim3(blocks), dim3(128), 0, s, g, a);
+  hipLaunchKernelGGL((csg64_kernel<KM, NB, WALKS>), dim3(blocks), dim3(128), csg_lds_bytes(g, sizeof(double), 128), s, g,
+                     a);
   return hipGetLastError();
+}
+
+bool csg_depths_ok(const CsgDev& g)
+{
+  return g.vrows >= 1 && g.vrows <= (uint32_t)kCsgMaxValues && g.prows <= (uint32_t)kCsgMaxPoints;
 }
 
 } // namespace
 
-hipError_t launch_csg32(const CsgDev& g, int KM, int banks, const QueryArgs& a, hipStream_t s)
+hipError_t launch_csg32(const CsgDev& g, int banks, const QueryArgs& a, hipStream_t s)
 {
-  if (KM == 4) {
-    if (banks <= 1) return launch32<4, 1>(g, a, s);
-    if (banks == 2) return launch32<4, 2>(g, a, s);
-    return launch32<4, 4>(g, a, s);
-  }
-  if (banks <= 1) return launch32<8, 1>(g, a, s);
-  if (banks == 2) return launch32<8, 2>(g, a, s);
-  return launch32<8, 4>(g, a, s);
+  if (!csg_depths_ok(g)) return hipErrorInvalidValue;
+  if (!g.walks) return launch32<1, false>(g, a, s);
+  if (banks <= 1) return launch32<1, true>(g, a, s);
+  if (banks == 2) return launch32<2, true>(g, a, s);
+  return launch32<4, true>(g, a, s);
 }
 
 hipError_t launch_csg64(const CsgDev& g, int KM, int banks, const QueryArgs& a, hipStream_t s)
 {
+  if (!csg_depths_ok(g)) return hipErrorInvalidValue;
+  if (!g.walks) return launch64<4, 1, false>(g, a, s);
   if (KM == 4) {
-    if (banks <= 1) return launch64<4, 1>(g, a, s);
-    if (banks == 2) return launch64<4, 2>(g, a, s);
-    return launch64<4, 4>(g, a, s);
+    if (banks <= 1) return launch64<4, 1, true>(g, a, s);
+    if (banks == 2) return launch64<4, 2, true>(g, a, s);
+    return launch64<4, 4, true>(g, a, s);
   }
-  if (banks <= 1) return launch64<8, 1>(g, a, s);
-  if (banks == 2) return launch64<8, 2>(g, a, s);
-  return launch64<8, 4>(g, a, s);
+  if (banks <= 1) return launch64<8, 1, true>(g, a, s);
+  if (banks == 2) return launch64<8, 2, true>(g, a, s);
+  return launch64<8, 4, true>(g, a, s);
 }
 
 } // namespace ebgpu

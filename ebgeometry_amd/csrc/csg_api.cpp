@@ -278,6 +278,9 @@ ebg_status ebg_csg_create(const ebg_csg_op* ops, uint64_t num_ops, uint64_t main
   g->dev.bvhs       = g->bvhs.as<CsgBvhDev>();
   g->dev.meshes     = g->meshdev.as<MeshDev>();
   g->dev.main_count = uint32_t(main_count);
+  g->dev.vrows      = uint32_t(std::max(vmax, 1));
+  g->dev.prows      = uint32_t(pmax);
+  g->dev.walks      = !g->nodes.empty() || !g->meshes.empty();
   g->dev.status     = g->status.as<uint32_t>();
   *out              = g;
   return EBG_OK;
@@ -311,9 +314,8 @@ ebg_status ebg_csg_query(const ebg_csg* cg, const float* d_pts, uint64_t n, floa
   // only tree walks (BVH unions, meshes) gain from neighbouring queries in a wavefront; a program of
   // analytic leaves runs the same instructions for any points, and in query order its reads and
   // writes are coalesced (2M queries, 12 blended parts: 368 -> 216 us)
-  const bool      walks = !g->nodes.empty() || !g->meshes.empty();
-  const uint32_t* idx   = nullptr;
-  if (o.presort && n > 1 && walks) {
+  const uint32_t* idx = nullptr;
+  if (o.presort && n > 1 && g->dev.walks) {
     EBG_HIP(ebgpu::presort(ws.view(), d_pts, n, s));
     idx = ws.perm.as<uint32_t>();
   }
@@ -326,7 +328,7 @@ ebg_status ebg_csg_query(const ebg_csg* cg, const float* d_pts, uint64_t n, floa
   a.recheck_abs   = o.fp64_all ? INFINITY : (recheck ? float(o.recheck_eps * g->scale) : 0.0f);
   a.recheck_list  = recheck ? ws.recheck_list() : nullptr;
   a.recheck_count = cnt;
-  EBG_HIP(ebgpu::launch_csg32(g->dev, g->KM, g->banks, a, s));
+  EBG_HIP(ebgpu::launch_csg32(g->dev, g->banks, a, s));
   if (recheck) {
     ebgpu::QueryArgs r = a;
     r.idx              = ws.recheck_list();

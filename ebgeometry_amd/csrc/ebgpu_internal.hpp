@@ -320,8 +320,9 @@ struct CsgDev
   const CsgInstr64* ops64;
   const CsgBvhDev*  bvhs;
   const MeshDev*    meshes;
-  uint32_t          main_count; // the program is ops[0, main_count)
-  uint32_t          pad;
+  uint32_t          main_count;   // the program is ops[0, main_count)
+  uint32_t          vrows, prows; // stack values (at least 1) and saved points the program reaches
+  uint32_t          walks;        // it holds BVH unions or meshes
   uint32_t*         status;     // kStatusStackOverflow: a BVH walk's stack was too small
 };
 

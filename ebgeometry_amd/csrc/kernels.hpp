@@ -189,7 +189,7 @@ hipError_t launch_batch64(const BatchArgs& a, int banks, hipStream_t s);
 
 // csg.hip: CSG programs. FP32 pass over a.n queries (a.idx: presort order), appending
 // |v| < a.recheck_abs to the recheck list; FP64 pass over that list (a.idx, *a.count_ptr).
-hipError_t launch_csg32(const CsgDev& g, int KM, int banks, const QueryArgs& a, hipStream_t s);
+hipError_t launch_csg32(const CsgDev& g, int banks, const QueryArgs& a, hipStream_t s);
 hipError_t launch_csg64(const CsgDev& g, int KM, int banks, const QueryArgs& a, hipStream_t s);
 
 // cloud.hip: k nearest cloud points (k <= kKnnMax) of n query points (pts, in the order idx) or,
