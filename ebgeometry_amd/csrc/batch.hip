@@ -129,7 +129,7 @@ __device__ __forceinline__ void batch_packet(const BatchArgs& a, uint32_t p, Pai
     mesh_walk<NB, COUNT, HAND>(m, wk, budget, HAND ? a.hand.spread[0] : 0, px, py, pz, bound, best, btri, n_inner, n_tris,
                                w_inner, w_tris, pl, &pc);
     if (!HAND || wk.top == 0) break;
-    if (hand_on(a.hand, wk, p, best, btri)) return; // whole wavefront
+    if (hand_on(a.hand, wk, p, best, btri) != kInvalid) return; // whole wavefront
     budget = ~0u;
   }
   batch_finish(a, it, m, p, active, qi, px, py, pz, best, btri);

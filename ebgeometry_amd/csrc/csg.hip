@@ -212,8 +212,11 @@ __device__ __forceinline__ void csg_step(const CsgDev& g, const CsgParams<R>& q,
     const MeshDev md   = sload_record(g.meshes + q.n);
     R             best = R(INFINITY);
     uint32_t      btri = kInvalid, bfeat = 0, c0 = 0, c1 = 0, c2 = 0, c3 = 0;
-    if constexpr (sizeof(R) == 4)
-      wide_walk<NB, false>(md, L.x, L.y, L.z, need ? R(INFINITY) : R(-1), best, btri, c0, c1, c2, c3);
+    if constexpr (sizeof(R) == 4) {
+      Walk<NB> wk;
+      wk.start(0u, 0u);
+      wide_walk<NB, false, false>(md, wk, 0u, 0, L.x, L.y, L.z, need ? R(INFINITY) : R(-1), best, btri, c0, c1, c2, c3);
+    }
     else
       traverse<KM, NB, R, false, true>(md, L.x, L.y, L.z, need ? R(INFINITY) : R(-1), best, btri, bfeat, c0, c1, c2, c3);
     R val = R(INFINITY);

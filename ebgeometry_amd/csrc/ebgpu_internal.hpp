@@ -171,6 +171,12 @@ struct HandOn
   HandItem*           items[2];
   uint32_t*           counts; // slots, items[0], items[1] (zero at the first launch)
 };
+// A scene's slot: the walk of mesh instance `prim` for a packet; the packet's slots are chained
+// through `next` (kInvalid: the last) from the one with head = 1.
+struct SceneSlot
+{
+  uint32_t packet, prim, next, head;
+};
 
 // ---------------------------------------------------------------------------------------------
 // CSG union scenes: primitives in BVH leaf order

@@ -116,7 +116,7 @@ hipError_t launch_sdf64(const MeshDev& m, int banks, const QueryArgs& a, hipStre
 // CSG union scenes (scene.hip). KM = branching of the instanced meshes (all equal); banks =
 // stack capacity / 64 for both the scene tree and the mesh trees. Work counters: [0] interior
 // nodes, [1] triangles, [4]/[5] their wave-level fetches, [6] primitives, [7] wave-level.
-hipError_t launch_scene32(const SceneDev& sc, int banks, const QueryArgs& a, bool count, hipStream_t s);
+hipError_t launch_scene32(const SceneDev& sc, int banks, const QueryArgs& a, SceneSlot* slots, bool count, hipStream_t s);
 // FP64 pass over a.idx / a.count_ptr, seeded with |v32| (1 + slack_rel) + slack_abs.
 hipError_t launch_scene64(const SceneDev& sc, int KM, int banks, const QueryArgs& a, hipStream_t s);
 
@@ -234,6 +234,8 @@ struct GridSpec
   double   origin[3], spacing[3];
   uint64_t dims[3];
 };
+// 64 points in each cell of dims[0] x dims[1] x dims[2] cells of size spacing (the cost grid's packets).
+hipError_t launch_cell_points(const GridSpec& g, float* out, hipStream_t s);
 hipError_t launch_grid_points(const GridSpec& g, float* out, hipStream_t s);
 hipError_t launch_f32_to_f64(const float* in, double* out, uint64_t n, hipStream_t s);
 hipError_t launch_add_counts(unsigned long long* work, const uint32_t* recheck, const uint32_t* fallback, hipStream_t s);

@@ -52,10 +52,30 @@ struct SceneCounts
   uint32_t n_inner = 0, n_prims = 0, n_tris = 0, w_inner = 0, w_prims = 0, w_tris = 0;
 };
 
+// The point in a mesh instance's own space, FP32 (pr.A = M / s).
+__device__ __forceinline__ void instance_point(const PrimRec& pr, float px, float py, float pz, float& qx, float& qy,
+                                               float& qz)
+{
+  const float ux = px - pr.t[0], uy = py - pr.t[1], uz = pz - pr.t[2];
+  qx = pr.A[0] * ux + pr.A[1] * uy + pr.A[2] * uz;
+  qy = pr.A[3] * ux + pr.A[4] * uy + pr.A[5] * uz;
+  qz = pr.A[6] * ux + pr.A[7] * uy + pr.A[8] * uz;
+}
+
+// Where a packet's long instance walks are handed on to.
+struct SceneHand
+{
+  const HandOn* h;
+  SceneSlot*    slots;
+  uint32_t      packet, head; // head: the packet's last slot (kInvalid: none)
+};
+
 // Union value of the scene at (px,py,pz) for this lane. v holds the starting value (+inf, or an
-// upper bound on the answer when seeded); bound < 0 marks a lane without a query.
-template <int KM, int NB, class R, bool COUNT>
-__device__ __forceinline__ void scene_traverse(const SceneDev& sc, R px, R py, R pz, R& v, R bound, SceneCounts& c)
+// upper bound on the answer when seeded); bound < 0 marks a lane without a query. HAND: instances
+// whose walks were handed on are missing from v, which costs the rest of the walk some culling.
+template <int KM, int NB, class R, bool COUNT, bool HAND>
+__device__ __forceinline__ void scene_traverse(const SceneDev& sc, R px, R py, R pz, R& v, R bound, SceneCounts& c,
+                                               SceneHand* hand)
 {
   [[maybe_unused]] const R    seed = v; // FP64: a bound on |value| (+inf: none)
   const Node<4>* __restrict__ nodes = static_cast<const Node<4>*>(sc.nodes);
@@ -110,12 +130,8 @@ __device__ __forceinline__ void scene_traverse(const SceneDev& sc, R px, R py, R
         const MeshDev  md = sload_record(sc.meshes + uni(pr.mesh));
         R              qx, qy, qz, s;
         if constexpr (sizeof(R) == 4) {
-          // pr.A = M / s
-          const float ux = px - pr.t[0], uy = py - pr.t[1], uz = pz - pr.t[2];
-          qx = pr.A[0] * ux + pr.A[1] * uy + pr.A[2] * uz;
-          qy = pr.A[3] * ux + pr.A[4] * uy + pr.A[5] * uz;
-          qz = pr.A[6] * ux + pr.A[7] * uy + pr.A[8] * uz;
-          s  = pr.s;
+          instance_point(pr, px, py, pz, qx, qy, qz);
+          s = pr.s;
         }
         else {
           const PrimRec64 q  = sload_record(sc.prims64 + i);
@@ -137,8 +153,23 @@ __device__ __forceinline__ void scene_traverse(const SceneDev& sc, R px, R py, R
         near             = pn ? near : R(-1);
         R        best    = INFINITY;
         uint32_t btri    = kInvalid, bfeat = 0;
-        if constexpr (sizeof(R) == 4)
-          wide_walk<NB, COUNT>(md, qx, qy, qz, near, best, btri, c.n_inner, c.n_tris, c.w_inner, c.w_tris);
+        if constexpr (sizeof(R) == 4) {
+          Walk<NB> wk;
+          wk.start(0u, 0u);
+          wide_walk<NB, COUNT, HAND>(md, wk, HAND ? hand->h->budget[0] : 0u, HAND ? hand->h->spread[0] : 0, qx, qy, qz, near,
+                                     best, btri, c.n_inner, c.n_tris, c.w_inner, c.w_tris);
+          if (HAND && wk.top > 0) {
+            const uint32_t j = hand_on(*hand->h, wk, hand->packet, pn ? best : -1.0f, btri);
+            if (j != kInvalid) {
+              if (lane == 0) hand->slots[j] = SceneSlot{hand->packet, i, hand->head, 0u};
+              hand->head = j;
+              continue;
+            }
+            // no room: walk on (a lane's bound is its best so far)
+            wide_walk<NB, COUNT, false>(md, wk, 0u, 0, qx, qy, qz, pn ? best : -1.0f, best, btri, c.n_inner, c.n_tris,
+                                        c.w_inner, c.w_tris);
+          }
+        }
         else
           traverse<KM, NB, R, COUNT, true>(md, qx, qy, qz, near, best, btri, bfeat, c.n_inner, c.n_tris, c.w_inner,
                                            c.w_tris);
@@ -161,9 +192,9 @@ __device__ __forceinline__ void scene_traverse(const SceneDev& sc, R px, R py, R
 
 // FP32 pass, one 64-query packet per wavefront, 4 per workgroup, XCD-aware block order. Bound by the
 // latency of its scalar loads: registers are held to what 7 wavefronts per SIMD have.
-template <int NB, bool COUNT>
+template <int NB, bool COUNT, bool HAND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 7 : 4))) void scene32_kernel(
-  const SceneDev sc, const QueryArgs a)
+  const SceneDev sc, const QueryArgs a, SceneSlot* const slots)
 {
   const uint32_t blk = xcd_remap(blockIdx.x, gridDim.x);
   const uint64_t n   = a.n;
@@ -184,14 +215,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 7
   const float seed = (active && a.seed_r) ? a.seed_r[qi] : INFINITY;
   float       v    = seed;
   SceneCounts c;
-  scene_traverse<4, NB, float, COUNT>(sc, px, py, pz, v, active ? seed * seed : -1.0f, c);
-  if (a.seed_r) {
+  SceneHand   hand{&a.hand, slots, uni(blk * 4u + (threadIdx.x >> 6)), kInvalid};
+  scene_traverse<4, NB, float, COUNT, HAND>(sc, px, py, pz, v, active ? seed * seed : -1.0f, c, &hand);
+  if (!HAND && a.seed_r) {
     const bool     redo  = active && !(v < seed);
     const uint64_t rmask = ballot(redo);
     if (rmask) {
       float       v2 = INFINITY;
       SceneCounts c2;
-      scene_traverse<4, NB, float, COUNT>(sc, px, py, pz, v2, redo ? INFINITY : -1.0f, c2);
+      scene_traverse<4, NB, float, COUNT, false>(sc, px, py, pz, v2, redo ? INFINITY : -1.0f, c2, nullptr);
       if (redo) v = v2;
       if (__lane_id() == 0 && a.fallback_count) atomicAdd(a.fallback_count, (uint32_t)__popcll(rmask));
       if (COUNT) {
@@ -201,6 +233,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 7
     }
   }
   if (active) a.out_d[qi] = v;
+  if (HAND && hand.head != kInvalid) { // the value is settled, and checked, when the slots are done
+    if (__lane_id() == 0) slots[hand.head].head = 1u;
+    return;
+  }
   if (a.recheck_list) wave_append(active && fabsf(v) < a.recheck_abs, qi, a.recheck_list, a.recheck_count);
   if (COUNT && a.work) {
     const uint64_t si = wave_sum_u64(active ? (uint64_t)c.n_inner : 0ull);
@@ -214,6 +250,78 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 7
       atomicAdd(a.work + 6, (unsigned long long)sp);
       atomicAdd(a.work + 7, (unsigned long long)c.w_prims);
     }
+  }
+}
+
+// The handed-on instance walks, as the mesh kernel's items: stage 0 hands on again, stage 1 walks to
+// the end.
+template <int NB, int STAGE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 7 : 4))) void scene_items_kernel(
+  const SceneDev sc, const QueryArgs a, const SceneSlot* const slots)
+{
+  const uint32_t n = min(a.hand.counts[1 + STAGE], a.hand.item_cap);
+  for (uint32_t w = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); w < n; w += gridDim.x * 4u) {
+    const SWords<4> hi = sload<4>(a.hand.items[STAGE] + w);
+    if (hi.w[0] == kInvalid) continue;
+    const uint32_t      slot = hi.w[0];
+    const SWords<4>     sl   = sload<4>(slots + slot);
+    const PrimRec       pr   = sload_record(sc.prims + sl.w[1]);
+    const MeshDev       md   = sload_record(sc.meshes + uni(pr.mesh));
+    unsigned long long* keys = a.hand.keys + 64 * (size_t)slot + __lane_id();
+    const uint64_t      key  = *keys;
+    const uint64_t      tid  = 64u * (uint64_t)sl.w[0] + __lane_id();
+    float               qx = 0.0f, qy = 0.0f, qz = 0.0f;
+    if (tid < a.n) {
+      const size_t qi = a.idx ? a.idx[tid] : (uint32_t)tid;
+      instance_point(pr, a.pts[3 * qi], a.pts[3 * qi + 1], a.pts[3 * qi + 2], qx, qy, qz);
+    }
+    float    best = __uint_as_float((uint32_t)(key >> 32)); // -1: a lane without a query
+    uint32_t btri = (uint32_t)key, n_inner = 0, n_tris = 0, w_inner = 0, w_tris = 0;
+    Walk<NB> wk;
+    wk.start(hi.w[1], hi.w[2]);
+    wide_walk<NB, false, STAGE == 0>(md, wk, a.hand.budget[1], a.hand.spread[1], qx, qy, qz, best, best, btri, n_inner,
+                                     n_tris, w_inner, w_tris);
+    if (STAGE == 0 && wk.top > 0 && !append_items(wk, slot, a.hand.items[1], a.hand.counts + 2, a.hand.item_cap))
+      wide_walk<NB, false, false>(md, wk, 0u, 0, qx, qy, qz, best, best, btri, n_inner, n_tris, w_inner, w_tris);
+    const uint64_t now = ((uint64_t)__float_as_uint(best) << 32) | btri;
+    if (now < key) atomicMin(keys, (unsigned long long)now);
+  }
+}
+
+// The handed-on packets' end: each lane's value is the least of the packet's own and its slots'.
+__global__ __launch_bounds__(256) void scene_resolve_kernel(const SceneDev sc, const QueryArgs a,
+                                                            const SceneSlot* const slots)
+{
+  const uint32_t n = min(a.hand.counts[0], a.hand.slot_cap);
+  for (uint32_t s = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); s < n; s += gridDim.x * 4u) {
+    const uint32_t p = uni(a.hand.list[s]);
+    if (p == kInvalid || uni(slots[s].head) == 0u) continue;
+    const uint64_t tid    = 64u * (uint64_t)p + __lane_id();
+    const bool     active = tid < a.n;
+    uint32_t       qi     = 0;
+    float          px = 0.0f, py = 0.0f, pz = 0.0f, v = INFINITY;
+    if (active) {
+      qi = a.idx ? a.idx[tid] : (uint32_t)tid;
+      px = a.pts[3 * (size_t)qi];
+      py = a.pts[3 * (size_t)qi + 1];
+      pz = a.pts[3 * (size_t)qi + 2];
+      v  = a.out_d[qi];
+    }
+    for (uint32_t k = s; k != kInvalid;) {
+      const SWords<4> sl   = sload<4>(slots + k);
+      const PrimRec   pr   = sload_record(sc.prims + sl.w[1]);
+      const MeshDev   md   = sload_record(sc.meshes + uni(pr.mesh));
+      const uint64_t  key  = a.hand.keys[64 * (size_t)k + __lane_id()];
+      const float     best = __uint_as_float((uint32_t)(key >> 32));
+      const uint32_t  btri = (uint32_t)key;
+      float           qx, qy, qz;
+      instance_point(pr, px, py, pz, qx, qy, qz);
+      if (active && best >= 0.0f && btri != kInvalid)
+        v = min(v, pr.s * resolve32(md, btri, closest_feature(md, btri, qx, qy, qz), best, qx, qy, qz));
+      k = sl.w[2];
+    }
+    if (active) a.out_d[qi] = v;
+    if (a.recheck_list) wave_append(active && fabsf(v) < a.recheck_abs, qi, a.recheck_list, a.recheck_count);
   }
 }
 
@@ -236,15 +344,15 @@ __device__ __forceinline__ void scene64_block(const SceneDev& sc, const QueryArg
   }
   double      v = seed;
   SceneCounts c;
-  scene_traverse<KM, NB, double, false>(sc, px, py, pz, v, active ? seed * seed : -1.0, c);
+  scene_traverse<KM, NB, double, false, false>(sc, px, py, pz, v, active ? seed * seed : -1.0, c, nullptr);
   if (active && v < seed) a.out_d[qi] = (float)v;
 }
 
-// The list's length is only known on the device: a fixed grid of wavefronts strides over it,
-// kScene64Lanes entries per wavefront (the other lanes sit out). The list holds near-surface
-// queries from all over the scene, so a wavefront walks about one path per entry; with 32
-// entries the slowest wavefront, which ends the launch, ends earlier (32M queries, 4,096 spheres + 1,024 boxes + 8 meshes: 0.98 -> 0.79 ms; 16
-// entries 0.81 ms).
+// The list's length is only known on the device: a fixed grid of wavefronts strides over it. The list
+// holds near-surface queries from all over the scene, so a wavefront walks about one path per entry,
+// and the slowest wavefront ends the launch: at most kScene64Lanes entries each (32M queries, 4,096
+// spheres + 1,024 boxes + 8 meshes: 64 entries 0.98 ms, 32 0.79, 16 0.81), fewer while the list does
+// not fill the grid twice (4M queries: 345 -> 280 us).
 constexpr uint32_t kScene64Lanes = 32;
 template <int KM, int NB>
 __global__ __launch_bounds__(256) void scene64_kernel(const SceneDev sc, const QueryArgs a)
@@ -252,26 +360,37 @@ __global__ __launch_bounds__(256) void scene64_kernel(const SceneDev sc, const Q
   const uint64_t n     = a.count_ptr ? (uint64_t)*a.count_ptr : a.n;
   const uint32_t lane  = __lane_id();
   const uint64_t waves = (uint64_t)gridDim.x * 4u;
-  for (uint64_t w = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); w * kScene64Lanes < n; w += waves) {
-    const uint64_t tid = lane < kScene64Lanes ? w * kScene64Lanes + lane : n; // n: inactive
+  uint32_t       width = 1;
+  while (width < kScene64Lanes && 2u * width * waves < n) width *= 2u;
+  for (uint64_t w = uni(blockIdx.x * 4u + (threadIdx.x >> 6)); w * width < n; w += waves) {
+    const uint64_t tid = lane < width ? w * width + lane : n; // n: inactive
     scene64_block<KM, NB>(sc, a, n, tid);
   }
 }
 
 template <int NB>
-hipError_t launch32(const SceneDev& sc, const QueryArgs& a, bool count, hipStream_t s)
+hipError_t launch32(const SceneDev& sc, const QueryArgs& a, SceneSlot* slots, bool count, hipStream_t s)
 {
   const uint32_t blocks = (uint32_t)((a.n + 255) / 256);
   if (blocks == 0) return hipSuccess;
-  if (count) hipLaunchKernelGGL((scene32_kernel<NB, true>), dim3(blocks), dim3(256), 0, s, sc, a);
-  else hipLaunchKernelGGL((scene32_kernel<NB, false>), dim3(blocks), dim3(256), 0, s, sc, a);
+  if (count) hipLaunchKernelGGL((scene32_kernel<NB, true, false>), dim3(blocks), dim3(256), 0, s, sc, a, slots);
+  else if (!slots) hipLaunchKernelGGL((scene32_kernel<NB, false, false>), dim3(blocks), dim3(256), 0, s, sc, a, slots);
+  else {
+    const HandOn& h = a.hand;
+    if (a.seed_r || !h.slot_cap || !h.list || !h.keys || !h.items[0] || !h.items[1] || !h.counts) return hipErrorInvalidValue;
+    const uint32_t g = std::clamp<uint32_t>(4u * blocks, 512u, 2048u);
+    hipLaunchKernelGGL((scene32_kernel<NB, false, true>), dim3(blocks), dim3(256), 0, s, sc, a, slots);
+    hipLaunchKernelGGL((scene_items_kernel<NB, 0>), dim3(g), dim3(256), 0, s, sc, a, slots);
+    hipLaunchKernelGGL((scene_items_kernel<NB, 1>), dim3(g), dim3(256), 0, s, sc, a, slots);
+    hipLaunchKernelGGL(scene_resolve_kernel, dim3(std::min(g, (h.slot_cap + 3u) / 4u)), dim3(256), 0, s, sc, a, slots);
+  }
   return hipGetLastError();
 }
 
 template <int KM, int NB>
 hipError_t launch64(const SceneDev& sc, const QueryArgs& a, hipStream_t s)
 {
-  const uint32_t blocks = std::min<uint32_t>((uint32_t)((a.n + 255) / 256), 2048u);
+  const uint32_t blocks = (uint32_t)std::min<uint64_t>((a.n + 3) / 4, 2048u);
   if (blocks == 0) return hipSuccess;
   hipLaunchKernelGGL((scene64_kernel<KM, NB>), dim3(blocks), dim3(256), 0, s, sc, a);
   return hipGetLastError();
@@ -279,11 +398,11 @@ hipError_t launch64(const SceneDev& sc, const QueryArgs& a, hipStream_t s)
 
 } // namespace
 
-hipError_t launch_scene32(const SceneDev& sc, int banks, const QueryArgs& a, bool count, hipStream_t s)
+hipError_t launch_scene32(const SceneDev& sc, int banks, const QueryArgs& a, SceneSlot* slots, bool count, hipStream_t s)
 {
-  if (banks <= 1) return launch32<1>(sc, a, count, s);
-  if (banks == 2) return launch32<2>(sc, a, count, s);
-  return launch32<4>(sc, a, count, s);
+  if (banks <= 1) return launch32<1>(sc, a, slots, count, s);
+  if (banks == 2) return launch32<2>(sc, a, slots, count, s);
+  return launch32<4>(sc, a, slots, count, s);
 }
 
 hipError_t launch_scene64(const SceneDev& sc, int KM, int banks, const QueryArgs& a, hipStream_t s)

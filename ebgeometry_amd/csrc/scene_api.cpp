@@ -29,6 +29,7 @@ struct ebg_scene
   double                 lo[3]{}, hi[3]{}, diag = 0;
   std::mutex             mu;
   Workspace              ws;
+  DevBuf                 handed;  // HandOn's lists, then the slots
   std::mutex             grid_mu; // held around the lattice buffer (ebg_scene_query_grid)
   DevBuf                 gridpts;
   hipEvent_t             ev0 = nullptr, ev1 = nullptr;
@@ -264,6 +265,13 @@ ebg_status ebg_scene_bounds(const ebg_scene* sc, double* lo3, double* hi3, doubl
   return EBG_OK;
 }
 
+// Visits before an instance's walk is handed on (HandOn::budget), far fewer than in the mesh kernels: a
+// visited leaf costs the wavefront every triangle that some lane may need. 4M points: (150, 60) 1.87 ms,
+// (80, 30) 1.64, (30, 30) 1.49, (15, 15) 1.35, (10, 20) 1.39; 10,000 points: 1.47, 1.04, 0.73, 0.58, 0.53.
+constexpr uint32_t kSceneBudget[2] = {15, 15};
+// Handed-on walks have room as for this many queries at most (27 MB); beyond it wavefronts walk on.
+constexpr uint64_t kHandMaxRoom = 1u << 24;
+
 ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n, float* d_value,
                            const ebg_query_opts* opts)
 {
@@ -286,7 +294,7 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
     EBG_HIP(hipEventCreate(&sc->ev1));
   }
   uint32_t* cnt = ws.counters();
-  EBG_HIP(ebgpu::launch_fill_u32(cnt, 2, 0u, s));
+  EBG_HIP(ebgpu::launch_fill_u32(cnt, 8, 0u, s));
   const uint32_t* idx = nullptr;
   if (o.presort && n > 1) {
     EBG_HIP(ebgpu::presort(ws.view(), d_pts, n, s));
@@ -312,9 +320,24 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
   a.recheck_count = cnt;
   a.work          = reinterpret_cast<unsigned long long*>(o.work);
   const bool count = o.work != nullptr;
+  // Long walks of mesh instances are handed on whatever the number of queries: a few packets inside a
+  // mesh last as long as millions elsewhere (10,000 points 2.67 ms, 4M points 3.3 ms before, now 0.58
+  // and 1.35).
+  ebgpu::SceneSlot* slots = nullptr;
+  if (!sc->meshes.empty() && !count && !seeds) {
+    const uint64_t    room  = std::min(n, kHandMaxRoom);
+    const std::size_t lists = Workspace::hand_bytes(room);
+    EBG_HIP(sc->handed.reserve(lists + sizeof(ebgpu::SceneSlot) * Workspace::hand_slots(room)));
+    a.hand = Workspace::hand_view(sc->handed.as<uint8_t>(), room, cnt + 2);
+    slots  = reinterpret_cast<ebgpu::SceneSlot*>(sc->handed.as<uint8_t>() + lists);
+    for (int i = 0; i < 2; i++) {
+      a.hand.budget[i] = kSceneBudget[i];
+      a.hand.spread[i] = ebgpu::kHandSpread[i];
+    }
+  }
 
   EBG_HIP(hipEventRecord(sc->ev0, s));
-  EBG_HIP(ebgpu::launch_scene32(sc->dev, sc->banks, a, count, s));
+  EBG_HIP(ebgpu::launch_scene32(sc->dev, sc->banks, a, slots, count, s));
   EBG_HIP(hipEventRecord(sc->ev1, s));
   sc->timed = true;
   if (recheck) {

@@ -106,7 +106,7 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
         wk.start(0u, 0u);
         if (__lane_id() == 0) atomicAdd(a.fallback_count, (uint32_t)__popcll(mmask));
       }
-      if (hand_on(a.hand, wk, (uint32_t)pk, best, btri)) return; // whole wavefront
+      if (hand_on(a.hand, wk, (uint32_t)pk, best, btri) != kInvalid) return; // whole wavefront
       if (MODE == kSeeded && !redo && active) bound = best;
       budget = ~0u;
       continue;

@@ -976,19 +976,19 @@ __device__ __forceinline__ bool append_items(const Walk<NB>& wk, uint32_t slot, 
   return fits;
 }
 
-// Hand the rest of the walk of `packet` on (see HandOn); false: no room, walk on.
+// Hand the rest of the walk of `packet` on (see HandOn): its slot, or kInvalid: no room, walk on.
 template <int NB>
-__device__ __forceinline__ bool hand_on(const HandOn& h, const Walk<NB>& wk, uint32_t packet, float best, uint32_t btri)
+__device__ __forceinline__ uint32_t hand_on(const HandOn& h, const Walk<NB>& wk, uint32_t packet, float best, uint32_t btri)
 {
   const uint32_t lane = __lane_id();
   uint32_t       j    = 0;
   if (lane == 0) j = atomicAdd(h.counts, 1u);
   j = rdlane(j, 0);
-  if (j >= h.slot_cap) return false;
+  if (j >= h.slot_cap) return kInvalid;
   const bool ok                = append_items(wk, j, h.items[0], h.counts + 1, h.item_cap);
   h.keys[64 * (size_t)j + lane] = ((unsigned long long)__float_as_uint(best) << 32) | btri;
   if (lane == 0) h.list[j] = ok ? packet : kInvalid;
-  return ok;
+  return ok ? j : kInvalid;
 }
 
 // Visit a node: test its children and push the ones some lane reaches, ranked so that the farthest
@@ -1049,6 +1049,24 @@ __device__ __forceinline__ void push_walk_children(const MeshDev& m, Walk<NB>& w
   }
 }
 
+// Spread the stack to about `spread` entries before it is handed on: nodes give way to their children,
+// from the bottom (the largest subtrees).
+template <int NB>
+__device__ __forceinline__ void spread_walk(const MeshDev& m, Walk<NB>& wk, int spread, float px, float py, float pz,
+                                            float b2, int rep)
+{
+  for (int bot = 0; bot < wk.top && wk.top < spread; bot++) {
+    const uint32_t ecnt = wk.st.cnt_at(bot);
+    if ((ecnt & (kBoxChild - 1u)) != 0u) continue; // a leaf stays as it is
+    const uint32_t eref = uni(wk.st.ref_at(bot));
+    float          v[8];
+    wk.top--; // the top entry takes its place
+    wk.st.bound_at(wk.top, v);
+    wk.st.put(bot, wk.st.ref_at(wk.top), wk.st.cnt_at(wk.top), v);
+    push_walk_children(m, wk, eref, px, py, pz, b2, rep);
+  }
+}
+
 // The walk over the mesh's WalkNodes from wk's stack until it is empty or (HAND) `budget` nodes and
 // leaves have been visited. Then the stack is spread for handing on: its lowest entries, the largest
 // subtrees, are replaced by their children until there are `spread` entries (a depth-first stack
@@ -1099,37 +1117,24 @@ __device__ __forceinline__ void mesh_walk(const MeshDev& m, Walk<NB>& wk, uint32
       }
     }
   }
-  if constexpr (HAND) {
-    // out of budget: spread the stack (rare)
-    for (int bot = 0; bot < top && top < spread; bot++) {
-      const uint32_t ecnt = st.cnt_at(bot);
-      if ((ecnt & (kBoxChild - 1u)) != 0u) continue; // a leaf stays as it is
-      const uint32_t eref = uni(st.ref_at(bot));
-      float          v[8];
-      top--; // the top entry takes its place
-      st.bound_at(top, v);
-      st.put(bot, st.ref_at(top), st.cnt_at(top), v);
-      push_walk_children(m, wk, eref, px, py, pz, b2, rep);
-    }
-  }
+  if constexpr (HAND) spread_walk(m, wk, spread, px, py, pz, b2, rep); // out of budget (rare)
 }
 
 // The walk for kernels without the pair-compacted leaves' LDS (mesh instances of scenes, mesh
 // leaves of programs): a triangle is evaluated by the whole wavefront when some lane's cull radius
 // reaches its disc, behind the lower-bound cull of tri_eval32_culled. px, py, pz, bound and best are
 // in the mesh's own units; bound < 0: a lane without a query. Lanes meet triangles that only others
-// asked for too, so with a finite bound `best` is the lane's minimum only if it is within it.
-template <int NB, bool COUNT>
-__device__ __forceinline__ void wide_walk(const MeshDev& m, float px, float py, float pz, float bound, float& best,
-                                          uint32_t& btri, uint32_t& n_inner, uint32_t& n_tris, uint32_t& w_inner,
-                                          uint32_t& w_tris)
+// asked for too, so with a finite bound `best` is the lane's minimum only if it is within it. HAND:
+// ends after `budget` visits, with wk's stack spread, and goes on from there when called again.
+template <int NB, bool COUNT, bool HAND>
+__device__ __forceinline__ void wide_walk(const MeshDev& m, Walk<NB>& wk, uint32_t budget, int spread, float px, float py,
+                                          float pz, float bound, float& best, uint32_t& btri, uint32_t& n_inner,
+                                          uint32_t& n_tris, uint32_t& w_inner, uint32_t& w_tris)
 {
   const int   lane = __lane_id(), rep = rep_lane(bound);
   const float ss = m.scale * m.scale, sx = px * m.scale, sy = py * m.scale, sz = pz * m.scale;
   float       b2   = cull_radius2(m, bound * ss);
-  Walk<NB>    wk;
-  wk.start(0u, 0u);
-  while (wk.top > 0) {
+  while (wk.top > 0 && (!HAND || budget > 0u)) {
     --wk.top;
     const uint32_t ecnt = wk.st.cnt_at(wk.top);
     bool           need = true;
@@ -1142,6 +1147,7 @@ __device__ __forceinline__ void wide_walk(const MeshDev& m, float px, float py, 
       if (COUNT) need = ((mask >> lane) & 1ull) != 0;
     }
     const uint32_t eref = uni(wk.st.ref_at(wk.top)), cnt = ecnt & (kBoxChild - 1u);
+    if constexpr (HAND) budget--;
     if (cnt == 0u) {
       if (COUNT) { n_inner += need ? 1u : 0u; w_inner++; }
       push_walk_children(m, wk, eref, sx, sy, sz, b2, rep);
@@ -1179,6 +1185,7 @@ __device__ __forceinline__ void wide_walk(const MeshDev& m, float px, float py, 
       b2 = cull_radius2(m, bound * ss);
     }
   }
+  if constexpr (HAND) spread_walk(m, wk, spread, sx, sy, sz, b2, rep); // out of budget
 }
 
 // The closest triangle in FP64, given a distance d32 that an FP32 walk found (|d32| for lanes with
