@@ -493,18 +493,15 @@ ebg_status ensure_cost_grid(ebg_mesh* m, hipStream_t s)
     m->grid_lo[c]    = float(lo[c]);
     m->grid_scale[c] = float(1.0 / step[c]);
   }
-  std::vector<float> pts(3 * 64 * ng);
-  for (uint32_t z = 0; z < g; z++)
-    for (uint32_t y = 0; y < g; y++)
-      for (uint32_t x = 0; x < g; x++)
-        for (uint32_t l = 0; l < 64; l++) {
-          float* p = &pts[3 * (64 * ((uint64_t(z) * g + y) * g + x) + l)];
-          p[0]     = float(lo[0] + (x + ((l & 3) + 0.5) / 4) * step[0]);
-          p[1]     = float(lo[1] + (y + (((l >> 2) & 3) + 0.5) / 4) * step[1]);
-          p[2]     = float(lo[2] + (z + ((l >> 4) + 0.5) / 4) * step[2]);
-        }
+  ebgpu::GridSpec cells{};
+  for (int c = 0; c < 3; c++) {
+    cells.dims[c]    = g;
+    cells.origin[c]  = lo[c];
+    cells.spacing[c] = step[c];
+  }
   ebgpu::DevBuf dp, dd;
-  EBG_HIP(upload(dp, pts));
+  EBG_HIP(dp.reserve(12 * 64 * ng));
+  EBG_HIP(ebgpu::launch_cell_points(cells, dp.as<float>(), s));
   EBG_HIP(dd.reserve(4 * 64 * ng));
   EBG_HIP(m->cost_grid.reserve(4 * ng));
   ebgpu::QueryArgs q{};
@@ -992,7 +989,8 @@ ebg_status ebg_mlp_train(ebg_mesh* m, const ebg_mlp_opts* opts, float* loss)
   ebg_query_opts q;
   ebg_query_opts_default(&q);
   q.stream           = o.stream;
-  const ebg_status st = ebg_query_sdf(m, pts.as<float>(), n, dist.as<float>(), nullptr, &q);
+  ebg_status st = ebg_query_sdf(m, pts.as<float>(), n, dist.as<float>(), nullptr, &q);
+  if (st == EBG_OK) st = ensure_cost_grid(m, s); // for the large queries that the network is trained for
   if (st != EBG_OK) return st;
 
   float       last = 0.0f;

@@ -49,6 +49,18 @@ __global__ void f32_to_f64_kernel(const float* __restrict__ in, double* __restri
 // Lattice points of a box of cells or nodes (x fastest, then y, then z: the layout of an AMReX
 // or Chombo FAB): point (i, j, k) = origin + (i, j, k) * spacing, each coordinate a separately
 // rounded FP64 product and sum, then rounded to FP32 (round to nearest even).
+// 64 points (4 x 4 x 4) in each cell of g.dims cells of size g.spacing, cell by cell
+__global__ void cell_points_kernel(GridSpec g, float* __restrict__ out)
+{
+  const uint64_t p = (uint64_t)blockIdx.x * 256 + threadIdx.x, c = p >> 6;
+  const uint32_t l = (uint32_t)p & 63u;
+  if (c >= g.dims[0] * g.dims[1] * g.dims[2]) return;
+  const uint64_t i = c % g.dims[0], r = c / g.dims[0], j = r % g.dims[1], k = r / g.dims[1];
+  out[3 * p]       = (float)(g.origin[0] + ((double)i + ((l & 3u) + 0.5) / 4) * g.spacing[0]);
+  out[3 * p + 1]   = (float)(g.origin[1] + ((double)j + (((l >> 2) & 3u) + 0.5) / 4) * g.spacing[1]);
+  out[3 * p + 2]   = (float)(g.origin[2] + ((double)k + ((l >> 4) + 0.5) / 4) * g.spacing[2]);
+}
+
 __global__ void grid_points_kernel(GridSpec g, float* __restrict__ out)
 {
   const uint64_t n = g.dims[0] * g.dims[1] * g.dims[2];
@@ -370,6 +382,14 @@ hipError_t launch_grid_points(const GridSpec& g, float* out, hipStream_t s)
   const uint64_t n = g.dims[0] * g.dims[1] * g.dims[2];
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(grid_points_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, g, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_cell_points(const GridSpec& g, float* out, hipStream_t s)
+{
+  const uint64_t n = 64 * g.dims[0] * g.dims[1] * g.dims[2];
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(cell_points_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, g, out);
   return hipGetLastError();
 }
 
