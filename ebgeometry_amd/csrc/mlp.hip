@@ -25,6 +25,7 @@ namespace {
 typedef __bf16   bf16x8 __attribute__((ext_vector_type(8)));
 typedef float    f32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
 
 // FP32 -> BF16, round to nearest even (v_cvt_pk_bf16_f32 on gfx950)
 __device__ __forceinline__ uint16_t f2bf(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
@@ -257,8 +258,8 @@ __global__ __launch_bounds__(64 * kInferWaves) void infer_kernel(const float* __
 
 // A training step is 12 small products; as separate launches (25 a step, 16 x 16 tiles, operands
 // through L2) it was bound by the launches: 262,144 samples in batches of 4,096, labelling included,
-// took 13.7 ms, now 3.8 ms (a step: 39 us here, 6 us in the sums and Adam). Here a workgroup takes
-// 64 rows through the whole network and back with every activation and delta in LDS (113 KB): only
+// took 13.7 ms, now 3.1 ms (a step: 30 us here, 6 us in the sums and Adam). Here a workgroup takes
+// 64 rows through the whole network and back with every activation and delta in LDS (160 KB): only
 // the points come in and the workgroup's gradient goes out. The gradient tiles stay in the
 // accumulators over the workgroup's 64-row tiles, and each workgroup writes its own partial
 // gradient, summed in a fixed order by the second launch: no atomics but the loss, so training is
@@ -269,41 +270,56 @@ __global__ __launch_bounds__(64 * kInferWaves) void infer_kernel(const float* __
 constexpr int kTrainRows  = 64;  // rows per tile
 constexpr int kTrainWaves = 8;   // wave w owns output columns 16 w .. 16 w + 15 of every product
 constexpr int kTrainBlk   = 128; // most workgroups of a step (each strides over tiles)
-constexpr int kTrainLd    = kMlpHidden + 8; // LDS row strides (16-byte aligned, rows on shifted banks)
-constexpr int kTrainLd0   = kMlpInPad + 8;
+constexpr int kTrainLd    = kMlpHidden + 8; // LDS strides of row-major tiles (16-byte aligned, rows on
+constexpr int kTrainLd0   = kMlpInPad + 8;  // shifted banks) ...
+constexpr int kTrainLdT   = kTrainRows + 8; // ... and of tiles stored column by column
 
+// Products along the network take a tile's rows as their operand, the weight gradients (in^T d) its
+// columns: activations and deltas are stored both ways where both are read, so that every operand is
+// one 16-byte read (gathering the columns from row-major tiles, 8 reads of 2 bytes each, a step of
+// 4,096 rows took 39 us, now 30).
 struct TrainLds
 {
-  uint16_t x0[kTrainRows * kTrainLd0];
-  uint16_t h[4][kTrainRows * kTrainLd];
-  uint16_t d[2][kTrainRows * kTrainLd];
+  uint16_t x0[kTrainRows * kTrainLd0], x0t[kMlpInPad * kTrainLdT];
+  uint16_t r[3][kTrainRows * kTrainLd];   // rows of h1, h4, d2; of h2, d4; of h3, d3 (layers from 1)
+  uint16_t ht[3][kMlpHidden * kTrainLdT]; // columns of h1, h2, h3
+  uint16_t dt[2][kMlpHidden * kTrainLdT]; // columns of the deltas, in turn
   float    w5[kMlpHidden], g[kTrainRows];
 };
 static_assert(sizeof(TrainLds) <= 160 * 1024, "one training workgroup's LDS");
 
 __device__ __forceinline__ u16x8 lds8(const uint16_t* p) { return *reinterpret_cast<const u16x8*>(p); }
-// 8 elements of a column, rows r .. r + 7
-__device__ __forceinline__ u16x8 lds_col8(const uint16_t* p, int ld)
-{
-  u16x8 v;
-#pragma unroll
-  for (int e = 0; e < 8; e++) v[e] = p[e * ld];
-  return v;
-}
+__device__ __forceinline__ uint16_t relu_gate(uint16_t h, float x) { return f2bf((h == 0 || (h & 0x8000u)) ? 0.0f : x); }
 
 // acc += in^T d over the tile's 64 rows: NT row tiles of in's columns, the wave's 16 columns of d
 template <int NT>
-__device__ __forceinline__ void train_wgrad(const uint16_t* in, int ld, const uint16_t* d, int wave, int nn, int g,
+__device__ __forceinline__ void train_wgrad(const uint16_t* in, const uint16_t* d, int wave, int nn, int g,
                                             f32x4 (&acc)[NT])
 {
-  const u16x8 b0 = lds_col8(d + (8 * g) * kTrainLd + 16 * wave + nn, kTrainLd);
-  const u16x8 b1 = lds_col8(d + (32 + 8 * g) * kTrainLd + 16 * wave + nn, kTrainLd);
+  const u16x8 b0 = lds8(d + (16 * wave + nn) * kTrainLdT + 8 * g);
+  const u16x8 b1 = lds8(d + (16 * wave + nn) * kTrainLdT + 32 + 8 * g);
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    acc[t] = mfma(lds_col8(in + (8 * g) * ld + 16 * t + nn, ld), b0, acc[t]);
-    acc[t] = mfma(lds_col8(in + (32 + 8 * g) * ld + 16 * t + nn, ld), b1, acc[t]);
-    __builtin_amdgcn_sched_barrier(0); // one tile's operands at a time: the registers hold the gradients
+    acc[t] = mfma(lds8(in + (16 * t + nn) * kTrainLdT + 8 * g), b0, acc[t]);
+    acc[t] = mfma(lds8(in + (16 * t + nn) * kTrainLdT + 32 + 8 * g), b1, acc[t]);
+    if (t & 1) __builtin_amdgcn_sched_barrier(0); // a few operands at a time: the registers hold the gradients
   }
+}
+// The wave's weight fragments of a layer of K inputs (K / 32 blocks), from the [out][in] copy.
+template <int K>
+__device__ __forceinline__ void train_weights(const uint16_t* w, int col, int g, u16x8 (&bf)[4])
+{
+#pragma unroll
+  for (int b = 0; b < K / 32; b++) bf[b] = *reinterpret_cast<const u16x8*>(w + col * K + 32 * b + 8 * g);
+}
+// Rows 16 t .. 16 t + 15 of (in W) for the wave's 16 columns
+template <int K>
+__device__ __forceinline__ f32x4 train_rows(const uint16_t* in, int ld, int t, int nn, int g, const u16x8 (&bf)[4])
+{
+  f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int b = 0; b < K / 32; b++) acc = mfma(lds8(in + (16 * t + nn) * ld + 32 * b + 8 * g), bf[b], acc);
+  return acc;
 }
 
 // wt: the BF16 weights row-major [in][out]; wtt: the same transposed, [out][in] per layer (same
@@ -334,108 +350,127 @@ __global__ __launch_bounds__(64 * kTrainWaves) void train_kernel(const float* __
     if (t < 4) a1[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     a2[t] = a3[t] = a4[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   }
-  float db[4] = {0.0f, 0.0f, 0.0f, 0.0f}, dw5 = 0.0f, db5 = 0.0f, lsum = 0.0f; // threads < 128: column tid
+  // column sums: column tid / 4, a quarter of the rows each; db5, lsum: threads 0 mod 8
+  float     db[4] = {0.0f, 0.0f, 0.0f, 0.0f}, dw5 = 0.0f, db5 = 0.0f, lsum = 0.0f;
+  const int sc = tid >> 2, sq = tid & 3;
+  const int wo[4] = {kBfW1, kBfW2, kBfW3, kBfW4};
 
   for (int row0 = blockIdx.x * kTrainRows; row0 < n; row0 += gridDim.x * kTrainRows) {
-    __syncthreads();
-    { // features: 8 threads per row, 8 features each
-      const int r = tid >> 3, i = row0 + r, f0 = (tid & 7) * 8;
-      float     x[3] = {0.0f, 0.0f, 0.0f};
-      if (i < n)
-        for (int c = 0; c < 3; c++) x[c] = (pts[3 * (size_t)i + c] - p.lo[c]) * p.sc[c] - 1.0f;
-#pragma unroll
-      for (int k = 0; k < 8; k++) S.x0[r * kTrainLd0 + f0 + k] = f2bf(feature(f0 + k, x[0], x[1], x[2]));
-    }
-    __syncthreads();
-    // the weights are read again for each tile: kept across tiles they would take the registers that
-    // hold the gradients
+    // the weights are read again for each tile (kept across tiles they would take the registers that
+    // hold the gradients), each layer's one layer ahead of its products
     const uint16_t *wl = wt, *wlt = wtt;
     asm volatile("" : "+s"(wl), "+s"(wlt));
-    // forward: h = relu(in W + b); the wave's B fragments come straight from the transposed copy
-    const int wo[4] = {kBfW1, kBfW2, kBfW3, kBfW4};
+    u16x8 bf[2][4];
+    train_weights<kMlpInPad>(wlt + wo[0], col, g, bf[0]);
+    const int r8 = tid >> 3, k8 = tid & 7; // 8 threads per row
+    float     tgt = 0.0f;
+    { // features: 8 per thread
+      const int i = row0 + r8, f0 = k8 * 8;
+      float     x[3] = {0.0f, 0.0f, 0.0f};
+      if (i < n) {
+        tgt = target[i];
+        for (int c = 0; c < 3; c++) x[c] = (pts[3 * (size_t)i + c] - p.lo[c]) * p.sc[c] - 1.0f;
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const uint16_t f = f2bf(feature(f0 + k, x[0], x[1], x[2]));
+        S.x0[r8 * kTrainLd0 + f0 + k]    = f;
+        S.x0t[(f0 + k) * kTrainLdT + r8] = f;
+      }
+    }
+    __syncthreads();
+    // forward: h = relu(in W + b)
 #pragma unroll
     for (int L = 0; L < 4; L++) {
-      const int       K  = L == 0 ? kMlpInPad : kMlpHidden, ld = L == 0 ? kTrainLd0 : kTrainLd;
-      const uint16_t* in = L == 0 ? S.x0 : S.h[L - 1];
-      u16x8           bf[4];
-#pragma unroll
-      for (int b = 0; b < K / 32; b++)
-        bf[b] = *reinterpret_cast<const u16x8*>(wlt + wo[L] + col * K + 32 * b + 8 * g);
+      if (L < 3) train_weights<kMlpHidden>(wlt + wo[L + 1], col, g, bf[(L + 1) & 1]);
+      uint16_t* h = S.r[L == 3 ? 0 : L];
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
+        const f32x4 acc = L == 0 ? train_rows<kMlpInPad>(S.x0, kTrainLd0, t, nn, g, bf[0])
+                                 : train_rows<kMlpHidden>(S.r[L - 1], kTrainLd, t, nn, g, bf[L & 1]);
+        u16x4       v;
 #pragma unroll
-        for (int b = 0; b < K / 32; b++) acc = mfma(lds8(in + (16 * t + nn) * ld + 32 * b + 8 * g), bf[b], acc);
-#pragma unroll
-        for (int e = 0; e < 4; e++) S.h[L][(16 * t + 4 * g + e) * kTrainLd + col] = f2bf(fmaxf(acc[e] + bias[L], 0.0f));
+        for (int e = 0; e < 4; e++) {
+          v[e] = f2bf(fmaxf(acc[e] + bias[L], 0.0f));
+          h[(16 * t + 4 * g + e) * kTrainLd + col] = v[e];
+        }
+        if (L < 3) *reinterpret_cast<u16x4*>(&S.ht[L][col * kTrainLdT + 16 * t + 4 * g]) = v;
         __builtin_amdgcn_sched_barrier(0);
       }
       __syncthreads();
     }
-    { // output layer and loss: 8 threads per row, 16 columns each
-      const int       r = tid >> 3, i = row0 + r, k0 = (tid & 7) * 16;
-      const uint16_t* h = S.h[3] + r * kTrainLd + k0;
+    train_weights<kMlpHidden>(wl + wo[3], col, g, bf[1]);
+    { // output layer and loss: 8 threads per row, columns 2 k8 + 16 j and the next
+      const uint16_t* h = S.r[0] + r8 * kTrainLd + 2 * k8;
+      uint32_t        hv[8];
       float           y = 0.0f;
 #pragma unroll
-      for (int k = 0; k < 16; k++) y += bf2f(h[k]) * S.w5[k0 + k];
+      for (int j = 0; j < 8; j++) {
+        hv[j] = *reinterpret_cast<const uint32_t*>(h + 16 * j);
+        y += bf2f((uint16_t)hv[j]) * S.w5[2 * k8 + 16 * j];
+        y += bf2f((uint16_t)(hv[j] >> 16)) * S.w5[2 * k8 + 16 * j + 1];
+      }
       for (int o = 1; o < 8; o <<= 1) y += __shfl_xor(y, o, 64);
       y += b5;
       float gi = 0.0f;
-      if (i < n) {
-        const float e = y - logf(fabsf(target[i]) * inv_diag + kMlpLogC);
+      if (row0 + r8 < n) {
+        const float e = y - logf(fabsf(tgt) * inv_diag + kMlpLogC);
         const float w = e < 0.0f ? under_weight : 1.0f;
         gi            = 2.0f * w * e * inv_n;
-        if ((tid & 7) == 0) lsum += w * e * e;
+        if (k8 == 0) lsum += w * e * e;
       }
-      if ((tid & 7) == 0) S.g[r] = gi;
+      if (k8 == 0) {
+        S.g[r8] = gi;
+        db5 += gi;
+      }
 #pragma unroll
-      for (int k = 0; k < 16; k++) {
-        const uint16_t hv = h[k];
-        S.d[1][r * kTrainLd + k0 + k] = f2bf((hv == 0 || (hv & 0x8000u)) ? 0.0f : gi * S.w5[k0 + k]);
+      for (int j = 0; j < 8; j++) {
+        const int      c  = 2 * k8 + 16 * j;
+        const uint16_t d0 = relu_gate((uint16_t)hv[j], gi * S.w5[c]), d1 = relu_gate((uint16_t)(hv[j] >> 16), gi * S.w5[c + 1]);
+        *reinterpret_cast<uint32_t*>(&S.r[1][r8 * kTrainLd + c]) = d0 | (uint32_t)d1 << 16;
+        S.dt[1][c * kTrainLdT + r8]                              = d0;
+        S.dt[1][(c + 1) * kTrainLdT + r8]                        = d1;
       }
     }
     __syncthreads();
-    if (tid < kMlpHidden) {
-#pragma unroll 4
-      for (int r = 0; r < kTrainRows; r++) dw5 += bf2f(S.h[3][r * kTrainLd + tid]) * S.g[r];
-    }
-    if (tid == 0)
-#pragma unroll 4
-      for (int r = 0; r < kTrainRows; r++) db5 += S.g[r];
-    // hidden layers, last to first: delta of layer L (0-based) in d[L & 1]
+#pragma unroll 8
+    for (int j = 0; j < kTrainRows / 4; j++) dw5 += bf2f(S.r[0][(4 * j + sq) * kTrainLd + sc]) * S.g[4 * j + sq];
+    // hidden layers, last to first: the delta of layer L (from 0) has its columns in dt[L & 1], its
+    // rows in r[1], r[2], r[0] for L = 3, 2, 1
 #pragma unroll
     for (int L = 3; L >= 0; L--) {
-      const uint16_t* d = S.d[L & 1];
-      if (tid < kMlpHidden) {
-        float s = 0.0f;
-#pragma unroll 8
-        for (int r = 0; r < kTrainRows; r++) s += bf2f(d[r * kTrainLd + tid]);
+      const uint16_t* d = S.dt[L & 1];
+      if (L > 1) train_weights<kMlpHidden>(wl + wo[L - 1], col, g, bf[(L - 1) & 1]);
+      {
+        const u16x8 lo = lds8(d + sc * kTrainLdT + 16 * sq), hi = lds8(d + sc * kTrainLdT + 16 * sq + 8);
+        float       s = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) s += bf2f(lo[e]);
+#pragma unroll
+        for (int e = 0; e < 8; e++) s += bf2f(hi[e]);
         db[L] += s;
       }
-      if (L == 3) train_wgrad<8>(S.h[2], kTrainLd, d, wave, nn, g, a4);
-      else if (L == 2) train_wgrad<8>(S.h[1], kTrainLd, d, wave, nn, g, a3);
-      else if (L == 1) train_wgrad<8>(S.h[0], kTrainLd, d, wave, nn, g, a2);
-      else train_wgrad<4>(S.x0, kTrainLd0, d, wave, nn, g, a1);
       if (L > 0) { // delta of the layer below: (d W^T) where its activation is positive
-        uint16_t* o = S.d[(L - 1) & 1];
-        u16x8     bf[4];
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-          bf[b] = *reinterpret_cast<const u16x8*>(wl + wo[L] + col * kMlpHidden + 32 * b + 8 * g);
+        const uint16_t* dr = S.r[L == 3 ? 1 : (L == 2 ? 2 : 0)];
+        uint16_t*       o  = S.r[L == 3 ? 2 : 0];
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-          f32x4 acc{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-          for (int b = 0; b < 4; b++) acc = mfma(lds8(d + (16 * t + nn) * kTrainLd + 32 * b + 8 * g), bf[b], acc);
+          const f32x4 acc = train_rows<kMlpHidden>(dr, kTrainLd, t, nn, g, bf[L & 1]);
+          const u16x4 h   = *reinterpret_cast<const u16x4*>(&S.ht[L - 1][col * kTrainLdT + 16 * t + 4 * g]);
+          u16x4       v;
 #pragma unroll
           for (int e = 0; e < 4; e++) {
-            const int      r  = 16 * t + 4 * g + e;
-            const uint16_t hv = S.h[L - 1][r * kTrainLd + col];
-            o[r * kTrainLd + col] = f2bf((hv == 0 || (hv & 0x8000u)) ? 0.0f : acc[e]);
+            v[e] = relu_gate(h[e], acc[e]);
+            if (L > 1) o[(16 * t + 4 * g + e) * kTrainLd + col] = v[e];
           }
+          *reinterpret_cast<u16x4*>(&S.dt[(L - 1) & 1][col * kTrainLdT + 16 * t + 4 * g]) = v;
           __builtin_amdgcn_sched_barrier(0);
         }
       }
+      if (L == 3) train_wgrad<8>(S.ht[2], d, wave, nn, g, a4);
+      else if (L == 2) train_wgrad<8>(S.ht[1], d, wave, nn, g, a3);
+      else if (L == 1) train_wgrad<8>(S.ht[0], d, wave, nn, g, a2);
+      else train_wgrad<4>(S.x0t, d, wave, nn, g, a1);
       __syncthreads();
     }
   }
@@ -451,14 +486,28 @@ __global__ __launch_bounds__(64 * kTrainWaves) void train_kernel(const float* __
       out[kOffW3 + r] = a3[t][e];
       out[kOffW4 + r] = a4[t][e];
     }
-  if (tid < kMlpHidden) {
+  for (int o = 1; o < 4; o <<= 1) {
+#pragma unroll
+    for (int L = 0; L < 4; L++) db[L] += __shfl_xor(db[L], o, 64);
+    dw5 += __shfl_xor(dw5, o, 64);
+  }
+  if (sq == 0) {
     const int bo[4] = {kOffB1, kOffB2, kOffB3, kOffB4};
 #pragma unroll
-    for (int L = 0; L < 4; L++) out[bo[L] + tid] = db[L];
-    out[kOffW5 + tid] = dw5;
+    for (int L = 0; L < 4; L++) out[bo[L] + sc] = db[L];
+    out[kOffW5 + sc] = dw5;
   }
-  if (tid == 0) out[kOffB5] = db5;
-  for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
+  for (int o = 32; o > 0; o >>= 1) {
+    lsum += __shfl_xor(lsum, o, 64);
+    db5 += __shfl_xor(db5, o, 64);
+  }
+  if (lane == 0) S.g[wave] = db5; // after the last tile's barrier
+  __syncthreads();
+  if (tid == 0) {
+    float s = 0.0f;
+    for (int w = 0; w < kTrainWaves; w++) s += S.g[w];
+    out[kOffB5] = s;
+  }
   if (lane == 0 && lsum != 0.0f) atomicAdd(loss_sum, lsum);
 }
 
