@@ -248,8 +248,9 @@ ebg_status enqueue(ebg_batch_plan* p, hipStream_t s, bool events)
 // mesh's grid mean start first (256-mesh workload: 66.8 -> 55.4 ms; 1.5x: 56.3, 3x: 55.4).
 constexpr uint64_t kEarlyMinFaces = 16384;
 // Plans of fewer queries hand long walks on (HandOn) besides: such a launch is over before its
-// longest packets are, early or not (32 meshes of 1,280 to 81,920 faces, 5M queries: 4.1 -> 1.6 ms).
-constexpr uint64_t kHandMaxTotal = 1u << 23;
+// longest packets are, early or not. 32 meshes of 1,280 to 81,920 faces, handed on and not: 3.0M
+// queries 1.52 and 3.95 ms, 5.9M 2.01 and 3.39, 8.9M 2.62 and 3.70, 11.9M 3.06 and 3.02.
+constexpr uint64_t kHandMaxTotal  = 11u << 20;
 constexpr double   kEarlyFactor   = 2.0;
 
 double elapsed_ms(hipEvent_t a, hipEvent_t b)

@@ -401,14 +401,16 @@ __device__ __forceinline__ void band_block(const MeshDev& m, const QueryArgs& a,
 }
 
 // Every query. The launch lasts as long as the packet with the most triangles in its lanes' bands (next
-// to the medial axis), and nothing is handed on here, so packets are narrowed until there are
-// kBandPackets of them: 100,000 closest faces on 81,920 faces, displaced, 1.95 ms with the FP32 pass's
-// packets, 1.18 with 4 queries each; 300,000 2.41 -> 1.51 (8 queries); 1M 2.60 -> 2.17 (16; 2.21 with
-// 32, 2.22 with 8); 2M 3.77 -> 3.30 (32; 3.91 with 8).
-constexpr uint64_t kBandPackets = 1u << 16;
+// to the medial axis), and nothing is handed on here, so packets are narrowed, down to 4 queries, until
+// there are kBandPackets of them. Times of the whole call with 64, 32, 16, 8, 4 queries a packet, in us:
+// 1M closest faces on 81,920 faces, displaced: 2582, 2198, 2143, 2206, 2748; 100,000 on it: 1953, 1954,
+// 1762, 1333, 1186. A mesh without such packets pays for paths that are no longer shared (1M on 4,600
+// triangles of a polygon mesh: 1383, 1404, 1558, 1730, 1998; 200,003: 628, 591, 611, 632, 694): the line
+// lies where it loses nothing yet.
+constexpr uint64_t kBandPackets = 1u << 15;
 inline uint32_t    band_narrow(uint64_t n, uint32_t narrow)
 {
-  while (narrow < 6 && num_packets(n, narrow + 1) <= kBandPackets) narrow++;
+  while (narrow < 4 && num_packets(n, narrow + 1) <= kBandPackets) narrow++;
   return narrow;
 }
 template <int NB>
