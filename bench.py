@@ -405,7 +405,7 @@ def scene_bench(a, dev):
             "mesh_leaf_size": 16, "learned_bound": learned,
             "value": round(n / dt, 1), "unit": "queries/s", "ms_per_step": round(dt * 1e3, 3),
             "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "scene32_kernel<4,1,false>",
+                         "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "scene32_kernel<1,false,true> and its items",
                          "kernel_ms": round(kms, 3), "algorithmic_bytes_per_launch": int(byts),
                          "per_wavefront": {"interior_nodes": round(w[4] / (n / 64), 1),
                                            "primitives": round(w[7] / (n / 64), 1),
@@ -470,7 +470,7 @@ def batched_bench(a):
                       "tune_ms": info["tune_ms"]},
            "graph_replay_ms": round(replay_ms, 3),
            "roofline": packet_roofline(nq, c, K, kms, f"batch32_kernel<{info['stack_capacity'] // 64},false,"
-                                       f"{str(plan.persistent).lower()}>",
+                                       f"{str(plan.persistent).lower()},false>",
                                        profiled_traffic("batch32", "batch32_many_meshes_256_counters.txt")),
            "correctness": {"sample": f"{checked} queries (200 strided of every 16th mesh) against the oracle",
                            "max_abs_err_over_diag": worst, "sign_mismatches": signs,

@@ -2,15 +2,20 @@
 //
 // HBM layout of one mesh (all arrays 64-byte aligned, in leaf order where per-triangle):
 //   nodes   Node<K>[num_nodes]   K child boxes as SoA (lo.x[K] .. hi.z[K]) + child refs.
-//                                K=4: 128 B, K=8: 256 B. Read with wave-uniform (scalar)
-//                                loads: one fetch serves all 64 queries of a wavefront.
+//                                K=4: 128 B, K=8: 256 B. Read by the FP64 walks of scenes and
+//                                programs, with wave-uniform (scalar) loads: one fetch serves all
+//                                64 queries of a wavefront.
+//   wnodes  WalkNode[]           the FP32 walk's tree: 4 children bounded by cylinders or boxes.
+//   tdisc   TriDisc[num_tris+16] per triangle the disc of its plane that holds it: the screen of
+//                                the FP32 walk's leaves, 4 triangles per scalar round trip.
+//   frames  FrameRec[num_tris]   each triangle in a frame of its own plane (FP32 pair evaluation).
 //   tris    TriRec[num_tris]     128 B FP32 record per triangle with the quantities the
 //                                point-triangle kernel needs precomputed (edges, face normal,
 //                                edge x normal, 1/|edge|^2). Also read with scalar loads.
 //   tripos  float[12*num_tris]   raw vertex positions (v0,v1,v2,pad) for the FP64 path.
 //   tsph    float8[num_tris+16]  per-triangle culling data, contiguous per leaf: bounding sphere
-//                                (centre, radius) and plane (unit normal, -n.v0), so that the
-//                                culling data of 4 leaf triangles arrives in one scalar round trip.
+//                                (centre, radius) and plane (unit normal, -n.v0) for the FP64
+//                                walks, 4 leaf triangles in one scalar round trip.
 //   feat    uint32[8*num_tris]   vertex ids, half-edge ids, original face id: lets the sign
 //                                step fetch the one pseudo-normal a query needs.
 //   vn32/vn64, en32/en64         vertex / half-edge pseudo-normals (float4 / double4).

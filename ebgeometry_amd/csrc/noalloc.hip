@@ -3,7 +3,7 @@
 // For callers that cannot allocate device memory (code under HIP graph capture, tight serving
 // loops, harnesses that forbid hipMalloc). The workspace of one call -- presort keys and
 // permutation, radix-sort scratch, FP64 recheck list, counters, seeded radii, recheck masks and
-// the split-packet schedule -- is carved from `scratch`, which every GPU the library runs on
+// the schedule of long walks (split or handed-on packets) -- is carved from `scratch`, which every GPU the library runs on
 // holds (its own copy) until the process ends. Its device address is looked up once per device
 // with hipGetSymbolAddress; host code uses that address, never the array's name.
 #include "host_common.hpp"
