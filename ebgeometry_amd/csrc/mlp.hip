@@ -601,12 +601,6 @@ __global__ __launch_bounds__(256) void sync_bf16_kernel(const float* __restrict_
   winfer[i]   = k < 0 ? (uint16_t)0 : f2bf(master[moff + k * kMlpHidden + r]); // W^T[out r][in k]
 }
 
-__global__ void scale_kernel(float* p, int n, float s)
-{
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] *= s;
-}
-
 // public order <-> master layout (W1 rows 51..63 are padding)
 __global__ void grad_public_kernel(const float* __restrict__ g, float* __restrict__ out)
 {
