@@ -186,6 +186,7 @@ static ebg_status build_walk(ebg_mesh* m, const ebgpu::PackedMesh& pm)
     return fail(EBG_STACK_OVERFLOW, "tree needs a traversal stack of " + std::to_string(wt.stack_need) +
                                       " entries (max 256); use a smaller branching factor");
   if (m->wbanks == 3) m->wbanks = 4;
+  m->walk_deep_need = wt.deep_need;
   const std::vector<ebgpu::SplitRoot> roots = split_frontier(wt, kSplitRoots);
   EBG_HIP(upload(m->split_roots, roots));
   m->num_split_roots = uint32_t(roots.size());
@@ -654,7 +655,7 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
     a.hand = ws.hand;
     for (int i = 0; i < 2; i++) {
       a.hand.budget[i] = ebgpu::kHandBudget[i];
-      a.hand.spread[i] = ebgpu::kHandSpread[i];
+      a.hand.spread[i] = ebgpu::hand_spread(i, 64 * m->wbanks, m->walk_deep_need);
     }
   }
 

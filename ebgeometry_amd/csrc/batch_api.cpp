@@ -21,7 +21,7 @@ struct ebg_batch
 {
   std::vector<ebg_mesh*> meshes; // owned
   DevBuf                 meshdev;
-  int                    K = 4, leaf = 8, banks = 1, wbanks = 1;
+  int                    K = 4, leaf = 8, banks = 1, wbanks = 1, deep_need = 1;
   bool                   tuned = false;
   double                 tune_ms[4]{-1, -1, -1, -1};
   double                 build_seconds = 0;
@@ -199,7 +199,7 @@ ebg_status enqueue(ebg_batch_plan* p, hipStream_t s, bool events)
     a.hand = ebgpu::Workspace::hand_view(p->handed.as<uint8_t>(), p->total, p->counter.as<uint32_t>() + 4);
     for (int i = 0; i < 2; i++) {
       a.hand.budget[i] = ebgpu::kHandBudget[i];
-      a.hand.spread[i] = ebgpu::kHandSpread[i];
+      a.hand.spread[i] = ebgpu::hand_spread(i, 64 * b->wbanks, b->deep_need);
     }
   }
   if (p->presort && p->total > 1) {
@@ -355,8 +355,9 @@ ebg_status ebg_batch_create(const float* const* xyz, const uint64_t* nv, const u
   std::vector<ebgpu::MeshDev> md(num_meshes);
   for (uint64_t i = 0; i < num_meshes; i++) {
     md[i]    = b->meshes[i]->dev;
-    b->banks  = std::max(b->banks, b->meshes[i]->banks);
-    b->wbanks = std::max(b->wbanks, b->meshes[i]->wbanks);
+    b->banks     = std::max(b->banks, b->meshes[i]->banks);
+    b->wbanks    = std::max(b->wbanks, b->meshes[i]->wbanks);
+    b->deep_need = std::max(b->deep_need, b->meshes[i]->walk_deep_need);
     b->num_triangles += b->meshes[i]->nt;
   }
   const hipError_t e = upload(b->meshdev, md);

@@ -5,6 +5,7 @@
 #include "../../include/ebgpu.h"
 #include "kernels.hpp"
 #include "mlp.hpp"
+#include "walk_schedule.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -98,9 +99,7 @@ struct WsView
 
 // Calls of fewer queries hand long walks on (HandOn); larger presorted ones split the packets that
 // their cost grid finds expensive.
-constexpr uint64_t kHandMaxQ      = 1u << 20;
-constexpr uint32_t kHandBudget[2] = {150, 60}; // HandOn::budget (measured: api.cpp)
-constexpr int32_t  kHandSpread[2] = {48, 32};
+constexpr uint64_t kHandMaxQ = 1u << 20;
 
 // Query workspace, grown on demand.
 struct Workspace
@@ -257,7 +256,7 @@ struct ebg_mesh
   // the FP32 walk's tree and records (MeshDev::wnodes, tdisc, frames) and its stack banks
   ebgpu::DevBuf          wnodes, tdisc, frames;
   ebgpu::DevBuf          nfirst; // MeshDev::nfirst
-  int                    wbanks = 1;
+  int                    wbanks = 1, walk_deep_need = 1; // WalkTree::deep_need
   // cost grid of the split schedule (built at the first large presorted query): per cell, the
   // work of a packet of 64 queries spread over the cell
   ebgpu::DevBuf          cost_grid;

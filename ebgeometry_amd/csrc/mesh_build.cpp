@@ -682,9 +682,9 @@ struct WalkEmitter
     return c;
   }
 
-  // A walk node over the children kids of in[i]; returns its index, the triangles below it and
-  // the stack its walk needs beyond its own entry.
-  uint32_t emit(uint32_t i, const std::vector<int>& kids, Range& all, int& need)
+  // A walk node over the children kids of in[i], `level` levels below the root; returns its index, the
+  // triangles below it and the stack its walk needs beyond its own entry.
+  uint32_t emit(uint32_t i, const std::vector<int>& kids, int level, Range& all, int& need)
   {
     const uint32_t me = uint32_t(out.nodes.size());
     out.nodes.emplace_back();
@@ -718,7 +718,8 @@ struct WalkEmitter
       }
       else {
         nd.cnt[k] = kBoxChild;
-        nd.ref[k] = part.size() == 1 ? emit(n.ref[part[0]], children(n.ref[part[0]]), r, deep) : emit(i, part, r, deep);
+        nd.ref[k] = part.size() == 1 ? emit(n.ref[part[0]], children(n.ref[part[0]]), level + 1, r, deep)
+                                     : emit(i, part, level + 1, r, deep);
       }
       deepest = std::max(deepest, deep);
       if (r.count == r.last - r.first) {
@@ -731,6 +732,7 @@ struct WalkEmitter
     }
     out.nodes[me] = nd;
     need          = slots - 1 + deepest;
+    if (level == 2) out.deep_need = std::max(out.deep_need, 1 + need);
     return me;
   }
 };
@@ -741,12 +743,13 @@ void build_walk_tree(const PackedMesh& pm, float scale, WalkTree& out)
 {
   out.nodes.clear();
   out.range.clear();
+  out.deep_need = 1;
   int  need = 0;
   auto run  = [&](auto tag) {
     constexpr int         KK = decltype(tag)::value;
     WalkEmitter<KK>       e{reinterpret_cast<const Node<KK>*>(pm.nodes.data()), scale, out};
     typename WalkEmitter<KK>::Range all;
-    e.emit(0, e.children(0), all, need);
+    e.emit(0, e.children(0), 0, all, need);
   };
   if (pm.K == 4) run(std::integral_constant<int, 4>{});
   else run(std::integral_constant<int, 8>{});

@@ -25,6 +25,7 @@ struct ebg_scene
   DevBuf                 nodes, prims, prims64, meshdev, status;
   ebgpu::SceneDev        dev{};
   int                    KM = 4, banks = 1, stack_need = 0;
+  int                    deep_need = 1; // of its meshes: WalkTree::deep_need
   std::size_t            num_prims = 0, num_nodes = 0;
   double                 lo[3]{}, hi[3]{}, diag = 0;
   std::mutex             mu;
@@ -85,12 +86,13 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
   const int leaf = o.leaf_size ? o.leaf_size : 4;
   if (leaf < 1 || leaf > ebgpu::kMaxLeaf) return fail(EBG_INVALID_ARG, "leaf_size must be 1..16");
 
-  int KM = 0, mesh_banks = 1;
+  int KM = 0, mesh_banks = 1, deep_need = 1;
   for (uint64_t j = 0; j < num_meshes; j++) {
     if (!meshes[j]) return fail(EBG_INVALID_ARG, "null mesh handle");
     if (KM && meshes[j]->K != KM) return fail(EBG_INVALID_ARG, "all scene meshes must have the same branching");
     KM         = meshes[j]->K;
     mesh_banks = std::max({mesh_banks, meshes[j]->banks, meshes[j]->wbanks});
+    deep_need  = std::max(deep_need, meshes[j]->walk_deep_need);
   }
   if (!KM) KM = 4;
 
@@ -215,6 +217,7 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
   auto* sc       = new ebg_scene;
   sc->KM         = KM;
   sc->banks      = banks;
+  sc->deep_need  = deep_need;
   sc->stack_need = wb.stack_need;
   sc->num_prims  = n;
   sc->num_nodes  = wb.num_nodes;
@@ -332,7 +335,7 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
     slots  = reinterpret_cast<ebgpu::SceneSlot*>(sc->handed.as<uint8_t>() + lists);
     for (int i = 0; i < 2; i++) {
       a.hand.budget[i] = kSceneBudget[i];
-      a.hand.spread[i] = ebgpu::kHandSpread[i];
+      a.hand.spread[i] = ebgpu::hand_spread(i, 64 * sc->banks, sc->deep_need);
     }
   }
 

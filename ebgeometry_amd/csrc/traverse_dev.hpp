@@ -1040,9 +1040,10 @@ __device__ __forceinline__ void push_walk_children(const MeshDev& m, Walk<NB>& w
     pushed++;
   }
   wk.top += pushed;
-  // The capacity is the tree's exact worst case, computed at build time; should a walk ever exceed
-  // it, the pushes beyond it were dropped: record that in the mesh's status word (the host reports
-  // it) and go on with the entries that are held.
+  // The capacity is the tree's exact worst case for a walk from one entry, computed at build time, and
+  // stacks are spread only so far that a walk that goes on from them keeps to it (hand_spread); should a
+  // walk ever exceed it, the pushes beyond it were dropped: record that in the mesh's status word (the
+  // host reports it) and go on with the entries that are held.
   if (wk.top > 64 * NB) {
     if (__lane_id() == 0 && m.status) atomicOr(m.status, kStatusStackOverflow);
     wk.top = 64 * NB;
@@ -1050,7 +1051,8 @@ __device__ __forceinline__ void push_walk_children(const MeshDev& m, Walk<NB>& w
 }
 
 // Spread the stack to about `spread` entries before it is handed on: nodes give way to their children,
-// from the bottom (the largest subtrees).
+// from the bottom (the largest subtrees). Only when the walk is out of its budget: at least its start
+// entry has been visited.
 template <int NB>
 __device__ __forceinline__ void spread_walk(const MeshDev& m, Walk<NB>& wk, int spread, float px, float py, float pz,
                                             float b2, int rep)
