@@ -56,3 +56,19 @@ def test_training_is_reproducible(cuda):
         m.train_bound(num_samples=5000, epochs=2, batch=1000, seed=4)
         w.append(m.get_bound_params())
     assert np.isfinite(w[0]).all() and np.array_equal(w[0], w[1])
+
+
+def test_weights_are_written_when_training_returns(cuda):
+    """A stream that does not wait for the training's (a torch stream: non-blocking) predicts with the
+    trained weights at once."""
+    import torch
+    v, f = wl.displaced_icosphere(3, 9)
+    q = torch.from_numpy(wl.mixed_queries(5000, v, f, 10)).to(cuda)
+    side = torch.cuda.Stream()
+    m = TriMeshSDF(v, f)
+    for seed in range(8):
+        m.train_bound(num_samples=4096, epochs=1, batch=4096, seed=seed)
+        with torch.cuda.stream(side):
+            at_once = m.predict_bound(q)
+        torch.cuda.synchronize()
+        assert torch.equal(at_once, m.predict_bound(q)), seed
