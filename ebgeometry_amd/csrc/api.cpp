@@ -833,6 +833,9 @@ double ebg_mesh_last_traversal_ms(const ebg_mesh* cm)
   return ms;
 }
 
+// Host-array calls keep a device buffer of up to this many bytes in the handle.
+constexpr std::size_t kHostKeep = 64u << 20;
+
 ebg_status ebg_query_sdf_host(const ebg_mesh* cm, const float* pts, uint64_t n, float* dist, uint32_t* tri,
                               const ebg_query_opts* opts)
 {
@@ -846,12 +849,14 @@ ebg_status ebg_query_sdf_host(const ebg_mesh* cm, const float* pts, uint64_t n, 
   if (opts) o = *opts;
   hipStream_t s = static_cast<hipStream_t>(o.stream);
   // The device copies lie one after the other in a buffer that the handle keeps (200,003 queries with
-  // faces: 798 us with three allocations per call, now 617). A call that meets another one in
-  // progress takes a buffer of its own.
-  std::unique_lock<std::mutex> kept(m->host_mu, std::try_to_lock);
+  // faces: 798 us with three allocations per call, now 617), unless they are large, where the copies
+  // take far longer than an allocation. A call that meets another one in progress takes a buffer of its
+  // own.
+  const std::size_t            bytes = std::size_t(tri ? 20 : 16) * n;
+  std::unique_lock<std::mutex> kept(m->host_mu, std::defer_lock);
   DevBuf                       own;
-  DevBuf&                      io = kept.owns_lock() ? m->host_io : own;
-  EBG_HIP(io.reserve((tri ? 20 : 16) * n));
+  DevBuf& io = bytes <= kHostKeep && kept.try_lock() ? m->host_io : own;
+  EBG_HIP(io.reserve(bytes));
   float*           p  = io.as<float>();
   float*           d  = p + 3 * n;
   uint32_t*        t  = tri ? reinterpret_cast<uint32_t*>(d + n) : nullptr;

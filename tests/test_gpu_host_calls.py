@@ -1,5 +1,5 @@
 """Host-array calls share one buffer of the handle: sizes up and down, and several threads at once,
-give the values of the device-array call."""
+give the values of the device-array call; a large call's buffer is given back."""
 import threading
 
 import numpy as np
@@ -33,3 +33,19 @@ def test_sizes_and_threads(cuda):
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_large_buffers_are_given_back(cuda):
+    """5M points take 80 MB of points and distances, above what the handle keeps (64 MiB). The query
+    workspace, which it does keep, is grown by a device-array call first."""
+    import torch
+    v, f = wl.displaced_icosphere(2, 35)
+    m = TriMeshSDF(v, f)
+    q = wl.mixed_queries(5_000_000, v, f, 36)
+    ref = m.query(torch.from_numpy(q).to(cuda)).cpu().numpy()
+    torch.cuda.empty_cache()
+    before, _ = torch.cuda.mem_get_info()
+    got = m.signed_distance(q)
+    after, _ = torch.cuda.mem_get_info()
+    assert np.array_equal(got, ref)
+    assert before - after < 32 << 20
