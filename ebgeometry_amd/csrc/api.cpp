@@ -860,12 +860,18 @@ ebg_status ebg_query_sdf_host(const ebg_mesh* cm, const float* pts, uint64_t n, 
   float*           p  = io.as<float>();
   float*           d  = p + 3 * n;
   uint32_t*        t  = tri ? reinterpret_cast<uint32_t*>(d + n) : nullptr;
-  EBG_HIP(hipMemcpyAsync(p, pts, 12 * n, hipMemcpyHostToDevice, s));
-  const ebg_status st = ebg_query_sdf(m, p, n, d, t, &o);
+  const ebg_status st = [&]() -> ebg_status {
+    EBG_HIP(hipMemcpyAsync(p, pts, 12 * n, hipMemcpyHostToDevice, s));
+    const ebg_status q = ebg_query_sdf(m, p, n, d, t, &o);
+    if (q != EBG_OK) return q;
+    EBG_HIP(hipMemcpyAsync(dist, d, 4 * n, hipMemcpyDeviceToHost, s));
+    if (tri) EBG_HIP(hipMemcpyAsync(tri, t, 4 * n, hipMemcpyDeviceToHost, s));
+    return EBG_OK;
+  }();
+  // waits whatever came of it: the next call may take the buffer on another stream
+  const hipError_t e = hipStreamSynchronize(s);
   if (st != EBG_OK) return st;
-  EBG_HIP(hipMemcpyAsync(dist, d, 4 * n, hipMemcpyDeviceToHost, s));
-  if (tri) EBG_HIP(hipMemcpyAsync(tri, t, 4 * n, hipMemcpyDeviceToHost, s));
-  EBG_HIP(hipStreamSynchronize(s));
+  EBG_HIP(e);
   return EBG_OK;
 }
 

@@ -1,5 +1,5 @@
-"""Host-array calls share one buffer of the handle: sizes up and down, and several threads at once,
-give the values of the device-array call; a large call's buffer is given back."""
+"""Host-array calls share one buffer of the handle: sizes up and down, several threads at once, and calls
+after a refused one give the values of the device-array call; a large call's buffer is given back."""
 import threading
 
 import numpy as np
@@ -7,6 +7,7 @@ import pytest
 
 from ebgeometry_amd import TriMeshSDF
 from ebgeometry_amd import workloads as wl
+from ebgeometry_amd._lib import EbgError
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +50,18 @@ def test_large_buffers_are_given_back(cuda):
     after, _ = torch.cuda.mem_get_info()
     assert np.array_equal(got, ref)
     assert before - after < 32 << 20
+
+
+def test_call_after_a_refused_one(cuda):
+    """The learned bound of an untrained mesh is refused after the points were sent to the device; the
+    next call, on another stream, has the buffer to itself."""
+    import torch
+    v, f = wl.displaced_icosphere(3, 37)
+    m = TriMeshSDF(v, f)
+    q = wl.mixed_queries(300_000, v, f, 38)
+    ref = m.query(torch.from_numpy(q).to(cuda)).cpu().numpy()
+    side = torch.cuda.Stream()
+    for _ in range(3):
+        with pytest.raises(EbgError):
+            m.signed_distance(q[::-1].copy(), learned_bound=True)
+        assert np.array_equal(m.signed_distance(q, stream=side.cuda_stream), ref)
