@@ -54,8 +54,8 @@ SOURCES = [
     ("mlp.hip", DEVICE),
     ("noalloc.hip", DEVICE),
 ]
-HEADERS = ["ebgpu_internal.hpp", "kernels.hpp", "mesh_build.hpp", "mlp.hpp", "traverse_dev.hpp", "walk_schedule.hpp",
-           "host_common.hpp", "gpu_build.hpp"]
+HEADERS = ["ebgpu_internal.hpp", "kernels.hpp", "mesh_build.hpp", "mlp.hpp", "mlp_schedule.hpp", "traverse_dev.hpp",
+           "walk_schedule.hpp", "host_common.hpp", "gpu_build.hpp"]
 
 
 def _mtime(p):

@@ -950,7 +950,7 @@ ebg_status ebg_mlp_check_schedule(uint64_t num_samples, int32_t batch)
 {
   if (num_samples < 1 || batch < 32 || batch > 65536) return fail(EBG_INVALID_ARG, "num_samples/batch out of range");
   std::string why;
-  if (!ebgpu::mlp_check_train_schedule(num_samples, batch, &why)) return fail(EBG_INVALID_ARG, why);
+  if (!ebgpu::check_train_schedule(num_samples, batch, num_samples, ebgpu::mlp_train_blocks(batch), &why)) return fail(EBG_INVALID_ARG, why);
   return EBG_OK;
 }
 
@@ -981,7 +981,7 @@ ebg_status ebg_mlp_train(ebg_mesh* m, const ebg_mlp_opts* opts, float* loss)
     return fail(EBG_INVALID_ARG, "lr, box_scale, near_sigma or under_weight out of range");
   {
     std::string why;
-    if (!ebgpu::mlp_check_train_schedule(o.num_samples, o.batch, &why)) return fail(EBG_INVALID_ARG, why);
+    if (!ebgpu::check_train_schedule(o.num_samples, o.batch, o.num_samples, ebgpu::mlp_train_blocks(o.batch), &why)) return fail(EBG_INVALID_ARG, why);
   }
   hipStream_t s = static_cast<hipStream_t>(o.stream);
   std::lock_guard<std::recursive_mutex> lock(m->mu);

@@ -267,9 +267,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void infer_kernel(const float* __
 // 4,096 rows fills 64 workgroups).
 // The operations and roundings are those of separate products: BF16 activations and deltas, FP32
 // accumulation, FP32 biases, output layer and loss.
-constexpr int kTrainRows  = 64;  // rows per tile
 constexpr int kTrainWaves = 8;   // wave w owns output columns 16 w .. 16 w + 15 of every product
-constexpr int kTrainBlk   = 128; // most workgroups of a step (each strides over tiles)
 constexpr int kTrainLd    = kMlpHidden + 8; // LDS strides of row-major tiles (16-byte aligned, rows on
 constexpr int kTrainLd0   = kMlpInPad + 8;  // shifted banks) ...
 constexpr int kTrainLdT   = kTrainRows + 8; // ... and of tiles stored column by column
@@ -722,8 +720,6 @@ MlpTrainBuffers::~MlpTrainBuffers()
     if (p) (void)hipFree(p);
 }
 
-int mlp_train_blocks(int n) { return std::min((n + kTrainRows - 1) / kTrainRows, kTrainBlk); }
-
 hipError_t MlpTrainBuffers::ensure(int b)
 {
   const int want = mlp_train_blocks(b);
@@ -844,29 +840,12 @@ hipError_t mlp_forward(const Mlp& m, const float* pts, const uint32_t* idx, uint
   return hipGetLastError();
 }
 
-// A training step over n rows on tb's partial gradients: the launch shape and the extents of what
-// it indexes, checked on the host. The workgroups stride over 64-row tiles and guard rows >= n;
-// weights, biases and gradients have fixed sizes; each workgroup writes kMaster floats of `part`.
-static hipError_t check_step(int n, int parts, std::string* why)
+// Enqueue the loss and the partial gradients of a step over n rows of `samples`; returns the partial
+// gradients' number in *parts. Weights, biases and gradients have fixed sizes; what depends on n is checked.
+static hipError_t train_launch(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, uint64_t samples, int n,
+                               hipStream_t s, int* parts, std::string* why)
 {
-  if (n < 1) {
-    if (why) *why = "empty training batch";
-    return hipErrorInvalidValue;
-  }
-  const int blocks = mlp_train_blocks(n);
-  if (blocks < 1 || blocks > parts) {
-    if (why) *why = "training batch larger than its buffers";
-    return hipErrorInvalidValue;
-  }
-  return hipSuccess;
-}
-
-// Enqueue the loss and the partial gradients; returns their number in *parts.
-static hipError_t train_launch(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, int n, hipStream_t s,
-                               int* parts, std::string* why)
-{
-  hipError_t e = check_step(n, tb.parts, why);
-  if (e != hipSuccess) return e;
+  if (!check_train_step(n, samples, uint64_t(tb.parts), why)) return hipErrorInvalidValue;
   *parts = mlp_train_blocks(n);
   hipLaunchKernelGGL(train_kernel, dim3(*parts), dim3(64 * kTrainWaves), 0, s, pts, target, n, dev_of(m), m.wtrain,
                      m.wtrain_t, 1.0f / m.diag, 1.0f / (float)n, m.under_weight, tb.loss, tb.part);
@@ -878,28 +857,18 @@ hipError_t mlp_loss_grad(Mlp& m, MlpTrainBuffers& tb, const float* pts, const fl
 {
   hipError_t e     = tb.ensure(n);
   int        parts = 0;
-  if (e != hipSuccess || (e = train_launch(m, tb, pts, target, n, s, &parts, why)) != hipSuccess) return e;
+  if (e != hipSuccess || (e = train_launch(m, tb, pts, target, uint64_t(n), n, s, &parts, why)) != hipSuccess)
+    return e;
   hipLaunchKernelGGL(train_update_kernel<false>, dim3((kMaster + 255) / 256), dim3(256), 0, s, tb.part, parts, m.grad,
                      nullptr, nullptr, nullptr, 0.0f, 0.0f, 0.0f, nullptr, nullptr);
   return hipGetLastError();
 }
 
-bool mlp_check_train_schedule(uint64_t num_samples, int batch, std::string* why)
-{
-  const int        parts = mlp_train_blocks(batch); // what ensure(batch) allocates
-  std::vector<int> sizes{(int)std::min<uint64_t>(num_samples, (uint64_t)batch)};
-  if (num_samples > (uint64_t)batch && num_samples % (uint64_t)batch) sizes.push_back(int(num_samples % batch));
-  bool ok = true;
-  for (int n : sizes)
-    if (check_step(n, parts, why) != hipSuccess) ok = false;
-  return ok;
-}
-
-hipError_t mlp_step(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, int n, float lr, hipStream_t s,
-                    std::string* why)
+hipError_t mlp_step(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, uint64_t samples, int n, float lr,
+                    hipStream_t s, std::string* why)
 {
   int        parts = 0;
-  hipError_t e     = train_launch(m, tb, pts, target, n, s, &parts, why);
+  hipError_t e     = train_launch(m, tb, pts, target, samples, n, s, &parts, why);
   if (e != hipSuccess) return e;
   m.step++;
   const float bc1 = 1.0f / (1.0f - std::pow(0.9f, (float)m.step));
@@ -941,16 +910,15 @@ hipError_t mlp_fit(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* d
   hipError_t e = tb.ensure(batch);
   if (e != hipSuccess) return e;
   // Adam with a cosine learning-rate decay to 5% over all steps
-  const uint64_t spe   = (n + batch - 1) / batch;
+  const uint64_t spe   = train_steps(n, batch);
   const double   total = double(spe) * epochs;
-  uint64_t       k     = 0;
   float          last  = 0.0f;
   for (int ep = 0; ep < epochs; ep++) {
     if ((e = hipMemsetAsync(tb.loss, 0, sizeof(float), s)) != hipSuccess) return e;
-    for (uint64_t b = 0; b < n; b += batch, k++) {
-      const int   nb = int(std::min<uint64_t>(batch, n - b));
-      const float lr = float(lr0 * (0.05 + 0.95 * 0.5 * (1.0 + std::cos(M_PI * double(k) / total))));
-      if ((e = mlp_step(m, tb, pts + 3 * b, dist + b, nb, lr, s, why)) != hipSuccess) return e;
+    for (uint64_t k = 0; k < spe; k++) {
+      const TrainStep t  = train_step(n, batch, k);
+      const float     lr = float(lr0 * (0.05 + 0.95 * 0.5 * (1.0 + std::cos(M_PI * double(ep * spe + k) / total))));
+      if ((e = mlp_step(m, tb, pts + 3 * t.first, dist + t.first, n - t.first, t.rows, lr, s, why)) != hipSuccess) return e;
     }
     // the inference copy of the trained weights, before the last wait: callers go on to other streams
     if (ep + 1 == epochs && (e = mlp_sync_bf16(m, s)) != hipSuccess) return e;

@@ -15,6 +15,7 @@
 #pragma once
 
 #include "ebgpu_internal.hpp"
+#include "mlp_schedule.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -98,19 +99,16 @@ struct MlpTrainBuffers
   ~MlpTrainBuffers();
   hipError_t ensure(int batch);
 };
-int mlp_train_blocks(int n); // workgroups, hence partial gradients, of a step of n rows
 
 // Loss and full parameter gradient (into m.grad, master layout) for n points
 // with targets |d| (physical units). The summed loss is added to tb.loss[0].
 // On failure *why (nullable) names the check that failed.
 hipError_t mlp_loss_grad(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, int n,
                          hipStream_t s, std::string* why = nullptr);
-// Host-only: run the shape and extent checks of every launch of the training steps that
-// ebg_mlp_train enqueues for these sizes (full batches and the last, partial one). No GPU.
-bool mlp_check_train_schedule(uint64_t num_samples, int batch, std::string* why);
-// One training step: loss, gradient, Adam and the BF16 training copies (not the inference copy).
-hipError_t mlp_step(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, int n, float lr, hipStream_t s,
-                    std::string* why);
+// One training step over n rows of `samples` at pts and target: loss, gradient, Adam and the BF16 training
+// copies (not the inference copy).
+hipError_t mlp_step(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* target, uint64_t samples, int n, float lr,
+                    hipStream_t s, std::string* why);
 // Copy the gradient out in the public parameter order (device pointer, kMlpParams floats).
 hipError_t mlp_grad_public(const Mlp& m, float* out, hipStream_t s);
 

@@ -370,7 +370,7 @@ ebg_status ebg_scene_mlp_train(ebg_scene* sc, const ebg_mlp_opts* opts, float* l
     return fail(EBG_INVALID_ARG, "lr, box_scale, near_sigma or under_weight out of range");
   {
     std::string why;
-    if (!ebgpu::mlp_check_train_schedule(o.num_samples, o.batch, &why)) return fail(EBG_INVALID_ARG, why);
+    if (!ebgpu::check_train_schedule(o.num_samples, o.batch, o.num_samples, ebgpu::mlp_train_blocks(o.batch), &why)) return fail(EBG_INVALID_ARG, why);
   }
   hipStream_t s = static_cast<hipStream_t>(o.stream);
   ebgpu::Mlp& mlp = sc->mlp;

@@ -577,10 +577,11 @@ ebg_status ebg_mlp_set_params(ebg_mesh* mesh, const float* params);
  * learned bound, so a network is trained once per mesh. No counterpart in the reference. */
 ebg_status ebg_mlp_save(const ebg_mesh* mesh, const char* path);
 ebg_status ebg_mlp_load(ebg_mesh* mesh, const char* path);
-/* Host-only check (no GPU needed, nothing is allocated or launched): the launch shapes and the
- * largest index of every buffer access of each training step ebg_mlp_train would enqueue for
- * num_samples pairs in batches of `batch` (full batches and the last, partial one) against the
- * buffers it allocates. EBG_INVALID_ARG names the failing check. ebg_mlp_train runs it first. */
+/* Host-only check (no GPU needed, nothing is allocated or launched): the steps that ebg_mlp_train would
+ * enqueue for num_samples pairs in batches of `batch` (full batches and the last, partial one) cover the
+ * samples, and keep within the arrays whose sizes depend on the two (samples, targets, partial
+ * gradients). EBG_INVALID_ARG names the failing check. ebg_mlp_train runs it first, and checks each
+ * step against its arrays when it is enqueued. */
 ebg_status ebg_mlp_check_schedule(uint64_t num_samples, int32_t batch);
 /* Training loss summed over n <= 65536 device points with device targets |d| (d_loss, one
  * float, nullable) and its gradient (d_grad, ebg_mlp_param_count floats, parameter order
