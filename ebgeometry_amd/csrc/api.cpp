@@ -704,7 +704,7 @@ ebg_status ebg_query_sdf(const ebg_mesh* cm, const float* d_pts, uint64_t n, flo
   if (opts) o = *opts;
   if (o.learned_bound && !m->mlp.trained) return fail(EBG_NOT_READY, "learned bound requested but no network trained");
   std::lock_guard<std::recursive_mutex> lock(m->mu);
-  EBG_HIP(m->ws.ensure(n));
+  EBG_HIP(m->ws.ensure(n, ebgpu::WsUse::mesh));
   return ebgpu::query_pipeline(m, d_pts, n, d_dist, d_tri, o, m->ws.view(), true);
 }
 

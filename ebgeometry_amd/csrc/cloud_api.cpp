@@ -100,7 +100,7 @@ ebg_status ebg_cloud_knn(const ebg_cloud* cc, const float* d_pts, uint64_t n, ui
   std::lock_guard<std::mutex> lock(c->mu);
   const uint32_t*             idx = nullptr;
   if (o.presort && n > 1) {
-    EBG_HIP(c->ws.ensure(n));
+    EBG_HIP(c->ws.ensure(n, ebgpu::WsUse::sorted));
     EBG_HIP(ebgpu::presort(c->ws.view(), d_pts, n, s));
     idx = c->ws.perm.as<uint32_t>();
   }

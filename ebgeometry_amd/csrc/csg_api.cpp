@@ -308,7 +308,7 @@ ebg_status ebg_csg_query(const ebg_csg* cg, const float* d_pts, uint64_t n, floa
 
   std::lock_guard<std::mutex> lock(g->mu);
   Workspace&                  ws = g->ws;
-  EBG_HIP(ws.ensure(n));
+  EBG_HIP(ws.ensure(n, g->dev.walks ? ebgpu::WsUse::sorted : ebgpu::WsUse::lists));
   uint32_t* cnt = ws.counters();
   EBG_HIP(ebgpu::launch_fill_u32(cnt, 2, 0u, s));
   // only tree walks (BVH unions, meshes) gain from neighbouring queries in a wavefront; a program of

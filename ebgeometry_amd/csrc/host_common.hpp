@@ -101,29 +101,43 @@ struct WsView
 // their cost grid finds expensive.
 constexpr uint64_t kHandMaxQ = 1u << 20;
 
+// What a handle's calls use of its workspace (the same for all of them): the counters and the recheck
+// list; the presort's arrays and the seeded radii too; or, a mesh, everything.
+enum class WsUse
+{
+  lists,
+  sorted,
+  mesh
+};
+
 // Query workspace, grown on demand.
 struct Workspace
 {
   DevBuf   codes, codes_sorted, perm, sort_scratch, box, lists, seeds, sched, handed, rmask;
   uint64_t cap = 0;
 
-  hipError_t ensure(uint64_t n)
+  hipError_t ensure(uint64_t n, WsUse use)
   {
     if (n <= cap && cap) return hipSuccess;
     const uint64_t m = std::max<uint64_t>(n, 1024);
     hipError_t     e;
-    if ((e = codes.reserve(8 * m)) != hipSuccess) return e;
-    if ((e = codes_sorted.reserve(8 * m)) != hipSuccess) return e;
-    if ((e = perm.reserve(4 * m)) != hipSuccess) return e;
-    if ((e = sort_scratch.reserve(radix_sort_scratch_bytes(m))) != hipSuccess) return e;
-    if ((e = box.reserve(sizeof(double) * 6 * (kBboxParts + 1))) != hipSuccess) return e;
-    // recheck list, fallback list, 2 counters (+pad)
+    cap = 0; // should growing fail
+    // recheck list, fallback list, counters (+pad)
     if ((e = lists.reserve(8 * m + 256)) != hipSuccess) return e;
-    if ((e = seeds.reserve(4 * m)) != hipSuccess) return e;
-    if ((e = rmask.reserve(8 * mask_packets(m))) != hipSuccess) return e; // recheck lane mask per packet
-    // split packets: one flag byte per packet, the list of split packets, 64 result keys each
-    if ((e = sched.reserve(sched_early_offset(m) + 4 * (size_t)early_cap(m))) != hipSuccess) return e;
-    if ((e = handed.reserve(hand_bytes(std::min(m, kHandMaxQ)))) != hipSuccess) return e;
+    if (use != WsUse::lists) {
+      if ((e = codes.reserve(8 * m)) != hipSuccess) return e;
+      if ((e = codes_sorted.reserve(8 * m)) != hipSuccess) return e;
+      if ((e = perm.reserve(4 * m)) != hipSuccess) return e;
+      if ((e = sort_scratch.reserve(radix_sort_scratch_bytes(m))) != hipSuccess) return e;
+      if ((e = box.reserve(sizeof(double) * 6 * (kBboxParts + 1))) != hipSuccess) return e;
+      if ((e = seeds.reserve(4 * m)) != hipSuccess) return e;
+    }
+    if (use == WsUse::mesh) {
+      if ((e = rmask.reserve(8 * mask_packets(m))) != hipSuccess) return e; // recheck lane mask per packet
+      // split packets: one flag byte per packet, the list of split packets, 64 result keys each
+      if ((e = sched.reserve(sched_early_offset(m) + 4 * (size_t)early_cap(m))) != hipSuccess) return e;
+      if ((e = handed.reserve(hand_bytes(std::min(m, kHandMaxQ)))) != hipSuccess) return e;
+    }
     cap = m;
     return hipSuccess;
   }
@@ -183,6 +197,7 @@ struct Workspace
     v.counters     = counters();
     v.seeds        = seeds.as<float>();
     v.rmask        = rmask.as<uint64_t>();
+    if (!handed.p) return v; // not a mesh's
     v.heavy_flag   = heavy_flag();
     v.heavy_list   = heavy_list();
     v.heavy_keys   = heavy_keys();

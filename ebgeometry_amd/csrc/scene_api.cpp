@@ -291,7 +291,7 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
 
   std::lock_guard<std::mutex> lock(sc->mu);
   Workspace&                  ws = sc->ws;
-  EBG_HIP(ws.ensure(n));
+  EBG_HIP(ws.ensure(n, ebgpu::WsUse::sorted));
   if (!sc->ev0) {
     EBG_HIP(hipEventCreate(&sc->ev0));
     EBG_HIP(hipEventCreate(&sc->ev1));

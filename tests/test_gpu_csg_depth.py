@@ -32,3 +32,19 @@ def test_stack_depths(cuda, n, depth, transform):
     big = np.abs(ref) > 1e-6 * span
     assert np.array_equal(np.sign(v[big]), np.sign(ref[big]))
     assert np.abs(f.value(q, fp64_all=True) - ref).max() <= 1e-7 * span
+
+
+def test_programs_without_walks_reserve_no_sort(cuda):
+    """Nothing is sorted for them: 2M points take lists of 16 MB, and none of the presort's arrays
+    (72 MB)."""
+    import torch
+    f = nested(3, True)
+    f.value(torch.zeros(8, 3, device=cuda))  # the program's own arrays
+    q = torch.rand(2_000_000, 3, device=cuda)
+    out = torch.empty(2_000_000, device=cuda)
+    torch.cuda.synchronize()
+    before, _ = torch.cuda.mem_get_info()
+    f.value(q, out=out)
+    torch.cuda.synchronize()
+    after, _ = torch.cuda.mem_get_info()
+    assert before - after < 40 << 20
