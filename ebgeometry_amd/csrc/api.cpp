@@ -628,7 +628,6 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   // (100 queries: one launch of seven less, 2% of the call)
   const bool masks = recheck && narrow < 6;
   a.recheck_mask   = masks ? ws.rmask : nullptr;
-  a.fallback_list  = nullptr;
   a.fallback_count = cnt + 1;
   a.work           = reinterpret_cast<unsigned long long*>(o.work);
   a.pair_work      = reinterpret_cast<unsigned long long*>(o.pair_work);

@@ -441,7 +441,6 @@ ebg_status ebg_batch_plan_create(ebg_batch* b, const ebg_batch_item* items, uint
       r.box_inv[c]     = h > 0 ? float(256.0 / (2.0 * h)) : 0.0f;
     }
     r.recheck_abs = o.fp64_all ? INFINITY : float(o.recheck_eps * m->diag);
-    r.slack_abs   = float(1e-5 * m->diag);
     total += it.n;
   }
   if (total > 0xFFFFFFFFull) return fail(EBG_INVALID_ARG, "at most 2^32-1 queries per plan");

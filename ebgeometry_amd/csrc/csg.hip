@@ -211,14 +211,15 @@ __device__ __forceinline__ void csg_step(const CsgDev& g, const CsgParams<R>& q,
   if (WALKS && op == kCsgMesh) {
     const MeshDev md   = sload_record(g.meshes + q.n);
     R             best = R(INFINITY);
-    uint32_t      btri = kInvalid, bfeat = 0, c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+    uint32_t      btri = kInvalid, bfeat = 0;
     if constexpr (sizeof(R) == 4) {
+      uint32_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;
       Walk<NB> wk;
       wk.start(0u, 0u);
       wide_walk<NB, false, false>(md, wk, 0u, 0, L.x, L.y, L.z, need ? R(INFINITY) : R(-1), best, btri, c0, c1, c2, c3);
     }
     else
-      traverse<KM, NB, R, false, true>(md, L.x, L.y, L.z, need ? R(INFINITY) : R(-1), best, btri, bfeat, c0, c1, c2, c3);
+      traverse64<KM, NB>(md, L.x, L.y, L.z, need ? R(INFINITY) : R(-1), best, btri, bfeat);
     R val = R(INFINITY);
     if (need && btri != kInvalid) {
       if constexpr (sizeof(R) == 4) val = resolve32(md, btri, closest_feature(md, btri, L.x, L.y, L.z), best, L.x, L.y, L.z);

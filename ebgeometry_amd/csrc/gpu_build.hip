@@ -751,11 +751,9 @@ __global__ __launch_bounds__(256) void pack_kernel(const float* __restrict__ xyz
   put(r.sc, cen);
   r.sr    = float(rad * (1.0 + 1e-5) + 1e-7 * (dlen(cen) + rad));
   tris[i] = r;
-  float* sp = tsph + 8 * i;
+  float* sp = tsph + 4 * i;
   for (int c = 0; c < 3; c++) sp[c] = r.sc[c];
   sp[3] = r.sr;
-  for (int c = 0; c < 3; c++) sp[4 + c] = r.n[c];
-  sp[7] = float(-(double(r.n[0]) * r.v0[0] + double(r.n[1]) * r.v0[1] + double(r.n[2]) * r.v0[2]));
   for (int v = 0; v < 3; v++)
     for (int c = 0; c < 3; c++) tripos[12 * i + 3 * v + c] = xyz[3 * (size_t)tri[3 * f + v] + c];
   for (int c = 9; c < 12; c++) tripos[12 * i + c] = 0.0f;
@@ -1106,7 +1104,7 @@ ebg_status build_mesh_gpu_sah(const float* xyz, std::size_t nv, const uint32_t* 
   EBG_GB(out.tripos.reserve(48 * nt));
   EBG_GB(out.feat.reserve(32 * nt));
   EBG_GB(out.fn64.reserve(32 * nt));
-  EBG_GB(zeros<float>(out.tsph, 8 * (nt + kSphPad)));
+  EBG_GB(zeros<float>(out.tsph, 4 * (nt + kSphPad)));
   EBG_GB(d_area.reserve(8 * nt));
   EBG_GB(out.area_cdf.reserve(4 * (nt + 1)));
   EBG_GB(upload(d_hmax, std::vector<unsigned long long>{0ull}));

@@ -122,8 +122,8 @@ struct Workspace
     const uint64_t m = std::max<uint64_t>(n, 1024);
     hipError_t     e;
     cap = 0; // should growing fail
-    // recheck list, fallback list, counters (+pad)
-    if ((e = lists.reserve(8 * m + 256)) != hipSuccess) return e;
+    // recheck list, counters (+pad)
+    if ((e = lists.reserve(4 * m + 256)) != hipSuccess) return e;
     if (use != WsUse::lists) {
       if ((e = codes.reserve(8 * m)) != hipSuccess) return e;
       if ((e = codes_sorted.reserve(8 * m)) != hipSuccess) return e;
@@ -181,8 +181,7 @@ struct Workspace
     return h;
   }
   uint32_t* recheck_list() const { return lists.as<uint32_t>(); }
-  uint32_t* fallback_list() const { return lists.as<uint32_t>() + cap; }
-  uint32_t* counters() const { return lists.as<uint32_t>() + 2 * cap; } // as WsView::counters
+  uint32_t* counters() const { return lists.as<uint32_t>() + cap; } // as WsView::counters
 
   WsView view() const
   {

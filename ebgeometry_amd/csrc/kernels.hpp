@@ -23,8 +23,7 @@ struct QueryArgs
   // non-null: instead of appending to recheck_list, each packet pk (threads 64 pk ..) writes the
   // lane mask of its recheck queries here; launch_recheck_compact then builds the list
   uint64_t*           recheck_mask;
-  uint32_t*           fallback_list;  // queries whose seeded radius held no triangle
-  uint32_t*           fallback_count;
+  uint32_t*           fallback_count; // queries whose seeded radius held no triangle
   unsigned long long* work;      // [inner nodes, triangles] accumulated (null = not counted)
   unsigned long long* pair_work; // counting launches: [pairs, pair batches, culling loads, leaves screened]
   float               slack_abs; // FP64 recheck: bound = (|d| + slack_abs + slack_rel*|d|)^2
@@ -131,8 +130,7 @@ struct alignas(16) BatchItemDev
   float        box_lo[3];  // key box of the item's mesh: bin = (p - lo) * inv, 8 bits per axis
   float        box_inv[3];
   float        recheck_abs; // |d| below this is redone in FP64 (recheck_eps * mesh diagonal)
-  float        slack_abs;   // FP64 seed slack (1e-5 * mesh diagonal)
-  uint32_t     pad[2];
+  uint32_t     pad[3];
 };
 static_assert(sizeof(BatchItemDev) == 80, "BatchItemDev layout");
 

@@ -171,8 +171,7 @@ __device__ __forceinline__ void scene_traverse(const SceneDev& sc, R px, R py, R
           }
         }
         else
-          traverse<KM, NB, R, COUNT, true>(md, qx, qy, qz, near, best, btri, bfeat, c.n_inner, c.n_tris, c.w_inner,
-                                           c.w_tris);
+          traverse64<KM, NB>(md, qx, qy, qz, near, best, btri, bfeat);
         // Lanes that did not ask for this instance (near = -1) or found nothing that near still saw
         // triangles the wavefront evaluated, so their btri names some triangle but not their nearest.
         val = R(INFINITY);

@@ -1246,141 +1246,89 @@ __device__ __forceinline__ uint32_t closest_feature(const MeshDev& m, uint32_t t
   return f;
 }
 
-// R = float: FP32 pass on TriRec records. R = double: FP64 recheck on raw positions.
-// The walk starts at `start` (the root, or a subtree root of a split packet).
-template <int K, int NB, class R, bool COUNT, bool WMIN = (sizeof(R) == 8)>
-__device__ __forceinline__ void traverse_from(const MeshDev& m, const Entry& start, R px, R py, R pz, R bound, R& best,
-                                              uint32_t& btri, uint32_t& bfeat, uint32_t& n_inner, uint32_t& n_tris,
-                                              uint32_t& w_inner, uint32_t& w_tris)
+// The FP64 walk of the packed tree (mesh instances of scenes, mesh leaves of programs), over the raw
+// vertex positions. bound < 0: a lane without a query.
+template <int K, int NB>
+__device__ __forceinline__ void traverse64(const MeshDev& m, double px, double py, double pz, double bound, double& best,
+                                           uint32_t& btri, uint32_t& bfeat)
 {
   const Node<K>* __restrict__ nodes = static_cast<const Node<K>*>(m.nodes);
   LaneStack<NB>               st;
   st.init();
-  const int lane = __lane_id();
-  const int rep  = rep_lane(bound);
-  int       top  = 0;
-  st.put(top++, start);
+  const int rep = rep_lane(bound);
+  int       top = 0;
+  st.put(top++, Entry{0u, 0u, m.root_lo[0], m.root_lo[1], m.root_lo[2], m.root_hi[0], m.root_hi[1], m.root_hi[2]});
   // Stamp of the bounds: it advances after every leaf that tightened some lane's bound, and each
   // pushed entry carries it above the count's bits. An entry whose stamp is current was pushed
   // because some lane's box distance^2 was within its bound, and no bound has changed since, so
   // the test at the pop would pass again: it is skipped (the box fields are not even read). A
-  // skipped test can only cost work, never change a result; the counting walk always tests.
+  // skipped test can only cost work, never change a result.
   uint32_t stamp = 1u; // the start entry carries 0: always tested
 
   while (top > 0) {
     --top;
     const uint32_t ecnt = st.cnt_at(top);
-    bool           need = true;
-    if (COUNT || (ecnt >> kStampShift) != stamp) {
-      const Entry e   = st.get(top);
-      const R     d2e = box_d2<R>(px, py, pz, e.lx, e.ly, e.lz, e.hx, e.hy, e.hz);
-      need            = d2e <= bound;
-      if (ballot(need) == 0) continue;
+    if ((ecnt >> kStampShift) != stamp) {
+      const Entry  e   = st.get(top);
+      const double d2e = box_d2<double>(px, py, pz, e.lx, e.ly, e.lz, e.hx, e.hy, e.hz);
+      if (ballot(d2e <= bound) == 0) continue;
     }
     const uint32_t eref = st.ref_at(top), cnt = ecnt & kCountMask;
 
     if (cnt == 0u) {
-      if (COUNT) { n_inner += need ? 1u : 0u; w_inner++; }
-      push_children<K, NB, R, WMIN>(sload_record(nodes + uni(eref)), px, py, pz, bound, st, top, rep,
-                                    stamp << kStampShift);
+      push_children<K, NB, double, true>(sload_record(nodes + uni(eref)), px, py, pz, bound, st, top, rep,
+                                         stamp << kStampShift);
       // The capacity is the tree's exact worst case, computed at build time; should a walk ever
       // exceed it, the pushes beyond it were dropped: record that in the mesh's status word
       // (the host reports it) and go on with the entries that are held.
       if (top > 64 * NB) {
-        if (lane == 0 && m.status) atomicOr(m.status, kStatusStackOverflow);
+        if (__lane_id() == 0 && m.status) atomicOr(m.status, kStatusStackOverflow);
         top = 64 * NB;
       }
     }
     else {
       // leaf: a triangle is evaluated by the whole wavefront (keeping the minimum is exact for
-      // every lane) unless, for every lane, its bounding sphere or its plane lies beyond the
-      // lane's bound (both are lower bounds on the distance to the triangle). Inactive lanes
-      // have bound < 0, so rb is NaN and they never ask for a triangle. The culling data of 4
-      // triangles arrives in one scalar round trip (the array is padded past the last leaf),
-      // then each needed triangle record in one more, where a lower bound (the plane and the
-      // edge lines, tri_eval32_culled) is tested against the bound as tightened by the leaf's
-      // earlier triangles.
+      // every lane) unless, for every lane, its bounding sphere lies beyond the lane's bound.
+      // Inactive lanes have bound < 0, so rb is NaN and they never ask for a triangle. The spheres
+      // of 4 triangles arrive in one scalar round trip (the array is padded past the last leaf),
+      // then each needed triangle in one more.
       const uint32_t first  = uni(eref);
-      const R        bound0 = bound;
-      R              rb;
-      [[maybe_unused]] float cull = 0.0f; // FP32 distance-only walks: the lower-bound cull's limit
-      if constexpr (sizeof(R) == 4) {
-        rb = __builtin_amdgcn_sqrtf(bound) * 1.000001f; // 1-ulp hardware root, rounded up
-        cull = cull_band(bound, m.hmax);
-      }
-      else rb = sqrt(bound);
+      const double   bound0 = bound, rb = sqrt(bound);
       for (uint32_t c0 = 0; c0 < cnt; c0 += 4) {
-        const SWords<32> sp   = sload<32>(m.tsph + 8 * (size_t)(first + c0));
+        const SWords<16> sp   = sload<16>(m.tsph + 4 * (size_t)(first + c0));
         uint32_t         need = 0;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           if (c0 + i < cnt) {
-            const R    sx  = px - R(__uint_as_float(sp.w[8 * i])), sy = py - R(__uint_as_float(sp.w[8 * i + 1])),
-                       sz  = pz - R(__uint_as_float(sp.w[8 * i + 2]));
-            const R    lim = rb + R(__uint_as_float(sp.w[8 * i + 3]));
-            const bool in_s = sx * sx + sy * sy + sz * sz <= lim * lim;
-            bool       in_p = true;
-            if constexpr (sizeof(R) == 4) {
-              // the FP32 plane (rounded normal and offset) may misjudge by a few ulps of the
-              // coordinates; the FP64 pass, whose seed only just contains the minimum, skips it
-              const float pd = fmaf(__uint_as_float(sp.w[8 * i + 4]), px,
-                                    fmaf(__uint_as_float(sp.w[8 * i + 5]), py,
-                                         fmaf(__uint_as_float(sp.w[8 * i + 6]), pz, __uint_as_float(sp.w[8 * i + 7]))));
-              in_p = fabsf(pd) <= rb;
-            }
-            if (COUNT) n_tris += (in_s && in_p) ? 1u : 0u;
-            // two ballots straight from the compares (a ballot of their conjunction went
-            // through a VGPR)
-            need |= (ballot(in_s) & ballot(in_p)) ? (1u << i) : 0u;
+            const double sx = px - (double)__uint_as_float(sp.w[4 * i]), sy = py - (double)__uint_as_float(sp.w[4 * i + 1]),
+                         sz = pz - (double)__uint_as_float(sp.w[4 * i + 2]);
+            const double lim = rb + (double)__uint_as_float(sp.w[4 * i + 3]);
+            need |= ballot(sx * sx + sy * sy + sz * sz <= lim * lim) ? (1u << i) : 0u;
           }
         }
         while (need) {
           const uint32_t t = first + c0 + (uint32_t)__builtin_ctz(need);
           need &= need - 1u;
-          R        d2;
-          uint32_t f = 0;
-          if constexpr (sizeof(R) == 4) {
-            const TriRec rec = sload_record(m.tris + t);
-            if (!tri_eval32_culled(rec, px, py, pz, cull, d2)) continue;
-            if (COUNT) w_tris++;
-          }
-          else {
-            if (COUNT) w_tris++;
-            const SWords<12> pos = sload<12>(m.tripos + 12 * (size_t)t);
-            const SWords<8>  fn  = sload<8>(m.fn64 + 4 * (size_t)t);
-            double           fnd[4];
-            __builtin_memcpy(fnd, fn.w, sizeof(fnd));
-            float posf[12];
-            __builtin_memcpy(posf, pos.w, sizeof(posf));
-            tri_eval64(posf, fnd, px, py, pz, d2, f);
-          }
+          double           d2;
+          uint32_t         f   = 0;
+          const SWords<12> pos = sload<12>(m.tripos + 12 * (size_t)t);
+          const SWords<8>  fn  = sload<8>(m.fn64 + 4 * (size_t)t);
+          double           fnd[4];
+          __builtin_memcpy(fnd, fn.w, sizeof(fnd));
+          float posf[12];
+          __builtin_memcpy(posf, pos.w, sizeof(posf));
+          tri_eval64(posf, fnd, px, py, pz, d2, f);
           if (d2 < best) {
             best  = d2;
             btri  = t;
             bfeat = f;
             bound = d2 < bound ? d2 : bound; // bound stays min(bound, best)
-            if constexpr (sizeof(R) == 4) cull = cull_band(bound, m.hmax);
           }
         }
       }
       if (ballot(bound < bound0)) stamp++;
     }
   }
-  // FP32: classify the winning triangle's closest feature (per-lane record load)
-  if constexpr (sizeof(R) == 4) {
-    if (btri != kInvalid) {
-      float d2w;
-      tri_eval32<true>(m.tris[btri], px, py, pz, d2w, bfeat);
-    }
-  }
-}
-
-template <int K, int NB, class R, bool COUNT, bool WMIN = (sizeof(R) == 8)>
-__device__ __forceinline__ void traverse(const MeshDev& m, R px, R py, R pz, R bound, R& best, uint32_t& btri,
-                                         uint32_t& bfeat, uint32_t& n_inner, uint32_t& n_tris, uint32_t& w_inner, uint32_t& w_tris)
-{
-  const Entry root{0u, 0u, m.root_lo[0], m.root_lo[1], m.root_lo[2], m.root_hi[0], m.root_hi[1], m.root_hi[2]};
-  traverse_from<K, NB, R, COUNT, WMIN>(m, root, px, py, pz, bound, best, btri, bfeat, n_inner, n_tris, w_inner, w_tris);
 }
 
 } // namespace dev

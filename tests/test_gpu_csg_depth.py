@@ -35,7 +35,7 @@ def test_stack_depths(cuda, n, depth, transform):
 
 
 def test_programs_without_walks_reserve_no_sort(cuda):
-    """Nothing is sorted for them: 2M points take lists of 16 MB, and none of the presort's arrays
+    """Nothing is sorted for them: 2M points take a list of 8 MB, and none of the presort's arrays
     (72 MB)."""
     import torch
     f = nested(3, True)
@@ -47,4 +47,4 @@ def test_programs_without_walks_reserve_no_sort(cuda):
     f.value(q, out=out)
     torch.cuda.synchronize()
     after, _ = torch.cuda.mem_get_info()
-    assert before - after < 40 << 20
+    assert before - after < 24 << 20
