@@ -922,14 +922,11 @@ hipError_t mlp_fit(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* d
     }
     float sum = 0.0f;
     if ((e = hipMemcpyAsync(&sum, tb.loss, sizeof(float), hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
-    // the inference copy of the trained weights, before the last wait: callers go on to other streams
-    // (262,144 samples: 3.16 ms with it ahead of the loss, 3.13 behind)
-    if (ep + 1 == epochs && (e = mlp_sync_bf16(m, s)) != hipSuccess) return e;
     if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
     last = sum / float(n);
   }
   if (last_loss) *last_loss = last;
-  return hipSuccess;
+  return mlp_sync_bf16(m, s); // the inference copy of the trained weights
 }
 
 } // namespace ebgpu

@@ -122,7 +122,8 @@ hipError_t mlp_scene_samples(const PrimRec* prims, uint32_t num_prims, const flo
                              float box_scale, float sigma, uint64_t seed, uint64_t n, float* pts, hipStream_t s);
 // Train m on n (point, distance) pairs (device arrays): epochs passes in batches of `batch`,
 // Adam with a cosine learning-rate decay from lr0 to 5%; *last_loss = the last epoch's mean loss.
-// Returns when the weights, the inference copy among them, are written.
+// Returns when the master weights are written; the refresh of the inference copy is enqueued on s, and the
+// caller waits for it.
 hipError_t mlp_fit(Mlp& m, MlpTrainBuffers& tb, const float* pts, const float* dist, uint64_t n, int epochs, int batch,
                    float lr0, hipStream_t s, float* last_loss, std::string* why);
 
