@@ -1,14 +1,15 @@
 // C-ABI layer: handle lifecycle, device memory, the query pipeline.
 //
 // Query pipeline for one batch (all on the caller's stream, no host synchronisation):
-//   1. Morton presort: query bbox -> 63-bit codes -> stable radix sort -> permutation
+//   1. presort: query bbox -> 30-bit Hilbert keys -> stable radix sort -> permutation (not for calls
+//      of one query per wavefront)
 //   2. [learned bound] MLP forward -> per-query seeded cull radius (on a second stream,
 //      concurrently with step 1)
 //   3. FP32 packet traversal over the permutation (writes d, face id by query index)
 //      with the exactness fallback inside the same wavefront: queries whose seeded radius held
-//      no triangle walk the tree again unseeded
-//   4. FP64 traversal for queries with |d| < recheck_eps * diag (sign is ill-conditioned in
-//      FP32 there), seeded with |d32| + slack
+//      no triangle walk the tree again unseeded; long walks are split or handed on
+//   4. FP64 decision (band_walk) of the queries with |d| < recheck_eps * diag, whose sign is
+//      ill-conditioned in FP32, or of all when closest faces are asked for
 #include "host_common.hpp"
 #include "gpu_build.hpp"
 #include "mesh_build.hpp"
@@ -67,8 +68,6 @@ static double heavy_factor(uint64_t n) { return n >= (1u << 22) ? 6.0 : 3.0; }
 // 1.49 ms handed on, 5.2M 2.14 against 2.45 ms, 16M on 327,680 faces 5.03 against 5.63 ms.
 // Budgets and spreads: (200, 100, 32, 16) 0.93 ms, (150, 60, 48, 32) 0.87, (100, 60, 32, 32) 0.86 on
 // the 1M queries.
-
-
 
 // Subtree roots for split packets: breadth-first from the root, each interior entry replaced by
 // its children until there are at least `target` roots (leaves stay as they are).
@@ -926,7 +925,7 @@ ebg_status ebg_morton_sort(const uint64_t* d_codes, uint64_t n, uint32_t* d_perm
 } // extern "C"
 
 // ------------------------------------------------------------------------------------------
-// learned bound (training lives in mlp_train.hip)
+// learned bound (the kernels live in mlp.hip)
 // ------------------------------------------------------------------------------------------
 extern "C" {
 

@@ -2,7 +2,7 @@
 //
 // The queries of all items (item = one query array against one mesh) form one flat index
 // space. The pipeline:
-//   1. keys: item id in the high bits, the query's Morton code (relative to a box around the
+//   1. keys: item id in the high bits, the query's Hilbert index (in a box around the
 //      item's mesh) in the low bits; one stable radix sort then orders every item's queries along
 //      the curve and keeps the items apart;
 //   2. batch32: a packet = up to 64 consecutive (sorted) queries of one item, one per lane of a
@@ -10,9 +10,9 @@
 //      wavefront to (item, first query). The wavefront loads its item and mesh records with
 //      scalar loads and runs the same packet traversal as the single-mesh kernel, so every
 //      wavefront works on one mesh while different wavefronts of a launch work on different
-//      meshes;
-//   3. batch64: packets that hold near-surface results were listed (one entry per packet with
-//      the lane mask); one wavefront per listed packet redoes those lanes in FP64.
+//      meshes. In smaller plans long walks are handed on (batch_items, batch_resolve);
+//   3. batch64: the near-surface queries were listed in packet order; a wavefront takes up to 64
+//      list entries and decides them in FP64, one of their items after the other (band_walk).
 #include "kernels.hpp"
 #include "sfc_dev.hpp"
 #include "traverse_dev.hpp"

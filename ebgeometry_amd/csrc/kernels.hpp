@@ -26,7 +26,7 @@ struct QueryArgs
   uint32_t*           fallback_count; // queries whose seeded radius held no triangle
   unsigned long long* work;      // [inner nodes, triangles] accumulated (null = not counted)
   unsigned long long* pair_work; // counting launches: [pairs, pair batches, culling loads, leaves screened]
-  float               slack_abs; // FP64 recheck: bound = (|d| + slack_abs + slack_rel*|d|)^2
+  float               slack_abs; // FP64 pass of scenes: seed |v32| (1 + slack_rel) + slack_abs
   float               slack_rel;
   // queries per packet (wavefront): 64 >> narrow
   uint32_t            narrow;

@@ -84,7 +84,7 @@ constexpr int kInferBias  = 4 * kMlpHidden; // b1..b4 in LDS
 // Layer-1 K order of the fused kernel: K index 32 b + 8 g + e holds, for g < 3, the Fourier
 // feature sin(w_j x_g) with j = 8 b + e, and for g = 3 the raw coordinate x_e (b = 0, e < 3)
 // or zero padding (-1). A lane's frequencies are then compile-time constants and its coordinate
-// is one select per query; features are bitwise those of features_kernel.
+// is one select per query; features are bitwise those of the training kernel.
 __host__ __device__ constexpr int infer_feature(int b, int g, int e)
 {
   return g < 3 ? 3 + 3 * (8 * b + e) + g : (b == 0 && e < 3 ? e : -1);

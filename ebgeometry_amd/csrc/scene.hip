@@ -11,12 +11,13 @@
 // The packet scheme is the one of the mesh kernel: one query per lane, a wave-uniform stack in
 // VGPR lanes, records read with scalar loads. A mesh instance that some lane needs is walked by
 // the whole wavefront, unseeded (the sign of its value is only known once its nearest triangle
-// is); lanes that do not need it carry a negative bound and take no part. In FP32 that walk is the
-// mesh kernel's over cylinder bounds and triangle discs, a leaf's pairs spread over the wavefront:
-// with box bounds and every lane testing every triangle the FP32 pass of 4M points against 4096
-// spheres, 1024 boxes and 8 meshes of 20,480 faces took 4.14 ms, now 2.80 ms, and a walk that
-// starts from the running value for lanes outside the mesh's box measured the same. The FP64 pass
-// only asks whether an instance comes within the query's |value|: 1.85 -> 0.30 ms.
+// is); lanes that do not need it carry a negative bound and take no part. In FP32 that walk goes over
+// the mesh's cylinder bounds and triangle discs, and the whole wavefront evaluates each triangle that
+// some lane may need (wide_walk): with box bounds and spheres the FP32 pass of 4M points against 4096
+// spheres, 1024 boxes and 8 meshes of 20,480 faces took 4.14 ms, so 2.80 ms (and less since long walks
+// are handed on), and a walk that starts from the running value for lanes outside the mesh's box
+// measured the same. The FP64 pass only asks whether an instance comes within the query's |value|:
+// 1.85 -> 0.30 ms.
 //
 // FP32 pass for all queries; an FP64 pass (same traversal in double, FP64 primitive parameters,
 // FP64 triangle math) redoes queries with |v| below the recheck threshold, seeded with the FP32

@@ -269,8 +269,9 @@ ebg_status ebg_scene_bounds(const ebg_scene* sc, double* lo3, double* hi3, doubl
 }
 
 // Visits before an instance's walk is handed on (HandOn::budget), far fewer than in the mesh kernels: a
-// visited leaf costs the wavefront every triangle that some lane may need. 4M points: (150, 60) 1.87 ms,
-// (80, 30) 1.64, (30, 30) 1.49, (15, 15) 1.35, (10, 20) 1.39; 10,000 points: 1.47, 1.04, 0.73, 0.58, 0.53.
+// visited leaf costs the wavefront every triangle that some lane may need. 4M points, one scene: (150, 60)
+// 1.87 ms, (80, 30) 1.64, (30, 30) 1.49, (15, 15) 1.35, (10, 20) 1.39; 10,000 points: 1.47, 1.04, 0.73, 0.58,
+// 0.53. Other scenes drawn alike: 4M points 1.25 to 2.8 ms (median of ten 1.37), 10,000 points 0.52 to 0.69.
 constexpr uint32_t kSceneBudget[2] = {15, 15};
 // Handed-on walks have room as for this many queries at most (27 MB); beyond it wavefronts walk on.
 constexpr uint64_t kHandMaxRoom = 1u << 24;
@@ -325,7 +326,7 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
   const bool count = o.work != nullptr;
   // Long walks of mesh instances are handed on whatever the number of queries: a few packets inside a
   // mesh last as long as millions elsewhere (10,000 points 2.67 ms, 4M points 3.3 ms before, now 0.58
-  // and 1.35).
+  // and 1.35 on that scene).
   ebgpu::SceneSlot* slots = nullptr;
   if (!sc->meshes.empty() && !count && !seeds) {
     const uint64_t    room  = std::min(n, kHandMaxRoom);

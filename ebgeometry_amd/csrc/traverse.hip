@@ -25,7 +25,7 @@
 // (e_i x n).(p - v_i) agree, else the closest of the three vertices and of the edges with
 // t in (0,1); the sign comes from the pseudo-normal of the chosen feature. The FP32 pass tracks
 // squared distance and the feature; the sign is resolved once per query at the end. The FP64
-// pass redoes near-surface queries in double with the reference's exact formulas.
+// pass decides near-surface queries, and closest faces, in double with the reference's formulas (band_walk).
 #include "kernels.hpp"
 #include "traverse_dev.hpp"
 

@@ -506,12 +506,12 @@ __device__ __forceinline__ void wave_append(bool pred, uint32_t idx, uint32_t* l
 
 // Interior node: test the K child boxes and push the ones some lane needs, ranked so that the
 // farthest lies deepest and the nearest is popped next. The order key is the box distance seen
-// by the representative lane `rep` (see rep_lane) for dense, curve-sorted mesh packets: one
+// by the representative lane `rep` (see rep_lane) for dense, curve-sorted packets (clouds): one
 // readlane instead of a wavefront minimum (DPP and 4 readlanes per child), and as good an
-// order there (16M queries, 327,680-face displaced sphere: 1.6% fewer triangle evaluations, 5.7% less time). With WMIN the key is the
-// minimum over the lanes that need the child: better for packets whose lanes are spread (the
-// FP64 passes over sparse lists, CSG scenes with primitives the size of a packet). `tag` is OR-ed
-// into each pushed count word (the mesh walk's stamp, above the leaf count's bits).
+// order there. With WMIN the key is the minimum over the lanes that need the child: better for
+// packets whose lanes are spread (the FP64 passes over sparse lists, CSG scenes with primitives the
+// size of a packet). `tag` is OR-ed into each pushed count word (traverse64's stamp, above the leaf
+// count's bits).
 template <int K, int NB, class R, bool WMIN>
 __device__ __forceinline__ void push_children(const Node<K>& nd, R px, R py, R pz, R bound, LaneStack<NB>& st,
                                               int& top, int rep, uint32_t tag = 0u)

@@ -46,9 +46,6 @@ __global__ void f32_to_f64_kernel(const float* __restrict__ in, double* __restri
   if (i < n) out[i] = (double)in[i];
 }
 
-// Lattice points of a box of cells or nodes (x fastest, then y, then z: the layout of an AMReX
-// or Chombo FAB): point (i, j, k) = origin + (i, j, k) * spacing, each coordinate a separately
-// rounded FP64 product and sum, then rounded to FP32 (round to nearest even).
 // 64 points (4 x 4 x 4) in each cell of g.dims cells of size g.spacing, cell by cell
 __global__ void cell_points_kernel(GridSpec g, float* __restrict__ out)
 {
@@ -61,6 +58,9 @@ __global__ void cell_points_kernel(GridSpec g, float* __restrict__ out)
   out[3 * p + 2]   = (float)(g.origin[2] + ((double)k + ((l >> 4) + 0.5) / 4) * g.spacing[2]);
 }
 
+// Lattice points of a box of cells or nodes (x fastest, then y, then z: the layout of an AMReX
+// or Chombo FAB): point (i, j, k) = origin + (i, j, k) * spacing, each coordinate a separately
+// rounded FP64 product and sum, then rounded to FP32 (round to nearest even).
 __global__ void grid_points_kernel(GridSpec g, float* __restrict__ out)
 {
   const uint64_t n = g.dims[0] * g.dims[1] * g.dims[2];

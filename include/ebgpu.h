@@ -189,8 +189,11 @@ ebg_status ebg_query_sdf(const ebg_mesh* mesh, const float* d_pts, uint64_t n, f
  * array of 40 MiB per GPU, held from the library's first use on that GPU until the process ends,
  * which limits a call to n <= EBG_NOALLOC_MAX_QUERIES (larger n: EBG_INVALID_ARG). Every call on
  * one GPU shares that array: calls that overlap on one GPU (other streams, other threads) race
- * and must be serialised by the caller. Differences from ebg_query_sdf: the learned bound's network runs on opts->stream before the traversal (no second stream); the
- * traversal is not timed (ebg_mesh_last_traversal_ms keeps the previous value). */
+ * and must be serialised by the caller. Differences from ebg_query_sdf: a call of the largest size
+ * (2^20, presorted) splits long packets only once an ebg_query_sdf call of at least that size, or a
+ * training of the bound network on at least 2^14 samples, has built the mesh's cost grid; the learned bound's network runs on
+ * opts->stream before the traversal (no second stream); the traversal is not timed
+ * (ebg_mesh_last_traversal_ms keeps the previous value). */
 #define EBG_NOALLOC_MAX_QUERIES 1048576u
 ebg_status ebg_query_sdf_noalloc(const ebg_mesh* mesh, const float* d_pts, uint64_t n, float* d_dist,
                                  uint32_t* d_tri, const ebg_query_opts* opts);

@@ -89,10 +89,10 @@ def test_mesh_create_validates_without_gpu():
 
 
 def test_training_schedule_checks_pass_without_a_gpu():
-    """Every launch of the training steps ebg_mlp_train enqueues (shapes, split-K chunks and the
-    largest index of each buffer access) is checked on the host for the schedules the tests and
-    the bench run: the learned-bound test's 400,000 pairs in batches of 2,048 (last batch 640),
-    the bench's 4M in 4,096, the gradient tests' single batches of 1,000 and 4,100 rows."""
+    """The training steps ebg_mlp_train enqueues (they cover the samples and keep within the arrays
+    sized for them) are checked on the host for the schedules the tests and the bench run: the
+    learned-bound test's 400,000 pairs in batches of 2,048 (last batch 640), the bench's 4M in
+    4,096, the gradient tests' single batches of 1,000 and 4,100 rows."""
     from ebgeometry_amd import _lib
     L = _lib.lib()
     for n, b in [(400_000, 2048), (4_000_000, 4096), (1000, 1024), (4100, 4100), (65536, 65536), (100, 32),
