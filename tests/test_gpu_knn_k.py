@@ -10,13 +10,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("k", list(range(1, 17)))
+@pytest.mark.parametrize("branching", [4, 8])
 @pytest.mark.parametrize("points,n,leaf", [(16, 1, 16), (17, 63, 1), (900, 65, 7), (5000, 500, 8)])
-def test_every_k(cuda, k, points, n, leaf):
+def test_every_k(cuda, k, points, n, leaf, branching):
     rng = np.random.default_rng(points + k)
     P = rng.normal(size=(points, 3)).astype(np.float32)
     P[1::5] = P[0::5][: len(P[1::5])]  # equal points: equal distances
     Q = np.concatenate([P[: n // 2], rng.normal(size=(n - n // 2, 3)).astype(np.float32)])
-    c = PointCloudBVH(P, leaf_size=leaf)
+    c = PointCloudBVH(P, leaf_size=leaf, branching=branching)
     idx, d2 = c.knn(Q, k)
     _, rd = cloud_ref.knn(P, Q, k)
     check_knn(P, Q, idx, d2, rd, f"k={k}")
