@@ -187,6 +187,7 @@ static ebg_status build_walk(ebg_mesh* m, const ebgpu::PackedMesh& pm)
                                       " entries (max 256); use a smaller branching factor");
   if (m->wbanks == 3) m->wbanks = 4;
   m->walk_deep_need = wt.deep_need;
+  m->walk_visits    = wt.visits;
   const std::vector<ebgpu::SplitRoot> roots = split_frontier(wt, kSplitRoots);
   EBG_HIP(upload(m->split_roots, roots));
   m->num_split_roots = uint32_t(roots.size());
@@ -539,7 +540,7 @@ ebg_status query_pipeline(ebg_mesh* m, const float* d_pts, uint64_t n, float* d_
   const bool timed = m->ev0 && may_alloc;
   // counting launches run unsplit: the counters describe the plain traversal's own work
   const bool face        = d_tri != nullptr;
-  const bool hand_on     = !o.work && n < kHandMaxQ;
+  const bool hand_on     = !o.work && n < kHandMaxQ && can_hand_on(m->walk_visits, kHandBudget[0]);
   const bool heavy_first = o.presort && n >= kHandMaxQ && !o.work && (may_alloc || m->grid_ready);
   m->last_split_cap      = face ? 0 : heavy_first ? Workspace::heavy_cap(n)
                                        : (hand_on && o.presort && n >= kHeavyMinQ ? ws.hand.slot_cap : 0);

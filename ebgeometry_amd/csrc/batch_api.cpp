@@ -22,6 +22,7 @@ struct ebg_batch
   std::vector<ebg_mesh*> meshes; // owned
   DevBuf                 meshdev;
   int                    K = 4, leaf = 8, banks = 1, wbanks = 1, deep_need = 1;
+  uint64_t               walk_visits = 0; // the most of its meshes
   bool                   tuned = false;
   double                 tune_ms[4]{-1, -1, -1, -1};
   double                 build_seconds = 0;
@@ -358,6 +359,7 @@ ebg_status ebg_batch_create(const float* const* xyz, const uint64_t* nv, const u
     b->banks     = std::max(b->banks, b->meshes[i]->banks);
     b->wbanks    = std::max(b->wbanks, b->meshes[i]->wbanks);
     b->deep_need = std::max(b->deep_need, b->meshes[i]->walk_deep_need);
+    b->walk_visits = std::max(b->walk_visits, b->meshes[i]->walk_visits);
     b->num_triangles += b->meshes[i]->nt;
   }
   const hipError_t e = upload(b->meshdev, md);
@@ -489,7 +491,7 @@ ebg_status ebg_batch_plan_create(ebg_batch* b, const ebg_batch_item* items, uint
   if ((e = p->rmask.reserve(8 * std::max<uint64_t>(p->num_packets, 1))) != hipSuccess) return bail(e, "recheck");
   if ((e = p->recheck.reserve(4 * (p->fp64 ? cap : 1))) != hipSuccess) return bail(e, "recheck");
   if ((e = p->counter.reserve(256)) != hipSuccess) return bail(e, "counter");
-  p->hand = total < kHandMaxTotal && !p->work;
+  p->hand = total < kHandMaxTotal && !p->work && ebgpu::can_hand_on(b->walk_visits, ebgpu::kHandBudget[0]);
   if (p->hand && (e = p->handed.reserve(ebgpu::Workspace::hand_bytes(total))) != hipSuccess) return bail(e, "hand-on lists");
   if ((e = hipEventCreate(&p->ev0)) != hipSuccess || (e = hipEventCreate(&p->ev1)) != hipSuccess)
     return bail(e, "events");

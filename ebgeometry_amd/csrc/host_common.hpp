@@ -271,6 +271,7 @@ struct ebg_mesh
   ebgpu::DevBuf          wnodes, tdisc, frames;
   ebgpu::DevBuf          nfirst; // MeshDev::nfirst
   int                    wbanks = 1, walk_deep_need = 1; // WalkTree::deep_need
+  uint64_t               walk_visits = 0;                // WalkTree::visits
   // cost grid of the split schedule (built at the first large presorted query): per cell, the
   // work of a packet of 64 queries spread over the cell
   ebgpu::DevBuf          cost_grid;

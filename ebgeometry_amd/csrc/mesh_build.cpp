@@ -752,6 +752,9 @@ void build_walk_tree(const PackedMesh& pm, float scale, WalkTree& out)
   if (pm.K == 4) run(std::integral_constant<int, 4>{});
   else run(std::integral_constant<int, 8>{});
   out.stack_need = 1 + std::max(0, need);
+  out.visits     = out.nodes.size();
+  for (const WalkNode& n : out.nodes)
+    for (uint32_t c : n.cnt) out.visits += c != kInvalid && (c & (kBoxChild - 1u)) != 0u;
 }
 
 namespace {

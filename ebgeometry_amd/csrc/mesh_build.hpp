@@ -112,6 +112,7 @@ struct WalkTree
   std::vector<WalkNode> nodes;
   std::vector<uint32_t> range;
   int                   stack_need = 0;
+  uint64_t              visits     = 0; // of a walk that visits every node and leaf
   int                   deep_need  = 1; // stack of a walk from any one entry two levels below the root
 };
 void build_walk_tree(const PackedMesh& pm, float scale, WalkTree& out);

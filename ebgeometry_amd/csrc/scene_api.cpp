@@ -26,6 +26,7 @@ struct ebg_scene
   ebgpu::SceneDev        dev{};
   int                    KM = 4, banks = 1, stack_need = 0;
   int                    deep_need = 1; // of its meshes: WalkTree::deep_need
+  uint64_t               walk_visits = 0; // the most of its meshes
   std::size_t            num_prims = 0, num_nodes = 0;
   double                 lo[3]{}, hi[3]{}, diag = 0;
   std::mutex             mu;
@@ -86,13 +87,15 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
   const int leaf = o.leaf_size ? o.leaf_size : 4;
   if (leaf < 1 || leaf > ebgpu::kMaxLeaf) return fail(EBG_INVALID_ARG, "leaf_size must be 1..16");
 
-  int KM = 0, mesh_banks = 1, deep_need = 1;
+  int      KM = 0, mesh_banks = 1, deep_need = 1;
+  uint64_t walk_visits = 0;
   for (uint64_t j = 0; j < num_meshes; j++) {
     if (!meshes[j]) return fail(EBG_INVALID_ARG, "null mesh handle");
     if (KM && meshes[j]->K != KM) return fail(EBG_INVALID_ARG, "all scene meshes must have the same branching");
     KM         = meshes[j]->K;
     mesh_banks = std::max({mesh_banks, meshes[j]->banks, meshes[j]->wbanks});
     deep_need  = std::max(deep_need, meshes[j]->walk_deep_need);
+    walk_visits = std::max(walk_visits, meshes[j]->walk_visits);
   }
   if (!KM) KM = 4;
 
@@ -218,6 +221,7 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
   sc->KM         = KM;
   sc->banks      = banks;
   sc->deep_need  = deep_need;
+  sc->walk_visits = walk_visits;
   sc->stack_need = wb.stack_need;
   sc->num_prims  = n;
   sc->num_nodes  = wb.num_nodes;
@@ -328,7 +332,7 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
   // mesh last as long as millions elsewhere (10,000 points 2.67 ms, 4M points 3.3 ms before, now 0.58
   // and 1.35 on that scene).
   ebgpu::SceneSlot* slots = nullptr;
-  if (!sc->meshes.empty() && !count && !seeds) {
+  if (!count && !seeds && ebgpu::can_hand_on(sc->walk_visits, kSceneBudget[0])) {
     const uint64_t    room  = std::min(n, kHandMaxRoom);
     const std::size_t lists = Workspace::hand_bytes(room);
     EBG_HIP(sc->handed.reserve(lists + sizeof(ebgpu::SceneSlot) * Workspace::hand_slots(room)));

@@ -19,4 +19,9 @@ inline int hand_spread(int stage, int capacity, int deep_need)
   return std::max(0, std::min(kHandSpread[stage], capacity - 1 - deep_need));
 }
 
+// Whether a walk of a tree of `visits` nodes and leaves can use up its budget. If not, its calls need none of
+// the launches that take up what was handed on (100 queries on 80 faces: 61 us with them, 46 without; 1
+// query 63 and 37).
+inline bool can_hand_on(uint64_t visits, uint32_t budget) { return visits > budget; }
+
 } // namespace ebgpu

@@ -1,6 +1,7 @@
 """How deep a walk's stack gets that is spread to be handed on, finds no room and goes on (hand_spread,
 WalkTree::deep_need): over the walk trees of deep meshes with every child reached, as next to a sphere's
-centre, it stays within the capacity that the tree's mesh is given, which the full spread does not."""
+centre, it stays within the capacity that the tree's mesh is given, which the full spread does not. And
+which trees' walks can use up a budget (WalkTree::visits)."""
 import os
 import shutil
 import subprocess
@@ -20,7 +21,7 @@ struct TreeWalk
 {
   const WalkTree&   t;
   std::vector<Item> st; // the top last
-  size_t            deepest = 0;
+  size_t            deepest = 0, visits = 0;
 
   void start(Item e) { st.assign(1, e); }
   void push_children(uint32_t node)
@@ -34,6 +35,7 @@ struct TreeWalk
     while (!st.empty() && budget--) {
       const Item e = st.back();
       st.pop_back();
+      visits++;
       if (e.second == 0u) push_children(e.first);
     }
   }
@@ -90,6 +92,11 @@ int main()
     std::printf("K=%d leaf=%d: stack_need %d deep_need %d spread %d %d: %zu (full spread %zu) of %d\n", K, leaf,
                 t.stack_need, t.deep_need, spread[0], spread[1], d, full, capacity);
     CHECK(t.deep_need <= t.stack_need && spread[0] > 0);
+    TreeWalk all{t};
+    all.start({0u, 0u});
+    all.walk(~0u);
+    CHECK(all.visits == t.visits && all.deepest <= size_t(t.stack_need));
+    CHECK(can_hand_on(t.visits, uint32_t(t.visits) - 1) && !can_hand_on(t.visits, uint32_t(t.visits)));
     CHECK(d <= size_t(capacity));
     over += full > size_t(capacity);
   }
