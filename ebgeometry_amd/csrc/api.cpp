@@ -193,7 +193,6 @@ static ebg_status build_walk(ebg_mesh* m, const ebgpu::PackedMesh& pm)
   m->num_split_roots = uint32_t(roots.size());
 
   std::vector<uint32_t> small, large;
-  std::vector<float>    none(8 * 4 * wt.nodes.size(), -1.0f);
   for (uint32_t i = 0; i < 4 * wt.nodes.size(); i++) {
     const uint32_t c = wt.range[2 * i + 1] - wt.range[2 * i];
     if (c) (c > ebgpu::kWalkLarge ? large : small).push_back(i);
@@ -203,7 +202,8 @@ static ebg_status build_walk(ebg_mesh* m, const ebgpu::PackedMesh& pm)
   EBG_HIP(upload(range, wt.range));
   EBG_HIP(upload(ls, small));
   EBG_HIP(upload(ll, large));
-  EBG_HIP(upload(discs, none));
+  EBG_HIP(discs.reserve(4 * 8 * 4 * wt.nodes.size()));
+  EBG_HIP(ebgpu::launch_fill_u32(discs.as<uint32_t>(), 8 * 4 * wt.nodes.size(), 0xBF800000u, nullptr)); // -1
   EBG_HIP(upload(off, std::vector<uint32_t>(16, 0u)));
   EBG_HIP(m->frames.reserve(sizeof(ebgpu::FrameRec) * std::max<uint64_t>(m->nt, 1)));
   EBG_HIP(m->tdisc.reserve(sizeof(ebgpu::TriDisc) * (m->nt + ebgpu::kSphPad)));

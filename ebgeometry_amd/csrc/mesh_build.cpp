@@ -672,31 +672,34 @@ struct WalkEmitter
     uint32_t first = kInvalid, last = 0, count = 0; // count: triangles in the subtree
   };
 
-  std::vector<int> children(uint32_t i) const
+  // A walk node over all children of in[i].
+  uint32_t emit(uint32_t i, int level, Range& all, int& need)
   {
-    std::vector<int> c;
+    int kids[K], m = 0;
     for (int k = 0; k < K; k++)
-      if (in[i].cnt[k] != kInvalid) c.push_back(k);
-    return c;
+      if (in[i].cnt[k] != kInvalid) kids[m++] = k;
+    return emit(i, kids, m, level, all, need);
   }
 
-  // A walk node over the children kids of in[i], `level` levels below the root; returns its index, the
+  // A walk node over the m children kids of in[i], `level` levels below the root; returns its index, the
   // triangles below it and the stack its walk needs beyond its own entry.
-  uint32_t emit(uint32_t i, const std::vector<int>& kids, int level, Range& all, int& need)
+  uint32_t emit(uint32_t i, const int* kids, int m, int level, Range& all, int& need)
   {
     const uint32_t me = uint32_t(out.nodes.size());
     out.nodes.emplace_back();
     out.range.resize(8 * out.nodes.size(), 0u);
     WalkNode nd{};
     for (int k = 0; k < 4; k++) nd.cnt[k] = kInvalid;
-    const int m = int(kids.size()), slots = std::min(m, 4);
+    const int slots = std::min(m, 4);
     int       deepest = 0;
     for (int k = 0; k < slots; k++) {
       // slots share the children evenly, in order
-      const std::vector<int> part(kids.begin() + k * m / slots, kids.begin() + (k + 1) * m / slots);
-      const Node<K>&         n = in[i];
-      float                  lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-      for (int c : part) {
+      const int*     part  = kids + k * m / slots;
+      const int      parts = (k + 1) * m / slots - k * m / slots;
+      const Node<K>& n     = in[i];
+      float          lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+      for (int p = 0; p < parts; p++) {
+        const int   c    = part[p];
         const float a[3] = {n.lox[c], n.loy[c], n.loz[c]}, b[3] = {n.hix[c], n.hiy[c], n.hiz[c]};
         for (int x = 0; x < 3; x++) {
           lo[x] = std::min(lo[x], a[x]);
@@ -709,15 +712,14 @@ struct WalkEmitter
       }
       Range r;
       int   deep = 0;
-      if (part.size() == 1 && n.cnt[part[0]] != 0u) {
+      if (parts == 1 && n.cnt[part[0]] != 0u) {
         nd.ref[k] = n.ref[part[0]];
         nd.cnt[k] = n.cnt[part[0]] | kBoxChild;
         r         = {nd.ref[k], nd.ref[k] + n.cnt[part[0]], n.cnt[part[0]]};
       }
       else {
         nd.cnt[k] = kBoxChild;
-        nd.ref[k] = part.size() == 1 ? emit(n.ref[part[0]], children(n.ref[part[0]]), level + 1, r, deep)
-                                     : emit(i, part, level + 1, r, deep);
+        nd.ref[k] = parts == 1 ? emit(n.ref[part[0]], level + 1, r, deep) : emit(i, part, parts, level + 1, r, deep);
       }
       deepest = std::max(deepest, deep);
       if (r.count == r.last - r.first) {
@@ -747,7 +749,9 @@ void build_walk_tree(const PackedMesh& pm, float scale, WalkTree& out)
     constexpr int         KK = decltype(tag)::value;
     WalkEmitter<KK>       e{reinterpret_cast<const Node<KK>*>(pm.nodes.data()), scale, out};
     typename WalkEmitter<KK>::Range all;
-    e.emit(0, e.children(0), 0, all, need);
+    out.nodes.reserve(std::size_t(KK / 2) * pm.num_nodes);
+    out.range.reserve(8 * std::size_t(KK / 2) * pm.num_nodes);
+    e.emit(0, 0, all, need);
   };
   if (pm.K == 4) run(std::integral_constant<int, 4>{});
   else run(std::integral_constant<int, 8>{});
