@@ -98,7 +98,8 @@ __device__ __forceinline__ void batch_finish(const BatchArgs& a, const BatchItem
   const bool found = active && btri != kInvalid;
   float      d     = 0.0f;
   if (found) {
-    d            = resolve32(m, btri, closest_feature(m, btri, px, py, pz), best, px, py, pz);
+    const uint32_t feat = closest_feature(m, btri, px, py, pz, best);
+    d            = resolve32(m, btri, feat, best, px, py, pz);
     it.out[qi]   = d;
     if (it.tri) it.tri[qi] = m.tris[btri].face;
   }

@@ -144,7 +144,8 @@ __device__ __forceinline__ void sdf32_packet(const MeshDev& m, const QueryArgs& 
   best *= m.inv_scale * m.inv_scale;
   float d = 0.0f;
   if (found) {
-    d = resolve32(m, btri, closest_feature(m, btri, px, py, pz), best, px, py, pz);
+    const uint32_t feat = closest_feature(m, btri, px, py, pz, best);
+    d                   = resolve32(m, btri, feat, best, px, py, pz);
     a.out_d[qi] = d;
     if (a.out_tri) a.out_tri[qi] = m.tris[btri].face;
   }
@@ -323,8 +324,9 @@ __global__ __launch_bounds__(256) void sdf32_resolve_kernel(const MeshDev m, con
       const uint32_t           t   = (uint32_t)key;
       if (t != kInvalid) {
         const float px = a.pts[3 * (size_t)qi], py = a.pts[3 * (size_t)qi + 1], pz = a.pts[3 * (size_t)qi + 2];
-        const float d2 = __uint_as_float((uint32_t)(key >> 32)) * (m.inv_scale * m.inv_scale); // the walk's, unscaled
-        d              = resolve32(m, t, closest_feature(m, t, px, py, pz), d2, px, py, pz);
+        float          d2   = __uint_as_float((uint32_t)(key >> 32)) * (m.inv_scale * m.inv_scale); // the walk's, unscaled
+        const uint32_t feat = closest_feature(m, t, px, py, pz, d2);
+        d              = resolve32(m, t, feat, d2, px, py, pz);
         a.out_d[qi]    = d;
         if (a.out_tri) a.out_tri[qi] = m.tris[t].face;
         found = true;

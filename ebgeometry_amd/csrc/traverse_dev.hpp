@@ -1237,13 +1237,20 @@ __device__ __forceinline__ float signed_distance64(const MeshDev& m, uint32_t t,
 }
 
 // The closest feature of the winning triangle (per-lane record load), at the point in the mesh's
-// own units.
-__device__ __forceinline__ uint32_t closest_feature(const MeshDev& m, uint32_t t, float px, float py, float pz)
+// own units. d2w: the walk's distance^2, in those units; where it overflowed in the walk's scaled ones
+// (a small mesh's query some 10^19 of its sizes away: every triangle is the same there) it is replaced.
+__device__ __forceinline__ uint32_t closest_feature(const MeshDev& m, uint32_t t, float px, float py, float pz, float& d2w)
 {
   float    d2;
   uint32_t f;
   tri_eval32<true>(m.tris[t], px, py, pz, d2, f);
+  d2w = d2w < INFINITY ? d2w : d2;
   return f;
+}
+__device__ __forceinline__ uint32_t closest_feature(const MeshDev& m, uint32_t t, float px, float py, float pz)
+{
+  float d2 = 0.0f;
+  return closest_feature(m, t, px, py, pz, d2);
 }
 
 // The FP64 walk of the packed tree (mesh instances of scenes, mesh leaves of programs), over the raw
