@@ -27,6 +27,7 @@ struct ebg_scene
   int                    KM = 4, banks = 1, stack_need = 0;
   int                    deep_need = 1; // of its meshes: WalkTree::deep_need
   uint64_t               walk_visits = 0; // the most of its meshes
+  uint64_t               instances   = 0; // mesh primitives
   std::size_t            num_prims = 0, num_nodes = 0;
   double                 lo[3]{}, hi[3]{}, diag = 0;
   std::mutex             mu;
@@ -88,7 +89,7 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
   if (leaf < 1 || leaf > ebgpu::kMaxLeaf) return fail(EBG_INVALID_ARG, "leaf_size must be 1..16");
 
   int      KM = 0, mesh_banks = 1, deep_need = 1;
-  uint64_t walk_visits = 0;
+  uint64_t walk_visits = 0, instances = 0;
   for (uint64_t j = 0; j < num_meshes; j++) {
     if (!meshes[j]) return fail(EBG_INVALID_ARG, "null mesh handle");
     if (KM && meshes[j]->K != KM) return fail(EBG_INVALID_ARG, "all scene meshes must have the same branching");
@@ -138,6 +139,7 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
       }
     }
     else if (p.type == EBG_PRIM_MESH) {
+      instances++;
       if (p.mesh < 0 || uint64_t(p.mesh) >= num_meshes) return fail(EBG_INVALID_ARG, where + "mesh index out of range");
       if (!(p.scale > 0.0)) return fail(EBG_INVALID_ARG, where + "mesh scale must be > 0");
       double M[9];
@@ -222,6 +224,7 @@ ebg_status ebg_scene_create(const ebg_prim* prims, uint64_t n, ebg_mesh* const* 
   sc->banks      = banks;
   sc->deep_need  = deep_need;
   sc->walk_visits = walk_visits;
+  sc->instances   = instances;
   sc->stack_need = wb.stack_need;
   sc->num_prims  = n;
   sc->num_nodes  = wb.num_nodes;
@@ -330,9 +333,10 @@ ebg_status ebg_scene_query(const ebg_scene* csc, const float* d_pts, uint64_t n,
   const bool count = o.work != nullptr;
   // Long walks of mesh instances are handed on whatever the number of queries: a few packets inside a
   // mesh last as long as millions elsewhere (10,000 points 2.67 ms, 4M points 3.3 ms before, now 0.58
-  // and 1.35 on that scene).
+  // and 1.35 on that scene). Each packet may hand each instance on once; the counter has to hold all that ask.
   ebgpu::SceneSlot* slots = nullptr;
-  if (!count && !seeds && ebgpu::can_hand_on(sc->walk_visits, kSceneBudget[0])) {
+  if (!count && !seeds && ebgpu::can_hand_on(sc->walk_visits, kSceneBudget[0]) &&
+      ebgpu::hand_counts_fit((n + 63) / 64 * sc->instances)) {
     const uint64_t    room  = std::min(n, kHandMaxRoom);
     const std::size_t lists = Workspace::hand_bytes(room);
     EBG_HIP(sc->handed.reserve(lists + sizeof(ebgpu::SceneSlot) * Workspace::hand_slots(room)));

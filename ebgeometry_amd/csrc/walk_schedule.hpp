@@ -24,4 +24,7 @@ inline int hand_spread(int stage, int capacity, int deep_need)
 // query 63 and 37).
 inline bool can_hand_on(uint64_t visits, uint32_t budget) { return visits > budget; }
 
+// Whether HandOn's 32-bit counter of slots can count `walks` requests (all of them, granted or not).
+inline bool hand_counts_fit(uint64_t walks) { return walks <= 0xFFFFFFFFull; }
+
 } // namespace ebgpu

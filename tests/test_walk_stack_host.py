@@ -102,6 +102,7 @@ int main()
   }
   CHECK(over >= 2); // the trees are deep enough to tell
   CHECK(hand_spread(0, 64, 64) == 0 && hand_spread(0, 64, 1) == kHandSpread[0]);
+  CHECK(hand_counts_fit(0xFFFFFFFFull) && !hand_counts_fit(0x100000000ull)); // 2^32 points in 64 instances
   std::printf("stack bound checked\n");
   return 0;
 }
